@@ -150,6 +150,9 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * channels a multiple of 64, rows of at most 63 pixels; any other convolution runs tiling 1 for it).  The patch
  * kernel adds up channel block by channel block, the others tap by tap: results agree to rounding, not bit for bit.
  * 6 / 7 = tilings 1 / 2 with two LDS tiles in flight instead of three (more workgroups per CU).
+ * 15 - 20 split the reduction over the wavefronts of a workgroup, for outputs of few tiles: 15 / 16 = 32x32 over four /
+ * eight wavefronts, 17 / 20 = 64x32 over four / eight, 18 / 19 = 64x64 with one / two workgroups per CU (input channels a
+ * multiple of 64 bytes; anything else runs tiling 2 for them).  Partial sums are added in the order of the wavefronts.
  * c_logical: input channels that carry data when C is zero-padded to a chunk (0 = C); it only enters the
  * algorithmic-work figure the profiler reports, never the arithmetic. */
 int tch_conv2d_fwd(tch_context* ctx, int dtype, const void* x, const void* w, void* y, const void* add,

@@ -319,23 +319,22 @@ __device__ inline void store_floats(float* dst, const float* v) {
 //                  sum(g * xhat), xhat = (bn_x - mean) * invstd: the two reductions of the
 //                  BatchNorm backward.
 // ---------------------------------------------------------------------------
-template <typename T, int MODE, int WM, int WN, int TM, int TN>
-__device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0,
-                                   int tile_m) {
+// The accumulators reach it through `walk(fin)`, which calls fin(visit, row of the tile, column of the tile, E values) for
+// every chunk this thread stores (column chunk tid % CH, so `row_of(visit)` alone names it beforehand).
+// NT of the workgroup's BLOCK threads store something; the others only keep the barriers company.
+template <typename T, int MODE, int BN, int NT, int BLOCK, int VISITS, int STAGE_BYTES, typename RowOf, typename Walk>
+__device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, int m0, int n0, int tile_m, RowOf row_of, Walk walk) {
   constexpr int E = Elem<T>::kPerChunk;
-  constexpr int BN = WN * TN * 32;
-  constexpr int NT = WM * WN * 64;
   constexpr int CH = BN / E;   // column chunks of the tile; a thread always gets chunk tid % CH
   constexpr int ROWS = NT / CH;
-  static_assert(NT % CH == 0, "stats mapping");
+  static_assert(NT % CH == 0 && NT <= BLOCK, "stats mapping");
+  const bool storing = NT == BLOCK || tid < NT;
   const bool want_stats = p.stats != nullptr || p.stat_acc != nullptr;
   float st_sum[E], st_sq[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) st_sum[e] = st_sq[e] = 0.f;
   // data gradient with BatchNorm sums: the chunks of bn_x and bn_mask this thread will meet are
   // requested up front, so that their latency overlaps the staging of the accumulators
-  constexpr int ITERS = (WM * 32 * CH) / NT;
-  constexpr int VISITS = TM * ITERS;
   float bn_mu[E], bn_is[E];
   uint4 pre_x[VISITS], pre_m[VISITS];
   if (MODE == kDgrad && want_stats) {
@@ -346,21 +345,17 @@ __device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], 
       bn_is[e] = col < p.gemm_n ? p.bn_invstd[col + e] : 0.f;
     }
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int it = 0; it < ITERS; ++it) {
-        const int q = tid + it * NT;
-        const int r = q / CH;
-        const int row = m0 + ((r >> 5) * TM + tm) * 32 + (r & 31);
-        const bool ok = row < p.gemm_m && col < p.gemm_n;
-        const int64_t idx = static_cast<int64_t>(row) * p.gemm_n + col;
-        pre_x[tm * ITERS + it] = ok ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_x) + idx) : make_uint4(0, 0, 0, 0);
-        pre_m[tm * ITERS + it] = (ok && p.bn_mask) ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_mask) + idx)
-                                                   : make_uint4(0, 0, 0, 0);
-      }
+    for (int visit = 0; visit < VISITS; ++visit) {
+      const int row = m0 + row_of(visit);
+      const bool ok = storing && row < p.gemm_m && col < p.gemm_n;
+      const int64_t idx = static_cast<int64_t>(row) * p.gemm_n + col;
+      pre_x[visit] = ok ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_x) + idx) : make_uint4(0, 0, 0, 0);
+      pre_m[visit] = (ok && p.bn_mask) ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_mask) + idx)
+                                       : make_uint4(0, 0, 0, 0);
+    }
   }
 
-  staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, [&](int visit, int tr, int tc, float* v) {
+  walk([&](int visit, int tr, int tc, float* v) {
     const int row = m0 + tr, col = n0 + tc;
     if (row >= p.gemm_m || col >= p.gemm_n) return;
     const int64_t idx = static_cast<int64_t>(row) * p.gemm_n + col;
@@ -449,12 +444,14 @@ __device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], 
     // banks, and the 64 lanes of a load below (8 values of e x 8 values of cc) land 8 banks apart per plane: neither
     // has a bank conflict (a [thread][2E] layout made every store a 16-way one)
     constexpr int PS = NT + 8;
-    static_assert(2 * E * PS * 4 <= WM * 32 * (BN + kStagePad) * 4, "the sums fit the staging tile");
+    static_assert(2 * E * PS * 4 <= STAGE_BYTES, "the sums fit the staging tile");
     float* red = stage;
+    if (storing) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      red[e * PS + tid] = st_sum[e];
-      red[(E + e) * PS + tid] = st_sq[e];
+      for (int e = 0; e < E; ++e) {
+        red[e * PS + tid] = st_sum[e];
+        red[(E + e) * PS + tid] = st_sq[e];
+      }
     }
     __syncthreads();
     if (tid < BN) {
@@ -484,6 +481,23 @@ __device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], 
     }
     if (p.fin_counters) finalize_column_tile<MODE, BN, NT>(p, stage, tid, n0);
   }
+}
+
+// The form for accumulators spread over the wavefronts of a tile, one 32-row band at a time.
+template <typename T, int MODE, int WM, int WN, int TM, int TN>
+__device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0,
+                                   int tile_m) {
+  constexpr int BN = WN * TN * 32;
+  constexpr int NT = WM * WN * 64;
+  constexpr int CH = BN / Elem<T>::kPerChunk;
+  constexpr int ITERS = (WM * 32 * CH) / NT;
+  finish_walk<T, MODE, BN, NT, NT, TM * ITERS, WM * 32 * (BN + kStagePad) * 4>(
+      p, stage, tid, m0, n0, tile_m,
+      [&](int visit) {
+        const int r = (tid + (visit % ITERS) * NT) / CH;
+        return ((r >> 5) * TM + visit / ITERS) * 32 + (r & 31);
+      },
+      [&](auto fin) { staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, fin); });
 }
 
 // ---------------------------------------------------------------------------
@@ -1231,6 +1245,247 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+// forward / data gradient where the grid of output tiles cannot fill the chip (and fp32 at every size): the
+// reduction is dealt out to the KG wavefronts of a workgroup
+// ---------------------------------------------------------------------------
+// Every wavefront owns the WHOLE TM*32 x TN*32 tile for every KG-th reduction step and has a ring of NBUF operand
+// tiles of its own in LDS, filled with direct loads: nothing is shared before the end, so the main loop has no
+// barrier and a wavefront waits for its own loads only.  The partial tiles meet in LDS once and are added in the
+// order of the wavefronts.  What this buys where workgroups are few: KG * (NBUF - 1) operand tiles in flight per
+// compute unit and a serial chain of nk / KG steps instead of nk.
+// A step is one 64-byte LDS row per GEMM row (32 bf16 or 16 fp32 elements), laid out as in igemm2_kernel with
+// 32-element steps; in_c must be a multiple of the step.
+template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
+__global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
+  constexpr int E = Elem<T>::kPerChunk;
+  constexpr int EB = sizeof(T);
+  constexpr int BM = TM * 32, BN = TN * 32;
+  constexpr int RB = 64;                 // bytes of one LDS row
+  constexpr int KS = RB / EB;            // reduction elements per step
+  constexpr int A_LD = BM / 16, B_LD = BN / 16;   // direct loads (sixteen rows each) per step
+  constexpr int A_BYTES = BM * RB, BUF_BYTES = (BM + BN) * RB;
+  constexpr int NT = KG * 64;
+  constexpr int CH = BN / E;
+  constexpr int ITEMS = BM * CH;
+  constexpr int NTE = ITEMS < NT ? ITEMS : NT;     // threads that store
+  constexpr int VISITS = (ITEMS + NT - 1) / NT;
+  static_assert(ITEMS % NTE == 0, "epilogue mapping");
+  constexpr int LD = BN + kStagePad;
+  constexpr int RED_BYTES = KG * BM * LD * 4;
+  constexpr int RING_BYTES = KG * NBUF * BUF_BYTES;
+  constexpr int LDS_BYTES = RED_BYTES > RING_BYTES ? RED_BYTES : RING_BYTES;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[LDS_BYTES];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+  // group_rows != 0: consecutive ids (one XCD) walk down the row tiles of one column tile, sharing its filter rows;
+  // 0: along the column tiles of one row tile, sharing its activation rows
+  const uint32_t run = p.group_rows ? p.tiles_m : p.tiles_n;
+  const int slow = id / run, fast = id - slow * run;
+  const int tile_m = p.group_rows ? fast : slow, tile_n = p.group_rows ? slow : fast;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+
+  const int in_h = (MODE == kFwd) ? p.H : p.Ho;
+  const int in_w = (MODE == kFwd) ? p.W : p.Wo;
+  const int in_c = (MODE == kFwd) ? p.C : p.K;
+  const int cblocks = in_c / KS;
+  const int nk = p.R * p.S * cblocks;
+  const int sl = p.stride_log2, sm = p.stride - 1;
+
+  // ---- per lane: the rows it feeds, their byte offset at tap (0,0) and which taps exist ----
+  const int sub_row = lane >> 2, slot = lane & 3;
+  int a_off[A_LD];
+  uint32_t a_taps[A_LD];
+#pragma unroll
+  for (int j = 0; j < A_LD; ++j) {
+    const int trow = j * 16 + sub_row;
+    const int chunk = slot ^ ((trow >> 2) & 3);
+    const int row = m0 + trow;
+    uint32_t taps = 0;
+    int base = 0;
+    if (row < p.gemm_m) {
+      if (p.pointwise) {
+        base = row * in_c;
+        taps = 1u;
+      } else {
+        uint32_t img, pix, oh, ow;
+        p.div_plane.divmod(static_cast<uint32_t>(row), img, pix);
+        p.div_width.divmod(pix, oh, ow);
+        // a tap exists where its row does and its column does
+        uint32_t cols = 0;
+        if (MODE == kFwd) {
+          const int h0 = static_cast<int>(oh) * p.stride - p.pad, w0 = static_cast<int>(ow) * p.stride - p.pad;
+          base = ((static_cast<int>(img) * in_h + h0) * in_w + w0) * in_c;
+          for (int s = 0; s < p.S; ++s)
+            if (static_cast<unsigned>(w0 + s) < static_cast<unsigned>(in_w)) cols |= 1u << s;
+          for (int r = 0; r < p.R; ++r)
+            if (static_cast<unsigned>(h0 + r) < static_cast<unsigned>(in_h)) taps |= cols << (r * p.S);
+        } else {
+          const int hp = static_cast<int>(oh) + p.pad, wp = static_cast<int>(ow) + p.pad;
+          base = ((static_cast<int>(img) * in_h + (hp >> sl)) * in_w + (wp >> sl)) * in_c;
+          for (int s = 0; s < p.S; ++s) {
+            const int tw = wp - s;
+            if (tw >= 0 && (tw & sm) == 0 && (tw >> sl) < in_w) cols |= 1u << s;
+          }
+          for (int r = 0; r < p.R; ++r) {
+            const int th = hp - r;
+            if (th >= 0 && (th & sm) == 0 && (th >> sl) < in_h) taps |= cols << (r * p.S);
+          }
+        }
+      }
+    }
+    a_off[j] = (base + chunk * E) * EB;
+    a_taps[j] = taps;
+  }
+  int b_off[B_LD];
+#pragma unroll
+  for (int j = 0; j < B_LD; ++j) {
+    const int trow = j * 16 + sub_row;
+    const int chunk = slot ^ ((trow >> 2) & 3);
+    const int row = n0 + trow;
+    b_off[j] = row < p.gemm_n ? (row * p.gemm_k + chunk * E) * EB : static_cast<int>(kOutOfRange);
+  }
+  const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(p.a_src, p.a_bytes);
+  const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(p.b_src, p.b_bytes);
+
+  // ---- this wavefront's steps: wave, wave + KG, ... as a scalar walk over (tap, channel block) ----
+  const int my_steps = nk > wave ? (nk - wave + KG - 1) / KG : 0;
+  int ld_kt = wave, ld_t = wave / cblocks;
+  int ld_cb = wave - ld_t * cblocks;
+  int ld_r = ld_t / p.S, ld_s = ld_t - (ld_t / p.S) * p.S;
+  unsigned char* ring = lds + wave * (NBUF * BUF_BYTES);
+  auto issue_loads = [&](int buf) {
+    const int tap_elems = (MODE == kFwd) ? (ld_r * in_w + ld_s) * in_c : -((ld_r >> sl) * in_w + (ld_s >> sl)) * in_c;
+    const int a_step = (tap_elems + ld_cb * KS) * EB;
+    const int b_step = ld_kt * RB;
+    unsigned char* dst = ring + buf * BUF_BYTES;
+#pragma unroll
+    for (int j = 0; j < A_LD; ++j) {
+      const bool ok = (a_taps[j] >> ld_t) & 1u;
+      load_to_lds(rsrc_a, dst + j * 1024, ok ? a_off[j] + a_step : static_cast<int>(kOutOfRange), 0);
+    }
+#pragma unroll
+    for (int j = 0; j < B_LD; ++j) load_to_lds(rsrc_b, dst + A_BYTES + j * 1024, b_off[j], b_step);
+    ld_kt += KG;
+    ld_cb += KG;
+    while (ld_cb >= cblocks) {
+      ld_cb -= cblocks;
+      ++ld_t;
+      if (++ld_s == p.S) {
+        ld_s = 0;
+        ++ld_r;
+      }
+    }
+  };
+
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  const int frag_row = lane & 31, frag_half = lane >> 5;
+  const int swz = (frag_row >> 2) & 3;
+  const uint32_t ring_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
+  const uint32_t rd = ring_base + frag_row * RB + swz * 16;
+  auto read_frags = [&](int buf, int kk, uint4_t* fa, uint4_t* fb) {
+    const uint32_t pa = (rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16)) + buf * BUF_BYTES;
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[tm]) : "v"(pa), "n"(tm * 32 * RB));
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn)
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[tn]) : "v"(pa), "n"(A_BYTES + tn * 32 * RB));
+  };
+  auto multiply = [&](uint4_t* fa, uint4_t* fb) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(fa[tm]));
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(fb[tn]));
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) {
+        Chunk a, b;
+        a.h = __builtin_bit_cast(bf16x8_t, fa[tm]);
+        b.h = __builtin_bit_cast(bf16x8_t, fb[tn]);
+        mma<T>(b, a, acc[tm][tn]);
+      }
+  };
+
+  // The tile of step i lands when at most the NBUF-2 tiles requested behind it are outstanding (near the end fewer
+  // follow: wait for everything).  The reads of step i-1 were waited for before its multiplies, so its buffer is free.
+  constexpr int AHEAD = (NBUF - 2) * (A_LD + B_LD);
+  static_assert(AHEAD < 64, "vmcnt range");
+  auto step = [&](int i, int buf) {
+    if (i + NBUF - 1 <= my_steps)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (i + NBUF - 1 < my_steps) issue_loads((buf + NBUF - 1) % NBUF);
+    uint4_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+    read_frags(buf, 0, fa0, fb0);
+    read_frags(buf, 1, fa1, fb1);
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN) : "memory");
+    multiply(fa0, fb0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    multiply(fa1, fb1);
+  };
+#pragma unroll
+  for (int i = 0; i < NBUF - 1; ++i)
+    if (i < my_steps) issue_loads(i);
+  int i0 = 0;
+  for (; i0 + NBUF <= my_steps; i0 += NBUF) {
+#pragma unroll
+    for (int u = 0; u < NBUF; ++u) step(i0 + u, u);
+  }
+#pragma unroll
+  for (int u = 0; u < NBUF - 1; ++u)
+    if (i0 + u < my_steps) step(i0 + u, u);
+
+  // ---- the partial tiles meet: [wave][BM][LD] fp32, over the rings ----
+  float* red = reinterpret_cast<float*>(lds);
+  finish_walk<T, MODE, BN, NTE, NT, VISITS, LDS_BYTES>(
+      p, red, tid, m0, n0, tile_m, [&](int visit) { return (tid + visit * NT) / CH; },
+      [&](auto fin) {
+        __syncthreads();   // every wavefront is done with its ring
+        float* mine = red + wave * (BM * LD);
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              *reinterpret_cast<float4*>(mine + (tm * 32 + frag_row) * LD + tn * 32 + 8 * j + 4 * frag_half) =
+                  make_float4(acc[tm][tn][4 * j], acc[tm][tn][4 * j + 1], acc[tm][tn][4 * j + 2], acc[tm][tn][4 * j + 3]);
+        __syncthreads();
+        if (NTE < NT && tid >= NTE) return;
+#pragma unroll
+        for (int visit = 0; visit < VISITS; ++visit) {
+          const int q = tid + visit * NT;
+          const int r = q / CH, c = (q - r * CH) * E;
+          float v[E];
+#pragma unroll
+          for (int e = 0; e < E; ++e) v[e] = 0.f;
+#pragma unroll
+          for (int g = 0; g < KG; ++g)
+#pragma unroll
+            for (int e = 0; e < E; e += 4) {
+              const float4 t = *reinterpret_cast<const float4*>(red + (g * BM + r) * LD + c + e);
+              v[e] += t.x;
+              v[e + 1] += t.y;
+              v[e + 2] += t.z;
+              v[e + 3] += t.w;
+            }
+          fin(visit, r, c, v);
+        }
+      });
+}
+
+// ---------------------------------------------------------------------------
 // 3x3, stride 1, pad 1 (forward and data gradient), 128 x 64*TN tile: the activation side of the nine
 // taps of a channel block is ONE patch in LDS.  The 128 output pixels of a tile are consecutive in the
 // flattened (image, row, column) order, and the input pixel of tap (r, s) lies (r-1)*W + (s-1) places
@@ -1572,6 +1827,25 @@ int launch_cfg2(Context* ctx, IgemmArgs& a, double flops) {
                 name.c_str(), flops, 0, conv_bytes<MODE>(a, 2));
 }
 
+template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
+int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
+  constexpr int BM = TM * 32, BN = TN * 32;
+  static const std::string name = std::string("igemm4_kernel<") + (sizeof(T) == 2 ? "bf16," : "f32,") +
+                                  (MODE == kFwd ? "fwd," : "dgrad,") + std::to_string(BM) + "x" + std::to_string(BN) + "," +
+                                  std::to_string(KG) + "way," + std::to_string(NBUF) + "buf>";
+  a.tiles_m = (a.gemm_m + BM - 1) / BM;
+  a.tiles_n = (a.gemm_n + BN - 1) / BN;
+  const int64_t wgs = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
+  if (wgs <= 0 || wgs > 0x7fffffff) {
+    set_error("igemm: grid out of range");
+    return -22;
+  }
+  // the larger operand is the one an XCD should fetch once
+  a.group_rows = static_cast<int64_t>(a.gemm_n) * a.gemm_k > static_cast<int64_t>(a.a_bytes / sizeof(T)) ? 1 : 0;
+  return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF>, dim3(static_cast<unsigned>(wgs)), dim3(KG * 64), a, name.c_str(),
+                flops, 0, conv_bytes<MODE>(a, sizeof(T)));
+}
+
 // The 3x3 patch kernel: stride 1, pad 1, input channels in blocks of 64, rows short enough for the patch
 template <int MODE>
 bool patch_kernel_fits(const IgemmArgs& a) {
@@ -1615,8 +1889,36 @@ int igemm2_setting() {
   return v;
 }
 
+// Tilings of igemm4_kernel (tile, wavefronts the reduction is dealt to, LDS tiles in flight of each).  LDS decides how
+// many workgroups share a CU: one (kSplit32Deep, kSplit64, kSplit64x32Deep) or two (the others).
+enum SplitTile : int {
+  kSplit32 = 15,         // 32 x 32, 4, 4
+  kSplit32Deep = 16,     // 32 x 32, 8, 2
+  kSplit64x32 = 17,      // 64 x 32, 4, 3
+  kSplit64 = 18,         // 64 x 64, 4, 4 (fp32: 8, 2)
+  kSplit64Pair = 19,     // 64 x 64, 4, 2
+  kSplit64x32Deep = 20,  // 64 x 32, 8, 3
+};
+
 template <typename T, int MODE>
 int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
+  switch (tile_cfg) {
+    case kSplit32:
+      return launch_cfg4<T, MODE, 1, 1, 4, 4>(ctx, a, flops);
+    case kSplit32Deep:
+      return launch_cfg4<T, MODE, 1, 1, 8, 2>(ctx, a, flops);
+    case kSplit64x32:
+      return launch_cfg4<T, MODE, 2, 1, 4, 3>(ctx, a, flops);
+    case kSplit64x32Deep:
+      return launch_cfg4<T, MODE, 2, 1, 8, 3>(ctx, a, flops);
+    case kSplit64:   // fp32 is bound by the matrix pipes: two wavefronts on each
+      if constexpr (sizeof(T) == 2) return launch_cfg4<T, MODE, 2, 2, 4, 4>(ctx, a, flops);
+      else return launch_cfg4<T, MODE, 2, 2, 8, 2>(ctx, a, flops);
+    case kSplit64Pair:
+      return launch_cfg4<T, MODE, 2, 2, 4, 2>(ctx, a, flops);
+    default:
+      break;
+  }
   if constexpr (sizeof(T) == 2 && (MODE == kFwd || MODE == kDgrad)) {
     const int in_c = MODE == kFwd ? a.C : a.K;
     const int setting = igemm2_setting();
@@ -1685,8 +1987,14 @@ double conv_flops(const ConvShape& s, int Ho, int Wo) {
 // rows of the workgroup tile of a tiling number (5 = the 3x3 patch kernel, or tiling 1 where it does not fit)
 int tile_rows(int tile_cfg) {
   if (tile_cfg == 9 || tile_cfg == 10) return 256;
+  if (tile_cfg >= kSplit32) return tile_cfg <= kSplit32Deep ? 32 : 64;
   if (tile_cfg >= 11 && tile_cfg <= 14) return tile_cfg == 14 ? 64 : 128;
   return (tile_cfg == 5 || tile_cfg == 6) ? 128 : tile_cfg >= 2 ? 64 : 128;
+}
+
+// column tiles of 32: callers of the in-kernel finalize provide a counter per 64 columns
+bool narrow_tile(int tile_cfg) {
+  return tile_cfg == kSplit32 || tile_cfg == kSplit32Deep || tile_cfg == kSplit64x32 || tile_cfg == kSplit64x32Deep;
 }
 
 int64_t tiles_for(int m, int n, int bm, int bn) {
@@ -1700,11 +2008,15 @@ bool wants_huge_tile(int dtype, int gemm_m, int gemm_n, int in_c, int taps) {
          tiles_for(gemm_m, gemm_n, 256, 256) >= 1024;
 }
 
+// igemm4_kernel: whole 64-byte steps of input channels, one bit per tap
+bool split_tile_fits(int dtype, int in_c, int taps) { return in_c % (dtype == kBF16 ? 32 : 16) == 0 && taps <= 32; }
+
 // The tiling that runs when `tile_cfg` is asked for: the 256 x 256 tilings exist for the direct-to-LDS kernel only
 // and stand for 128 x 128 elsewhere (the statistics' row tiles follow the tiling that runs).
 int effective_tile(int tile_cfg, int dtype, int in_c, int taps) {
   if ((tile_cfg == 9 || tile_cfg == 10) && !(dtype == kBF16 && in_c % 64 == 0 && taps <= 32 && igemm2_setting() != 0))
     return 0;
+  if (tile_cfg >= kSplit32 && !split_tile_fits(dtype, in_c, taps)) return 2;
   return tile_cfg;
 }
 
@@ -1714,6 +2026,31 @@ int pick_tile(int gemm_m, int gemm_n, int splits) {
   if (gemm_n > 64 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= 384) return 0;
   if (tiles_for(gemm_m, gemm_n, 128, 64) * splits >= 384) return 1;
   return 2;
+}
+
+// Where the output has too few tiles to fill the chip, the reduction is split inside the workgroup (igemm4_kernel):
+// smaller tiles as the grid shrinks, and from a reduction depth on that pays for the partial tiles that meet in LDS.
+// The lines lie where the layers of ResNet-152 at batches 1-64 and the projections of Swin-B and GPT-2 at 200-2331 rows
+// crossed over, timed back to back with cold filters (bf16, us, before -> after): 196 x 256 over 2304 13.2 -> 6.1,
+// 49 x 512 over 4608 22.1 -> 8.1 (32 x 32); 784 x 512 over 4608 36.9 -> 14.8 (64 x 32); 3920 x 256 over 2304
+// 20.6 -> 13.9, 1024 x 768 over 3072 24.3 -> 15.9 (64 x 64, one workgroup per CU); 4704 x 256 over 2304 21.0 -> 15.9
+// (two).  Beyond those sizes the shared operand tiles of the other kernels win.  fp32 multiplies at 1/16 of the rate,
+// so it gains from spreading them over every SIMD at shallower reductions (784 x 256 over 2304: 77.6 -> 14.8 us) and
+// keeps the 64 x 64 split tile on large grids too (2048 x 3072 over 768: 100 -> 86 us).  -1: none of them.
+int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
+  if (igemm2_setting() == 0 || !split_tile_fits(dtype, in_c, taps)) return -1;
+  const int64_t t32 = tiles_for(gemm_m, gemm_n, 32, 32), t64 = tiles_for(gemm_m, gemm_n, 64, 64);
+  if (t32 <= 256) return gemm_k >= 1024 ? kSplit32Deep : kSplit32;
+  if (dtype == kBF16) {
+    if (t32 <= 512) return gemm_k >= 1536 ? kSplit64x32 : kSplit32;
+    if (t64 <= 256 && gemm_k >= 512) return kSplit64;
+    if (t64 <= 448 && gemm_k >= 1024) return kSplit64Pair;
+    return -1;
+  }
+  if (t32 <= 512) return gemm_k >= 768 ? kSplit64x32Deep : kSplit32;
+  if (t64 <= 256 && gemm_k >= 768) return kSplit64;
+  if (t64 <= 512 && gemm_k >= 512) return kSplit64x32;
+  return gemm_k >= 256 && tiles_for(gemm_m, gemm_n, 128, 128) < 384 ? kSplit64Pair : -1;
 }
 
 // The heuristic's tiling for a pointwise product with a shallow reduction (at most 256 channels): the same tile
@@ -1729,6 +2066,12 @@ int shallow_tile(int tile_cfg, int dtype, int in_c, int taps) {
       tile_cfg <= 2)
     return tile_cfg + 12;
   return tile_cfg;
+}
+
+// The tiling the library takes by itself
+int heuristic_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
+  const int split = split_tile(dtype, gemm_m, gemm_n, gemm_k, in_c, taps);
+  return split >= 0 ? split : shallow_tile(pick_tile(gemm_m, gemm_n, 1), dtype, in_c, taps);
 }
 
 int fill_common(IgemmArgs& a, const ConvShape& s, int dtype) {
@@ -1834,13 +2177,13 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    tile_cfg = shallow_tile(pick_tile(a.gemm_m, a.gemm_n, 1), dtype, s.C, s.R * s.S);
+    tile_cfg = heuristic_tile(dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S);
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int row_tiles = (a.gemm_m + tile_rows(tile_cfg) - 1) / tile_rows(tile_cfg);
-  const bool in_kernel = finalize && row_tiles <= kBnFinalizeInKernelTiles;
+  const bool in_kernel = finalize && row_tiles <= kBnFinalizeInKernelTiles && !narrow_tile(tile_cfg);
   if (in_kernel) bind_finalize(a, finalize);
   int rc = dtype == kBF16 ? launch_mode<bf16, kFwd>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
                           : launch_mode<float, kFwd>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));
@@ -1854,7 +2197,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int gemm_m = s.N * Ho * Wo;
-  if (tile_cfg < 0) tile_cfg = pick_tile(gemm_m, s.K, 1);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S);
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -1862,7 +2205,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
 
 int conv2d_dgrad_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   const int gemm_m = s.N * s.H * s.W;
-  if (tile_cfg < 0) tile_cfg = pick_tile(gemm_m, s.C, 1);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S);
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -1906,13 +2249,13 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
   if (tile_cfg < 0) {
-    tile_cfg = shallow_tile(pick_tile(a.gemm_m, a.gemm_n, 1), dtype, s.K, s.R * s.S);
+    tile_cfg = heuristic_tile(dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S);
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
   const BnFinalize* finalize = bn ? bn->finalize : nullptr;
   const int row_tiles = (a.gemm_m + tile_rows(tile_cfg) - 1) / tile_rows(tile_cfg);
-  const bool in_kernel = finalize && row_tiles <= kBnFinalizeInKernelTiles;
+  const bool in_kernel = finalize && row_tiles <= kBnFinalizeInKernelTiles && !narrow_tile(tile_cfg);
   if (in_kernel) bind_finalize(a, finalize);
   int rc = dtype == kBF16 ? launch_mode<bf16, kDgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
                           : launch_mode<float, kDgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));

@@ -295,7 +295,7 @@ class ResNetEngine(EngineBase):
         """The fastest tiling, or a larger tile that is within `tile_margin` of it: alone on the chip a small tile
         can win by a few percent and still lose in the step, where it shares L2 bandwidth with the weight gradients
         (a larger tile fetches fewer operand bytes per flop)."""
-        area = lambda cfg: {0: 4, 11: 4, 12: 4, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2}.get(cfg, 1)
+        area = lambda cfg: {0: 4, 11: 4, 12: 4, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2, 15: 0.25, 16: 0.25, 17: 0.5, 20: 0.5}.get(cfg, 1)
         best = min(timings.values())
         ok = [cfg for cfg, t in timings.items() if t <= best * (1.0 + self.tile_margin)]
         return min(ok, key=lambda cfg: (-area(cfg), timings[cfg]))
@@ -312,7 +312,8 @@ class ResNetEngine(EngineBase):
         x = self._scratch((n, h, w, c.cin_store), T)
         z = self._scratch((n, ho, wo, c.cout), T)
         wgt, wt = self._w(c.name + ".weight"), self._wt(c.name + ".weight")
-        part = self._scratch((ops.conv2d_fwd_stat_rows(x, c.cout, c.k, c.k, c.stride, c.pad, 2) * c.cout * 2,),
+        # row tiles of the statistics: tiling 15 has the smallest
+        part = self._scratch((ops.conv2d_fwd_stat_rows(x, c.cout, c.k, c.k, c.stride, c.pad, 15) * c.cout * 2,),
                              torch.float32)
         reps = 4
 
@@ -325,7 +326,7 @@ class ResNetEngine(EngineBase):
         mean = self._scratch((c.cin_store,), torch.float32)
         invstd = self._scratch((c.cin_store,), torch.float32, 1.0)
         x2 = self._scratch(tuple(x.shape), T, 1.0)
-        dpart = self._scratch((ops.conv2d_dgrad_stat_rows(x, c.cout, c.k, c.k, c.stride, c.pad, 2) * c.cin_store * 2,),
+        dpart = self._scratch((ops.conv2d_dgrad_stat_rows(x, c.cout, c.k, c.k, c.stride, c.pad, 15) * c.cin_store * 2,),
                               torch.float32)
         torch.cuda.synchronize()
 
@@ -344,9 +345,13 @@ class ResNetEngine(EngineBase):
         # 11 - 14 = 128 x 128 (three / two LDS tiles), 128 x 64, 64 x 64 with 32-element reduction steps: half the LDS
         # per workgroup, which the wide, shallow products of the first two stages prefer
         cfgs = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14) if c.cout > 64 else (1, 2, 3, 6, 7, 13, 14)) + patch
+        # 15 - 20 = the reduction split over the wavefronts of a workgroup: only where a 64 x 64 tiling cannot fill the chip
+        few = lambda pixels, channels: (15, 16, 17, 18, 19) if -(-pixels // 64) * -(-channels // 64) <= 512 else ()
+        cfgs += few(n * ho * wo, c.cout)
         t_f = {cfg: self._time_program(fwd(cfg)) / reps for cfg in cfgs}
         tf = self._pick_tiling(t_f)
         cfgs_d = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14) if c.cin_store > 64 else (1, 2, 3, 6, 7, 13, 14)) + patch
+        cfgs_d += few(n * h * w, c.cin_store)
         t_d = {cfg: self._time_program(dgrad(cfg)) / reps for cfg in cfgs_d} if c.cin_store >= 64 else {-1: 0.0}
         td = self._pick_tiling(t_d)
         self._tile_cache[key] = (tf, td)
@@ -466,8 +471,8 @@ class ResNetEngine(EngineBase):
             xm = torch.empty((n_, h_, w_, c_.cin_store), dtype=T, device="meta")
             # sized for the smallest row tile, whichever tiling is picked
             stat_elems[0] = max(stat_elems[0],
-                                ops.conv2d_fwd_stat_rows(xm, c_.cout, c_.k, c_.k, c_.stride, c_.pad, 2) * c_.cout * 2,
-                                ops.conv2d_dgrad_stat_rows(xm, c_.cout, c_.k, c_.k, c_.stride, c_.pad, 2) * c_.cin_store * 2)
+                                ops.conv2d_fwd_stat_rows(xm, c_.cout, c_.k, c_.k, c_.stride, c_.pad, 15) * c_.cout * 2,
+                                ops.conv2d_dgrad_stat_rows(xm, c_.cout, c_.k, c_.k, c_.stride, c_.pad, 15) * c_.cin_store * 2)
             tiles[c_.name] = self._tune_conv(c_, n_, h_, w_) if self.autotune else (-1, -1)
         stat_partial = act(max(stat_elems[0], 2), dtype=torch.float32)
         bn_scratch = act(3 * max(max(c_.cout, c_.cin_store) for c_, _ in conv_inputs), dtype=torch.float32)

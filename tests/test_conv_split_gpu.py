@@ -1,0 +1,44 @@
+"""The convolution tilings that split the reduction over the wavefronts of a workgroup (15 - 20), at the edges of their
+tiles and rings, against the CPU oracle: the operator tests of test_ops_gpu.py run on them."""
+import pytest
+import torch
+
+import test_ops_gpu as T
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # N, H, W, C, K, R, S, stride, pad
+    (1, 7, 7, 64, 64, 1, 1, 1, 0),        # fewer reduction steps than wavefronts (bf16: 2), rows and columns off the tile
+    (1, 7, 9, 192, 72, 3, 3, 1, 1),       # a step count that is no multiple of the wavefronts, ragged columns
+    (3, 14, 14, 64, 32, 3, 3, 2, 1),      # strided: taps that exist for every second pixel only
+    (2, 16, 16, 64, 128, 1, 1, 2, 0),     # strided 1x1
+    (65, 1, 1, 1088, 200, 1, 1, 1, 0),    # one row over a tile, a deep pointwise reduction
+    (1, 5, 5, 24, 40, 3, 3, 1, 1),        # channels that are no whole step: another kernel runs
+]
+TILES = [15, 16, 17, 18, 19, 20]
+dtypes = pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+
+
+@dtypes
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("tile_cfg", TILES)
+def test_forward_and_data_gradient(ctx, dtype, case, tile_cfg):
+    T.test_conv_fwd(ctx, dtype, case, tile_cfg)
+    T.test_conv_dgrad(ctx, dtype, case, tile_cfg)
+
+
+@dtypes
+@pytest.mark.parametrize("case", CASES[:5])
+@pytest.mark.parametrize("tile_cfg", TILES)
+def test_batchnorm_sums(ctx, dtype, case, tile_cfg):
+    T.test_conv_with_bn_statistics(ctx, dtype, case, tile_cfg)
+    T.test_conv_dgrad_with_bn_backward_sums(ctx, dtype, case, tile_cfg, True)
+
+
+@dtypes
+@pytest.mark.parametrize("rows,K,C", [(196, 256, 1024), (196, 512, 2048), (784, 512, 2048), (1024, 256, 1024), (4704, 256, 1024),
+                                      (343, 1024, 1024), (2048, 768, 768)])
+def test_library_choice(ctx, dtype, rows, K, C):
+    """One size on each side of the lines of the library's own choice."""
+    T.test_conv_fwd(ctx, dtype, (rows, 1, 1, C, K, 1, 1, 1, 0), -1)
