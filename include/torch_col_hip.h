@@ -444,6 +444,13 @@ int tch_flash_attn_fwd(tch_context* ctx, int dtype, const void* q, const void* k
 int tch_flash_attn_bwd(tch_context* ctx, int dtype, const void* q, const void* k, const void* v, const void* o,
                        const void* dout, const float* lse, float* delta, void* dq, void* dk, void* dv, int B, int H,
                        int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal);
+/* The same for any sequence length (the two above refuse one that is no multiple of 128). */
+int tch_flash_attn_any_fwd(tch_context* ctx, int dtype, const void* q, const void* k, const void* v, void* o, float* lse,
+                           int B, int H, int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale,
+                           int causal);
+int tch_flash_attn_any_bwd(tch_context* ctx, int dtype, const void* q, const void* k, const void* v, const void* o,
+                           const void* dout, const float* lse, float* delta, void* dq, void* dk, void* dv, int B, int H,
+                           int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal);
 
 /* Window attention of the Swin-B step in one launch per direction (train/swin_b_tiny.py:94-110: q k^T * scale +
  * relative position bias (+ shift mask), softmax, @ v; torchvision's shifted_window_attention for

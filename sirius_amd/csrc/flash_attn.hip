@@ -18,6 +18,14 @@
 // {16s + 8t + 4(lane/32) + i}, which is a permutation of the 16 reduction indices of one MFMA step; the other
 // operand is read from LDS with the same permutation (transposing reads, ds_read_b64_tr_b16).
 //
+// RAGGED (a sequence length that is no multiple of 128): the last fixed block and the last walked tile reach past the
+// sequence.  Loads of rows beyond it fetch the last row again (no branch, always a finite value), and nothing is
+// stored for them.  A walked key beyond the end is masked like a future key (a causal mask covers it already); a walked
+// query beyond the end gets a log-sum-exp of +inf, so that its probabilities are exp2(-inf) = 0: the inner loops
+// are those of the whole-tile form.  The whole-tile form keeps its own instantiation (no clamps in its address path).
+// Against the three-launch chain over materialised scores that such lengths took before: 12 layers of 3 x 777
+// tokens, forward + backward, 5.36 -> 0.7 ms (the step 10.7 -> 6.1 ms).
+//
 // Numerics: scores and statistics in fp32 from the bf16 products, exponentials as exp2 of pre-scaled values,
 // probabilities rounded to bf16 for the second product (as the unfused path stores them).  The backward
 // recomputes the probabilities from the saved log-sum-exp; dQ and (dK, dV) are two launches so that nothing is
@@ -66,6 +74,16 @@ __device__ inline TileRegs tile_load(const bf16* base, int64_t rs, int tid) {
   r.hi = *reinterpret_cast<const uint4*>(src + 32 * rs);
   return r;
 }
+// rows `first` .. `first` + 63 of a sequence of T rows; rows beyond it repeat the last one
+template <bool RAGGED>
+__device__ inline TileRegs tile_load_at(const bf16* base, int64_t rs, int first, int T, int tid) {
+  if (!RAGGED) return tile_load(base + first * rs, rs, tid);
+  const int r0 = first + (tid >> 3), r1 = r0 + 32;
+  TileRegs r;
+  r.lo = *reinterpret_cast<const uint4*>(base + (r0 < T ? r0 : T - 1) * rs + (tid & 7) * 8);
+  r.hi = *reinterpret_cast<const uint4*>(base + (r1 < T ? r1 : T - 1) * rs + (tid & 7) * 8);
+  return r;
+}
 __device__ inline void tile_store(unsigned char* lds, int tid, const TileRegs& r) {
   unsigned char* dst = lds + (tid >> 3) * kRowB + (tid & 7) * 16;
   *reinterpret_cast<uint4*>(dst) = r.lo;
@@ -73,16 +91,20 @@ __device__ inline void tile_store(unsigned char* lds, int tid, const TileRegs& r
 }
 
 // this wave's fragments of 32 fixed rows (row = first + lane % 32): 4 chunks cover the lane half's 32 columns
-__device__ inline void load_fixed(const bf16* base, int64_t rs, int first, int lane, Chunk (&f)[4]) {
-  const bf16* row = base + static_cast<int64_t>(first + (lane & 31)) * rs + 8 * (lane >> 5);
+template <bool RAGGED>
+__device__ inline void load_fixed(const bf16* base, int64_t rs, int first, int T, int lane, Chunk (&f)[4]) {
+  int r = first + (lane & 31);
+  if (RAGGED && r >= T) r = T - 1;
+  const bf16* row = base + static_cast<int64_t>(r) * rs + 8 * (lane >> 5);
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) f[ks].u = *reinterpret_cast<const uint4*>(row + ks * 16);
 }
 
 // acc[ct] holds the transposed result: column 32 ct + 8 (r / 4) + 4 (lane / 32) + r % 4 of fixed row lane % 32.
 // Goes through this wave's LDS patch so that a row leaves as 16-byte pieces.
+template <bool RAGGED>
 __device__ inline void store_fixed(f32x16_t (&acc)[2], float mul, unsigned char* patch, bf16* base, int64_t rs, int first,
-                                   int lane) {
+                                   int T, int lane) {
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
@@ -97,14 +119,15 @@ __device__ inline void store_fixed(f32x16_t (&acc)[2], float mul, unsigned char*
   for (int i = 0; i < 4; ++i) {
     const int q = lane + 64 * i;
     const uint4 v = *reinterpret_cast<const uint4*>(patch + (q >> 3) * kRowB + (q & 7) * 16);
-    *reinterpret_cast<uint4*>(base + static_cast<int64_t>(first + (q >> 3)) * rs + (q & 7) * 8) = v;
+    if (!RAGGED || first + (q >> 3) < T)
+      *reinterpret_cast<uint4*>(base + static_cast<int64_t>(first + (q >> 3)) * rs + (q & 7) * 8) = v;
   }
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // forward (DQ = false) and the dQ half of the backward (DQ = true): fixed queries, walked keys
 // ---------------------------------------------------------------------------------------------------------
-template <bool CAUSAL, bool DQ>
+template <bool CAUSAL, bool DQ, bool RAGGED>
 __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kTileB];
   unsigned char* kt = lds;
@@ -114,21 +137,24 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
   // placement: the blocks of one head keep one residue of the id modulo 8 (one XCD, one L2 for its keys and
   // values), and the long blocks of a causal problem come first so that each compute unit's share of
   // consecutive ids mixes long and short ones.
-  const int nbh = gridDim.x / (p.T / kFixed);
-  const int qb = p.T / kFixed - 1 - blockIdx.x / nbh;
+  const int blocks = RAGGED ? (p.T + kFixed - 1) / kFixed : p.T / kFixed;
+  const int nbh = gridDim.x / blocks;
+  const int qb = blocks - 1 - blockIdx.x / nbh;
   const int bh = blockIdx.x % nbh;
   const int b = bh / p.H, h = bh - b * p.H;
   const int64_t qkv_off = b * p.qkv_bs + h * kHd, o_off = b * p.o_bs + h * kHd;
   const int q0 = qb * kFixed, qw0 = q0 + 32 * wave;
   const int query = qw0 + (lane & 31);
+  const bool real = !RAGGED || query < p.T;
+  const int64_t stat_at = static_cast<int64_t>(bh) * p.T + (real ? query : p.T - 1);
 
   Chunk qf[4], dof[4];
-  load_fixed(p.q + qkv_off, p.qkv_rs, qw0, lane, qf);
+  load_fixed<RAGGED>(p.q + qkv_off, p.qkv_rs, qw0, p.T, lane, qf);
   float lse2 = 0.f, delta = 0.f;
   if (DQ) {
-    load_fixed(p.dout + o_off, p.o_rs, qw0, lane, dof);
+    load_fixed<RAGGED>(p.dout + o_off, p.o_rs, qw0, p.T, lane, dof);
     Chunk of[4];
-    load_fixed(p.o + o_off, p.o_rs, qw0, lane, of);
+    load_fixed<RAGGED>(p.o + o_off, p.o_rs, qw0, p.T, lane, of);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       float a[8], g[8];
@@ -138,15 +164,17 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
       for (int e = 0; e < 8; ++e) delta += a[e] * g[e];
     }
     delta += __shfl_xor(delta, 32, 64);
-    if (half == 0) p.delta[static_cast<int64_t>(bh) * p.T + query] = delta;
-    lse2 = p.lse[static_cast<int64_t>(bh) * p.T + query] * kLog2e;
+    if (half == 0 && real) p.delta[stat_at] = delta;
+    lse2 = p.lse[stat_at] * kLog2e;
   }
 
-  const int steps = CAUSAL ? (q0 + kFixed) / kWalk : p.T / kWalk;
+  const int tiles = RAGGED ? (p.T + kWalk - 1) / kWalk : p.T / kWalk;
+  const int seen = (q0 + kFixed) / kWalk;   // tiles a causal block of queries sees
+  const int steps = CAUSAL ? (RAGGED && seen > tiles ? tiles : seen) : tiles;
   const bf16* kbase = p.k + qkv_off;
   const bf16* vbase = p.v + qkv_off;
-  TileRegs rk = tile_load(kbase, p.qkv_rs, tid);
-  TileRegs rv = tile_load(vbase, p.qkv_rs, tid);
+  TileRegs rk = tile_load_at<RAGGED>(kbase, p.qkv_rs, 0, p.T, tid);
+  TileRegs rv = tile_load_at<RAGGED>(vbase, p.qkv_rs, 0, p.T, tid);
 
   f32x16_t acc[2];
   zero_acc(acc[0]);
@@ -161,9 +189,9 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
     __syncthreads();
     {
       // the last step fetches its own tile again rather than branching around the loads
-      const int64_t next = static_cast<int64_t>(kb + 1 < steps ? kb + 1 : kb) * kWalk * p.qkv_rs;
-      rk = tile_load(kbase + next, p.qkv_rs, tid);
-      rv = tile_load(vbase + next, p.qkv_rs, tid);
+      const int next = (kb + 1 < steps ? kb + 1 : kb) * kWalk;
+      rk = tile_load_at<RAGGED>(kbase, p.qkv_rs, next, p.T, tid);
+      rv = tile_load_at<RAGGED>(vbase, p.qkv_rs, next, p.T, tid);
     }
     const int k0 = kb * kWalk;
     if (CAUSAL && k0 > qw0 + 31) continue;   // nothing of this tile is visible to this wave's queries
@@ -180,7 +208,9 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
         for (int ks = 0; ks < 4; ++ks) dp[t] = mma16(frag_rows<kRowB>(vt, 32 * t, ks, lane), dof[ks], dp[t]);
       }
     }
-    const bool diagonal = CAUSAL && k0 + kWalk - 1 > qw0;   // some key of the tile lies beyond some query
+    // some key of the tile lies beyond some query, or beyond the sequence
+    const bool diagonal = CAUSAL ? k0 + kWalk - 1 > qw0 : RAGGED && k0 + kWalk > p.T;
+    const int last = CAUSAL ? query : p.T - 1;   // the last key this lane's query sees
     float pr[2][16];
     if (!DQ) {
       // running maximum on the raw scores (the scale is positive), then exp2(s * c - m * c) as one fused
@@ -191,7 +221,7 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float v = s[t][r];
-          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > query) v = -INFINITY;
+          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > last) v = -INFINITY;
           pr[t][r] = v;
           bmax = fmaxf(bmax, v);
         }
@@ -223,7 +253,7 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float pv = __builtin_amdgcn_exp2f(s[t][r] * c - lse2);
-          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > query) pv = 0.f;
+          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > last) pv = 0.f;
           pr[t][r] = pv * (dp[t][r] - delta);
         }
     }
@@ -242,23 +272,24 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
   if (!DQ) {
     l += __shfl_xor(l, 32, 64);
     mul = 1.f / l;
-    if (half == 0) p.lse[static_cast<int64_t>(bh) * p.T + query] = m * p.scale + __builtin_amdgcn_logf(l) * kLn2;
+    if (half == 0 && real) p.lse[stat_at] = m * p.scale + __builtin_amdgcn_logf(l) * kLn2;
   }
   __syncthreads();   // every wave is done with the tiles: the space becomes four output patches
-  store_fixed(acc, mul, lds + wave * 32 * kRowB, p.out + (DQ ? qkv_off : o_off), DQ ? p.qkv_rs : p.o_rs, qw0, lane);
+  store_fixed<RAGGED>(acc, mul, lds + wave * 32 * kRowB, p.out + (DQ ? qkv_off : o_off), DQ ? p.qkv_rs : p.o_rs, qw0, p.T,
+                      lane);
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // dK and dV: fixed keys, walked queries
 // ---------------------------------------------------------------------------------------------------------
-template <bool CAUSAL>
+template <bool CAUSAL, bool RAGGED>
 __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kTileB];
   __shared__ __attribute__((aligned(16))) float stat[2][kWalk];   // log-sum-exp (base 2) and delta of the staged queries
   unsigned char* qt = lds;
   unsigned char* dot = lds + kTileB;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
-  const int nbh = gridDim.x / (p.T / kFixed);   // placement as in flash_query_kernel: early keys see most queries
+  const int nbh = gridDim.x / (RAGGED ? (p.T + kFixed - 1) / kFixed : p.T / kFixed);   // placement as in flash_query_kernel: early keys see most queries
   const int kblk = blockIdx.x / nbh;
   const int bh = blockIdx.x % nbh;
   const int b = bh / p.H, h = bh - b * p.H;
@@ -267,11 +298,11 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   const int key = kw0 + (lane & 31);
 
   Chunk kf[4], vf[4];
-  load_fixed(p.k + qkv_off, p.qkv_rs, kw0, lane, kf);
-  load_fixed(p.v + qkv_off, p.qkv_rs, kw0, lane, vf);
+  load_fixed<RAGGED>(p.k + qkv_off, p.qkv_rs, kw0, p.T, lane, kf);
+  load_fixed<RAGGED>(p.v + qkv_off, p.qkv_rs, kw0, p.T, lane, vf);
 
   const int first = CAUSAL ? k0 / kWalk : 0;   // queries before the first key see none of these keys
-  const int steps = p.T / kWalk;
+  const int steps = RAGGED ? (p.T + kWalk - 1) / kWalk : p.T / kWalk;
   const bf16* qbase = p.q + qkv_off;
   const bf16* dobase = p.dout + o_off;
   const float* lse = p.lse + static_cast<int64_t>(bh) * p.T;
@@ -279,10 +310,13 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   TileRegs rq, rd;
   float rstat = 0.f;
   auto fetch = [&](int qb) {
-    rq = tile_load(qbase + static_cast<int64_t>(qb) * kWalk * p.qkv_rs, p.qkv_rs, tid);
-    rd = tile_load(dobase + static_cast<int64_t>(qb) * kWalk * p.o_rs, p.o_rs, tid);
-    if (tid < kWalk) rstat = lse[qb * kWalk + tid] * kLog2e;
-    else if (tid < 2 * kWalk) rstat = dlt[qb * kWalk + tid - kWalk];
+    rq = tile_load_at<RAGGED>(qbase, p.qkv_rs, qb * kWalk, p.T, tid);
+    rd = tile_load_at<RAGGED>(dobase, p.o_rs, qb * kWalk, p.T, tid);
+    const int row = qb * kWalk + (tid & (kWalk - 1));
+    const bool real = !RAGGED || row < p.T;
+    const int at = real ? row : p.T - 1;
+    if (tid < kWalk) rstat = real ? lse[at] * kLog2e : INFINITY;
+    else if (tid < 2 * kWalk) rstat = dlt[at];
   };
   fetch(first);
 
@@ -348,17 +382,19 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   }
   __syncthreads();
   unsigned char* patch = lds + wave * 32 * kRowB;
-  store_fixed(dv, 1.f, patch, p.dv + qkv_off, p.qkv_rs, kw0, lane);
+  store_fixed<RAGGED>(dv, 1.f, patch, p.dv + qkv_off, p.qkv_rs, kw0, p.T, lane);
   __syncthreads();
-  store_fixed(dk, p.scale, patch, p.dk + qkv_off, p.qkv_rs, kw0, lane);
+  store_fixed<RAGGED>(dk, p.scale, patch, p.dk + qkv_off, p.qkv_rs, kw0, p.T, lane);
 }
 
 int check_geometry(const char* who, int dtype, int B, int H, int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs,
-                   int64_t o_bs) {
+                   int64_t o_bs, int any_length) {
   const std::string w(who);
   TCH_CHECK_ARG(dtype == kBF16, w + ": bf16 only");
-  TCH_CHECK_ARG(B >= 1 && H >= 1 && T >= kFixed && T % kFixed == 0, w + ": the sequence length must be a multiple of 128");
-  TCH_CHECK_ARG(static_cast<int64_t>(B) * H * (T / kFixed) < (1ll << 31), w + ": too many blocks for one grid");
+  TCH_CHECK_ARG(B >= 1 && H >= 1 && T >= 1 && (any_length || T % kFixed == 0),
+                w + ": the sequence length must be a multiple of 128");
+  TCH_CHECK_ARG(T <= (1 << 30) && static_cast<int64_t>(B) * H * ((T + kFixed - 1) / kFixed) < (1ll << 31),
+                w + ": too many blocks for one grid");
   TCH_CHECK_ARG(qkv_rs >= static_cast<int64_t>(H) * kHd && o_rs >= static_cast<int64_t>(H) * kHd,
                 w + ": row strides shorter than the heads");
   TCH_CHECK_ARG(qkv_rs % 8 == 0 && qkv_bs % 8 == 0 && o_rs % 8 == 0 && o_bs % 8 == 0,
@@ -371,8 +407,9 @@ bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15)
 }  // namespace
 
 int flash_attn_fwd(Context* ctx, int dtype, const void* q, const void* k, const void* v, void* o, float* lse, int B,
-                   int H, int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal) {
-  if (int rc = check_geometry("flash_attn_fwd", dtype, B, H, T, qkv_rs, qkv_bs, o_rs, o_bs)) return rc;
+                   int H, int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal,
+                   int any_length) {
+  if (int rc = check_geometry("flash_attn_fwd", dtype, B, H, T, qkv_rs, qkv_bs, o_rs, o_bs, any_length)) return rc;
   TCH_CHECK_ARG(q && k && v && o && lse, "flash_attn_fwd: null tensor");
   TCH_CHECK_ARG(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o), "flash_attn_fwd: tensors must be 16-byte aligned");
   FlashArgs a{};
@@ -388,16 +425,19 @@ int flash_attn_fwd(Context* ctx, int dtype, const void* q, const void* k, const 
   a.H = H;
   a.T = T;
   a.scale = scale;
-  const dim3 grid(static_cast<unsigned>(T / kFixed) * B * H);
+  const dim3 grid(static_cast<unsigned>((T + kFixed - 1) / kFixed) * B * H);
   const double flops = 4.0 * B * H * static_cast<double>(T) * T * kHd * (causal ? 0.5 : 1.0);
-  return causal ? launch(ctx, flash_query_kernel<true, false>, grid, dim3(256), a, "flash_attn_fwd<causal>", flops, 0)
-                : launch(ctx, flash_query_kernel<false, false>, grid, dim3(256), a, "flash_attn_fwd<full>", flops, 0);
+  const bool ragged = T % kFixed != 0;
+  void (*const kernel)(FlashArgs) =
+      causal ? (ragged ? flash_query_kernel<true, false, true> : flash_query_kernel<true, false, false>)
+             : (ragged ? flash_query_kernel<false, false, true> : flash_query_kernel<false, false, false>);
+  return launch(ctx, kernel, grid, dim3(256), a, causal ? "flash_attn_fwd<causal>" : "flash_attn_fwd<full>", flops, 0);
 }
 
 int flash_attn_bwd(Context* ctx, int dtype, const void* q, const void* k, const void* v, const void* o, const void* dout,
                    const float* lse, float* delta, void* dq, void* dk, void* dv, int B, int H, int T, int64_t qkv_rs,
-                   int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal) {
-  if (int rc = check_geometry("flash_attn_bwd", dtype, B, H, T, qkv_rs, qkv_bs, o_rs, o_bs)) return rc;
+                   int64_t qkv_bs, int64_t o_rs, int64_t o_bs, float scale, int causal, int any_length) {
+  if (int rc = check_geometry("flash_attn_bwd", dtype, B, H, T, qkv_rs, qkv_bs, o_rs, o_bs, any_length)) return rc;
   TCH_CHECK_ARG(q && k && v && o && dout && lse && delta && dq && dk && dv, "flash_attn_bwd: null tensor");
   TCH_CHECK_ARG(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && aligned16(dout) && aligned16(dq) &&
                     aligned16(dk) && aligned16(dv),
@@ -420,14 +460,18 @@ int flash_attn_bwd(Context* ctx, int dtype, const void* q, const void* k, const 
   a.H = H;
   a.T = T;
   a.scale = scale;
-  const dim3 grid(static_cast<unsigned>(T / kFixed) * B * H);
+  const dim3 grid(static_cast<unsigned>((T + kFixed - 1) / kFixed) * B * H);
   const double pair = 2.0 * B * H * static_cast<double>(T) * T * kHd * (causal ? 0.5 : 1.0);   // one T x T x 64 product
   // the dQ launch leaves delta for the dK / dV launch
-  int rc = causal ? launch(ctx, flash_query_kernel<true, true>, grid, dim3(256), a, "flash_attn_dq<causal>", 3.0 * pair, 0)
-                  : launch(ctx, flash_query_kernel<false, true>, grid, dim3(256), a, "flash_attn_dq<full>", 3.0 * pair, 0);
-  if (rc) return rc;
-  return causal ? launch(ctx, flash_key_kernel<true>, grid, dim3(256), a, "flash_attn_dkv<causal>", 4.0 * pair, 0)
-                : launch(ctx, flash_key_kernel<false>, grid, dim3(256), a, "flash_attn_dkv<full>", 4.0 * pair, 0);
+  const bool ragged = T % kFixed != 0;
+  void (*const dq_kernel)(FlashArgs) =
+      causal ? (ragged ? flash_query_kernel<true, true, true> : flash_query_kernel<true, true, false>)
+             : (ragged ? flash_query_kernel<false, true, true> : flash_query_kernel<false, true, false>);
+  void (*const dkv_kernel)(FlashArgs) = causal ? (ragged ? flash_key_kernel<true, true> : flash_key_kernel<true, false>)
+                                               : (ragged ? flash_key_kernel<false, true> : flash_key_kernel<false, false>);
+  if (int rc = launch(ctx, dq_kernel, grid, dim3(256), a, causal ? "flash_attn_dq<causal>" : "flash_attn_dq<full>", 3.0 * pair, 0))
+    return rc;
+  return launch(ctx, dkv_kernel, grid, dim3(256), a, causal ? "flash_attn_dkv<causal>" : "flash_attn_dkv<full>", 4.0 * pair, 0);
 }
 
 }  // namespace tch

@@ -10,7 +10,7 @@ recorded program of hand-written kernels per batch size:
 * the vocabulary is padded to a multiple of 128 rows of zeros (they never receive a gradient), so the
   output head and its two gradients run on the direct-to-LDS GEMM kernel;
 * attention reads the packed [B, T, 3, heads, head_dim] projection in place: in bf16 with heads 64 wide
-  and a sequence length that is a multiple of 128 it is one fused launch forward (scores never leave the
+  it is one fused launch forward (scores never leave the
   chip, the log-sum-exp is kept) and two backward; otherwise batched strided GEMMs and a causal softmax
   over materialised [B, heads, T, T] scores (kept for the backward);
 * backward is written out by hand; the gradient that bypasses a LayerNorm is added inside the
@@ -280,7 +280,7 @@ class GPT2Engine(EngineBase):
         s_b, o_b = (H * T * T, T * T), (T * C, D)
         scale = 1.0 / math.sqrt(D)
         # one fused pass per direction where the kernel's shape limits hold; the three-launch chain otherwise
-        fused = self.fused_attention and self.dtype == torch.bfloat16 and D == 64 and T % 128 == 0
+        fused = self.fused_attention and self.dtype == torch.bfloat16 and D == 64
 
         prog = ops.Program()
         marks = []
@@ -306,7 +306,7 @@ class GPT2Engine(EngineBase):
                     # P is the log-sum-exp here: all the backward needs to rebuild the probabilities
                     P = act(B * H, T, dtype=torch.float32)
                     ops.flash_attn_fwd(ctx, flat, flat[C:], flat[2 * C:], o.view(-1), P, B, H, T, (qkv_row, T * qkv_row),
-                                       (C, T * C), scale, causal=True)
+                                       (C, T * C), scale, causal=True, any_length=True)
                 else:
                     P = act(B, H, T, T)
                     ops.batched_gemm(ctx, flat, flat[C:], P, T, T, D, (qkv_row, 1), (qkv_row, 1), T, (B, H), qkv_b, qkv_b,
@@ -370,7 +370,7 @@ class GPT2Engine(EngineBase):
                 if fused:
                     ops.flash_attn_bwd(ctx, flat, flat[C:], flat[2 * C:], o.view(-1), d_o.view(-1), P, dP, gflat,
                                        gflat[C:], gflat[2 * C:], B, H, T, (qkv_row, T * qkv_row), (C, T * C), scale,
-                                       causal=True)
+                                       causal=True, any_length=True)
                 else:
                     ops.batched_gemm(ctx, P, d_o, gflat[2 * C:], T, D, T, (1, T), (1, C), qkv_row, (B, H), s_b, o_b, qkv_b,
                                      causal=3)
