@@ -2068,9 +2068,11 @@ int shallow_tile(int tile_cfg, int dtype, int in_c, int taps) {
   return tile_cfg;
 }
 
-// The tiling the library takes by itself
-int heuristic_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
-  const int split = split_tile(dtype, gemm_m, gemm_n, gemm_k, in_c, taps);
+// The tiling the library takes by itself.  kAutoInOrder: one that adds up every reduction front to back, as all but the
+// split ones do, so that a row's result is the same bits whatever the number of rows.
+constexpr int kAutoInOrder = -2;
+int heuristic_tile(int asked, int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
+  const int split = asked == kAutoInOrder ? -1 : split_tile(dtype, gemm_m, gemm_n, gemm_k, in_c, taps);
   return split >= 0 ? split : shallow_tile(pick_tile(gemm_m, gemm_n, 1), dtype, in_c, taps);
 }
 
@@ -2177,7 +2179,7 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S);
+    tile_cfg = heuristic_tile(tile_cfg, dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S);
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
@@ -2197,7 +2199,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int gemm_m = s.N * Ho * Wo;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S);
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2205,7 +2207,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
 
 int conv2d_dgrad_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   const int gemm_m = s.N * s.H * s.W;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S);
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2249,7 +2251,7 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S);
+    tile_cfg = heuristic_tile(tile_cfg, dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S);
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);

@@ -262,9 +262,13 @@ class GPT2Engine(EngineBase):
         def as4(t):
             return t.view(t.shape[0], 1, 1, t.shape[1])
 
+        # No sample depends on another here, so no sample's bf16 roundings should depend on how many others the
+        # batch has: forward products in one order of additions.  (fp32: the order is below the tolerance of any use.)
+        order = ops.IN_ORDER if self.dtype == torch.bfloat16 else -1
+
         def lin_fwd(name, x, y, add=None):
             ops.conv2d_fwd(ctx, as4(x), self._w(name + ".weight"), as4(y), 1, 0,
-                           bias=self._view(self.params, name + ".bias"), add=None if add is None else as4(add))
+                           bias=self._view(self.params, name + ".bias"), add=None if add is None else as4(add), tile_cfg=order)
 
         def side():
             return ctx.side_lane(wait_main=True) if self.overlap_wgrad else contextlib.nullcontext()
@@ -328,7 +332,7 @@ class GPT2Engine(EngineBase):
             hf = act(R, C)
             ln_fwd("transformer.ln_f", 2 * L, h, hf)
             logits = act(R, Vp, dtype=torch.float32)
-            ops.conv2d_fwd(ctx, as4(hf), self._w("transformer.wte.weight"), as4(logits), 1, 0)
+            ops.conv2d_fwd(ctx, as4(hf), self._w("transformer.wte.weight"), as4(logits), 1, 0, tile_cfg=order)
             dlogits = act(R, Vp).zero_()   # the padding columns stay zero: no kernel writes them
             ops.softmax_ce_lm(ctx, logits, plan.labels, plan.loss_rows, plan.loss, dlogits, V, B * (T - 1), loss_scale)
             plan.n_forward = len(prog)

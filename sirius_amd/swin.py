@@ -310,10 +310,14 @@ class SwinEngine(EngineBase):
         def as4(t):
             return t.view(t.shape[0], 1, 1, t.shape[1])
 
+        # No sample depends on another here, so no sample's bf16 roundings should depend on how many others the
+        # batch has: forward products in one order of additions.  (fp32: the order is below the tolerance of any use.)
+        order = ops.IN_ORDER if self.dtype == torch.bfloat16 else -1
+
         def lin_fwd(name, x, y, add=None, bias=True):
             ops.conv2d_fwd(ctx, as4(x), self._w(name + ".weight"), as4(y), 1, 0,
                            bias=self._view(self.params, name + ".bias") if bias else None,
-                           add=None if add is None else as4(add))
+                           add=None if add is None else as4(add), tile_cfg=order)
 
         def side():
             return ctx.side_lane(wait_main=True) if self.overlap_wgrad else contextlib.nullcontext()
