@@ -377,6 +377,9 @@ __global__ __launch_bounds__(256) void bn_apply_cols_kernel(ApplyArgs p) {
 // per-tile partials of its 64 channels itself (every workgroup of a column block repeats that sum, in the
 // same fixed order, from L2: row_blocks x 512 bytes), then applies.  The workgroups of slab 0 also write the
 // per-channel outputs (saved statistics, running statistics / dgamma, dbeta).
+// At small batches the launch is one chain of latencies, so everything that does not depend on the sums is requested
+// ahead of them (the channel's parameters, the thread's first row): the chain is one trip to memory instead of three
+// (20 images, 14x14 stage: forward 6.1 -> 5.8 us per launch, backward 7.4 -> 6.1).
 constexpr int kFusedCols = 64;
 constexpr int kFusedMaxRowBlocks = 256;
 
@@ -410,6 +413,36 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
   __shared__ float coef[3][kFusedCols];
   const int tid = threadIdx.x;
   const int c0 = blockIdx.x * kFusedCols;
+  const bool writer = blockIdx.y == 0;
+  const int tx = tid % CPR, ty = tid / CPR;
+  const int64_t cc = p.C / E;                    // chunks per full row
+  const int64_t col_chunk = c0 / E + tx;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * p.rows_per_slab;
+  int64_t r1 = r0 + p.rows_per_slab;
+  if (r1 > p.rows) r1 = p.rows;
+  const bool has_b = BWD || p.b != nullptr;
+  float par0 = 0.f, par1 = 0.f, par2 = 0.f, par3 = 0.f;   // gamma; beta or saved mean; saved 1/std or the running pair
+  if (tid < kFusedCols) {
+    const int c = c0 + tid;
+    par0 = p.gamma[c];
+    if (BWD) {
+      par1 = p.save_mean[c];
+      par2 = p.save_invstd[c];
+    } else {
+      par1 = p.beta[c];
+      if (writer && p.running_mean) {
+        par2 = p.running_mean[c];
+        par3 = p.running_var[c];
+      }
+    }
+  }
+  // the first row of this thread (a thread beyond the slab fetches the slab's last row and stores nothing)
+  Chunk fa, fb = zero_chunk();
+  {
+    const int64_t r = r0 + ty < r1 ? r0 + ty : r1 - 1;
+    fa.u = static_cast<const uint4*>(p.a)[r * cc + col_chunk];
+    if (has_b) fb.u = static_cast<const uint4*>(p.b)[r * cc + col_chunk];
+  }
   {
     const int pr = tid & 31, part = tid >> 5;
     double s0 = 0.0, q0 = 0.0, s1 = 0.0, q1 = 0.0;
@@ -455,29 +488,28 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
       q += red[k][tid >> 1][(tid & 1) * 2 + 1];
     }
     const double n = static_cast<double>(p.rows);
-    const bool writer = blockIdx.y == 0;
     if (!BWD) {
       const double mean = s / n;
       double var = q / n - mean * mean;
       if (var < 0.0) var = 0.0;
       const float invstd = 1.0f / sqrtf(static_cast<float>(var) + p.eps);
-      const float sc = p.gamma[c] * invstd;
+      const float sc = par0 * invstd;
       coef[0][tid] = sc;
-      coef[1][tid] = p.beta[c] - static_cast<float>(mean) * sc;
+      coef[1][tid] = par1 - static_cast<float>(mean) * sc;
       if (writer) {
         p.save_mean[c] = static_cast<float>(mean);
         p.save_invstd[c] = invstd;
         if (p.running_mean) {
           const double unbiased = p.rows > 1 ? var * n / (n - 1.0) : var;
-          p.running_mean[c] = (1.f - p.momentum) * p.running_mean[c] + p.momentum * static_cast<float>(mean);
-          p.running_var[c] = (1.f - p.momentum) * p.running_var[c] + p.momentum * static_cast<float>(unbiased);
+          p.running_mean[c] = (1.f - p.momentum) * par2 + p.momentum * static_cast<float>(mean);
+          p.running_var[c] = (1.f - p.momentum) * par3 + p.momentum * static_cast<float>(unbiased);
         }
       }
     } else {
-      const double invstd = p.save_invstd[c];
-      const double scale = static_cast<double>(p.gamma[c]) * invstd;
+      const double invstd = par2;
+      const double scale = static_cast<double>(par0) * invstd;
       const double cb = -scale * invstd * (q / n);
-      const double cz = -scale * (s / n) - cb * p.save_mean[c];
+      const double cz = -scale * (s / n) - cb * par1;
       coef[0][tid] = static_cast<float>(scale);
       coef[1][tid] = static_cast<float>(cb);
       coef[2][tid] = static_cast<float>(cz);
@@ -490,7 +522,6 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
   }
   __syncthreads();
 
-  const int tx = tid % CPR, ty = tid / CPR;
   float k0[E], k1[E], k2[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -498,12 +529,6 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
     k1[e] = coef[1][tx * E + e];
     k2[e] = BWD ? coef[2][tx * E + e] : 0.f;
   }
-  const int64_t cc = p.C / E;                    // chunks per full row
-  const int64_t col_chunk = c0 / E + tx;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.y) * p.rows_per_slab;
-  int64_t r1 = r0 + p.rows_per_slab;
-  if (r1 > p.rows) r1 = p.rows;
-  const bool has_b = BWD || p.b != nullptr;
   auto finish = [&](int64_t i, const Chunk& ca, const Chunk& cb) {
     float va[E], vb[E], vo[E];
     chunk_to_float<T>(ca, va);
@@ -525,8 +550,9 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
     }
     static_cast<uint4*>(p.out)[i] = float_to_chunk<T>(vo).u;
   };
-  // two rows per trip: both rows' chunks are requested before either is used
-  for (int64_t r = r0 + ty; r < r1; r += 2 * RPP) {
+  if (r0 + ty < r1) finish((r0 + ty) * cc + col_chunk, fa, fb);
+  // the rest two rows per trip: both rows' chunks are requested before either is used
+  for (int64_t r = r0 + ty + RPP; r < r1; r += 2 * RPP) {
     const int64_t i0 = r * cc + col_chunk, i1 = i0 + RPP * cc;
     const bool second = r + RPP < r1;
     Chunk a0, a1, b0 = zero_chunk(), b1 = zero_chunk();
