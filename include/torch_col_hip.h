@@ -422,6 +422,11 @@ int tch_embedding_fwd(tch_context* ctx, int dtype, const int64_t* ids, const voi
                       int T, int C, int vocab);
 int tch_embedding_bwd(tch_context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B,
                       int T, int C, int vocab, int accumulate_wpe, int32_t* chain);
+/* The links between the positions that share a token depend on the ids alone: made ahead (beside the forward pass), and
+ * a backward that finds them in `chain` (the same ids, B, T and vocab). */
+int tch_embedding_chain(tch_context* ctx, const int64_t* ids, int32_t* chain, int B, int T, int vocab);
+int tch_embedding_bwd_chained(tch_context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B,
+                              int T, int C, int vocab, int accumulate_wpe, int32_t* chain);
 /* C[z](m, n) (+)= alpha * sum_k A[z](m, k) B[z](n, k), z = zo * batch_inner + zi; A(m, k) at
  * a + zo * a_bo + zi * a_bi + m * a_rs + k * a_cs (elements), B alike with n; C row-major with ldc.
  * One stride of each operand must be 1.  causal (square problems under a causal mask): 0 nothing is known;

@@ -354,7 +354,16 @@ int tch_embedding_fwd(tch_context* ctx, int dtype, const int64_t* ids, const voi
 
 int tch_embedding_bwd(tch_context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B,
                       int T, int Cc, int vocab, int accumulate_wpe, int32_t* chain) {
-  return embedding_bwd(C(ctx), dtype, ids, dy, dwte, dwpe, B, T, Cc, vocab, accumulate_wpe, chain);
+  return embedding_bwd(C(ctx), dtype, ids, dy, dwte, dwpe, B, T, Cc, vocab, accumulate_wpe, chain, 0);
+}
+
+int tch_embedding_chain(tch_context* ctx, const int64_t* ids, int32_t* chain, int B, int T, int vocab) {
+  return embedding_chain(C(ctx), ids, chain, B, T, vocab);
+}
+
+int tch_embedding_bwd_chained(tch_context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B,
+                      int T, int Cc, int vocab, int accumulate_wpe, int32_t* chain) {
+  return embedding_bwd(C(ctx), dtype, ids, dy, dwte, dwpe, B, T, Cc, vocab, accumulate_wpe, chain, 1);
 }
 
 int tch_batched_gemm(tch_context* ctx, int dtype, const void* a, const void* b, void* c, int M, int N, int K,

@@ -160,7 +160,8 @@ int adamw_step(Context* ctx, float* param, const float* grad, float* exp_avg, fl
 int embedding_fwd(Context* ctx, int dtype, const int64_t* ids, const void* wte, const void* wpe, void* out, int B, int T,
                   int C, int vocab);
 int embedding_bwd(Context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B, int T,
-                  int C, int vocab, int accumulate_wpe, int32_t* chain);
+                  int C, int vocab, int accumulate_wpe, int32_t* chain, int chain_ready);
+int embedding_chain(Context* ctx, const int64_t* ids, int32_t* chain, int B, int T, int vocab);
 
 // swin_ops.hip
 int window_partition(Context* ctx, int dtype, const void* src, void* dst, const void* add, int B, int H, int W, int C,

@@ -871,19 +871,24 @@ int embedding_fwd(Context* ctx, int dtype, const int64_t* ids, const void* wte, 
                         : launch(ctx, embed_fwd_kernel<float>, grid, dim3(256), a, "embed_fwd_kernel<f32>", bytes, 1);
 }
 
+int embedding_chain(Context* ctx, const int64_t* ids, int32_t* chain, int B, int T, int vocab) {
+  TCH_CHECK_ARG(ids && chain && B > 0 && T > 0 && vocab > 0, "embedding_chain: null tensor or empty");
+  TCH_CHECK_ARG(static_cast<int64_t>(B) * T <= 0x7fffffff - 4096, "embedding_chain: too many tokens");
+  const int n = B * T;
+  ChainArgs ca{ids, chain, chain + n, n, vocab};
+  return launch(ctx, embed_chain_kernel, dim3((n + 63) / 64), dim3(256), ca, "embed_chain_kernel", 16.0 * n, 1);
+}
+
 int embedding_bwd(Context* ctx, int dtype, const int64_t* ids, const void* dy, float* dwte, float* dwpe, int B, int T,
-                  int C, int vocab, int accumulate_wpe, int32_t* chain) {
+                  int C, int vocab, int accumulate_wpe, int32_t* chain, int chain_ready) {
   if (int rc = check_rows("embedding_bwd", dtype, static_cast<int64_t>(B) * T, C)) return rc;
   TCH_CHECK_ARG(ids && dy && dwte && dwpe && vocab > 0, "embedding_bwd: null tensor");
   const int E = dtype == kBF16 ? 8 : 4;
   const int n = B * T;
   EmbedArgs a{ids, nullptr, nullptr, nullptr, dy, dwte, dwpe, static_cast<int64_t>(B) * T, T, C, C / E, vocab, B,
               accumulate_wpe, chain, chain ? chain + n : nullptr};
-  if (chain) {
-    ChainArgs ca{ids, chain, chain + n, n, vocab};
-    if (int rc = launch(ctx, embed_chain_kernel, dim3((n + 63) / 64), dim3(256), ca, "embed_chain_kernel", 16.0 * n, 1))
-      return rc;
-  }
+  if (chain && !chain_ready)
+    if (int rc = embedding_chain(ctx, ids, chain, B, T, vocab)) return rc;
   const double bytes = static_cast<double>(a.tokens) * C * (dtype == kBF16 ? 2.0 : 4.0) + 8.0 * a.tokens * C;
   const dim3 grid(flat_blocks(a.tokens * a.cc));
   return dtype == kBF16 ? launch(ctx, embed_bwd_kernel<bf16>, grid, dim3(256), a, "embed_bwd_kernel<bf16>", bytes, 1)

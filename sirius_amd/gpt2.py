@@ -298,6 +298,11 @@ class GPT2Engine(EngineBase):
             h = act(R, C)
             ops.embedding_fwd(ctx, plan.ids, self._w("transformer.wte.weight").view(Vp, C),
                               self._w("transformer.wpe.weight"), h.view(B, T, C))
+            # the embedding gradient's links depend on the ids alone: made on the idle second lane, off the tail of the step
+            # (a fork needs a main-lane launch ahead of it: the copy of the ids is none of the program's)
+            chain = act(2 * B * T, dtype=torch.int32)
+            with side():
+                ops.embedding_chain(ctx, plan.ids, chain, Vp)
             saved = []
             for i in range(L):
                 pre = f"transformer.h.{i}."
@@ -400,7 +405,7 @@ class GPT2Engine(EngineBase):
                 ctx.join()
             # tied weights: the scattered embedding gradient lands on top of the head's weight gradient
             ops.embedding_bwd(ctx, plan.ids, g.view(B, T, C), self._view(self.grads, "transformer.wte.weight").view(Vp, C),
-                              self._view(self.grads, "transformer.wpe.weight"), chain=act(2 * B * T, dtype=torch.int32))
+                              self._view(self.grads, "transformer.wpe.weight"), chain=chain, chain_ready=True)
         finally:
             ctx.end_record()
         plan.prog, plan.marks, plan.keep, plan.logits = prog, marks, keep, logits

@@ -861,15 +861,25 @@ def embedding_fwd(ctx, ids, wte, wpe, out):
           "tch_embedding_fwd")
 
 
-def embedding_bwd(ctx, ids, dy, dwte, dwpe, accumulate_wpe=False, chain=None):
+def embedding_chain(ctx, ids, chain, vocab):
+    """The links embedding_bwd follows between positions that share a token, into `chain` (int32, 2 * B * T)."""
+    B, T = ids.shape
+    assert chain.dtype == torch.int32 and chain.numel() >= 2 * B * T
+    check(lib().tch_embedding_chain(ctx.handle, _p(ids), _p(chain), B, T, vocab), "tch_embedding_chain")
+
+
+def embedding_bwd(ctx, ids, dy, dwte, dwpe, accumulate_wpe=False, chain=None, chain_ready=False):
     """chain: int32 scratch of 2 * B * T elements; with it the result is the same bit for bit every run (rows that
-    share a token are added in position order), without it fp32 atomics decide the order."""
+    share a token are added in position order), without it fp32 atomics decide the order.  chain_ready: it holds
+    what embedding_chain made of the same ids."""
     B, T = ids.shape
     vocab, C = dwte.shape
     assert tuple(dy.shape) == (B, T, C) and dwte.dtype == dwpe.dtype == torch.float32 and dwpe.shape[0] >= T
+    assert chain is not None or not chain_ready
     assert chain is None or (chain.dtype == torch.int32 and chain.numel() >= 2 * B * T)
-    check(lib().tch_embedding_bwd(ctx.handle, dtype_code(dy), _p(ids), _p(dy), _p(dwte), _p(dwpe), B, T, C, vocab,
-                                  int(accumulate_wpe), _p(chain)), "tch_embedding_bwd")
+    entry = lib().tch_embedding_bwd_chained if chain_ready else lib().tch_embedding_bwd
+    check(entry(ctx.handle, dtype_code(dy), _p(ids), _p(dy), _p(dwte), _p(dwpe), B, T, C, vocab, int(accumulate_wpe),
+                _p(chain)), "tch_embedding_bwd")
 
 
 def batched_gemm(ctx, a, b, c, M, N, K, a_strides, b_strides, ldc, batch=(1, 1), a_batch=(0, 0), b_batch=(0, 0),
