@@ -960,6 +960,12 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
 //   * a step never straddles a filter tap (channels % 64 == 0), so the tap walk is scalar:
 //     a lane keeps one byte offset and one validity bit per tap for each row it loads;
 //   * NBUF tiles in flight, one barrier per step;
+//   * ROT = 2 reads the operands of the next step into a second register set while this step is multiplied: the barrier
+//     hands over a tile one step before it is needed and the LDS latency passes behind the multiplies.  What bounds
+//     the small tiles then is LDS itself (a 64 x 64 tile: 32 KB read, 16 KB written per step).  1024 x 768 over 3072:
+//     24.3 us with a whole trip to memory per step (0.47 us each), 16.3 with the loads really in flight, 13.5 pipelined;
+//     2048 rows 25.3 / 20.6 / 17.8 (128 x 64 on eight wavefronts); 8192 rows 54 / 50.6 / 43.2 (128 x 128, 935 TFLOP/s
+//     of the 1310 a library product of 8192^3 reaches here);
 //   * KS = 32 halves the step (64-byte rows, sixteen rows per direct load): half the LDS per tile in flight, so
 //     more workgroups share a CU and a small grid is resident in one round.
 constexpr int kStep2 = 64;                  // reduction elements per step
@@ -974,8 +980,26 @@ __device__ inline void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char* d
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)dst, 16, voff, soff, 0, 0);
 }
 
+// the registers belong to their values up to this point of the program
+template <int A, int B>
+__device__ inline void hold(uint4_t (&r)[A][B]) {
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int j = 0; j < B; ++j) asm volatile("" : "+v"(r[i][j]));
+}
+
+// All but the newest N of this wave's direct loads have landed, all its LDS accesses are done, and every wave of the
+// workgroup is here.  Not __syncthreads(): the compiler puts a wait for EVERY outstanding direct load in front of
+// that (a direct load is an LDS write to it), which leaves no tile in flight across the barrier whatever NBUF is:
+// each step then pays a whole trip to memory (a 64 x 64 tile: 0.47 us per 64-element step with two buffers or three).
+template <int N>
+__device__ inline void wait_and_meet() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 template <int MODE, int WM, int WN, int TM, int TN, int NBUF, int ROT = 0, int KS = kStep2>
-__global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
+__global__ __launch_bounds__(WM* WN * 64, ROT == 2 ? 2 : 1) void igemm2_kernel(IgemmArgs p) {
   using T = bf16;
   constexpr int E = 8;
   constexpr int BM = WM * TM * 32;
@@ -1083,26 +1107,29 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     const int tap_elems = (MODE == kFwd) ? (ld_r * in_w + ld_s) * in_c : -((ld_r >> sl) * in_w + (ld_s >> sl)) * in_c;
     const int a_step = (tap_elems + ld_cb * KS) * 2;
     const int b_step = ld_kt * RB;
+    // a tile behind the last one: every offset out of range, so zeros land and memory is not asked
+    const uint32_t tap_bit = ld_kt < nk ? 1u << ld_t : 0u;
+    const int beyond = ld_kt < nk ? 0 : static_cast<int>(kOutOfRange);
     unsigned char* dst_a = lds + buf * BUF_BYTES + wave * A_LD * 1024;
     unsigned char* dst_b = lds + buf * BUF_BYTES + A_BYTES + wave * B_LD * 1024;
 #pragma unroll
     for (int j = 0; j < A_LD; ++j) {
-      const bool ok = (a_taps[j] >> ld_t) & 1u;
+      const bool ok = (a_taps[j] & tap_bit) != 0;
       const int off = ok ? a_off[j] + a_step : static_cast<int>(kOutOfRange);
       load_to_lds(rsrc_a, dst_a + j * 1024, off, 0);
     }
 #pragma unroll
     for (int j = 0; j < B_LD; ++j)
-      load_to_lds(rsrc_b, dst_b + j * 1024, b_off[j], b_step);
+      load_to_lds(rsrc_b, dst_b + j * 1024, b_off[j] | beyond, b_step);
     ++ld_kt;
-    if (++ld_cb == cblocks) {
-      ld_cb = 0;
-      ++ld_t;
-      if (++ld_s == p.S) {
-        ld_s = 0;
-        ++ld_r;
-      }
-    }
+    // selects, not branches: no block boundary while operand reads are in flight
+    const int next_tap = ++ld_cb == cblocks ? 1 : 0;
+    ld_cb = next_tap ? 0 : ld_cb;
+    ld_t += next_tap;
+    ld_s += next_tap;
+    const int next_row = ld_s == p.S ? 1 : 0;
+    ld_s = next_row ? 0 : ld_s;
+    ld_r += next_row;
   };
 
   f32x16_t acc[TM][TN];
@@ -1168,10 +1195,9 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     multiply(fa1, fb1);
   };
 
-  // vmcnt(n): at most n of this wave's loads still in flight (gfx9 encoding, nothing else waited for)
+  // at most this many of a wave's loads may still be in flight when its part of the oldest tile must have landed
   constexpr int LOADS = A_LD + B_LD;
   constexpr int AHEAD = (NBUF - 2) * LOADS;
-  constexpr int WAIT_IMM = (AHEAD & 0xF) | ((AHEAD >> 4) << 14) | (0x7 << 4) | (0xF << 8);
   static_assert(AHEAD < 64, "vmcnt range");
 
   // One step = wait until only the newer tiles' loads are outstanding (then this wave's part of tile kt has
@@ -1182,14 +1208,68 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
   // classes in every step); the last nk % NBUF steps follow one by one.
   auto step = [&](int kt, int u) {
     if (kt + NBUF - 1 <= nk)
-      __builtin_amdgcn_s_waitcnt(WAIT_IMM);
+      wait_and_meet<AHEAD>();
     else
-      __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));
-    __syncthreads();
+      wait_and_meet<0>();
     if (kt + NBUF - 1 < nk) issue_loads((u + NBUF - 1) % NBUF);
     compute(u);
   };
-  if constexpr (ROT) {
+  if constexpr (ROT == 2) {
+    // Pipelined over the reduction steps: the operands of tile kt+1 are read into a second register set while tile kt
+    // is multiplied.
+    static_assert(NBUF == 2 || NBUF == 4, "the register sets alternate with the buffers");
+    constexpr int SL = KS / 16;
+    uint4_t fa[2][SL][TM], fb[2][SL][TN];
+    // the buffer is part of the reads' immediate offset where that reaches (64 KB)
+    auto read_tile = [&](auto buf_c, uint4_t (&ra)[SL][TM], uint4_t (&rb)[SL][TN]) {
+      constexpr int AT = decltype(buf_c)::value * BUF_BYTES;
+      constexpr bool IMM = AT + BUF_BYTES <= 65536;
+#pragma unroll
+      for (int kk = 0; kk < SL; ++kk) {
+        const uint32_t cx = (2 * kk + frag_half) * 16;
+        const uint32_t pa = (a_rd ^ cx) + (IMM ? 0 : AT), pb = (b_rd ^ cx) + (IMM ? 0 : AT);
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+          asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(ra[kk][tm]) : "v"(pa), "n"(tm * 32 * RB + (IMM ? AT : 0)));
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(rb[kk][tn]) : "v"(pb), "n"(tn * 32 * RB + (IMM ? AT : 0)));
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < NBUF; ++s) issue_loads(s);
+    wait_and_meet<(NBUF - 1) * LOADS>();
+    read_tile(std::integral_constant<int, 0>{}, fa[0], fb[0]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    auto pstep = [&](auto u_c) {
+      constexpr int u = decltype(u_c)::value, set = u & 1;
+      wait_and_meet<AHEAD>();
+      read_tile(std::integral_constant<int, (u + 1) % NBUF>{}, fa[set ^ 1], fb[set ^ 1]);
+      issue_loads(u);
+#pragma unroll
+      for (int kk = 0; kk < SL; ++kk) multiply(fa[set][kk], fb[set][kk]);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      // the registers being filled stay theirs until here, also behind the last tile where nobody multiplies them
+      hold(fa[set ^ 1]);
+      hold(fb[set ^ 1]);
+    };
+    int kt0 = 0;
+    for (; kt0 + NBUF <= nk; kt0 += NBUF) {
+      pstep(std::integral_constant<int, 0>{});
+      pstep(std::integral_constant<int, 1>{});
+      if constexpr (NBUF == 4) {
+        pstep(std::integral_constant<int, 2>{});
+        pstep(std::integral_constant<int, 3>{});
+      }
+    }
+    if (kt0 < nk) pstep(std::integral_constant<int, 0>{});
+    if constexpr (NBUF == 4) {
+      if (kt0 + 1 < nk) pstep(std::integral_constant<int, 1>{});
+      if (kt0 + 2 < nk) pstep(std::integral_constant<int, 2>{});
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile: the epilogue uses their place
+  } else if constexpr (ROT == 1) {
     // Rotated loop for the large tiles, whose workgroup has a compute unit to itself (nobody else fills the
     // gap a barrier leaves): the barrier that hands over tile kt+1 sits BEFORE the last quarter of tile kt's
     // multiplies, whose operands are in registers by then, and the first operand reads of tile kt+1 are issued
@@ -1497,8 +1577,6 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
 // The reduction runs channel block by channel block (taps innermost), so sums round differently from
 // igemm2_kernel's tap-major order.
 // ---------------------------------------------------------------------------
-constexpr int vmcnt_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
 template <int MODE, int TN, int NBUF, int P_LD>
 __global__ __launch_bounds__(256) void igemm3_kernel(IgemmArgs p) {
   using T = bf16;
@@ -1661,12 +1739,11 @@ __global__ __launch_bounds__(256) void igemm3_kernel(IgemmArgs p) {
     for (int tap = 0; tap < 9; ++tap) {
       const int kt = cb * 9 + tap;
       if (kt + AHEAD > nk)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        wait_and_meet<0>();
       else if (tap >= 1 && tap <= AHEAD && next_patch)
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NBUF - 2) * B_LD + P_LD));
+        wait_and_meet<(NBUF - 2) * B_LD + P_LD>();
       else
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NBUF - 2) * B_LD));
-      __syncthreads();
+        wait_and_meet<(NBUF - 2) * B_LD>();
       // 9 taps per channel block: with three buffers the buffer of a step is a constant of the unrolled loop
       const int buf = NBUF == 3 ? tap % 3 : kt % NBUF;
       const int buf_ahead = NBUF == 3 ? (tap + AHEAD) % 3 : (kt + AHEAD) % NBUF;
@@ -1810,7 +1887,7 @@ int launch_cfg2(Context* ctx, IgemmArgs& a, double flops) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
   static const std::string name = std::string("igemm2_kernel<bf16,") + (MODE == kFwd ? "fwd," : "dgrad,") +
                                   std::to_string(BM) + "x" + std::to_string(BN) + "," + std::to_string(NBUF) + "buf" +
-                                  (WM * WN == 8 ? ",8w" : "") + (KS == 32 ? ",k32" : "") + (ROT ? ",rot>" : ">");
+                                  (WM * WN == 8 ? ",8w" : "") + (KS == 32 ? ",k32" : "") + (ROT == 1 ? ",rot>" : ROT == 2 ? ",pipe>" : ">");
   a.tiles_m = (a.gemm_m + BM - 1) / BM;
   a.tiles_n = (a.gemm_n + BN - 1) / BN;
   static const int group_env = [] {
@@ -1847,6 +1924,9 @@ int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
 }
 
 // The 3x3 patch kernel: stride 1, pad 1, input channels in blocks of 64, rows short enough for the patch
+bool patch_kernel_fits(const ConvShape& s, int in_c) {
+  return s.R == 3 && s.S == 3 && s.stride == 1 && s.pad == 1 && in_c % kStep2 == 0 && 128 + 2 * (s.W + 1) <= 256;
+}
 template <int MODE>
 bool patch_kernel_fits(const IgemmArgs& a) {
   const int in_c = MODE == kFwd ? a.C : a.K;
@@ -1899,6 +1979,16 @@ enum SplitTile : int {
   kSplit64Pair = 19,     // 64 x 64, 4, 2
   kSplit64x32Deep = 20,  // 64 x 32, 8, 3
 };
+
+// Tilings of igemm2_kernel with pipelined operand reads
+enum PipeTile : int {
+  kPipe64 = 21,       // 64 x 64
+  kPipe128x64 = 22,   // 128 x 64, eight wavefronts
+  kPipe128 = 23,      // 128 x 128
+};
+
+// the tiling of the same shape that runs where a pipelined one does not exist
+int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : tile_cfg == kPipe128x64 ? 1 : 0; }
 
 template <typename T, int MODE>
 int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
@@ -1955,6 +2045,13 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
         return tile_cfg == 6 ? launch_cfg2<MODE, 2, 2, 2, 1, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 1, 1, 2>(ctx, a, flops);
       tile_cfg -= 5;
     }
+    // 21 - 23: operand reads pipelined over the reduction steps (see igemm2_kernel): 64 x 64 with four tiles in LDS,
+    // 128 x 64 on eight wavefronts with four, 128 x 128 with two
+    if (tile_cfg >= kPipe64 && setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32) {
+      if (tile_cfg == kPipe64) return launch_cfg2<MODE, 2, 2, 1, 1, 4, 2>(ctx, a, flops);
+      if (tile_cfg == kPipe128x64) return launch_cfg2<MODE, 4, 2, 1, 1, 4, 2>(ctx, a, flops);
+      return launch_cfg2<MODE, 2, 2, 2, 2, 2, 2>(ctx, a, flops);
+    }
     if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32 && tile_cfg >= 0 && tile_cfg <= 2) {
       if (tile_cfg == 0)
         return setting == 3 ? launch_cfg2<MODE, 2, 2, 2, 2, 3>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 2, 2, 2>(ctx, a, flops);
@@ -1967,6 +2064,7 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
   if (tile_cfg == 6 || tile_cfg == 7) tile_cfg -= 5;
   if (tile_cfg == 9 || tile_cfg == 10) tile_cfg = 0;
   if (tile_cfg >= 11 && tile_cfg <= 14) tile_cfg = tile_cfg <= 12 ? 0 : tile_cfg - 12;
+  if (tile_cfg >= kPipe64) tile_cfg = pipe_stand_in(tile_cfg);
   switch (tile_cfg) {
     case 0:
       return launch_cfg<T, MODE, 2, 2, 2, 2>(ctx, a, flops);  // 128 x 128
@@ -1987,6 +2085,7 @@ double conv_flops(const ConvShape& s, int Ho, int Wo) {
 // rows of the workgroup tile of a tiling number (5 = the 3x3 patch kernel, or tiling 1 where it does not fit)
 int tile_rows(int tile_cfg) {
   if (tile_cfg == 9 || tile_cfg == 10) return 256;
+  if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 ? 64 : 128;
   if (tile_cfg >= kSplit32) return tile_cfg <= kSplit32Deep ? 32 : 64;
   if (tile_cfg >= 11 && tile_cfg <= 14) return tile_cfg == 14 ? 64 : 128;
   return (tile_cfg == 5 || tile_cfg == 6) ? 128 : tile_cfg >= 2 ? 64 : 128;
@@ -2011,11 +2110,17 @@ bool wants_huge_tile(int dtype, int gemm_m, int gemm_n, int in_c, int taps) {
 // igemm4_kernel: whole 64-byte steps of input channels, one bit per tap
 bool split_tile_fits(int dtype, int in_c, int taps) { return in_c % (dtype == kBF16 ? 32 : 16) == 0 && taps <= 32; }
 
+// igemm2_kernel: whole 128-byte steps of bf16 input channels, one bit per tap
+bool direct_tile_fits(int dtype, int in_c, int taps) {
+  return dtype == kBF16 && in_c % 64 == 0 && taps <= 32 && igemm2_setting() != 0;
+}
+
 // The tiling that runs when `tile_cfg` is asked for: the 256 x 256 tilings exist for the direct-to-LDS kernel only
 // and stand for 128 x 128 elsewhere (the statistics' row tiles follow the tiling that runs).
 int effective_tile(int tile_cfg, int dtype, int in_c, int taps) {
   if ((tile_cfg == 9 || tile_cfg == 10) && !(dtype == kBF16 && in_c % 64 == 0 && taps <= 32 && igemm2_setting() != 0))
     return 0;
+  if (tile_cfg >= kPipe64) return direct_tile_fits(dtype, in_c, taps) ? tile_cfg : pipe_stand_in(tile_cfg);
   if (tile_cfg >= kSplit32 && !split_tile_fits(dtype, in_c, taps)) return 2;
   return tile_cfg;
 }
@@ -2028,52 +2133,85 @@ int pick_tile(int gemm_m, int gemm_n, int splits) {
   return 2;
 }
 
-// Where the output has too few tiles to fill the chip, the reduction is split inside the workgroup (igemm4_kernel):
-// smaller tiles as the grid shrinks, and from a reduction depth on that pays for the partial tiles that meet in LDS.
-// The lines lie where the layers of ResNet-152 at batches 1-64 and the projections of Swin-B and GPT-2 at 200-2331 rows
-// crossed over, timed back to back with cold filters (bf16, us, before -> after): 196 x 256 over 2304 13.2 -> 6.1,
-// 49 x 512 over 4608 22.1 -> 8.1 (32 x 32); 784 x 512 over 4608 36.9 -> 14.8 (64 x 32); 3920 x 256 over 2304
-// 20.6 -> 13.9, 1024 x 768 over 3072 24.3 -> 15.9 (64 x 64, one workgroup per CU); 4704 x 256 over 2304 21.0 -> 15.9
-// (two).  Beyond those sizes the shared operand tiles of the other kernels win.  fp32 multiplies at 1/16 of the rate,
-// so it gains from spreading them over every SIMD at shallower reductions (784 x 256 over 2304: 77.6 -> 14.8 us) and
-// keeps the 64 x 64 split tile on large grids too (2048 x 3072 over 768: 100 -> 86 us).  -1: none of them.
+// What a bf16 product on the direct-to-LDS kernels takes with each of the tilings worth having, in microseconds:
+//   start + round * r + steps * max(alone, shared * r) + store * (outputs / 10^6)
+// with r = workgroups per compute unit, rounded up, and steps = 64-element reduction steps.  `alone` is a step of one
+// workgroup on a CU (a chain of latencies), `shared` what a step costs each of several that share the CU's operand
+// path; `round` is the epilogue, which those take in turn.  The constants are least-squares fits (mean error 3-7 %) to
+// kernel times of 280 products and convolutions: the projections of GPT-2 at 128-8192 rows and of Swin-B at 2-32
+// images forward, ResNet's 1x1 and 3x3 layers at 1-64 images (forward with batch sums, inference epilogue) for the
+// first table; ResNet's data gradients with the BatchNorm sums, whose epilogue reads two more tensors, for the second.
+// Choosing by them is within 2 % of always taking the fastest tiling; the tile-count thresholds they replace were
+// 8 % off at the sizes they were tuned on, up to 1.9x between.
+struct TileCost {
+  int cfg, bm, bn;
+  float start, round, alone, shared, store;
+};
+const TileCost kPlainCost[] = {
+    {0, 128, 128, 3.72f, 2.39f, 0.596f, 0.377f, 0.05f},  {1, 128, 64, 3.69f, 1.28f, 0.377f, 0.243f, 0.24f},
+    {2, 64, 64, 3.51f, 0.64f, 0.261f, 0.158f, 0.14f},    {5, 128, 64, 0.93f, 4.74f, 0.267f, 0.067f, 0.47f},
+    {12, 128, 128, 4.48f, 0.88f, 0.798f, 0.474f, 0.20f}, {13, 128, 64, 4.47f, 0.15f, 0.495f, 0.347f, 0.35f},
+    {14, 64, 64, 3.72f, 0.00f, 0.391f, 0.235f, 0.40f},   {kPipe64, 64, 64, 3.43f, 1.05f, 0.199f, 0.145f, 0.40f},
+    {kPipe128, 128, 128, 3.67f, 2.67f, 0.625f, 0.352f, 0.08f},
+    {kPipe128x64, 128, 64, 2.75f, 2.21f, 0.108f, 0.262f, 0.48f},
+    {kSplit32, 32, 32, 3.28f, 0.21f, 0.092f, 0.079f, 2.14f},
+    {kSplit32Deep, 32, 32, 3.47f, 0.07f, 0.075f, 0.082f, 3.11f},
+    {kSplit64x32, 64, 32, 3.46f, 0.19f, 0.147f, 0.127f, 1.27f}};
+const TileCost kSumsCost[] = {
+    {0, 128, 128, 5.71f, 2.89f, 0.629f, 0.424f, 0.40f},  {1, 128, 64, 4.73f, 2.32f, 0.413f, 0.280f, 0.26f},
+    {2, 64, 64, 4.58f, 1.30f, 0.285f, 0.184f, 0.25f},    {5, 128, 64, 1.28f, 6.10f, 0.266f, 0.067f, 0.55f},
+    {12, 128, 128, 6.18f, 1.64f, 0.818f, 0.501f, 0.55f}, {13, 128, 64, 5.57f, 1.10f, 0.528f, 0.363f, 0.31f},
+    {14, 64, 64, 4.79f, 0.70f, 0.408f, 0.242f, 0.47f},   {kPipe64, 64, 64, 4.09f, 1.97f, 0.225f, 0.148f, 0.55f},
+    {kPipe128, 128, 128, 5.95f, 3.00f, 0.665f, 0.408f, 0.45f},
+    {kPipe128x64, 128, 64, 2.69f, 5.40f, 0.272f, 0.291f, 0.57f},
+    {kSplit32, 32, 32, 3.44f, 0.48f, 0.108f, 0.087f, 3.96f},
+    {kSplit32Deep, 32, 32, 4.20f, 0.38f, 0.062f, 0.082f, 5.42f},
+    {kSplit64x32, 64, 32, 4.16f, 0.44f, 0.168f, 0.134f, 2.81f}};
+
+// fp32 where the output has too few tiles to fill the chip, and on large grids too: the reduction is split inside the
+// workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 multiplies at 1/16 of the bf16 rate, so it
+// gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us; 2048 x 3072 over 768: 100 -> 86).
+// -1: none of them.
+// (bf16 with channels that are no whole 64-element step: the two smallest forms only.)
 int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
   if (igemm2_setting() == 0 || !split_tile_fits(dtype, in_c, taps)) return -1;
   const int64_t t32 = tiles_for(gemm_m, gemm_n, 32, 32), t64 = tiles_for(gemm_m, gemm_n, 64, 64);
   if (t32 <= 256) return gemm_k >= 1024 ? kSplit32Deep : kSplit32;
-  if (dtype == kBF16) {
-    if (t32 <= 512) return gemm_k >= 1536 ? kSplit64x32 : kSplit32;
-    if (t64 <= 256 && gemm_k >= 512) return kSplit64;
-    if (t64 <= 448 && gemm_k >= 1024) return kSplit64Pair;
-    return -1;
-  }
+  if (dtype == kBF16) return t32 <= 512 ? kSplit32 : -1;
   if (t32 <= 512) return gemm_k >= 768 ? kSplit64x32Deep : kSplit32;
   if (t64 <= 256 && gemm_k >= 768) return kSplit64;
   if (t64 <= 512 && gemm_k >= 512) return kSplit64x32;
   return gemm_k >= 256 && tiles_for(gemm_m, gemm_n, 128, 128) < 384 ? kSplit64Pair : -1;
 }
 
-// The heuristic's tiling for a pointwise product with a shallow reduction (at most 256 channels): the same tile
-// shape with 32-element reduction steps (half the LDS per workgroup, more workgroups per CU), which measured faster
-// on every such layer of the three models (0 -> 12, 1 -> 13, 2 -> 14: same tile rows, so the statistics' row
-// tiles do not change).  TCH_IGEMM_K32=0 keeps the 64-element steps.
-int shallow_tile(int tile_cfg, int dtype, int in_c, int taps) {
-  static const bool on = [] {
-    const char* e = getenv("TCH_IGEMM_K32");
-    return !(e && atoi(e) == 0);
-  }();
-  if (on && dtype == kBF16 && taps == 1 && in_c % 64 == 0 && in_c <= 256 && igemm2_setting() != 0 && tile_cfg >= 0 &&
-      tile_cfg <= 2)
-    return tile_cfg + 12;
-  return tile_cfg;
-}
-
 // The tiling the library takes by itself.  kAutoInOrder: one that adds up every reduction front to back, as all but the
-// split ones do, so that a row's result is the same bits whatever the number of rows.
+// split ones do, so that a row's result is the same bits whatever the number of rows.  (The patch kernel, tiling 5, has
+// an order of its own: never with kAutoInOrder.)
 constexpr int kAutoInOrder = -2;
-int heuristic_tile(int asked, int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
-  const int split = asked == kAutoInOrder ? -1 : split_tile(dtype, gemm_m, gemm_n, gemm_k, in_c, taps);
-  return split >= 0 ? split : shallow_tile(pick_tile(gemm_m, gemm_n, 1), dtype, in_c, taps);
+struct TileQuery {
+  int dtype, gemm_m, gemm_n, gemm_k, in_c, taps;
+  bool patch;   // the 3x3 patch kernel fits
+  bool sums;    // data gradient with the BatchNorm sums in its epilogue
+};
+int heuristic_tile(int asked, const TileQuery& q) {
+  if (!direct_tile_fits(q.dtype, q.in_c, q.taps)) {
+    const int split = asked == kAutoInOrder ? -1 : split_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k, q.in_c, q.taps);
+    return split >= 0 ? split : pick_tile(q.gemm_m, q.gemm_n, 1);
+  }
+  const float steps = static_cast<float>(q.gemm_k) / 64.f, store = static_cast<float>(q.gemm_m) * q.gemm_n * 1e-6f;
+  int best = 2;
+  float best_us = INFINITY;
+  for (const TileCost& t : q.sums ? kSumsCost : kPlainCost) {
+    if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;
+    if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
+    const float r = static_cast<float>((tiles_for(q.gemm_m, q.gemm_n, t.bm, t.bn) + 255) / 256);
+    const float us = t.start + t.round * r + steps * fmaxf(t.alone, t.shared * r) + t.store * store;
+    if (us < best_us) {
+      best_us = us;
+      best = t.cfg;
+    }
+  }
+  return best;
 }
 
 int fill_common(IgemmArgs& a, const ConvShape& s, int dtype) {
@@ -2179,7 +2317,7 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S);
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false});
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
@@ -2199,7 +2337,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int gemm_m = s.N * Ho * Wo;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false});
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2207,7 +2345,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
 
 int conv2d_dgrad_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   const int gemm_m = s.N * s.H * s.W;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S);
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S, patch_kernel_fits(s, s.K), true});
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2251,7 +2389,7 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S);
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr});
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
