@@ -37,6 +37,8 @@
 #include "context.h"
 #include "ops.h"
 
+#include <utility>
+
 #include <mutex>
 #include <string>
 
@@ -95,13 +97,6 @@ struct IgemmArgs {
   uint32_t a_bytes, b_bytes;  // extents of a_src / b_src for the bounds-checked buffer loads
   FastDiv div_plane;  // pixels per image on the gather side
   FastDiv div_width;  // row width on the gather side
-};
-
-typedef short short4_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) short4_t* lds_short4_ptr;
-union TrPart {
-  short4_t s;
-  uint32_t w[2];
 };
 
 // first operand = filter-side fragment (its rows become accumulator registers),
@@ -674,12 +669,323 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
   finish_tile<T, MODE, WM, WN, TM, TN>(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
 }
 
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+
+// 16 bytes per lane from `rsrc` at byte offset voff (+ the wave-uniform soff) to dst + lane*16 in
+// LDS; an offset outside the resource stores zeros.  (Kept in a device function: named directly
+// in a kernel body, the builtin makes the host pass drop the kernel's launch stub.)
+__device__ inline void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char* dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)dst, 16, voff, soff, 0, 0);
+}
+
+// the registers belong to their values up to this point of the program
+template <int A, int B>
+__device__ inline void hold(uint4_t (&r)[A][B]) {
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int j = 0; j < B; ++j) asm volatile("" : "+v"(r[i][j]));
+}
+
+__device__ inline const void* wave_uniform(const void* ptr) {
+  const uint64_t v = reinterpret_cast<uint64_t>(ptr);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+  return reinterpret_cast<const void*>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+// fn(0), fn(1), .. fn(N - 1) with the index as a constant
+template <int... I, typename F>
+__device__ __forceinline__ void unrolled_steps(std::integer_sequence<int, I...>, F&& fn) {
+  (fn(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(F&& fn) {
+  unrolled_steps(std::make_integer_sequence<int, N>{}, fn);
+}
+
+// All but the newest N of this wave's direct loads have landed, all its LDS accesses are done, and every wave of the
+// workgroup is here.  Not __syncthreads(): the compiler puts a wait for EVERY outstanding direct load in front of
+// that (a direct load is an LDS write to it), which leaves no tile in flight across the barrier whatever NBUF is:
+// each step then pays a whole trip to memory (a 64 x 64 tile: 0.47 us per 64-element step with two buffers or three).
+template <int N>
+__device__ inline void wait_and_meet() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 // ---------------------------------------------------------------------------
 // weight gradient
 // ---------------------------------------------------------------------------
+// The bf16 weight gradient: dy and x tiles of 32 pixels go from global memory straight into LDS rows [pixel][channel]
+// and are read transposed (ds_read_b64_tr_b16: a lane gets 4 pixels of one channel).  A 16-byte slot of a row is
+// XOR-ed by the row so that the 4 x 32-byte patches of a transposing read spread over all banks although rows are
+// unpadded.  64 KB of tiles in flight, four of 128 x 128 or eight of 64 x 64: a workgroup's step is a trip to memory
+// divided by the tiles in flight until the operand path of the CU is full (64 x 64, 147 / 75 / 53 us with two / three /
+// four tiles where eight steps' worth of splits are missing).  Against the form that staged tiles in registers (two in
+// flight, LDS stores of its own): 256 x 2304 over 12 544 pixels 44 -> 31 us, 3072 x 768 over 8192 62 -> 47, 128 x 1152 over
+// 50 176 34 -> 26; reading a step ahead of its multiplication into a second register set (169 instead of 136
+// registers) gained nothing on top.
+// POINTWISE: x is read at dy's pixels (no tap arithmetic).  BIAS: the launch may be asked for the bias gradient.
+template <int WM, int WN, int TM, int TN>
+constexpr int wgrad_direct_buffers() {
+  return 65536 / (32 * (WM * TM + WN * TN) * 64);
+}
+template <int WM, int WN, int TM, int TN>
+constexpr int wgrad_direct_lds() {
+  constexpr int ring = wgrad_direct_buffers<WM, WN, TM, TN>() * 32 * (WM * TM + WN * TN) * 64, stage = WM * 32 * (WN * TN * 32 + kStagePad) * 4;
+  return ring > stage ? ring : stage;
+}
+template <int WM, int WN, int TM, int TN, bool POINTWISE, bool BIAS>
+__device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t id, unsigned char* lds) {
+  constexpr int BKP = 32, NBUF = wgrad_direct_buffers<WM, WN, TM, TN>();
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, NW = WM * WN;
+  constexpr int RA = BM * 2, RB = BN * 2;              // bytes of one pixel row
+  constexpr int SA = RA / 16, SB = RB / 16;            // 16-byte slots of it
+  constexpr int A_BYTES = BKP * RA, BUF_BYTES = BKP * (RA + RB);
+  constexpr int A_LD = A_BYTES / 1024 / NW, B_LD = BKP * RB / 1024 / NW;
+  static_assert(A_BYTES % (1024 * NW) == 0 && (BKP * RB) % (1024 * NW) == 0, "tile/loader mismatch");
+  static_assert((RA == 256 || RA == 128) && (RB == 256 || RB == 128), "row swizzle");
+  static_assert(NBUF * BUF_BYTES <= 65536, "the buffer is part of the reads' immediate offset");
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tiles_mn = p.tiles_m * p.tiles_n;
+  const int split = id / tiles_mn;
+  id -= split * tiles_mn;
+  const int tile_m = id / p.tiles_n;
+  const int tile_n = id - tile_m * p.tiles_n;
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int k_begin = split * p.k_per_split;
+  int k_end = k_begin + p.k_per_split;
+  if (k_end > p.gemm_k) k_end = p.gemm_k;
+  const int nk = (k_end - k_begin + BKP - 1) / BKP;
+
+  // two 128-byte rows span the 64 banks, or one 256-byte row does: four consecutive rows land on different quarters
+  auto swz_a = [](int row) { return RA == 256 ? (row & 3) << 2 : ((row >> 1) & 1) << 2; };
+  auto swz_b = [](int row) { return RB == 256 ? (row & 3) << 2 : ((row >> 1) & 1) << 2; };
+
+  // ---- what this lane loads: a fixed channel chunk of dy and of x, one pixel row per direct load ----
+  const int a_row = lane / SA, b_row = lane / SB;
+  const int a_ch = m0 + ((lane % SA) ^ swz_a(a_row)) * 8;
+  const int b_n = n0 + ((lane % SB) ^ swz_b(b_row)) * 8;
+  // a channel beyond the tensor has no pixels
+  const int a_end = a_ch < p.gemm_m ? k_end : 0, b_end = b_n < p.gemm_n ? k_end : 0;
+  // (a grouped launch reads its arguments from memory: told that they are the same in every lane)
+  const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(wave_uniform(p.a_src), __builtin_amdgcn_readfirstlane(p.a_bytes));
+  const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(wave_uniform(p.b_src), __builtin_amdgcn_readfirstlane(p.b_bytes));
+  int a_pix[A_LD], a_off[A_LD], b_pix[B_LD], b_off[B_LD];   // the pixel each direct load takes next, its byte offset
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) {
+    a_pix[i] = k_begin + (wave * A_LD + i) * (64 / SA) + a_row;
+    a_off[i] = (a_pix[i] * p.K + a_ch) * 2;
+  }
+  const int a_step = BKP * p.K * 2;
+  // not pointwise: the lane's tap and channel, and every load's place in the image, moved on by 32 pixels per step
+  int b_c = b_n, b_h = 0, b_w = 0;
+  uint32_t b_img[B_LD], b_oh[B_LD], b_ow[B_LD];
+  uint32_t step_img = 0, step_oh = 0, step_ow = 0;
+  if (!POINTWISE) {
+    const int tap = b_n / p.C;
+    const int r = tap / p.S;
+    b_c = b_n - tap * p.C;
+    b_h = r - p.pad;
+    b_w = tap - r * p.S - p.pad;
+    p.div_plane.divmod(BKP, step_img, step_oh);
+    p.div_width.divmod(step_oh, step_oh, step_ow);
+  }
+#pragma unroll
+  for (int i = 0; i < B_LD; ++i) {
+    b_pix[i] = k_begin + (wave * B_LD + i) * (64 / SB) + b_row;
+    b_off[i] = (b_pix[i] * p.C + b_c) * 2;
+    b_img[i] = b_oh[i] = b_ow[i] = 0;
+    if (!POINTWISE) {
+      uint32_t rem;
+      p.div_plane.divmod(static_cast<uint32_t>(b_pix[i]), b_img[i], rem);
+      p.div_width.divmod(rem, b_oh[i], b_ow[i]);
+    }
+  }
+  const int b_step = BKP * p.C * 2;
+  // Every lane issues every load whatever it asks for (the counted waits rely on it): an offset out of range where
+  // there is no pixel, a tap outside the image, or a tile behind the last one.
+  auto issue_loads = [&](int buf) {
+    unsigned char* dst_a = lds + buf * BUF_BYTES + wave * A_LD * 1024;
+    unsigned char* dst_b = lds + buf * BUF_BYTES + A_BYTES + wave * B_LD * 1024;
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) {
+      load_to_lds(rsrc_a, dst_a + i * 1024, a_pix[i] < a_end ? a_off[i] : static_cast<int>(kOutOfRange), 0);
+      a_pix[i] += BKP;
+      a_off[i] += a_step;
+    }
+#pragma unroll
+    for (int i = 0; i < B_LD; ++i) {
+      int off = b_off[i];
+      bool ok = b_pix[i] < b_end;
+      if (POINTWISE) {
+        b_off[i] += b_step;
+      } else {
+        const int hi = static_cast<int>(b_oh[i]) * p.stride + b_h, wi = static_cast<int>(b_ow[i]) * p.stride + b_w;
+        ok = ok & (static_cast<unsigned>(hi) < static_cast<unsigned>(p.H)) & (static_cast<unsigned>(wi) < static_cast<unsigned>(p.W));
+        off = (((static_cast<int>(b_img[i]) * p.H + hi) * p.W + wi) * p.C + b_c) * 2;
+        b_ow[i] += step_ow;
+        const uint32_t row = b_ow[i] >= static_cast<uint32_t>(p.Wo) ? 1u : 0u;
+        b_ow[i] -= row * p.Wo;
+        b_oh[i] += step_oh + row;
+        const uint32_t img = b_oh[i] >= static_cast<uint32_t>(p.Ho) ? 1u : 0u;
+        b_oh[i] -= img * p.Ho;
+        b_img[i] += step_img + img;
+      }
+      load_to_lds(rsrc_b, dst_b + i * 1024, ok ? off : static_cast<int>(kOutOfRange), 0);
+      b_pix[i] += BKP;
+    }
+  };
+
+  f32x16_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  // transposing reads: lane = 16 G + q; the 16 lanes of a group read pixels {8 (G/2) + q/4} x channels {16 (G%2) + 4 (q%4) ..};
+  // afterwards lane q owns channel 16 (G%2) + q of the band and four pixels
+  const int grp = lane >> 4, q16 = lane & 15;
+  const int tr_pix = 8 * (grp >> 1) + (q16 >> 2);
+  const int tr_b = (16 * (grp & 1) + 4 * (q16 & 3)) * 2;   // bytes within the 64-byte band
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  // address of pixel row tr_pix, band w * T + t: the band is four slots, so the row's XOR only moves whole bands
+  auto band = [&](int row_bytes, int w_band, int swz) {
+    return static_cast<uint32_t>(tr_pix * row_bytes + ((w_band * 4) ^ swz) * 16 + tr_b);
+  };
+  uint32_t rd_a[TM], rd_b[TN];
+#pragma unroll
+  for (int t = 0; t < TM; ++t) rd_a[t] = lds_base + band(RA, wm * TM + t, swz_a(tr_pix));
+#pragma unroll
+  for (int t = 0; t < TN; ++t) rd_b[t] = lds_base + A_BYTES + band(RB, wn * TN + t, swz_b(tr_pix));
+  typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
+  constexpr int SL = BKP / 16;
+  uint2_t fa[SL][TM][2], fb[SL][TN][2];
+  // rows + 16 and + 4 keep the row's swizzle (a multiple of four rows)
+  auto read_tile = [&](auto buf_c) {
+    constexpr int AT = decltype(buf_c)::value * BUF_BYTES;
+    auto &ra = fa;
+    auto &rb = fb;
+#pragma unroll
+    for (int ks = 0; ks < SL; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const uint32_t at = rd_a[tm];
+          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(ra[ks][tm][t]) : "v"(at), "n"(AT + (ks * 16 + 4 * t) * RA));
+        }
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) {
+          const uint32_t at = rd_b[tn];
+          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(rb[ks][tn][t]) : "v"(at), "n"(AT + (ks * 16 + 4 * t) * RB));
+        }
+      }
+  };
+  auto hold_tile = [&] {
+#pragma unroll
+    for (int ks = 0; ks < SL; ++ks)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(fa[ks][tm][t]));
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(fb[ks][tn][t]));
+      }
+  };
+  auto chunk = [](const uint2_t (&v)[2]) {
+    Chunk c;
+    c.w[0] = v[0][0];
+    c.w[1] = v[0][1];
+    c.w[2] = v[1][0];
+    c.w[3] = v[1][1];
+    return c;
+  };
+
+  // The bias gradient of a linear layer is the column sum of dy: the wavefronts of the first column of tiles add up the
+  // dy operands they multiply anyway (a lane: one channel of each band, half of the pixels).
+  const bool sum_dy = BIAS && p.dbias != nullptr && tile_n == 0 && wn == 0;
+  float bsum[TM];
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm) bsum[tm] = 0.f;
+
+  constexpr int LOADS = A_LD + B_LD;
+  constexpr int AHEAD = (NBUF - 2) * LOADS;
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s) issue_loads(s);
+  auto step = [&](auto u_c) {
+    constexpr int u = decltype(u_c)::value;
+    wait_and_meet<AHEAD>();
+    read_tile(u_c);
+    issue_loads((u + NBUF - 1) % NBUF);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_tile();
+#pragma unroll
+    for (int ks = 0; ks < SL; ++ks) {
+      Chunk ca[TM], cb[TN];
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) ca[tm] = chunk(fa[ks][tm]);
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) cb[tn] = chunk(fb[ks][tn]);
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) mma<bf16>(cb[tn], ca[tm], acc[tm][tn]);
+      if (sum_dy) {
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          float v[8];
+          chunk_to_float<bf16>(ca[tm], v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) bsum[tm] += v[e];
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);   // the next step's addresses stay in the next step (36 registers less)
+  };
+  int kt = 0;
+  for (; kt + NBUF <= nk; kt += NBUF) unrolled<NBUF>(step);
+  unrolled<NBUF - 1>([&](auto u_c) {
+    if (kt + decltype(u_c)::value < nk) step(u_c);
+  });
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile: the epilogue uses their place
+
+  float* out = static_cast<float*>(p.out);
+  if (p.splits > 1) out += static_cast<int64_t>(split) * p.gemm_m * p.gemm_n;
+  const bool accumulate = p.splits == 1 && p.accumulate;
+  staged_epilogue<bf16, WM, WN, TM, TN>(acc, reinterpret_cast<float*>(lds), tid, [&](int, int tr, int tc, float* v) {
+    const int row = m0 + tr, col = n0 + tc;
+    if (row >= p.gemm_m || col >= p.gemm_n) return;
+    float* dst = out + static_cast<int64_t>(row) * p.gemm_n + col;
+    if (accumulate) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] += dst[e];
+    }
+    store_floats<8>(dst, v);
+  });
+  if (sum_dy) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      const float sum = bsum[tm] + __shfl_xor(bsum[tm], 32, 64);
+      const int ch = m0 + (wm * TM + tm) * 32 + (lane & 31);
+      if (lane < 32 && ch < p.gemm_m) {
+        float* dst = p.dbias + (p.splits > 1 ? static_cast<int64_t>(split) * p.gemm_m : 0) + ch;
+        *dst = accumulate ? *dst + sum : sum;
+      }
+    }
+  }
+}
+
 // `id`: the workgroup's place among the tiles_m * tiles_n * splits workgroups of this weight gradient
-template <typename T, int WM, int WN, int TM, int TN>
-__device__ __forceinline__ void wgrad_body(const IgemmArgs& p, uint32_t id) {
+template <int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) {
+  typedef float T;
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int BKP = 4 * E;  // pixels per reduction step
   constexpr int BM = WM * TM * 32;
@@ -796,63 +1102,23 @@ __device__ __forceinline__ void wgrad_body(const IgemmArgs& p, uint32_t id) {
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
 
-  // transpose-read geometry (bf16): lane = 16*G + q; the 16 lanes of a group read
-  // pixels {base + q/4 ...} x channels {16*(G%2) + 4*(q%4) ...}; after the transpose
-  // lane q owns channel 16*(G%2) + q of the band and 4 pixels.
-  const int grp = lane >> 4, q16 = lane & 15;
-  const int tr_pix = 8 * (grp >> 1) + (q16 >> 2);
-  const int tr_ch = 16 * (grp & 1) + 4 * (q16 & 3);
-
   auto compute = [&](int buf) {
-    if constexpr (sizeof(T) == 2) {
-      const uint16_t* la = reinterpret_cast<const uint16_t*>(lds_a + buf * BKP * LDA);
-      const uint16_t* lb = reinterpret_cast<const uint16_t*>(lds_b + buf * BKP * LDB);
+    // fp32: one reduction element per lane and MFMA, no transposition needed
+    const float* la = reinterpret_cast<const float*>(lds_a + buf * BKP * LDA);
+    const float* lb = reinterpret_cast<const float*>(lds_b + buf * BKP * LDB);
 #pragma unroll
-      for (int ks = 0; ks < BKP / 16; ++ks) {
-        Chunk fa[TM], fb[TN];
+    for (int ks = 0; ks < BKP / 2; ++ks) {
+      const int prow = ks * 2 + (lane >> 5);
+      float fa[TM], fb[TN];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int prow = ks * 16 + tr_pix + 4 * t;
+      for (int tm = 0; tm < TM; ++tm) fa[tm] = la[prow * (LDA * 4) + (wm * TM + tm) * 32 + (lane & 31)];
 #pragma unroll
-          for (int tm = 0; tm < TM; ++tm) {
-            const uint16_t* ptr = la + prow * (LDA * 8) + (wm * TM + tm) * 32 + tr_ch;
-            TrPart v;
-            v.s = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(ptr));
-            fa[tm].w[2 * t] = v.w[0];
-            fa[tm].w[2 * t + 1] = v.w[1];
-          }
+      for (int tn = 0; tn < TN; ++tn) fb[tn] = lb[prow * (LDB * 4) + (wn * TN + tn) * 32 + (lane & 31)];
 #pragma unroll
-          for (int tn = 0; tn < TN; ++tn) {
-            const uint16_t* ptr = lb + prow * (LDB * 8) + (wn * TN + tn) * 32 + tr_ch;
-            TrPart v;
-            v.s = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(ptr));
-            fb[tn].w[2 * t] = v.w[0];
-            fb[tn].w[2 * t + 1] = v.w[1];
-          }
-        }
+      for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn) mma<T>(fb[tn], fa[tm], acc[tm][tn]);
-      }
-    } else {
-      // fp32: one reduction element per lane and MFMA, no transposition needed
-      const float* la = reinterpret_cast<const float*>(lds_a + buf * BKP * LDA);
-      const float* lb = reinterpret_cast<const float*>(lds_b + buf * BKP * LDB);
-#pragma unroll
-      for (int ks = 0; ks < BKP / 2; ++ks) {
-        const int prow = ks * 2 + (lane >> 5);
-        float fa[TM], fb[TN];
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) fa[tm] = la[prow * (LDA * 4) + (wm * TM + tm) * 32 + (lane & 31)];
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) fb[tn] = lb[prow * (LDB * 4) + (wn * TN + tn) * 32 + (lane & 31)];
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[tn], fa[tm], acc[tm][tn], 0, 0, 0);
-      }
+        for (int tn = 0; tn < TN; ++tn)
+          acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[tn], fa[tm], acc[tm][tn], 0, 0, 0);
     }
   };
 
@@ -917,13 +1183,23 @@ struct WgradArgs {
   uint32_t gemm_wgs;
 };
 
-template <typename T, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(WM* WN * 64) void wgrad_kernel(WgradArgs w) {
+template <int WM, int WN, int TM, int TN>
+__global__ __launch_bounds__(WM* WN * 64) void wgrad_f32_kernel(WgradArgs w) {
   if (blockIdx.x >= w.gemm_wgs) {
     splitk_reduce_body(w.red, blockIdx.x - w.gemm_wgs);
     return;
   }
-  wgrad_body<T, WM, WN, TM, TN>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs));
+  wgrad_body_f32<WM, WN, TM, TN>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs));
+}
+
+template <int WM, int WN, int TM, int TN, bool POINTWISE, bool BIAS>
+__global__ __launch_bounds__(WM* WN * 64) void wgrad_kernel(WgradArgs w) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[wgrad_direct_lds<WM, WN, TM, TN>()];
+  if (blockIdx.x >= w.gemm_wgs) {
+    splitk_reduce_body(w.red, blockIdx.x - w.gemm_wgs);
+    return;
+  }
+  wgrad_body_direct<WM, WN, TM, TN, POINTWISE, BIAS>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs), lds);
 }
 
 // The weight gradients of several convolutions in one launch.  `table` holds one argument block per convolution,
@@ -940,10 +1216,14 @@ struct WgradGroupArgs {
 
 template <typename T, int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs g) {
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[sizeof(T) == 2 ? wgrad_direct_lds<WM, WN, TM, TN>() : 16];
   for (uint32_t gid = xcd_remap(blockIdx.x, gridDim.x); gid < g.entries; gid += gridDim.x) {
     const uint2 e = g.map[gid];
     const IgemmArgs p = g.table[__builtin_amdgcn_readfirstlane(e.x)];
-    wgrad_body<T, WM, WN, TM, TN>(p, __builtin_amdgcn_readfirstlane(e.y));
+    const uint32_t id = __builtin_amdgcn_readfirstlane(e.y);
+    if constexpr (sizeof(T) == 4) wgrad_body_f32<WM, WN, TM, TN>(p, id);
+    else if (p.pointwise) wgrad_body_direct<WM, WN, TM, TN, true, true>(p, id, lds);
+    else wgrad_body_direct<WM, WN, TM, TN, false, true>(p, id, lds);
     __syncthreads();   // the next entry's operand tiles overwrite what the epilogue staged in LDS
   }
 }
@@ -964,42 +1244,14 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
 //     hands over a tile one step before it is needed and the LDS latency passes behind the multiplies.  What bounds
 //     the small tiles then is LDS itself (a 64 x 64 tile: 32 KB read, 16 KB written per step).  1024 x 768 over 3072:
 //     24.3 us with a whole trip to memory per step (0.47 us each), 16.3 with the loads really in flight, 13.5 pipelined;
-//     2048 rows 25.3 / 20.6 / 17.8 (128 x 64 on eight wavefronts); 8192 rows 54 / 50.6 / 43.2 (128 x 128, 935 TFLOP/s
-//     of the 1310 a library product of 8192^3 reaches here);
+//     2048 rows 25.3 / 20.6 / 17.8 (128 x 64 on eight wavefronts);
 //   * KS = 32 halves the step (64-byte rows, sixteen rows per direct load): half the LDS per tile in flight, so
 //     more workgroups share a CU and a small grid is resident in one round.
 constexpr int kStep2 = 64;                  // reduction elements per step
 constexpr int kRowBytes2 = kStep2 * 2;      // 128
 
-typedef __attribute__((address_space(3))) void* lds_void_ptr;
-
-// 16 bytes per lane from `rsrc` at byte offset voff (+ the wave-uniform soff) to dst + lane*16 in
-// LDS; an offset outside the resource stores zeros.  (Kept in a device function: named directly
-// in a kernel body, the builtin makes the host pass drop the kernel's launch stub.)
-__device__ inline void load_to_lds(__amdgpu_buffer_rsrc_t rsrc, unsigned char* dst, int voff, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_ptr)dst, 16, voff, soff, 0, 0);
-}
-
-// the registers belong to their values up to this point of the program
-template <int A, int B>
-__device__ inline void hold(uint4_t (&r)[A][B]) {
-#pragma unroll
-  for (int i = 0; i < A; ++i)
-#pragma unroll
-    for (int j = 0; j < B; ++j) asm volatile("" : "+v"(r[i][j]));
-}
-
-// All but the newest N of this wave's direct loads have landed, all its LDS accesses are done, and every wave of the
-// workgroup is here.  Not __syncthreads(): the compiler puts a wait for EVERY outstanding direct load in front of
-// that (a direct load is an LDS write to it), which leaves no tile in flight across the barrier whatever NBUF is:
-// each step then pays a whole trip to memory (a 64 x 64 tile: 0.47 us per 64-element step with two buffers or three).
-template <int N>
-__device__ inline void wait_and_meet() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
 template <int MODE, int WM, int WN, int TM, int TN, int NBUF, int ROT = 0, int KS = kStep2>
-__global__ __launch_bounds__(WM* WN * 64, ROT == 2 ? 2 : 1) void igemm2_kernel(IgemmArgs p) {
+__global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
   using T = bf16;
   constexpr int E = 8;
   constexpr int BM = WM * TM * 32;
@@ -1217,7 +1469,7 @@ __global__ __launch_bounds__(WM* WN * 64, ROT == 2 ? 2 : 1) void igemm2_kernel(I
   if constexpr (ROT == 2) {
     // Pipelined over the reduction steps: the operands of tile kt+1 are read into a second register set while tile kt
     // is multiplied.
-    static_assert(NBUF == 2 || NBUF == 4, "the register sets alternate with the buffers");
+    static_assert(NBUF == 4, "two register sets, alternating with the buffers");
     constexpr int SL = KS / 16;
     uint4_t fa[2][SL][TM], fb[2][SL][TN];
     // the buffer is part of the reads' immediate offset where that reaches (64 KB)
@@ -1255,19 +1507,10 @@ __global__ __launch_bounds__(WM* WN * 64, ROT == 2 ? 2 : 1) void igemm2_kernel(I
       hold(fb[set ^ 1]);
     };
     int kt0 = 0;
-    for (; kt0 + NBUF <= nk; kt0 += NBUF) {
-      pstep(std::integral_constant<int, 0>{});
-      pstep(std::integral_constant<int, 1>{});
-      if constexpr (NBUF == 4) {
-        pstep(std::integral_constant<int, 2>{});
-        pstep(std::integral_constant<int, 3>{});
-      }
-    }
-    if (kt0 < nk) pstep(std::integral_constant<int, 0>{});
-    if constexpr (NBUF == 4) {
-      if (kt0 + 1 < nk) pstep(std::integral_constant<int, 1>{});
-      if (kt0 + 2 < nk) pstep(std::integral_constant<int, 2>{});
-    }
+    for (; kt0 + NBUF <= nk; kt0 += NBUF) unrolled<NBUF>(pstep);
+    unrolled<NBUF - 1>([&](auto u_c) {
+      if (kt0 + decltype(u_c)::value < nk) pstep(u_c);
+    });
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile: the epilogue uses their place
   } else if constexpr (ROT == 1) {
     // Rotated loop for the large tiles, whose workgroup has a compute unit to itself (nobody else fills the
@@ -1875,8 +2118,14 @@ int launch_cfg(Context* ctx, IgemmArgs& a, double flops) {
       blocks += tr.blocks;
       tr.valid = false;
     }
-    return launch(ctx, wgrad_kernel<T, WM, WN, TM, TN>, dim3(blocks), block, w, igemm_name<T, MODE, WM, WN, TM, TN>(), flops, 0,
-                  bytes);
+    void (*kernel)(WgradArgs);
+    if constexpr (sizeof(T) == 4)
+      kernel = wgrad_f32_kernel<WM, WN, TM, TN>;
+    else if (a.pointwise)
+      kernel = a.dbias ? wgrad_kernel<WM, WN, TM, TN, true, true> : wgrad_kernel<WM, WN, TM, TN, true, false>;
+    else
+      kernel = a.dbias ? wgrad_kernel<WM, WN, TM, TN, false, true> : wgrad_kernel<WM, WN, TM, TN, false, false>;
+    return launch(ctx, kernel, dim3(blocks), block, w, igemm_name<T, MODE, WM, WN, TM, TN>(), flops, 0, bytes);
   } else
     return launch(ctx, igemm_kernel<T, MODE, WM, WN, TM, TN>, grid, block, a, igemm_name<T, MODE, WM, WN, TM, TN>(),
                   flops, 0, conv_bytes<MODE>(a, sizeof(T)));
@@ -1984,11 +2233,10 @@ enum SplitTile : int {
 enum PipeTile : int {
   kPipe64 = 21,       // 64 x 64
   kPipe128x64 = 22,   // 128 x 64, eight wavefronts
-  kPipe128 = 23,      // 128 x 128
 };
 
 // the tiling of the same shape that runs where a pipelined one does not exist
-int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : tile_cfg == kPipe128x64 ? 1 : 0; }
+int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : 1; }
 
 template <typename T, int MODE>
 int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
@@ -2045,12 +2293,12 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
         return tile_cfg == 6 ? launch_cfg2<MODE, 2, 2, 2, 1, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 1, 1, 2>(ctx, a, flops);
       tile_cfg -= 5;
     }
-    // 21 - 23: operand reads pipelined over the reduction steps (see igemm2_kernel): 64 x 64 with four tiles in LDS,
-    // 128 x 64 on eight wavefronts with four, 128 x 128 with two
+    // 21 / 22: operand reads pipelined over the reduction steps (see igemm2_kernel), four tiles in LDS: 64 x 64, and
+    // 128 x 64 on eight wavefronts.  (128 x 128 with two tiles, 229 registers: 43.2 us for 8192 x 768 over 3072 alone
+    // against 50.6, but the GPT-2 step is 0.2 ms slower with it, beside the weight gradients: not built.)
     if (tile_cfg >= kPipe64 && setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32) {
       if (tile_cfg == kPipe64) return launch_cfg2<MODE, 2, 2, 1, 1, 4, 2>(ctx, a, flops);
-      if (tile_cfg == kPipe128x64) return launch_cfg2<MODE, 4, 2, 1, 1, 4, 2>(ctx, a, flops);
-      return launch_cfg2<MODE, 2, 2, 2, 2, 2, 2>(ctx, a, flops);
+      return launch_cfg2<MODE, 4, 2, 1, 1, 4, 2>(ctx, a, flops);
     }
     if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32 && tile_cfg >= 0 && tile_cfg <= 2) {
       if (tile_cfg == 0)
@@ -2152,7 +2400,6 @@ const TileCost kPlainCost[] = {
     {2, 64, 64, 3.51f, 0.64f, 0.261f, 0.158f, 0.14f},    {5, 128, 64, 0.93f, 4.74f, 0.267f, 0.067f, 0.47f},
     {12, 128, 128, 4.48f, 0.88f, 0.798f, 0.474f, 0.20f}, {13, 128, 64, 4.47f, 0.15f, 0.495f, 0.347f, 0.35f},
     {14, 64, 64, 3.72f, 0.00f, 0.391f, 0.235f, 0.40f},   {kPipe64, 64, 64, 3.43f, 1.05f, 0.199f, 0.145f, 0.40f},
-    {kPipe128, 128, 128, 3.67f, 2.67f, 0.625f, 0.352f, 0.08f},
     {kPipe128x64, 128, 64, 2.75f, 2.21f, 0.108f, 0.262f, 0.48f},
     {kSplit32, 32, 32, 3.28f, 0.21f, 0.092f, 0.079f, 2.14f},
     {kSplit32Deep, 32, 32, 3.47f, 0.07f, 0.075f, 0.082f, 3.11f},
@@ -2162,7 +2409,6 @@ const TileCost kSumsCost[] = {
     {2, 64, 64, 4.58f, 1.30f, 0.285f, 0.184f, 0.25f},    {5, 128, 64, 1.28f, 6.10f, 0.266f, 0.067f, 0.55f},
     {12, 128, 128, 6.18f, 1.64f, 0.818f, 0.501f, 0.55f}, {13, 128, 64, 5.57f, 1.10f, 0.528f, 0.363f, 0.31f},
     {14, 64, 64, 4.79f, 0.70f, 0.408f, 0.242f, 0.47f},   {kPipe64, 64, 64, 4.09f, 1.97f, 0.225f, 0.148f, 0.55f},
-    {kPipe128, 128, 128, 5.95f, 3.00f, 0.665f, 0.408f, 0.45f},
     {kPipe128x64, 128, 64, 2.69f, 5.40f, 0.272f, 0.291f, 0.57f},
     {kSplit32, 32, 32, 3.44f, 0.48f, 0.108f, 0.087f, 3.96f},
     {kSplit32Deep, 32, 32, 4.20f, 0.38f, 0.062f, 0.082f, 5.42f},
@@ -2199,9 +2445,13 @@ int heuristic_tile(int asked, const TileQuery& q) {
     return split >= 0 ? split : pick_tile(q.gemm_m, q.gemm_n, 1);
   }
   const float steps = static_cast<float>(q.gemm_k) / 64.f, store = static_cast<float>(q.gemm_m) * q.gemm_n * 1e-6f;
+  const bool large = tiles_for(q.gemm_m, q.gemm_n, 128, 128) >= 384;
   int best = 2;
   float best_us = INFINITY;
   for (const TileCost& t : q.sums ? kSumsCost : kPlainCost) {
+    // one and a half 128 x 128 tiles per compute unit or more, beside a second lane of weight gradients: smaller tiles
+    // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 8 x 1024 12.05 -> 11.76 ms)
+    if (!q.sums && large && t.bm * t.bn < 128 * 128) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
     const float r = static_cast<float>((tiles_for(q.gemm_m, q.gemm_n, t.bm, t.bn) + 255) / 256);
@@ -2411,29 +2661,50 @@ int64_t conv2d_wgrad_workspace_bytes(const ConvShape& s, int dtype, int splits) 
   return static_cast<int64_t>(splits) * (static_cast<int64_t>(s.K) * s.R * s.S * s.C + s.K) * 4;
 }
 
+// tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups
+bool wgrad_big_tile(int gemm_m, int gemm_n, int64_t splits) {
+  return gemm_m >= 128 && gemm_n >= 128 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= 128;
+}
+
 int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
   const int BK = dtype == kBF16 ? 32 : 16;
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int64_t pixels = static_cast<int64_t>(s.N) * Ho * Wo;
   const int gemm_m = s.K, gemm_n = s.R * s.S * s.C;
-  int64_t tiles = tiles_for(gemm_m, gemm_n, 128, 128);
-  if (tiles < 8) tiles = tiles_for(gemm_m, gemm_n, 64, 64);
-  // Workgroups to aim for.  The weight gradients run beside the data-gradient chain on a second stream: a
-  // launch that does not fill the chip by itself shares it better, and every split costs a partial filter
-  // written and read again, so filters of few tiles over short reductions aim lower than wide or long products.
-  static const int target_env = [] {
-    const char* e = getenv("TCH_WGRAD_WGS");
-    return e && atoi(e) > 0 ? atoi(e) : 0;
-  }();
-  const int target_wgs = target_env ? target_env : (tiles <= 64 && pixels <= 16384) ? 192 : 384;
-  int64_t want = (target_wgs + tiles - 1) / tiles;
-  int64_t max_by_k = pixels / (4 * BK);  // at least four reduction steps per split
-  if (max_by_k < 1) max_by_k = 1;
-  if (want > max_by_k) want = max_by_k;
-  if (want > 512) want = 512;
-  if (want < 1) want = 1;
-  return static_cast<int>(want);
+  // The split count with the shortest start + steps * max(alone, shared * r) + store * (10^6 results written), r =
+  // workgroups per compute unit, rounded up: least-squares fits (6-8 % mean error) to 1 500 launches of every split count
+  // on the layers of the three models at 128-8192 rows and 1-64 images, per dtype for 128 x 128 and 64 x 64 tiles.  A
+  // partial filter is read again by the reduction that rides the next launch: kReread on top of what it
+  // costs to write.  (Aiming at 192-384 workgroups instead split short reductions that were launch latency and
+  // partial filters already: 1024 -> 3072 over 343 rows 17.8 us with two splits, 10.1 with one; 256 -> 768 over 5488
+  // rows 15.6 with 16, 10.8 with 4.)
+  struct Cost {
+    float start, alone, shared, store;
+  };
+  static const Cost cost[2][2] = {{{3.39f, 0.229f, 0.383f, 1.55f}, {8.56f, 0.371f, 0.912f, 0.71f}},     // fp32: 64, 128
+                                  {{3.08f, 0.109f, 0.089f, 2.33f}, {6.37f, 0.249f, 0.179f, 0.94f}}};   // bf16
+  constexpr float kReread = 1.f;   // microseconds per 10^6 results; 0 - 2 in the steps: within 1 %, 1 the best of most
+  int64_t most = pixels / (4 * BK);   // at least four reduction steps per split
+  if (most > 512) most = 512;
+  int best = 1;
+  float best_us = INFINITY;
+  for (int64_t want = 1; want <= most || want == 1; ++want) {
+    const int64_t steps = ((pixels + want - 1) / want + BK - 1) / BK;
+    const int64_t splits = (pixels + steps * BK - 1) / (steps * BK);
+    if (splits != want) continue;   // the same as a smaller count
+    const bool big = wgrad_big_tile(gemm_m, gemm_n, splits);
+    const Cost& c = cost[dtype == kBF16][big];
+    const int side = big ? 128 : 64;
+    const float r = static_cast<float>((tiles_for(gemm_m, gemm_n, side, side) * splits + 255) / 256);
+    const float results = static_cast<float>(gemm_m) * gemm_n * splits * 1e-6f;
+    const float us = c.start + steps * fmaxf(c.alone, c.shared * r) + (c.store + (splits > 1 ? kReread : 0.f)) * results;
+    if (us < best_us) {
+      best_us = us;
+      best = static_cast<int>(splits);
+    }
+  }
+  return best;
 }
 
 int conv2d_wgrad_flush(Context* ctx) {
@@ -2472,11 +2743,7 @@ int conv2d_wgrad(Context* ctx, int dtype, const ConvShape& s, const void* x, con
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    static const int big_from = [] {
-      const char* e = getenv("TCH_WGRAD_BIG_TILE_WGS");
-      return e && atoi(e) > 0 ? atoi(e) : 128;
-    }();
-    tile_cfg = (a.gemm_m >= 128 && a.gemm_n >= 128 && tiles_for(a.gemm_m, a.gemm_n, 128, 128) * splits >= big_from) ? 0 : 2;
+    tile_cfg = wgrad_big_tile(a.gemm_m, a.gemm_n, splits) ? 0 : 2;
   }
   int rc = dtype == kBF16 ? launch_mode<bf16, kWgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
                           : launch_mode<float, kWgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));
