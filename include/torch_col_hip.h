@@ -376,6 +376,11 @@ int tch_layernorm_fwd(tch_context* ctx, int dtype, const void* x, void* y, const
 /* dx = LayerNorm'(dy) (+ residual, laid out like dx, may be NULL: the gradient that bypasses the LayerNorm);
  * partial: fp32 scratch of tch_layernorm_bwd_partial_rows(rows) * C * 2 floats; dgamma / dbeta (+)= */
 int tch_layernorm_bwd_partial_rows(int64_t rows);
+/* on != 0: the column sums (dgamma, dbeta) of the LayerNorm backwards from here on are not launched with them but ride the
+ * next tch_conv2d_wgrad_trailing of the context as extra workgroups (tch_conv2d_wgrad_flush launches what is left; a
+ * backward behind another with no such call between them launches the older sums first).  `partial` must stay
+ * untouched until that launch is done.  Same bits. */
+int tch_layernorm_defer_sums(tch_context* ctx, int on);
 int tch_layernorm_bwd(tch_context* ctx, int dtype, const void* dy, const void* x, void* dx, const void* residual,
                       const float* gamma,
                       const float* mean, const float* rstd, float* dgamma, float* dbeta, int accumulate, int64_t rows,

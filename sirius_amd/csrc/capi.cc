@@ -312,6 +312,15 @@ int tch_layernorm_bwd_windowed(tch_context* ctx, int dtype, const void* dy, cons
                        partial, &win);
 }
 
+int tch_layernorm_defer_sums(tch_context* ctx, int on) {
+  if (!ctx) {
+    set_error("null context");
+    return -22;
+  }
+  C(ctx)->defer_col_sums = on != 0;
+  return 0;
+}
+
 int tch_layernorm_bwd_partial_rows(int64_t rows) { return layernorm_bwd_partial_rows(rows); }
 
 int tch_layernorm_bwd(tch_context* ctx, int dtype, const void* dy, const void* x, void* dx, const void* residual,

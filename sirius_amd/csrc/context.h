@@ -161,6 +161,12 @@ class Context {
     unsigned blocks = 0;
     double bytes = 0.0;
   } trailing_reduce;
+  // The same for the column sums of a LayerNorm backward while defer_col_sums is up (layernorm_bwd).
+  bool defer_col_sums = false;
+  struct {
+    bool valid = false;
+    LnSumArgs args{};
+  } trailing_col_sum;
 
   // `next`: the record that follows in the program being replayed (nullptr: none or unknown).  A lane-0 launch
   // that is followed by a lane-1 launch which has to wait for it carries the event of that wait as its own stop

@@ -284,6 +284,14 @@ struct ReduceArgs {
   unsigned first_blocks;
 };
 
+// the column sums of a LayerNorm backward's partial rows (col_sum.h)
+struct LnSumArgs {
+  const float* partial;  // [blocks][C][2]
+  float* out0;           // (+)= sum_b partial[b][c][0]
+  float* out1;           // (+)= sum_b partial[b][c][1]
+  int blocks, C, accumulate;
+};
+
 class Context;  // defined in context.h
 
 int submit(Context* ctx, const void* fn, dim3 grid, dim3 block, const void* args, size_t arg_bytes,

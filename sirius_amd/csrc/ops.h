@@ -148,6 +148,7 @@ int layernorm_bwd_partial_rows(int64_t rows);  // rows of [C][2] fp32 scratch la
 int layernorm_bwd(Context* ctx, int dtype, const void* dy, const void* x, void* dx, const void* residual, const float* gamma,
                   const float* mean, const float* rstd, float* dgamma, float* dbeta, int accumulate, int64_t rows,
                   int C, float* partial, const LnWindow* win = nullptr);
+int col_sum_flush(Context* ctx);   // the column sums a layernorm_bwd deferred, as a launch of their own
 int gelu_fwd(Context* ctx, int dtype, const void* x, void* y, int64_t n, int tanh_form);
 int gelu_bwd(Context* ctx, int dtype, const void* dy, const void* x, void* dx, int64_t n, int tanh_form);
 int attn_softmax_fwd(Context* ctx, int dtype, const void* scores, void* probs, int64_t batch, int heads, int Lq, int Lk,

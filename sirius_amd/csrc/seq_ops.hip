@@ -9,6 +9,8 @@
 //   and the shift mask                        train/swin_b_tiny.py:8-172, train/swin_b.py:38
 //   GPT-2 gelu_new, causal attention, wte + wpe   train/gpt2.py:26
 //   torch.optim.AdamW                         train/gpt2.py:31, train/swin_b.py:43 (variants)
+#include "col_sum.h"
+#include "context.h"
 #include "kernels.h"
 #include "ops.h"
 
@@ -281,51 +283,9 @@ __global__ __launch_bounds__(256) void ln_bwd_kernel(LnArgs p) {
   }
 }
 
-struct ColSumArgs {
-  const float* partial;  // [blocks][C][2]
-  float* out0;           // (+)= sum_b partial[b][c][0]
-  float* out1;           // (+)= sum_b partial[b][c][1]
-  int blocks, C, accumulate;
-};
-
-// 8 columns x 32 lanes per workgroup, fp64 sums in a fixed order
-__global__ __launch_bounds__(256) void col_sum_kernel(ColSumArgs p) {
-  __shared__ double red[32][8][2];
-  const int cl = threadIdx.x & 7, lane = threadIdx.x >> 3;
-  const int c = blockIdx.x * 8 + cl;
-  double s = 0.0, q = 0.0;
-  if (c < p.C) {
-    constexpr int U = 16;   // 512 row blocks in one round trip to memory
-    for (int b = lane; b < p.blocks; b += U * 32) {
-      float2 v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int bb = b + u * 32;
-        v[u] = bb < p.blocks ? *reinterpret_cast<const float2*>(p.partial + (static_cast<int64_t>(bb) * p.C + c) * 2)
-                             : make_float2(0.f, 0.f);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        s += v[u].x;
-        q += v[u].y;
-      }
-    }
-  }
-  red[lane][cl][0] = s;
-  red[lane][cl][1] = q;
-  __syncthreads();
-  for (int off = 16; off > 0; off >>= 1) {
-    if (lane < off) {
-      red[lane][cl][0] += red[lane + off][cl][0];
-      red[lane][cl][1] += red[lane + off][cl][1];
-    }
-    __syncthreads();
-  }
-  if (lane == 0 && c < p.C) {
-    const float a = static_cast<float>(red[0][cl][0]), b = static_cast<float>(red[0][cl][1]);
-    p.out0[c] = p.accumulate ? p.out0[c] + a : a;
-    p.out1[c] = p.accumulate ? p.out1[c] + b : b;
-  }
+__global__ __launch_bounds__(256) void col_sum_kernel(LnSumArgs p) {
+  __shared__ double red[kColSumLds];
+  col_sum_body(p, blockIdx.x, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -781,8 +741,23 @@ int layernorm_bwd(Context* ctx, int dtype, const void* dy, const void* x, void* 
   int rc = dtype == kBF16 ? launch(ctx, ln_kernel_for<bf16, true>(sh), dim3(blocks), dim3(256), a, "ln_bwd_kernel<bf16>", bytes, 1)
                           : launch(ctx, ln_kernel_for<float, true>(sh), dim3(blocks), dim3(256), a, "ln_bwd_kernel<f32>", bytes, 1);
   if (rc) return rc;
-  ColSumArgs s{partial, dgamma, dbeta, blocks, C, accumulate};
+  LnSumArgs s{partial, dgamma, dbeta, blocks, C, accumulate};
+  if (ctx->defer_col_sums) {
+    // rides the next weight gradient (one at a time: an older one goes out now)
+    if (int frc = col_sum_flush(ctx)) return frc;
+    ctx->trailing_col_sum.valid = true;
+    ctx->trailing_col_sum.args = s;
+    return 0;
+  }
   return launch(ctx, col_sum_kernel, dim3((C + 7) / 8), dim3(256), s, "col_sum_kernel", 8.0 * blocks * C, 1);
+}
+
+int col_sum_flush(Context* ctx) {
+  auto& tr = ctx->trailing_col_sum;
+  if (!tr.valid) return 0;
+  tr.valid = false;
+  return launch(ctx, col_sum_kernel, dim3((tr.args.C + 7) / 8), dim3(256), tr.args, "col_sum_kernel",
+                8.0 * tr.args.blocks * tr.args.C, 1);
 }
 
 int gelu_fwd(Context* ctx, int dtype, const void* x, void* y, int64_t n, int tanh_form) {

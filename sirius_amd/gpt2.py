@@ -226,7 +226,13 @@ class GPT2Engine(EngineBase):
         plan.loss_rows = act(R, dtype=torch.float32)
         plan.loss = act(1, dtype=torch.float32)
         ln_mean, ln_rstd = act((2 * L + 1) * R, dtype=torch.float32), act((2 * L + 1) * R, dtype=torch.float32)
-        ln_partial = act(ops.layernorm_bwd_partial_rows(R) * C * 2, dtype=torch.float32)
+        # The column sums of a LayerNorm backward ride the next weight gradient, from a partial buffer of their own.  Six
+        # taken in turn: the one a LayerNorm writes was read by a weight gradient two layers ago at the latest, which
+        # the main lane has waited for (one layer behind, see below).
+        n_partial = ops.layernorm_bwd_partial_rows(R) * C * 2
+        ln_ride = self.trailing_reduce
+        ln_partials = [act(n_partial, dtype=torch.float32) for _ in range(6 if ln_ride else 1)]
+        ln_turn = [0]
 
         # the weight-gradient workspace over every projection of the plan
         ws_bytes = 4
@@ -255,9 +261,10 @@ class GPT2Engine(EngineBase):
 
         def ln_bwd(name, idx, dy, x, dx, residual=None):
             m, r = ln_stats(idx)
+            ln_turn[0] += 1
             ops.layernorm_bwd(ctx, dy, x, dx, self._view(self.params, name + ".weight"), m, r,
-                              self._view(self.grads, name + ".weight"), self._view(self.grads, name + ".bias"), ln_partial,
-                              residual=residual)
+                              self._view(self.grads, name + ".weight"), self._view(self.grads, name + ".bias"),
+                              ln_partials[ln_turn[0] % len(ln_partials)], residual=residual, ride=ln_ride)
 
         def as4(t):
             return t.view(t.shape[0], 1, 1, t.shape[1])

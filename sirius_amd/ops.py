@@ -787,9 +787,17 @@ def layernorm_bwd_partial_rows(rows):
 
 
 def layernorm_bwd(ctx, dy, x, dx, gamma, mean, rstd, dgamma, dbeta, partial, accumulate=False, residual=None,
-                  window=None, windowed=()):
+                  window=None, windowed=(), ride=False):
     """window = (H, W, window size, shift) and windowed, a subset of ("dx", "dy", "residual"): those tensors are laid
-    out as window tokens, everything else ([B*H*W, C] x, the statistics) in pixel order."""
+    out as window tokens, everything else ([B*H*W, C] x, the statistics) in pixel order.  ride: dgamma and dbeta are
+    added up by the next TrailingWgrad call (or its flush) from `partial`, which must stay untouched until then."""
+    if ride:
+        check(lib().tch_layernorm_defer_sums(ctx.handle, 1), "tch_layernorm_defer_sums")
+        try:
+            layernorm_bwd(ctx, dy, x, dx, gamma, mean, rstd, dgamma, dbeta, partial, accumulate, residual, window, windowed)
+        finally:
+            check(lib().tch_layernorm_defer_sums(ctx.handle, 0), "tch_layernorm_defer_sums")
+        return
     C = x.shape[-1]
     rows = x.numel() // C
     assert dy.dtype == x.dtype == dx.dtype and (residual is None or residual.dtype == x.dtype)

@@ -267,8 +267,12 @@ class SwinEngine(EngineBase):
         max_rc = max(B * st["Rp"] ** 2 * st["C"] for st in self.stages)         # elements of the largest [rows, C]
         n_ln = 2 + sum(2 * st["depth"] for st in self.stages) + (len(self.stages) - 1)
         ln_mean, ln_rstd = act(n_ln * rows0, dtype=torch.float32), act(n_ln * rows0, dtype=torch.float32)
-        ln_partial = act(max(ops.layernorm_bwd_partial_rows(B * st["R"] ** 2) * 4 * st["C"] * 2 for st in self.stages),
-                         dtype=torch.float32)
+        # the column sums of a LayerNorm backward ride the next weight gradient, from a partial buffer of their own; four
+        # taken in turn, and the lanes meet at the end of every block: a buffer is written again two such points later
+        n_partial = max(ops.layernorm_bwd_partial_rows(B * st["R"] ** 2) * 4 * st["C"] * 2 for st in self.stages)
+        ln_ride = self.trailing_reduce
+        ln_partials = [act(n_partial, dtype=torch.float32) for _ in range(4 if ln_ride else 1)]
+        ln_turn = [0]
         ln_slot = [0]
 
         def new_ln(rows):
@@ -303,9 +307,11 @@ class SwinEngine(EngineBase):
                               stats[0], stats[1], window=window, **kw)
 
         def ln_bwd(name, dy, x, dx, stats, residual=None, window=None, windowed=()):
+            ln_turn[0] += 1
             ops.layernorm_bwd(ctx, dy, x, dx, self._view(self.params, name + ".weight"), stats[0], stats[1],
-                              self._view(self.grads, name + ".weight"), self._view(self.grads, name + ".bias"), ln_partial,
-                              residual=residual, window=window, windowed=windowed)
+                              self._view(self.grads, name + ".weight"), self._view(self.grads, name + ".bias"),
+                              ln_partials[ln_turn[0] % len(ln_partials)], residual=residual, window=window, windowed=windowed,
+                              ride=ln_ride)
 
         def as4(t):
             return t.view(t.shape[0], 1, 1, t.shape[1])

@@ -40,3 +40,36 @@ def test_order_of_additions_does_not_depend_on_the_rows(ctx, rows):
         outs.append(y[:rows])
     ctx.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layernorm_sums_that_ride_a_weight_gradient(ctx, dtype):
+    """dgamma / dbeta from the next trailing weight gradient, from the backward behind it, and from the flush: the same
+    bits as from the launch of their own."""
+    from sirius_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    rows, C, K = 700, 264, 72
+    x, dy = (torch.randn(rows, C, device="cuda", generator=g).to(dtype) for _ in range(2))
+    gamma, mean, rstd = torch.ones(C, device="cuda"), torch.zeros(rows, device="cuda"), torch.ones(rows, device="cuda")
+    wx, wdy = (torch.randn(rows, 1, 1, n, device="cuda", generator=g).to(dtype) for n in (C, K))
+    n_partial = ops.layernorm_bwd_partial_rows(rows) * C * 2
+    sp = ops.conv2d_wgrad_splits(wx, K, 1, 1, 1, 0)
+    half = ops.conv2d_wgrad_workspace_bytes(ops.dtype_code(wx), K, 1, 1, C, sp) // 4 + 64
+    trail = ops.TrailingWgrad(ctx, torch.empty(2 * half, device="cuda"), half)
+
+    def backward(ride):
+        out = [torch.full((C,), 7.0, device="cuda") for _ in range(2)]
+        ops.layernorm_bwd(ctx, dy, x, torch.empty_like(x), gamma, mean, rstd, *out, torch.empty(n_partial, device="cuda"), ride=ride)
+        return out
+    want = backward(False)
+    dw, ref = torch.empty(K, 1, 1, C, device="cuda"), torch.empty(K, 1, 1, C, device="cuda")
+    ops.conv2d_wgrad(ctx, wx, wdy, ref, 1, 0, workspace=torch.empty(half, device="cuda"), splits=sp)
+    got = [backward(True), backward(True)]      # the first goes out with the second backward
+    trail.wgrad(wx, wdy, dw, 1, 0)
+    got.append(backward(True))
+    trail.flush()
+    ctx.synchronize()
+    assert torch.equal(dw, ref)
+    for pair in got:
+        assert torch.equal(pair[0], want[0]) and torch.equal(pair[1], want[1])
