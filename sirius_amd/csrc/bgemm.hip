@@ -14,9 +14,14 @@
 // A batch index z splits into (z / inner, z % inner) with separate
 // offsets, which addresses head h of sample b inside a packed [B, T, 3C] projection.
 //
-// Tile 64 x 64 x 32, four wavefronts of 32 x 32 (one mfma 32x32 accumulator each).  Operands go
-// global -> registers -> LDS in the [row][k] layout the MFMA fragments read; a chunk that is not
-// contiguous along k is scattered element by element on its way into LDS.
+// Tile 64 x 64 x 64, four wavefronts of 32 x 32 (one mfma 32x32 accumulator each).  Operands go global -> registers ->
+// LDS; the registers of the next 64 reduction steps are loaded before the multiplications of the present ones, because a
+// GPT-2 step at 2x256 has 96 to 384 workgroups of four wavefronts here: one trip to memory per step was what they waited
+// for.  In LDS a k-contiguous operand lies as [row][k], as the MFMA fragments read it; one that is contiguous along the
+// rows is scattered to that layout in bf16, but stays [k][row] in fp32, where a fragment is one element per lane and
+// reads from there without conflicts.
+// fp32, 24 heads, out of a step: P V and dS K 24.8 -> 10.4 us, P^T dO and dS^T Q 24.8 -> 12.8 us, the scores 10.2 -> 7.4 us,
+// against steps of 32 with nothing in flight.
 //
 // Reference call sites of the products: window attention q @ k^T and attn @ v
 // (train/swin_b_tiny.py:94-110); GPT-2 attention inside transformers (train/gpt2.py:26).
@@ -27,7 +32,7 @@ namespace tch {
 namespace {
 
 constexpr int kTile = 64;
-constexpr int kBK = 32;
+constexpr int kBK = 64;
 
 struct BgemmArgs {
   const void* a;
@@ -55,67 +60,86 @@ __device__ inline void mma_step<float>(const Chunk& first, const Chunk& second, 
   for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(first.f[e], second.f[e], acc, 0, 0, 0);
 }
 
-// One operand tile [64 rows][kBK] into LDS rows of (kBK / E + 1) chunks.  `rows`/`ks` are what is
-// left of the matrix from this tile's origin; everything beyond reads as zero.
-template <typename T>
-__device__ inline void stage_tile(const T* base, int64_t rs, int64_t cs, int rows, int ks, unsigned char* lds, int tid) {
-  constexpr int E = Elem<T>::kPerChunk;
-  constexpr int KCH = kBK / E;                    // chunks along k per row
-  constexpr int ROW_BYTES = (KCH + 1) * 16;
-  constexpr int CHUNKS = kTile * kBK / E;          // per tile
-  constexpr int PER_THREAD = CHUNKS / 256;
-  static_assert(CHUNKS % 256 == 0, "tile/loader mismatch");
+// One operand tile [64 rows][kBK] on its way into LDS.  KC: the operand is contiguous along k, otherwise along the rows.
+template <typename T, bool KC>
+struct Tile {
+  static constexpr int E = Elem<T>::kPerChunk;
+  static constexpr int PER_THREAD = kTile * kBK / E / 256;
+  static constexpr bool KMAJOR = !KC && sizeof(T) == 4;      // [k][row] in LDS
+  static constexpr int PITCH = KMAJOR ? (kTile + 4) * 4 : (kBK / E + 1) * 16;
+  static constexpr int BYTES = (KMAJOR ? kBK : kTile) * PITCH;
+  Chunk reg[PER_THREAD];
+
+  // first: where the chunk q begins along the contiguous axis; second: its place along the other
+  __device__ static int first(int q) { return q % (kTile / E) * E; }
+  __device__ static int second(int q) { return q / (kTile / E); }
+
+  // `rows` / `ks` are what is left of the matrix from this tile's origin; everything beyond reads as zero
+  __device__ inline void load(const T* base, int64_t stride, int rows, int ks, int tid) {
+    const int n1 = KC ? ks : rows, n2 = KC ? rows : ks;
+    const bool aligned = (reinterpret_cast<uintptr_t>(base) & 15) == 0 && stride % E == 0;
+    if (aligned && n1 >= 64 && n2 >= 64) {
 #pragma unroll
-  for (int it = 0; it < PER_THREAD; ++it) {
-    const int q = tid + it * 256;
-    if (cs == 1) {
-      // chunk = E consecutive k of one row
-      const int r = q / KCH, kc = (q - r * KCH) * E;
-      const T* src = base + static_cast<int64_t>(r) * rs + kc;
+      for (int it = 0; it < PER_THREAD; ++it) {
+        const int q = tid + it * 256;
+        reg[it].u = *reinterpret_cast<const uint4*>(base + second(q) * stride + first(q));
+      }
+      return;
+    }
+#pragma unroll
+    for (int it = 0; it < PER_THREAD; ++it) {
+      const int q = tid + it * 256, i = first(q);
+      const T* src = base + second(q) * stride + i;
       Chunk ch = zero_chunk();
-      if (r < rows) {
-        if (kc + E <= ks && (reinterpret_cast<uintptr_t>(src) & 15) == 0) {
+      if (second(q) < n2) {
+        if (aligned && i + E <= n1) {
           ch.u = *reinterpret_cast<const uint4*>(src);
         } else {
           T* dst = reinterpret_cast<T*>(&ch);
 #pragma unroll
           for (int e = 0; e < E; ++e)
-            if (kc + e < ks) dst[e] = src[e];
+            if (i + e < n1) dst[e] = src[e];
         }
       }
-      *reinterpret_cast<uint4*>(lds + r * ROW_BYTES + kc * sizeof(T)) = ch.u;
-    } else {
-      // chunk = E consecutive rows at one k (rs == 1)
-      constexpr int RCH = kTile / E;
-      const int k = q / RCH, r0 = (q - k * RCH) * E;
-      const T* src = base + static_cast<int64_t>(k) * cs + r0;
-      Chunk ch = zero_chunk();
-      if (k < ks) {
-        if (r0 + E <= rows && (reinterpret_cast<uintptr_t>(src) & 15) == 0) {
-          ch.u = *reinterpret_cast<const uint4*>(src);
-        } else {
-          T* dst = reinterpret_cast<T*>(&ch);
-#pragma unroll
-          for (int e = 0; e < E; ++e)
-            if (r0 + e < rows) dst[e] = src[e];
-        }
-      }
-      const T* vals = reinterpret_cast<const T*>(&ch);
-#pragma unroll
-      for (int e = 0; e < E; ++e) *reinterpret_cast<T*>(lds + (r0 + e) * ROW_BYTES + k * sizeof(T)) = vals[e];
+      reg[it] = ch;
     }
   }
-}
 
-template <typename T>
+  __device__ inline void store(unsigned char* lds, int tid) const {
+#pragma unroll
+    for (int it = 0; it < PER_THREAD; ++it) {
+      const int q = tid + it * 256;
+      if constexpr (KC || KMAJOR) {
+        *reinterpret_cast<uint4*>(lds + second(q) * PITCH + first(q) * sizeof(T)) = reg[it].u;
+      } else {
+        const T* vals = reinterpret_cast<const T*>(&reg[it]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) *reinterpret_cast<T*>(lds + (first(q) + e) * PITCH + second(q) * sizeof(T)) = vals[e];
+      }
+    }
+  }
+
+  // E reduction elements of one row, from chunk kc on
+  __device__ static inline Chunk fragment(const unsigned char* lds, int row, int kc) {
+    Chunk c;
+    if constexpr (KMAJOR) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) c.f[e] = *reinterpret_cast<const float*>(lds + (kc * E + e) * PITCH + row * 4);
+    } else {
+      c.u = *reinterpret_cast<const uint4*>(lds + row * PITCH + kc * 16);
+    }
+    return c;
+  }
+};
+
+template <typename T, bool A_KC, bool B_KC>
 __global__ __launch_bounds__(256) void bgemm_kernel(BgemmArgs p) {
   constexpr int E = Elem<T>::kPerChunk;
-  constexpr int KCH = kBK / E;
-  constexpr int ROW_BYTES = (KCH + 1) * 16;
-  constexpr int TILE_BYTES = kTile * ROW_BYTES;
+  using TA = Tile<T, A_KC>;
+  using TB = Tile<T, B_KC>;
   constexpr int STAGE_LD = kTile + 4;  // floats per row of the output staging tile
   constexpr int STAGE_BYTES = kTile * STAGE_LD * 4;
-  constexpr int LDS_BYTES = 2 * TILE_BYTES > STAGE_BYTES ? 2 * TILE_BYTES : STAGE_BYTES;
+  constexpr int LDS_BYTES = TA::BYTES + TB::BYTES > STAGE_BYTES ? TA::BYTES + TB::BYTES : STAGE_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char lds[LDS_BYTES];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -129,23 +153,32 @@ __global__ __launch_bounds__(256) void bgemm_kernel(BgemmArgs p) {
   const int zo = z / p.batch_inner, zi = z - zo * p.batch_inner;
   const T* A = static_cast<const T*>(p.a) + zo * p.a_bo + zi * p.a_bi + static_cast<int64_t>(m0) * p.a_rs;
   const T* B = static_cast<const T*>(p.b) + zo * p.b_bo + zi * p.b_bi + static_cast<int64_t>(n0) * p.b_rs;
+  TA ta;
+  TB tb;
+  auto load = [&](int k0) {
+    ta.load(A + static_cast<int64_t>(k0) * p.a_cs, A_KC ? p.a_rs : p.a_cs, p.M - m0, k_end - k0, tid);
+    tb.load(B + static_cast<int64_t>(k0) * p.b_cs, B_KC ? p.b_rs : p.b_cs, p.N - n0, k_end - k0, tid);
+  };
 
   f32x16_t acc;
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0.f;
   const int frag_row = lane & 31, frag_half = lane >> 5;
+  load(k_begin);
   for (int k0 = k_begin; k0 < k_end; k0 += kBK) {
     __syncthreads();
-    stage_tile<T>(A + static_cast<int64_t>(k0) * p.a_cs, p.a_rs, p.a_cs, p.M - m0, k_end - k0, lds, tid);
-    stage_tile<T>(B + static_cast<int64_t>(k0) * p.b_cs, p.b_rs, p.b_cs, p.N - n0, k_end - k0, lds + TILE_BYTES, tid);
+    ta.store(lds, tid);
+    tb.store(lds + TA::BYTES, tid);
     __syncthreads();
+    if (k0 + kBK < k_end) load(k0 + kBK);
+    auto half = [&](int h) {
 #pragma unroll
-    for (int kk = 0; kk < KCH / 2; ++kk) {
-      Chunk fa, fb;
-      fa.u = *reinterpret_cast<const uint4*>(lds + (wm * 32 + frag_row) * ROW_BYTES + (kk * 2 + frag_half) * 16);
-      fb.u = *reinterpret_cast<const uint4*>(lds + TILE_BYTES + (wn * 32 + frag_row) * ROW_BYTES + (kk * 2 + frag_half) * 16);
-      mma_step<T>(fb, fa, acc);  // B rows -> accumulator registers, A rows -> lanes
-    }
+      for (int kk = h * (kBK / E / 4); kk < (h + 1) * (kBK / E / 4); ++kk)   // B rows -> accumulator registers, A rows -> lanes
+        mma_step<T>(TB::fragment(lds + TA::BYTES, wn * 32 + frag_row, kk * 2 + frag_half),
+                    TA::fragment(lds, wm * 32 + frag_row, kk * 2 + frag_half), acc);
+    };
+    half(0);
+    if (k0 + kBK / 2 < k_end) half(1);   // a head of 32 fills half a step
   }
   // lane (l & 31) holds row m; register 4 j + i holds column 8 j + 4 (l >> 5) + i.  The tile goes through
   // LDS so that every lane then owns E consecutive columns of one row: 16-byte stores along the rows of C.
@@ -211,9 +244,13 @@ int batched_gemm(Context* ctx, int dtype, const void* a, const void* b, void* c,
   static const char* const names[2][4] = {
       {"bgemm_kernel<f32,kk>", "bgemm_kernel<f32,kt>", "bgemm_kernel<f32,tk>", "bgemm_kernel<f32,tt>"},
       {"bgemm_kernel<bf16,kk>", "bgemm_kernel<bf16,kt>", "bgemm_kernel<bf16,tk>", "bgemm_kernel<bf16,tt>"}};
-  const char* name = names[dtype == kBF16][(a_cs == 1 ? 0 : 2) + (b_cs == 1 ? 0 : 1)];
-  return dtype == kBF16 ? launch(ctx, bgemm_kernel<bf16>, grid, dim3(256), g, name, flops, 0)
-                        : launch(ctx, bgemm_kernel<float>, grid, dim3(256), g, name, flops, 0);
+  static void (*const kernels[2][4])(BgemmArgs) = {
+      {bgemm_kernel<float, true, true>, bgemm_kernel<float, true, false>, bgemm_kernel<float, false, true>,
+       bgemm_kernel<float, false, false>},
+      {bgemm_kernel<bf16, true, true>, bgemm_kernel<bf16, true, false>, bgemm_kernel<bf16, false, true>,
+       bgemm_kernel<bf16, false, false>}};
+  const int way = (a_cs == 1 ? 0 : 2) + (b_cs == 1 ? 0 : 1);
+  return launch(ctx, kernels[dtype == kBF16][way], grid, dim3(256), g, names[dtype == kBF16][way], flops, 0);
 }
 
 }  // namespace tch
