@@ -2396,10 +2396,13 @@ int effective_tile(int tile_cfg, int dtype, int in_c, int taps) {
 }
 
 // Enough workgroups to give each of the 256 CUs some, with bigger tiles as
-// soon as the problem can afford them.
-int pick_tile(int gemm_m, int gemm_n, int splits) {
-  if (gemm_n > 64 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= 384) return 0;
-  if (tiles_for(gemm_m, gemm_n, 128, 64) * splits >= 384) return 1;
+// soon as the problem can afford them.  fp32 over short reductions is epilogue and latency: small tiles share a CU and
+// overlap theirs (data gradients with the batch sums, 12544 x 256 over 64: 16.8 us as 128 x 128, 14.8 as 64 x 64; 25088
+// rows 26.8 and 21.8).
+int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
+  if (dtype == kF32 && gemm_k <= 128) return 2;
+  if (gemm_n > 64 && tiles_for(gemm_m, gemm_n, 128, 128) >= 384) return 0;
+  if (tiles_for(gemm_m, gemm_n, 128, 64) >= 384) return 1;
   return 2;
 }
 
@@ -2446,7 +2449,9 @@ int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps
   const int64_t t32 = tiles_for(gemm_m, gemm_n, 32, 32), t64 = tiles_for(gemm_m, gemm_n, 64, 64);
   if (t32 <= 256) return gemm_k >= 1024 ? kSplit32Deep : kSplit32;
   if (dtype == kBF16) return t32 <= 512 ? kSplit32 : -1;
-  if (t32 <= 512) return gemm_k >= 768 ? kSplit64x32Deep : kSplit32;
+  // up to two 32 x 32 tiles per CU: they hide each other's latencies until the reduction is long enough to do so alone
+  // (3136 x 128 over 1152 with the batch sums: 17.4 us as 64 x 32, 16.2 as 32 x 32; 640 x 768 over 3072: 32.4 and 33.9)
+  if (t32 <= 512) return gemm_k >= 1536 ? kSplit64x32Deep : kSplit32;
   if (t64 <= 256 && gemm_k >= 768) return kSplit64;
   if (t64 <= 512 && gemm_k >= 512) return kSplit64x32;
   return gemm_k >= 256 && tiles_for(gemm_m, gemm_n, 128, 128) < 384 ? kSplit64Pair : -1;
@@ -2464,7 +2469,7 @@ struct TileQuery {
 int heuristic_tile(int asked, const TileQuery& q) {
   if (!direct_tile_fits(q.dtype, q.in_c, q.taps)) {
     const int split = asked == kAutoInOrder ? -1 : split_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k, q.in_c, q.taps);
-    return split >= 0 ? split : pick_tile(q.gemm_m, q.gemm_n, 1);
+    return split >= 0 ? split : pick_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k);
   }
   const float steps = static_cast<float>(q.gemm_k) / 64.f, store = static_cast<float>(q.gemm_m) * q.gemm_n * 1e-6f;
   const bool large = tiles_for(q.gemm_m, q.gemm_n, 128, 128) >= 384;
