@@ -267,11 +267,12 @@ class SwinEngine(EngineBase):
         max_rc = max(B * st["Rp"] ** 2 * st["C"] for st in self.stages)         # elements of the largest [rows, C]
         n_ln = 2 + sum(2 * st["depth"] for st in self.stages) + (len(self.stages) - 1)
         ln_mean, ln_rstd = act(n_ln * rows0, dtype=torch.float32), act(n_ln * rows0, dtype=torch.float32)
-        # the column sums of a LayerNorm backward ride the next weight gradient, from a partial buffer of their own; four
-        # taken in turn, and the lanes meet at the end of every block: a buffer is written again two such points later
+        # the column sums of a LayerNorm backward ride the next weight gradient, from a partial buffer of their own; six
+        # taken in turn: the last one a section of the backward pass writes is read by the first weight gradient of the
+        # next section and written again two sections after that at the earliest
         n_partial = max(ops.layernorm_bwd_partial_rows(B * st["R"] ** 2) * 4 * st["C"] * 2 for st in self.stages)
         ln_ride = self.trailing_reduce
-        ln_partials = [act(n_partial, dtype=torch.float32) for _ in range(4 if ln_ride else 1)]
+        ln_partials = [act(n_partial, dtype=torch.float32) for _ in range(6 if ln_ride else 1)]
         ln_turn = [0]
         ln_slot = [0]
 
@@ -339,10 +340,16 @@ class SwinEngine(EngineBase):
         def flat(n):
             return act(n)
         s_n1 = flat(max_rc)                                    # LayerNorm output before it is gathered
-        # gradients of [rows, C] tensors, handed round; six, so that inside a block nothing the second lane
-        # still reads (the block's incoming gradient, the gathered projection gradient) is written again
-        g_bufs = [flat(max_rc) for _ in range(6)]
-        g_3c, g_4c_a, g_4c_b = flat(3 * max_rc), flat(4 * max_rc), flat(4 * max_rc)
+        # The backward pass is cut into sections (one per block and patch merging).  The second lane may trail the main
+        # one by a section: when section k begins, the main lane has waited for the weight gradients of section k - 2.
+        # (Meeting at the end of every section cost the main lane the tail of the weight gradient that its last projection
+        # forks: 1 % of a Swin-B step over 32 images.)  So what the second lane reads of a section's own gradients comes in two sets, taken in turn, and
+        # the gradient handed from section to section, read in the section behind the one that writes it, in three.
+        n_sets = 2 if self.overlap_wgrad else 1
+        g_sets = [[flat(max_rc) for _ in range(4)] for _ in range(n_sets)]
+        g_ring = [flat(max_rc) for _ in range(n_sets + 1)]
+        g_3c_sets, g_4c_sets = ([flat(n * max_rc) for _ in range(n_sets)] for n in (3, 4))
+        g_4c_a = flat(4 * max_rc)        # main lane only
         # One launch per direction for the attention of a block where the kernel's limits hold (bf16, heads 32
         # wide and even in number, at most 64 tokens per window): score rows are then padded to 64 keys.
         for st in self.stages:
@@ -351,10 +358,10 @@ class SwinEngine(EngineBase):
             st["keys_ld"] = 64 if st["fused"] else st["ws"] ** 2      # leading dimension of a score row
             st["bias_elems"] = st["heads"] * (64 * 64 if st["fused"] else st["ws"] ** 4)
         max_scores = max(B * (st["Rp"] // st["ws"]) ** 2 * st["heads"] * st["ws"] ** 2 * st["keys_ld"] for st in self.stages)
-        d_scores = flat(max_scores)
+        d_scores_sets = [flat(max_scores) for _ in range(n_sets)]
         max_bias = max(st["bias_elems"] for st in self.stages)
         bias_buf = act(max_bias, dtype=torch.float32)
-        dbias_buf = act(max_bias, dtype=torch.float32)
+        dbias_buf = act(max_bias, dtype=torch.float32)         # second lane only
         colsum_ws = act(max(ops.column_sum_workspace_floats(B * (st["Rp"] // st["ws"]) ** 2,
                                                             st["heads"] * st["ws"] ** 2 * st["keys_ld"])
                             for st in self.stages), dtype=torch.float32)
@@ -514,12 +521,12 @@ class SwinEngine(EngineBase):
             # ================= backward =================
             if self.overlap_wgrad:
                 ctx.join()      # the second lane may still be writing the transposed filters of the last optimizer step
-            g_pooled = v2(g_bufs[0], B, CL)
+            section = 0
+            g_pooled = v2(g_sets[0][0], B, CL)
             lin_bwd("head", pooled, dlogits, g_pooled)
-            g_hf = v2(g_bufs[1], rowsL, CL)
+            g_hf = v2(g_sets[0][1], rowsL, CL)
             ops.avgpool_bwd(ctx, g_pooled, g_hf.view(B, stL["R"], stL["R"], CL))
-            gi = 2                                            # index of the buffer that holds the running gradient
-            g = v2(g_bufs[gi], rowsL, CL)
+            g = v2(g_ring[0], rowsL, CL)                      # the running gradient: ring place `section`
             ln_bwd("norm", g_hf, x, g, final_stats)
             mark("bwd", "norm")
             merges = {si: m for si, *m in saved_merges}
@@ -540,27 +547,27 @@ class SwinEngine(EngineBase):
                     # g is the gradient of the merged tokens [rows/4, 2C]
                     xm, nm, mstats = merges[si]
                     pre = f"features.{st['f'] + 1}."
-                    spare = [k for k in range(len(g_bufs)) if k != gi]
+                    section += 1
                     d_nm = v2(g_4c_a, mrows, 4 * C)
                     with side():
                         wgrad(as4(nm), as4(g), self._view(self.grads, pre + "reduction.weight"))
                     ops.conv2d_dgrad(ctx, as4(g), self._wt(pre + "reduction.weight"), as4(d_nm), 1, 0)
-                    d_xm = v2(g_4c_b, mrows, 4 * C)
+                    d_xm = v2(g_4c_sets[section % n_sets], mrows, 4 * C)
                     ln_bwd(pre + "norm", d_nm, xm, d_xm, mstats)
-                    gi = spare[0]
-                    g = v2(g_bufs[gi], rows, C)
+                    g = v2(g_ring[section % len(g_ring)], rows, C)
                     ops.patch_merge_gather(ctx, d_xm, g, (B, R, R, C), reverse=True)
                     if self.overlap_wgrad:
-                        ctx.join()
+                        ctx.join(behind=True)
                     mark("bwd", pre[:-1])
                 for i in range(st["depth"] - 1, -1, -1):
                     bi -= 1
                     _, _, shift, x_in, xw, qkv, Pm, o, x1, n2, f1, f2, stats1, stats2 = saved_blocks[bi]
                     pre = f"features.{st['f']}.{i}."
-                    spare = [k for k in range(len(g_bufs)) if k != gi]
+                    section += 1
+                    g_bufs, g_3c, g_4c_b, d_scores = (of[section % n_sets] for of in (g_sets, g_3c_sets, g_4c_sets, d_scores_sets))
                     # t_b, t_c, t_d carry window-ordered gradients (the padded frame's rows) wherever the block has windows
-                    t_a, t_e = v2(g_bufs[spare[0]], rows, C), v2(g_bufs[spare[4]], rows, C)
-                    t_b, t_c, t_d = (v2(g_bufs[k], wrows, C) for k in spare[1:4])
+                    t_a = v2(g_bufs[0], rows, C)
+                    t_b, t_c, t_d = (v2(g_bufs[k], wrows, C) for k in (1, 2, 3))
                     d_f2, d_f1, d_qkv = v2(g_4c_a, rows, 4 * C), v2(g_4c_b, rows, 4 * C), v2(g_3c, wrows, 3 * C)
                     fq, fg = qkv.view(-1), d_qkv.view(-1)
                     dP = d_scores[:B_ * Hh * N * st["keys_ld"]].view(B_, Hh, N, st["keys_ld"])
@@ -613,9 +620,7 @@ class SwinEngine(EngineBase):
                                          qkv_b, alpha=scale)
                     d_xw = t_d
                     lin_bwd(pre + "attn.qkv", xw, d_qkv, d_xw)
-                    # the new running gradient goes into a buffer of its own: the old one may still be read by
-                    # this block's first weight gradient on the second lane
-                    g_next = t_e
+                    g_next = v2(g_ring[section % len(g_ring)], rows, C)
                     if fuse_w:
                         ln_bwd(pre + "norm1", d_xw, x_in, g_next, stats1, residual=g1, window=win,
                                windowed=("dy", "residual"))
@@ -626,15 +631,16 @@ class SwinEngine(EngineBase):
                             d_n1 = t_c
                             ops.window_partition(ctx, d_xw, d_n1, ws, shift, reverse=True, image_shape=(B, R, R, C))
                         ln_bwd(pre + "norm1", d_n1, x_in, g_next, stats1, residual=g1)
-                    g, gi = g_next, spare[4]
+                    g = g_next
                     if self.overlap_wgrad:
-                        ctx.join()
+                        ctx.join(behind=True)
                     mark("bwd", pre[:-1])
             # patch embedding: LayerNorm, then the 4x4 stride-4 convolution (no data gradient: it is the input)
-            spare = [k for k in range(len(g_bufs)) if k != gi]
-            d_e0 = v2(g_bufs[spare[0]], rows0, C0)
+            d_e0 = v2(g_sets[(section + 1) % n_sets][0], rows0, C0)
             ln_bwd("features.0.2", g, e0, d_e0, embed_stats)
-            # on the main lane, behind the join that ended the last block: the second lane's last weight gradient has
+            if self.overlap_wgrad:
+                ctx.join()
+            # on the main lane, behind the join: the second lane's last weight gradient has
             # finished, so its pending reduction may ride this launch; this one's own reduction follows at once
             wgrad(x0, d_e0.view(B, R0, R0, C0), self._view(self.grads, "features.0.0.weight"), stride=P, c_logical=3)
             if trail is not None:
