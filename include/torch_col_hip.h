@@ -92,7 +92,9 @@ typedef struct tch_launch_stat {
   int lane;           /* 0 = main lane, 1 = the lane that may run beside it */
   int64_t workgroups;
 } tch_launch_stat;
-/* The same replay, one row per program position (out[i] is launch i): what each launch of a step costs alone
+/* What the program would launch, one row per program position, without running anything (ms = 0; needs no GPU). */
+int tch_program_launches(const tch_program* prog, tch_launch_stat* out, int64_t max_out, int64_t* n_out);
+/* A replay as tch_program_profile makes it, one row per program position (out[i] is launch i): what each launch of a step costs alone
  * on the chip, next to the work it states -- the input of a per-layer roofline table. */
 int tch_program_profile_launches(tch_context* ctx, const tch_program* prog, int reps, tch_launch_stat* out,
                                  int64_t max_out, int64_t* n_out);
@@ -238,7 +240,9 @@ int tch_bn_eval_coef(tch_context* ctx, const float* gamma, const float* beta, co
 int tch_bn_apply_bwd(tch_context* ctx, int dtype, const void* g, const void* x, void* dx, int64_t rows, int C,
                      const float* coef);
 /* dw[K,R,S,C] (fp32) (+)= sum over pixels of dy x x.  splits > 1 needs a workspace of
- * tch_conv2d_wgrad_workspace_bytes(); splits <= 0 lets the library choose (query with _pick_splits). */
+ * tch_conv2d_wgrad_workspace_bytes(); splits <= 0 lets the library choose (query with _pick_splits).  tile_cfg, here and in
+ * every form below: 0 = 128x128, 1 = 128x64, 2 = 64x64; the other numbers of the list above stand for the one of their
+ * shape (15 - 20: for 2). */
 int tch_conv2d_wgrad_pick_splits(int dtype, int N, int H, int W, int C, int K, int R, int S, int stride, int pad);
 int64_t tch_conv2d_wgrad_workspace_bytes(int dtype, int K, int R, int S, int C, int splits);
 int tch_conv2d_wgrad(tch_context* ctx, int dtype, const void* x, const void* dy, float* dw, float* workspace,

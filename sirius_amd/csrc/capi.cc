@@ -703,6 +703,26 @@ extern "C" int tch_program_time_kernel(tch_context* ctx, const tch_program* prog
   return time_kernel_in_program(&ctx->ctx, prog->prog, kernel_name, reps, mean_us, launches_per_replay);
 }
 
+extern "C" int tch_program_launches(const tch_program* prog, tch_launch_stat* out, int64_t max_out, int64_t* n_out) {
+  if (!prog || !n_out || max_out < 0 || (!out && max_out > 0)) {
+    set_error("tch_program_launches: bad arguments");
+    return -22;
+  }
+  int64_t n = 0;
+  for (const LaunchRecord& l : prog->prog.launches) {
+    if (n >= max_out) break;
+    tch_launch_stat& o = out[n++];
+    snprintf(o.name, sizeof(o.name), "%s", l.fn && l.name ? l.name : "");
+    o.ms = 0.0;
+    o.flops = l.fn && !l.work_is_bytes ? l.work : 0.0;
+    o.bytes = l.fn ? l.bytes : 0.0;
+    o.lane = l.lane;
+    o.workgroups = l.fn ? static_cast<int64_t>(l.grid.x) * l.grid.y * l.grid.z : 0;
+  }
+  *n_out = n;
+  return 0;
+}
+
 extern "C" int tch_program_profile_launches(tch_context* ctx, const tch_program* prog, int reps, tch_launch_stat* out,
                                             int64_t max_out, int64_t* n_out) {
   if (!ctx || !prog || !out || !n_out || max_out < 1) {

@@ -2260,8 +2260,44 @@ enum PipeTile : int {
 // the tiling of the same shape that runs where a pipelined one does not exist
 int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : 1; }
 
+// The weight-gradient kernel's tile (0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64) for a tiling number: the same shape where
+// there is one.  How the other kernels walk a tile (steps, LDS tiles, reductions split over wavefronts, the 3x3 patch) has
+// no meaning here, whose reduction is split over workgroups.
+int wgrad_tile(int tile_cfg) {
+  switch (tile_cfg) {
+    case 0:
+    case 9:
+    case 10:
+    case 11:
+    case 12:
+      return 0;
+    case 1:
+    case 5:
+    case 6:
+    case 13:
+    case kPipe128x64:
+      return 1;
+    default:
+      return 2;
+  }
+}
+
+template <typename T>
+int launch_wgrad(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
+  switch (wgrad_tile(tile_cfg)) {
+    case 0:
+      return launch_cfg<T, kWgrad, 2, 2, 2, 2>(ctx, a, flops);
+    case 1:
+      return launch_cfg<T, kWgrad, 2, 2, 2, 1>(ctx, a, flops);
+    default:
+      return launch_cfg<T, kWgrad, 2, 2, 1, 1>(ctx, a, flops);
+  }
+}
+
+// forward and data gradient
 template <typename T, int MODE>
 int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
+  static_assert(MODE == kFwd || MODE == kDgrad, "weight gradients go through launch_wgrad");
   switch (tile_cfg) {
     case kSplit32:
       return launch_cfg4<T, MODE, 1, 1, 4, 4>(ctx, a, flops);
@@ -2279,7 +2315,7 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
     default:
       break;
   }
-  if constexpr (sizeof(T) == 2 && (MODE == kFwd || MODE == kDgrad)) {
+  if constexpr (sizeof(T) == 2) {
     const int in_c = MODE == kFwd ? a.C : a.K;
     const int setting = igemm2_setting();
     if (tile_cfg == 5) {   // 128 x 64 with the 3x3 patch in LDS; convolutions it does not fit run as tiling 1
@@ -2773,8 +2809,8 @@ int conv2d_wgrad(Context* ctx, int dtype, const ConvShape& s, const void* x, con
   if (tile_cfg < 0) {
     tile_cfg = wgrad_big_tile(a.gemm_m, a.gemm_n, splits) ? 0 : 2;
   }
-  int rc = dtype == kBF16 ? launch_mode<bf16, kWgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
-                          : launch_mode<float, kWgrad>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));
+  int rc = dtype == kBF16 ? launch_wgrad<bf16>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
+                          : launch_wgrad<float>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));
   if (rc) return rc;
   if (splits > 1) {
     ReduceArgs r{workspace, dw, static_cast<int64_t>(a.gemm_m) * a.gemm_n, splits, accumulate, dbias_partial, dbias,

@@ -42,3 +42,34 @@ def test_batchnorm_sums(ctx, dtype, case, tile_cfg):
 def test_library_choice(ctx, dtype, rows, K, C):
     """One size on each side of the lines of the library's own choice."""
     T.test_conv_fwd(ctx, dtype, (rows, 1, 1, C, K, 1, 1, 1, 0), -1)
+
+
+@dtypes
+@pytest.mark.parametrize("tile_cfg", TILES)
+@pytest.mark.parametrize("splits", [1, 3])
+def test_weight_gradient_ignores_the_split_tilings(ctx, dtype, tile_cfg, splits):
+    """15 - 20 are no tilings of a weight gradient: the bits of tiling 2 (the same kernel), alone and with a pending
+    reduction to take along, and both against the float64 product."""
+    from sirius_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    rows, C, K = 500, 72, 136
+    x, dy = (torch.randn(rows, 1, 1, n, device="cuda", generator=g).to(dtype) for n in (C, K))
+    half = ops.conv2d_wgrad_workspace_bytes(ops.dtype_code(x), K, 1, 1, C, 8) // 4
+    ws = torch.empty(2 * half, device="cuda")
+    got, ref, other = (torch.empty(K, 1, 1, C, device="cuda") for _ in range(3))
+    ops.conv2d_wgrad(ctx, x, dy, ref, 1, 0, workspace=ws, splits=splits, tile_cfg=2)
+    ops.conv2d_wgrad(ctx, x, dy, got, 1, 0, workspace=ws, splits=splits, tile_cfg=tile_cfg)
+    ctx.synchronize()
+    want = (dy.double().view(rows, K).t() @ x.double().view(rows, C)).view_as(ref)
+    # products of exact operands summed in fp32 over 500 rows: 500 * 2^-24 of the sum of magnitudes at the very worst
+    scale = (dy.double().abs().view(rows, K).t() @ x.double().abs().view(rows, C)).view_as(ref)
+    assert ((ref - want).abs() <= 500 * 2.0 ** -24 * scale).all()
+    assert torch.equal(got, ref)
+    trail = ops.TrailingWgrad(ctx, ws, half)
+    trail.wgrad(x, dy, other, 1, 0)
+    trail.wgrad(x, dy, got, 1, 0, tile_cfg=tile_cfg)
+    trail.flush()
+    ops.conv2d_wgrad(ctx, x, dy, ref, 1, 0, workspace=ws, splits=ops.conv2d_wgrad_splits(x, K, 1, 1, 1, 0), tile_cfg=2)
+    ctx.synchronize()
+    assert torch.equal(other, got) and torch.equal(got, ref)

@@ -1,0 +1,89 @@
+"""What a recorded program holds (tch_program_launches): which kernel a call is sent to, on the CPU.  Nothing runs: the
+addresses are made up."""
+import ctypes
+
+import pytest
+
+from sirius_amd._lib import LaunchStat, check, lib
+
+F32, BF16 = 0, 1
+dtypes = pytest.mark.parametrize("dtype", [F32, BF16], ids=["f32", "bf16"])
+
+
+def address(i):
+    return ctypes.c_void_p(0x10000000 * (i + 1))
+
+
+class Recorder:
+    """A context and the programs recorded on it."""
+
+    def __init__(self):
+        self.ctx = ctypes.c_void_p()
+        check(lib().tch_context_create(None, ctypes.byref(self.ctx)))
+        self.progs = []
+
+    def begin(self):
+        prog = ctypes.c_void_p()
+        check(lib().tch_program_create(ctypes.byref(prog)))
+        check(lib().tch_program_begin_record(self.ctx, prog))
+        self.progs.append(prog)
+
+    def end(self):
+        """End the recording; [(kernel name, workgroups, lane)] of the launches in it (joins of the lanes: '')."""
+        check(lib().tch_program_end_record(self.ctx))
+        prog = self.progs[-1]
+        cap = int(lib().tch_program_size(prog))
+        rows, n = (LaunchStat * max(cap, 1))(), ctypes.c_int64()
+        check(lib().tch_program_launches(prog, rows, cap, ctypes.byref(n)))
+        assert n.value == cap
+        return [(r.name.decode(), int(r.workgroups), int(r.lane)) for r in rows[:cap]]
+
+    def close(self):
+        for p in self.progs:
+            lib().tch_program_destroy(p)
+        lib().tch_context_destroy(self.ctx)
+
+
+@pytest.fixture
+def rec():
+    r = Recorder()
+    yield r
+    r.close()
+
+
+K, C, ROWS = 256, 192, 4096
+NAMES = {F32: "f32", BF16: "bf16"}
+
+
+def wgrad(rec, dtype, tile_cfg, splits, trailing=False):
+    args = [rec.ctx, dtype, address(0), address(1), address(2)]
+    tail = [address(3), splits, 0, ROWS, 1, 1, C, K, 1, 1, 1, 0, tile_cfg, 0]
+    if trailing:
+        check(lib().tch_conv2d_wgrad_trailing(*args, None, *tail))
+    else:
+        check(lib().tch_conv2d_wgrad(*args, *tail))
+
+
+@dtypes
+@pytest.mark.parametrize("tile_cfg", range(23))
+def test_every_tiling_number_of_a_weight_gradient_runs_its_kernel(rec, dtype, tile_cfg):
+    """The tilings of the other directions stand for a shape; none of their kernels may get a weight gradient's operands."""
+    side = {0: (128, 128), 1: (128, 64)}.get({9: 0, 10: 0, 11: 0, 12: 0, 5: 1, 6: 1, 13: 1, 22: 1}.get(tile_cfg, tile_cfg), (64, 64))
+    tiles = (K // side[0]) * (-(-C // side[1]))
+    for splits in (1, 4):
+        rec.begin()
+        wgrad(rec, dtype, tile_cfg, splits)
+        got = rec.end()
+        assert got[0][:2] == (f"wgrad_kernel<{NAMES[dtype]},{side[0]}x{side[1]}>", tiles * splits)
+        assert [g[0] for g in got[1:]] == ["splitk_reduce_kernel"] * (splits > 1)
+
+
+@dtypes
+@pytest.mark.parametrize("tile_cfg", [2, 15, 20])
+def test_a_pending_reduction_rides_whatever_tiling_is_asked_for(rec, dtype, tile_cfg):
+    rec.begin()
+    wgrad(rec, dtype, 2, 4, trailing=True)
+    wgrad(rec, dtype, tile_cfg, 4, trailing=True)
+    check(lib().tch_conv2d_wgrad_flush(rec.ctx))
+    first, second, last = rec.end()
+    assert last[0] == "splitk_reduce_kernel" and second[1] == first[1] + last[1]
