@@ -63,7 +63,9 @@ int tch_context_synchronize(tch_context* ctx); /* both streams of the context */
 int tch_program_create(tch_program** out);
 void tch_program_destroy(tch_program* prog);
 int64_t tch_program_size(const tch_program* prog);
-/* Between begin and end every operator call on ctx appends to prog instead of launching. */
+/* Between begin and end every operator call on ctx appends to prog instead of launching.  Sums that wait for a launch to
+ * ride (tch_conv2d_wgrad_trailing, tch_layernorm_defer_sums) do not cross either line: begin launches those of calls made
+ * before it, end appends those of the program to it, as tch_conv2d_wgrad_flush would, behind a join of the lanes. */
 int tch_program_begin_record(tch_context* ctx, tch_program* prog);
 int tch_program_end_record(tch_context* ctx);
 /* Replay launches [first, last) (last < 0: to the end).  The reject flag is a

@@ -102,6 +102,8 @@ int tch_program_begin_record(tch_context* ctx, tch_program* prog) {
     set_error("tch_program_begin_record: context is already recording");
     return -16;
   }
+  // sums left pending by launches that ran are due now, not at every replay of this program
+  if (int rc = conv2d_wgrad_flush(&ctx->ctx)) return rc;
   ctx->ctx.recording = &prog->prog;
   return 0;
 }
@@ -111,10 +113,19 @@ int tch_program_end_record(tch_context* ctx) {
     set_error("tch_program_end_record: context is not recording");
     return -22;
   }
-  ctx->ctx.recording = nullptr;
-  ctx->ctx.lane = 0;
-  ctx->ctx.wait_main = false;
-  return 0;
+  Context& c = ctx->ctx;
+  c.lane = 0;
+  c.wait_main = false;
+  // A sum that still waits for a launch to ride belongs to this program: left on the context it would ride into the next
+  // one, whose replays then read buffers that may be gone (a plan whose building failed half-way ends up here too).
+  int rc = 0;
+  if (c.trailing_reduce.valid || c.trailing_col_sum.valid) {
+    rc = c.record_join();   // the partials may be lane 1's
+    if (rc == 0) rc = conv2d_wgrad_flush(&c);
+    c.trailing_reduce.valid = c.trailing_col_sum.valid = false;
+  }
+  c.recording = nullptr;
+  return rc;
 }
 
 int tch_program_run(tch_context* ctx, const tch_program* prog, int64_t first, int64_t last) {

@@ -73,3 +73,31 @@ def test_layernorm_sums_that_ride_a_weight_gradient(ctx, dtype):
     assert torch.equal(dw, ref)
     for pair in got:
         assert torch.equal(pair[0], want[0]) and torch.equal(pair[1], want[1])
+
+
+def test_an_eager_reduction_does_not_enter_a_recording(ctx):
+    """A reduction that pends when a recording begins is launched then; the program holds its own alone."""
+    from sirius_amd import ops
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    rows, C, K = 2000, 72, 136
+    x, dy = (torch.randn(rows, 1, 1, n, device="cuda", generator=g).bfloat16() for n in (C, K))
+    sp = ops.conv2d_wgrad_splits(x, K, 1, 1, 1, 0)
+    assert sp > 1
+    half = ops.conv2d_wgrad_workspace_bytes(ops.dtype_code(x), K, 1, 1, C, sp) // 4
+    trail = ops.TrailingWgrad(ctx, torch.empty(2 * half, device="cuda"), half)
+    ref, eager, recorded = (torch.full((K, 1, 1, C), 7.0, device="cuda") for _ in range(3))
+    ops.conv2d_wgrad(ctx, x, dy, ref, 1, 0, workspace=torch.empty(half, device="cuda"), splits=sp)
+    trail.wgrad(x, dy, eager, 1, 0)
+    prog = ops.Program()
+    ctx.begin_record(prog)
+    trail.wgrad(x, dy, recorded, 1, 0)
+    ctx.end_record()
+    ctx.synchronize()
+    assert torch.equal(eager, ref) and (recorded == 7).all()
+    eager.fill_(7)
+    for _ in range(2):
+        recorded.fill_(7)
+        ctx.run(prog)
+        ctx.synchronize()
+        assert torch.equal(recorded, ref) and (eager == 7).all()

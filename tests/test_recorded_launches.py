@@ -87,3 +87,44 @@ def test_a_pending_reduction_rides_whatever_tiling_is_asked_for(rec, dtype, tile
     check(lib().tch_conv2d_wgrad_flush(rec.ctx))
     first, second, last = rec.end()
     assert last[0] == "splitk_reduce_kernel" and second[1] == first[1] + last[1]
+
+
+@dtypes
+def test_pending_sums_end_with_the_recording(rec, dtype):
+    """A recording that ends before its flush (a plan whose building raised) leaves nothing for the next one to take along:
+    the sums are the last launches of their own program, behind a join of the lanes."""
+    rec.begin()
+    wgrad(rec, dtype, 2, 4, trailing=True)
+    check(lib().tch_conv2d_wgrad_flush(rec.ctx))
+    clean = rec.end()
+
+    rec.begin()
+    check(lib().tch_layernorm_defer_sums(rec.ctx, 1))
+    check(lib().tch_layernorm_bwd(rec.ctx, dtype, *[address(i) for i in range(3)], None, *[address(i) for i in range(3, 8)],
+                                  0, ROWS, C, address(8)))
+    check(lib().tch_layernorm_defer_sums(rec.ctx, 0))
+    check(lib().tch_context_set_lane(rec.ctx, 1, 1))
+    wgrad(rec, dtype, 2, 4)                     # not one that takes sums along: the column sums stay pending ...
+    check(lib().tch_conv2d_wgrad_flush(rec.ctx))
+    wgrad(rec, dtype, 2, 4, trailing=True)      # ... until the flush; this reduction pends when the recording ends
+    cut = rec.end()
+    names = [c[0] for c in cut]
+    assert names[0].startswith("ln_bwd_kernel") and "col_sum_kernel" in names
+    assert names[-2:] == ["", "splitk_reduce_kernel"] and cut[-1][2] == 0
+
+    rec.begin()
+    wgrad(rec, dtype, 2, 4, trailing=True)
+    check(lib().tch_conv2d_wgrad_flush(rec.ctx))
+    assert rec.end() == clean
+
+
+def test_pending_column_sums_end_with_the_recording(rec):
+    rec.begin()
+    check(lib().tch_layernorm_defer_sums(rec.ctx, 1))
+    check(lib().tch_layernorm_bwd(rec.ctx, BF16, *[address(i) for i in range(3)], None, *[address(i) for i in range(3, 8)],
+                                  0, ROWS, C, address(8)))
+    check(lib().tch_layernorm_defer_sums(rec.ctx, 0))
+    assert [r[0] for r in rec.end()] == ["ln_bwd_kernel<bf16>", "", "col_sum_kernel"]
+    rec.begin()
+    check(lib().tch_conv2d_wgrad_flush(rec.ctx))
+    assert rec.end() == []
