@@ -148,8 +148,10 @@ int tch_context_get_cu_limit(tch_context* ctx);
 
 /* ---- convolution (implicit GEMM on MFMA) ---------------------------------------- */
 /* y[N,Ho,Wo,K] = conv(x[N,H,W,C], w[K,R,S,C]) (+ bias[K]) (+ add, optionally gated by mask > 0).
- * out_f32 != 0 stores y as fp32 whatever dtype is.  tile_cfg: -1 auto, -2 auto among the tilings
- * that add up a reduction front to back (a row's result does not depend on the number of rows), 0 = 128x128, 1 = 128x64, 2 = 64x64,
+ * out_f32 != 0 stores y as fp32 whatever dtype is.  tile_cfg: -1 auto: the choice, and with it the order a reduction is
+ * added up in, follows the number of rows, so a sample's result may differ in rounding with the samples batched beside it
+ * (bf16 ResNet-152 logits by about 2e-3).  -2 auto among the tilings that add up a reduction front to back (a row's result
+ * does not depend on the number of rows).  0 = 128x128, 1 = 128x64, 2 = 64x64,
  * 3 = 64x64 on the register-staged kernel even where the direct-to-LDS kernel applies, 5 = 128x64 with the
  * activation side of all nine taps of a channel block held in LDS as one patch (bf16, 3x3, stride 1, pad 1,
  * channels a multiple of 64, rows of at most 63 pixels; any other convolution runs tiling 1 for it).  The patch

@@ -52,7 +52,7 @@ class ResNetEngine(EngineBase):
                  lr=0.1, momentum=0.9, weight_decay=1e-4, bn_momentum=0.1, bn_eps=1e-5, stream=None, allocator=None,
                  overlap_wgrad=True, fuse_bn_stats=True, fuse_bn_bwd=True, fuse_bn_finalize=False, autotune=False,
                  retain_gradients=False, group_wgrad=False, wgrad_group_wgs=256, wgrad_group_blocks=2,
-                 wgrad_group_max_wgs=0, bn_acc=None, trailing_reduce=None):
+                 wgrad_group_max_wgs=0, bn_acc=None, trailing_reduce=None, eval_in_order=False):
         self._init_engine(dtype, stream, allocator)
         assert num_classes % 8 == 0, "class count must be a multiple of one 16-byte chunk"
         self.image_size, self.num_classes = image_size, num_classes
@@ -76,6 +76,12 @@ class ResNetEngine(EngineBase):
         # fuse_eval_bn: the forward-only (inference) plan runs convolution + BatchNorm (+ residual) (+ ReLU) as one
         # launch each instead of two
         self.fuse_eval_bn = True
+        # eval_in_order: every sum of the forward-only plan is taken front to back, so that an image's logits are the same
+        # bits whatever images are batched with it.  Off by default: the tilings that split a reduction over wavefronts,
+        # which few rows call for, are then left out, and they are what a small request gains from (ResNet-152, 1 / 4 / 16 /
+        # 24 / 64 images: 0.87 / 1.16 / 2.01 / 2.29 / 3.73 ms without, 1.24 / 1.46 / 2.04 / 2.29 / 3.89 with).  Without it bf16
+        # logits of one image differ by about 2e-3 between batch sizes; at one batch size they are the same bits every time.
+        self.eval_in_order = bool(eval_in_order)
         # compact_downsample_dgrad: the data gradient of a stride-2 downsample convolution stays on the small grid
         self.compact_downsample_dgrad = True
         self.group_wgrad = group_wgrad and overlap_wgrad
@@ -810,6 +816,8 @@ class ResNetEngine(EngineBase):
             keep.append(t)
             return t
 
+        order = ops.IN_ORDER if self.eval_in_order else -1
+
         def conv_bn(c, name, x, residual=None, relu=True):
             Ho, Wo = ops.conv_out_hw(x.shape[1], x.shape[2], c.k, c.k, c.stride, c.pad)
             y = act(B, Ho, Wo, c.cout)
@@ -818,10 +826,10 @@ class ResNetEngine(EngineBase):
             if self.fuse_eval_bn:
                 # the BatchNorm is a per-channel scale and shift here: applied to the accumulators in the epilogue
                 ops.conv2d_fwd_affine(ctx, x, self._w(c.name + ".weight"), y, c.stride, c.pad, scale=coef[:ch], shift=coef[ch:],
-                                      residual=residual, relu=relu, c_logical=c.cin)
+                                      residual=residual, relu=relu, c_logical=c.cin, tile_cfg=order)
                 return y
             z = act(B, Ho, Wo, c.cout)
-            ops.conv2d_fwd(ctx, x, self._w(c.name + ".weight"), z, c.stride, c.pad, c_logical=c.cin)
+            ops.conv2d_fwd(ctx, x, self._w(c.name + ".weight"), z, c.stride, c.pad, c_logical=c.cin, tile_cfg=order)
             ops.bn_apply_fwd(ctx, z, y, coef, residual=residual, relu=relu)
             return y
 
@@ -846,7 +854,8 @@ class ResNetEngine(EngineBase):
             ops.avgpool_fwd(ctx, x, pooled)
             plan.logits = act(B, self.num_classes, dtype=torch.float32)
             ops.conv2d_fwd(ctx, pooled.view(B, 1, 1, self.feat), self._w("fc.weight"),
-                           plan.logits.view(B, 1, 1, self.num_classes), 1, 0, bias=self._view(self.params, "fc.bias"))
+                           plan.logits.view(B, 1, 1, self.num_classes), 1, 0, bias=self._view(self.params, "fc.bias"),
+                           tile_cfg=order)
         finally:
             ctx.end_record()
         plan.prog, plan.keep, plan.batch = prog, keep, B
@@ -863,7 +872,8 @@ class ResNetEngine(EngineBase):
 
     def forward_eval(self, x):
         """x [B,3,S,S] fp32 on the GPU -> the plan whose `logits` [B, classes] (fp32) the launches fill.  The
-        caller synchronises (ctx.synchronize()) before reading them."""
+        caller synchronises (ctx.synchronize()) before reading them.  An image's logits may differ in rounding between
+        batch sizes (eval_in_order: never)."""
         p = self.eval_plan(x.shape[0])
         p.x_in.copy_(x, non_blocking=True)
         self.ctx.run(p.prog)

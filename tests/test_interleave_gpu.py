@@ -48,6 +48,23 @@ def _calibrated_model(depths, classes, width, image, seed, residual_gain=0.1):
     return model.eval()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("fused", [True, False])
+def test_logits_of_an_image_do_not_depend_on_its_batch_with_eval_in_order(dtype, fused):
+    """eval_in_order: the same bits for an image alone and beside 2 to 39 others (one tile of rows to many)."""
+    from sirius_amd.resnet import ResNetEngine
+    eng = ResNetEngine((1, 2, 2, 1), 64, 64, dtype=dtype, image_size=96, eval_in_order=True)
+    eng.init_kaiming(0)
+    eng.fuse_eval_bn = fused
+    x = torch.randn(40, 3, 96, 96, device="cuda", generator=torch.Generator(device="cuda").manual_seed(9))
+    got = {}
+    for b in (40, 1, 3, 17):
+        p = eng.forward_eval(x[:b].contiguous())
+        eng.ctx.synchronize()
+        got[b] = p.logits.clone()
+        assert torch.isfinite(got[b]).all() and torch.equal(got[b], got[40][:b]), b
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-3), (torch.bfloat16, 2e-2)])
 @pytest.mark.parametrize("batch", [1, 4])
 def test_resnet152_eval_forward_against_the_oracle(dtype, tol, batch):
