@@ -12,15 +12,15 @@ from . import _C
 # (base MB, slope MB / sample), shared-tensor mode (train_adjuster.cc:647-698)
 MODEL_MEM_PARAM = {"resnet152": (1150, 85), "swin_b": (1700, 145), "swin_b_ddp": (2560, 140),
                    "gpt2": (2700, 490), "qwen": (9000, 600)}
-# This engine on MI355X, bf16 compute with fp32 master state, from pool readings (bytes held by torch before any
-# plan exists, and the bytes of the plans at three batch sizes; the plan grows linearly, its intercept is < 30 MB):
-#   resnet152  state 920 MB (+ 241 MB of accumulated gradients in colocate mode), plans 1109 / 2190 / 8673 MB at
-#              batch 8 / 16 / 64
-#   swin_b     state 1675 MB (+ 351 MB), plans 544 / 1083 / 4200 MB at batch 4 / 8 / 32
-#   gpt2       state 2375 MB (+ 498 MB); 256-token rows as train/gpt2.py:45 builds them: plans 1306 / 2585 / 10258 MB
-#              at batch 8 / 16 / 64 (1024-token rows: 640 MB per row)
-# base = state + accumulated gradients + the plan's intercept, slope = plan bytes per sample.
-MODEL_MEM_PARAM_MI355X = {"resnet152": (1190, 136), "swin_b": (2050, 131), "gpt2": (2900, 160)}
+# This engine on MI355X, bf16 compute with fp32 master state, in MB of 2^20 bytes: what the engine holds before any plan
+# exists, and the plans at several batch sizes (they grow linearly, with an intercept below 30 MB):
+#   resnet152  state 920 (+ 230 of accumulated gradients in colocate mode), plans 1091 / 2178 / 8706 at batch 8 / 16 / 64
+#   swin_b     state 1675 (+ 335), plans 597 / 1178 / 4610 at batch 4 / 8 / 32
+#   gpt2       state 2375 (+ 475); 256-token rows as train/gpt2.py:45 builds them: plans 1296 / 2628 / 10315 at batch
+#              8 / 16 / 64 (1024-token rows: 648 per row)
+# base = state + accumulated gradients + the plan's intercept, slope = plan bytes per sample, both rounded up.
+# tests/test_colocate_gpu.py holds the engines to these figures.
+MODEL_MEM_PARAM_MI355X = {"resnet152": (1190, 136), "swin_b": (2050, 144), "gpt2": (2900, 162)}
 
 
 class TrainAdjuster:

@@ -572,3 +572,24 @@ def test_handover_64_16_64_on_the_real_resnet152(clean_runtime, monkeypatch, tmp
     assert stat.killed_batch >= 1
     assert all(torch.isfinite(v).all() for v in out["model"].state_dict().values())
     assert tc.GetXQueueSizeAllStreams() == 0
+
+
+@pytest.mark.parametrize("model,batches", [("resnet152", (16, 64)), ("swin_b", (8, 32)), ("gpt2", (8, 64))])
+def test_engines_hold_the_memory_the_peer_reckons_with(model, batches):
+    """MODEL_MEM_PARAM_MI355X: what the peer predicts for a batch size is what the engine holds, or up to 4 % more (the
+    slope and the base are rounded up), never less: a peer that reckons with less finds training in its memory."""
+    import gc
+    from sirius_amd.gpt2 import GPT2Engine
+    from sirius_amd.resnet import ResNetEngine
+    from sirius_amd.swin import SwinEngine
+    from sirius_amd.torch_col.train_adjuster import MODEL_MEM_PARAM_MI355X, TrainAdjuster
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    eng = {"resnet152": ResNetEngine, "swin_b": SwinEngine, "gpt2": lambda: GPT2Engine(seq_len=256)}[model]()
+    eng.ensure_global_grads()
+    state = torch.cuda.memory_allocated() - before
+    adjuster = TrainAdjuster(model, MODEL_MEM_PARAM_MI355X)
+    for batch in batches:
+        held = (state + eng.plan(batch).bytes) / 2 ** 20
+        eng.release_activations()
+        assert held <= adjuster.predict_train_mem_usage_mb(batch) <= 1.04 * held, (batch, held)
