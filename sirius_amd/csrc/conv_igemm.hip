@@ -2240,6 +2240,15 @@ int igemm2_setting() {
   return v;
 }
 
+// TCH_IGEMM_K32 = 0: the library's own choice leaves out the tilings with 32-element reduction steps
+bool short_steps() {
+  static const bool on = [] {
+    const char* e = getenv("TCH_IGEMM_K32");
+    return !(e && atoi(e) == 0);
+  }();
+  return on;
+}
+
 // Tilings of igemm4_kernel (tile, wavefronts the reduction is dealt to, LDS tiles in flight of each).  LDS decides how
 // many workgroups share a CU: one (kSplit32Deep, kSplit64, kSplit64x32Deep) or two (the others).
 enum SplitTile : int {
@@ -2515,6 +2524,7 @@ int heuristic_tile(int asked, const TileQuery& q) {
     // one and a half 128 x 128 tiles per compute unit or more, beside a second lane of weight gradients: smaller tiles
     // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 8 x 1024 12.05 -> 11.76 ms)
     if (!q.sums && large && t.bm * t.bn < 128 * 128) continue;
+    if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
     const float r = static_cast<float>((tiles_for(q.gemm_m, q.gemm_n, t.bm, t.bn) + 255) / 256);
@@ -2725,8 +2735,13 @@ int64_t conv2d_wgrad_workspace_bytes(const ConvShape& s, int dtype, int splits) 
 }
 
 // tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups
+// (TCH_WGRAD_BIG_TILE_WGS: another count)
 bool wgrad_big_tile(int gemm_m, int gemm_n, int64_t splits) {
-  return gemm_m >= 128 && gemm_n >= 128 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= 128;
+  static const int from = [] {
+    const char* e = getenv("TCH_WGRAD_BIG_TILE_WGS");
+    return e && atoi(e) > 0 ? atoi(e) : 128;
+  }();
+  return gemm_m >= 128 && gemm_n >= 128 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= from;
 }
 
 int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
@@ -2735,6 +2750,19 @@ int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
   conv_output_hw(s, &Ho, &Wo);
   const int64_t pixels = static_cast<int64_t>(s.N) * Ho * Wo;
   const int gemm_m = s.K, gemm_n = s.R * s.S * s.C;
+  int64_t most = pixels / (4 * BK);   // at least four reduction steps per split
+  if (most > 512) most = 512;
+  if (most < 1) most = 1;
+  // TCH_WGRAD_WGS: a workgroup count to aim for instead
+  static const int aim = [] {
+    const char* e = getenv("TCH_WGRAD_WGS");
+    return e && atoi(e) > 0 ? atoi(e) : 0;
+  }();
+  if (aim) {
+    int64_t tiles = tiles_for(gemm_m, gemm_n, 128, 128);
+    if (tiles < 8) tiles = tiles_for(gemm_m, gemm_n, 64, 64);
+    return static_cast<int>(std::min((aim + tiles - 1) / tiles, most));
+  }
   // The split count with the shortest start + steps * max(alone, shared * r) + store * (10^6 results written), r =
   // workgroups per compute unit, rounded up: least-squares fits (6-8 % mean error) to 1 500 launches of every split count
   // on the layers of the three models at 128-8192 rows and 1-64 images, per dtype for 128 x 128 and 64 x 64 tiles.  A
@@ -2748,11 +2776,9 @@ int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
   static const Cost cost[2][2] = {{{3.39f, 0.229f, 0.383f, 1.55f}, {8.56f, 0.371f, 0.912f, 0.71f}},     // fp32: 64, 128
                                   {{3.08f, 0.109f, 0.089f, 2.33f}, {6.37f, 0.249f, 0.179f, 0.94f}}};   // bf16
   constexpr float kReread = 1.f;   // microseconds per 10^6 results; 0 - 2 in the steps: within 1 %, 1 the best of most
-  int64_t most = pixels / (4 * BK);   // at least four reduction steps per split
-  if (most > 512) most = 512;
   int best = 1;
   float best_us = INFINITY;
-  for (int64_t want = 1; want <= most || want == 1; ++want) {
+  for (int64_t want = 1; want <= most; ++want) {
     const int64_t steps = ((pixels + want - 1) / want + BK - 1) / BK;
     const int64_t splits = (pixels + steps * BK - 1) / (steps * BK);
     if (splits != want) continue;   // the same as a smaller count

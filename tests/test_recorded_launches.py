@@ -1,6 +1,9 @@
 """What a recorded program holds (tch_program_launches): which kernel a call is sent to, on the CPU.  Nothing runs: the
 addresses are made up."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -128,3 +131,33 @@ def test_pending_column_sums_end_with_the_recording(rec):
     rec.begin()
     check(lib().tch_conv2d_wgrad_flush(rec.ctx))
     assert rec.end() == []
+
+
+def choice(**env):
+    """In a process of its own (the settings are read once): splits and kernel of a weight gradient of 128 x 128 tiles, and
+    the kernel of a shallow pointwise product."""
+    code = """if True:
+        import sys
+        sys.path[:0] = [%r, %r]
+        import test_recorded_launches as T
+        rec = T.Recorder()
+        sp = T.lib().tch_conv2d_wgrad_pick_splits(1, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0)
+        rec.begin()
+        a = T.address
+        T.check(T.lib().tch_conv2d_wgrad(rec.ctx, 1, a(0), a(1), a(2), a(3), sp, 0, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0, -1, 0))
+        T.check(T.lib().tch_conv2d_fwd(rec.ctx, 1, a(0), a(1), a(2), None, None, None, 0, 200704, 1, 1, 64, 256, 1, 1, 1, 0, -1, 0))
+        names = [r[0] for r in rec.end()]
+        print(sp, names[0], names[-1], sep="|")
+    """ % (os.path.dirname(os.path.abspath(__file__)), os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, **env), stdout=subprocess.PIPE, check=True)
+    sp, wgrad_name, fwd_name = out.stdout.decode().split()[-1].split("|")
+    return int(sp), wgrad_name, fwd_name
+
+
+def test_settings_of_the_library_s_own_choice():
+    """TCH_WGRAD_WGS, TCH_WGRAD_BIG_TILE_WGS and TCH_IGEMM_K32 override what the tables of costs say."""
+    splits, wgrad_name, fwd_name = choice()
+    assert wgrad_name == "wgrad_kernel<bf16,128x128>" and ",k32" in fwd_name
+    assert choice(TCH_WGRAD_WGS="64")[0] == 1 and choice(TCH_WGRAD_WGS="1024")[0] == 16 and 1 < splits < 16
+    assert choice(TCH_WGRAD_BIG_TILE_WGS="100000")[1] == "wgrad_kernel<bf16,64x64>"
+    assert ",k32" not in choice(TCH_IGEMM_K32="0")[2]
