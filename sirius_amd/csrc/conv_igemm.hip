@@ -2230,8 +2230,8 @@ int launch_cfg3(Context* ctx, IgemmArgs& a, double flops) {
   return launch_cfg3_rows<MODE, TN, NBUF, 8>(ctx, a, flops);
 }
 
-// TCH_IGEMM2 = 0 keeps every convolution on igemm_kernel; 2 or 3 picks the number of LDS tiles
-// in flight of igemm2_kernel (default: 2 for 128x128, 3 for 128x64)
+// TCH_IGEMM2 = 0 keeps every convolution on igemm_kernel, whatever tiling is asked for; 2 or 3 picks the number of
+// LDS tiles of tilings 0 - 2 (default: 2 for 128x128, 3 for 128x64 and 64x64)
 int igemm2_setting() {
   static const int v = [] {
     const char* e = getenv("TCH_IGEMM2");
@@ -2423,7 +2423,9 @@ bool wants_huge_tile(int dtype, int gemm_m, int gemm_n, int in_c, int taps) {
 }
 
 // igemm4_kernel: whole 64-byte steps of input channels, one bit per tap
-bool split_tile_fits(int dtype, int in_c, int taps) { return in_c % (dtype == kBF16 ? 32 : 16) == 0 && taps <= 32; }
+bool split_tile_fits(int dtype, int in_c, int taps) {
+  return in_c % (dtype == kBF16 ? 32 : 16) == 0 && taps <= 32 && igemm2_setting() != 0;
+}
 
 // igemm2_kernel: whole 128-byte steps of bf16 input channels, one bit per tap
 bool direct_tile_fits(int dtype, int in_c, int taps) {
@@ -2490,7 +2492,7 @@ const TileCost kSumsCost[] = {
 // -1: none of them.
 // (bf16 with channels that are no whole 64-element step: the two smallest forms only.)
 int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
-  if (igemm2_setting() == 0 || !split_tile_fits(dtype, in_c, taps)) return -1;
+  if (!split_tile_fits(dtype, in_c, taps)) return -1;
   const int64_t t32 = tiles_for(gemm_m, gemm_n, 32, 32), t64 = tiles_for(gemm_m, gemm_n, 64, 64);
   if (t32 <= 256) return gemm_k >= 1024 ? kSplit32Deep : kSplit32;
   if (dtype == kBF16) return t32 <= 512 ? kSplit32 : -1;

@@ -133,24 +133,24 @@ def test_pending_column_sums_end_with_the_recording(rec):
     assert rec.end() == []
 
 
+def in_own_process(body, **env):
+    """What `body` prints, with the settings of `env` (they are read once per process)."""
+    head = "import sys\nsys.path[:0] = [%r, %r]\nimport test_recorded_launches as T\nrec, a = T.Recorder(), T.address\n" % (
+        os.path.dirname(os.path.abspath(__file__)), os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    out = subprocess.run([sys.executable, "-c", head + body], env=dict(os.environ, **env), stdout=subprocess.PIPE, check=True)
+    return out.stdout.decode().split("|")
+
+
 def choice(**env):
-    """In a process of its own (the settings are read once): splits and kernel of a weight gradient of 128 x 128 tiles, and
-    the kernel of a shallow pointwise product."""
-    code = """if True:
-        import sys
-        sys.path[:0] = [%r, %r]
-        import test_recorded_launches as T
-        rec = T.Recorder()
-        sp = T.lib().tch_conv2d_wgrad_pick_splits(1, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0)
-        rec.begin()
-        a = T.address
-        T.check(T.lib().tch_conv2d_wgrad(rec.ctx, 1, a(0), a(1), a(2), a(3), sp, 0, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0, -1, 0))
-        T.check(T.lib().tch_conv2d_fwd(rec.ctx, 1, a(0), a(1), a(2), None, None, None, 0, 200704, 1, 1, 64, 256, 1, 1, 1, 0, -1, 0))
-        names = [r[0] for r in rec.end()]
-        print(sp, names[0], names[-1], sep="|")
-    """ % (os.path.dirname(os.path.abspath(__file__)), os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, **env), stdout=subprocess.PIPE, check=True)
-    sp, wgrad_name, fwd_name = out.stdout.decode().split()[-1].split("|")
+    """Splits and kernel of a weight gradient, and the kernel of a shallow pointwise product."""
+    sp, wgrad_name, fwd_name = in_own_process("""
+sp = T.lib().tch_conv2d_wgrad_pick_splits(1, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0)
+rec.begin()
+T.check(T.lib().tch_conv2d_wgrad(rec.ctx, 1, a(0), a(1), a(2), a(3), sp, 0, 8192, 1, 1, 1024, 1024, 1, 1, 1, 0, -1, 0))
+T.check(T.lib().tch_conv2d_fwd(rec.ctx, 1, a(0), a(1), a(2), None, None, None, 0, 200704, 1, 1, 64, 256, 1, 1, 1, 0, -1, 0))
+names = [r[0] for r in rec.end()]
+print(sp, names[0], names[-1], sep="|", end="")
+""", **env)
     return int(sp), wgrad_name, fwd_name
 
 
@@ -161,3 +161,29 @@ def test_settings_of_the_library_s_own_choice():
     assert choice(TCH_WGRAD_WGS="64")[0] == 1 and choice(TCH_WGRAD_WGS="1024")[0] == 16 and 1 < splits < 16
     assert choice(TCH_WGRAD_BIG_TILE_WGS="100000")[1] == "wgrad_kernel<bf16,64x64>"
     assert ",k32" not in choice(TCH_IGEMM_K32="0")[2]
+
+
+@dtypes
+@pytest.mark.parametrize("setting", ["", "0", "2", "3"])
+def test_row_tiles_of_the_statistics_are_those_of_the_kernel(dtype, setting):
+    """Callers size the BatchNorm sums by tch_conv2d_fwd_stat_rows / tch_conv2d_dgrad_stat_rows: the kernel that runs has that
+    many row tiles, for every tiling and setting of TCH_IGEMM2.  0: igemm_kernel whatever tiling is asked for."""
+    got = in_own_process("""
+dtype, staged, L = %d, %r, T.lib()
+for cfg in [-2, -1] + list(range(23)):
+    for shape in ((2, 14, 14, 128, 256, 3, 3, 1, 1), (1, 56, 56, 64, 128, 1, 1, 2, 0), (3, 9, 7, 24, 40, 3, 3, 1, 1),
+                  (64, 56, 56, 256, 64, 1, 1, 1, 0), (1, 7, 7, 32, 512, 1, 1, 1, 0)):
+        rec.begin()
+        T.check(L.tch_conv2d_fwd_bnstats(rec.ctx, dtype, a(0), a(1), a(2), *shape, cfg, 0, a(3)))
+        T.check(L.tch_conv2d_dgrad_bnsums(rec.ctx, dtype, a(0), a(1), a(2), None, None, *shape, cfg, 0, a(3), a(4), a(5), a(6),
+                                          a(7), 1))
+        rows = (L.tch_conv2d_fwd_stat_rows(dtype, *shape, cfg), L.tch_conv2d_dgrad_stat_rows(dtype, *shape, cfg))
+        n, h, w, c, k, r, s, stride, pad = shape
+        out = (h + 2 * pad - r) // stride + 1, (w + 2 * pad - r) // stride + 1
+        for (name, wgs, _), row_tiles, m, cols in zip(rec.end(), rows, (n * out[0] * out[1], n * h * w), (k, c)):
+            bm, bn = map(int, name.split(",")[2].rstrip(">").split("x"))
+            assert row_tiles == -(-m // bm) and wgs == row_tiles * -(-cols // bn), (cfg, name)
+            assert not staged or name.startswith("igemm_kernel<"), (cfg, name)
+print("ok", end="")
+""" % (dtype, setting == "0"), **({"TCH_IGEMM2": setting} if setting else {}))
+    assert got == ["ok"]
