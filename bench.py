@@ -22,30 +22,20 @@ sys.path.insert(0, ROOT)
 PEAK_BF16_FLOPS = 2.5e15   # MI355X dense bf16 MFMA
 PEAK_HBM_BYTES = 8.0e12    # MI355X HBM3E
 METRIC = "ResNet-152 bf16 bs64 train images/sec on 1 GPU; conv MFMA util %"
-# HBM bytes per launch of the kernels that can top the step, from two rocprofv3 --pmc runs of this file
-# (FETCH_SIZE and WRITE_SIZE, KiB per dispatch, scaled by what the same counters read for the --calibrate
-# copy of known size: factors 2.000 and 1.000); the summary is profiles/resnet152_bf16_bs64_step_kernel_stats_and_traffic.txt
 # The handover measurement: a pool of nearly the whole part in 128 MB pages (the reference's 32 MB page costs one
 # driver call per page on the way out: 9 GB take 68 ms there, 18 ms in 128 MB pages).
 HANDOVER_POOL_GB = 256
 HANDOVER_PAGE_MB = 128
 # The rocprofv3 summaries of this file's default run: kernel trace (average durations inside the step) and the
-# FETCH_SIZE / WRITE_SIZE counter runs the traffic figures below are taken from.
+# FETCH_SIZE / WRITE_SIZE counter runs the traffic figures below are taken from (KiB per dispatch, scaled by what the same
+# counters read for the --calibrate copy of known size: factors 2.000 and 1.000).  HBM MiB per launch of the kernels whose launches
+# do not depend on the tiling tuner; another kernel at the top of the step has no figure.
 PROFILE_FILE = "profiles/resnet152_bf16_bs64_step_kernel_stats_and_traffic.txt"
 MEASURED_TRAFFIC_MIB = {
-    "wgrad_kernel<bf16,128x128>": 44.18 + 15.41,
-    "wgrad_kernel<bf16,64x64>": 93.22 + 6.32,
-    "igemm2_kernel<bf16,dgrad,128x64,3buf,k32>": 73.34 + 33.50,
-    "igemm2_kernel<bf16,dgrad,128x128,2buf>": 63.51 + 30.53,
-    "igemm2_kernel<bf16,dgrad,128x128,3buf,k32>": 66.89 + 35.55,
-    "igemm2_kernel<bf16,dgrad,128x128,2buf,k32>": 89.75 + 34.04,
-    "igemm2_kernel<bf16,dgrad,128x64,3buf>": 70.39 + 31.94,
-    "igemm2_kernel<bf16,fwd,128x128,2buf>": 28.05 + 15.45,
-    "igemm2_kernel<bf16,fwd,128x128,2buf,k32>": 32.77 + 29.51,
-    "igemm2_kernel<bf16,fwd,128x64,3buf>": 37.96 + 16.22,
-    "igemm3_kernel<bf16,dgrad,128x64,3buf,patch160>": 29.50 + 5.99,
-    "bn_fin_apply_kernel<bf16,bwd>": 24.39 + 11.91,
-    "bn_fin_apply_kernel<bf16,fwd>": 20.39 + 12.03,
+    "wgrad_kernel<bf16,64x64>": 64.44 + 5.60,
+    "wgrad_kernel<bf16,128x128>": 34.36 + 17.23,
+    "bn_fin_apply_kernel<bf16,bwd>": 24.40 + 11.91,
+    "bn_fin_apply_kernel<bf16,fwd>": 20.40 + 12.03,
 }
 
 
@@ -72,7 +62,7 @@ def grouped_wgrad_step(batch, x, y, steps, warmup, tile_cache):
     plan = eng.plan(batch)
     rows = eng.ctx.profile(plan.prog, 1) + eng.ctx.profile(eng._opt_prog, 1)
     wg = [r for r in rows if r["name"].startswith(("wgrad_", "splitk_reduce"))]
-    conv = [r for r in rows if r["name"].startswith(("igemm_kernel", "igemm2_kernel", "igemm3_kernel", "wgrad_"))]
+    conv = [r for r in rows if r["name"].startswith(("igemm", "wgrad_"))]
     grp = [r for r in rows if r["name"].startswith("wgrad_group_kernel<bf16,128x128>")]
     res = {"ms_per_step": ms, "images_per_s": batch / (ms * 1e-3), "launches_per_step": len(plan.prog) + len(eng._opt_prog),
            "wgrad_and_reduce_kernel_ms": sum(r["total_ms"] for r in wg),
@@ -463,7 +453,7 @@ def main():
     rows = eng.ctx.profile(plan.prog, reps) + eng.ctx.profile(eng._opt_prog, reps)
     rows.sort(key=lambda r: -r["total_ms"])
     total_ms = sum(r["total_ms"] for r in rows) / reps
-    conv = [r for r in rows if r["name"].startswith(("igemm_kernel", "igemm2_kernel", "igemm3_kernel", "wgrad_kernel"))]
+    conv = [r for r in rows if r["name"].startswith(("igemm", "wgrad_"))]
     conv_ms = sum(r["total_ms"] for r in conv) / reps
     conv_flops = sum(r["work"] for r in conv) / reps
     top = rows[0]

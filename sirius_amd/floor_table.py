@@ -20,7 +20,7 @@ PEAK_BYTES = 8.0e12
 
 def family(name):
     """Kernel family of a launch: what the kernel does, without its tiling."""
-    if name.startswith(("igemm2_kernel", "igemm3_kernel", "igemm_kernel")):
+    if name.startswith("igemm"):
         return "conv data gradient" if ",dgrad" in name else "conv forward"
     if name.startswith("wgrad"):
         return "conv weight gradient"

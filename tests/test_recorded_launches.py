@@ -187,3 +187,16 @@ for cfg in [-2, -1] + list(range(23)):
 print("ok", end="")
 """ % (dtype, setting == "0"), **({"TCH_IGEMM2": setting} if setting else {}))
     assert got == ["ok"]
+
+
+@dtypes
+@pytest.mark.parametrize("tile_cfg", range(23))
+def test_floor_table_files_every_convolution_kernel_under_its_direction(rec, dtype, tile_cfg):
+    from sirius_amd.floor_table import family
+    rec.begin()
+    check(lib().tch_conv2d_fwd(rec.ctx, dtype, address(0), address(1), address(2), None, None, None, 0, 2, 14, 14, 128, 128, 3, 3, 1, 1,
+                               tile_cfg, 0))
+    check(lib().tch_conv2d_dgrad(rec.ctx, dtype, address(0), address(1), address(2), None, None, 2, 14, 14, 128, 128, 3, 3, 1, 1,
+                                 tile_cfg, 0, 1))
+    wgrad(rec, dtype, tile_cfg, 1)
+    assert [family(r[0]) for r in rec.end()] == ["conv forward", "conv data gradient", "conv weight gradient"]
