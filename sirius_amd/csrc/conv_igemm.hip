@@ -15,7 +15,11 @@
 //   DGRAD  (N*H*W)   x C,        over R*S*K     (filter pre-transposed to [C][R][S][K])
 //   WGRAD  K         x (R*S*C),  over N*Ho*Wo, split across workgroups
 //
-// FWD / DGRAD: a tile row in LDS holds one GEMM row (or column) and BK reduction
+// Kernels: igemm2_kernel (bf16 forward / data gradient, direct-to-LDS), igemm3_kernel (3x3 layers with the activation
+// patch in LDS), igemm4_kernel (few output tiles, and fp32: the reduction dealt to the wavefronts of a workgroup),
+// igemm_kernel (what those do not take), wgrad_kernel (bf16) / wgrad_f32_kernel.
+//
+// FWD / DGRAD in igemm_kernel: a tile row in LDS holds one GEMM row (or column) and BK reduction
 // elements = 4 chunks of 16 bytes (+1 chunk of padding); a lane's MFMA operand is
 // one chunk (lanes 0-31 chunk 2j, lanes 32-63 chunk 2j+1 of their row).
 //
@@ -47,7 +51,7 @@ namespace tch {
 namespace {
 
 constexpr int kLdsStride = 5;  // FWD/DGRAD: chunks per LDS tile row: 4 data + 1 pad
-constexpr int kRowPad = 4;     // WGRAD: chunks of padding per [pixel] row (64 bytes)
+constexpr int kRowPad = 4;     // WGRAD, fp32: chunks of padding per [pixel] row (64 bytes)
 constexpr int kStagePad = 4;   // epilogue staging: floats of padding per row
 
 enum Mode : int { kFwd = 0, kDgrad = 1, kWgrad = 2 };
@@ -1254,7 +1258,10 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
 //     operand read touches every bank once;
 //   * a step never straddles a filter tap (channels % 64 == 0), so the tap walk is scalar:
 //     a lane keeps one byte offset and one validity bit per tap for each row it loads;
-//   * NBUF tiles in flight, one barrier per step;
+//   * NBUF tiles in LDS, one barrier per step: one is multiplied, one is being requested, and NBUF - 2 are in flight
+//     across the barrier (none with two, where the other workgroups of the CU fill the trip to memory: 8192 x 768 over
+//     3072 takes 45.2 us as 128 x 128 with two 64-element tiles, 61 with three, 51.5 with three of 32; 8192 x 2304
+//     over 768 44.8, 53.5 and 43.2);
 //   * ROT = 2 reads the operands of the next step into a second register set while this step is multiplied: the barrier
 //     hands over a tile one step before it is needed and the LDS latency passes behind the multiplies.  What bounds
 //     the small tiles then is LDS itself (a 64 x 64 tile: 32 KB read, 16 KB written per step).  1024 x 768 over 3072:
@@ -1583,9 +1590,12 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
-// forward / data gradient where the grid of output tiles cannot fill the chip (and fp32 at every size): the
-// reduction is dealt out to the KG wavefronts of a workgroup
+// forward / data gradient where the grid of output tiles cannot fill the chip (fp32: where it has fewer than one and a
+// half 128 x 128 tiles per compute unit): the reduction is dealt out to the KG wavefronts of a workgroup
 // ---------------------------------------------------------------------------
+// What bounds it: the trip to memory behind every launch boundary and the chain of steps behind it.  196 x 256 over 2304 (a
+// 3x3 layer of one image) 13.2 -> 6.1 us, 784 x 512 over 4608 36.9 -> 14.8, fp32 784 x 256 over 2304 77.6 -> 14.8 against
+// 64 x 64 tiles of igemm2_kernel / igemm_kernel; the 151 launches of a ResNet-152 request take 4.4-6.9 us each.
 // Every wavefront owns the WHOLE TM*32 x TN*32 tile for every KG-th reduction step and has a ring of NBUF operand
 // tiles of its own in LDS, filled with direct loads: nothing is shared before the end, so the main loop has no
 // barrier and a wavefront waits for its own loads only.  The partial tiles meet in LDS once and are added in the
@@ -2328,15 +2338,12 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
     const int in_c = MODE == kFwd ? a.C : a.K;
     const int setting = igemm2_setting();
     if (tile_cfg == 5) {   // 128 x 64 with the 3x3 patch in LDS; convolutions it does not fit run as tiling 1
-      // (measured and not built: a 128 x 128 tile with two or three filter tiles in flight and four filter
-      // tiles for this one were 4-30 % slower on every 3x3 layer of ResNet-152 at batch 64)
       if (setting != 0 && patch_kernel_fits<MODE>(a)) return launch_cfg3<MODE, 1, 3>(ctx, a, flops);
       tile_cfg = 1;
     }
-    // 9 / 10: 256 x 256 on eight wavefronts (128 x 64 each), two LDS tiles in flight, plain / rotated loop: for
-    // products with a thousand such tiles or more (measured on 65 536 x 4096 x 4096: 1.13-1.21 PFLOP/s rotated,
-    // 1.02 plain, 0.82-0.91 for 128 x 128; four wavefronts of 128 x 128 each: 0.99-1.05, and slower than 128 x 128
-    // on every layer of the three models, like this one)
+    // 9 / 10: 256 x 256 on eight wavefronts (128 x 64 each), two LDS tiles, plain / rotated loop: for products with a
+    // thousand such tiles or more (65 536 x 4096 x 4096: 1.22 PFLOP/s both, 1.04 for 128 x 128; 8192 x 3072 over 768: 50 us
+    // rotated, 53 plain, 52 for 128 x 128; slower than 128 x 128 on the other layers of the three models, by up to 1.7x)
     if (tile_cfg == 9 || tile_cfg == 10) {
       if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32)
         return tile_cfg == 9 ? launch_cfg2<MODE, 2, 4, 4, 2, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 4, 4, 2, 2, 1>(ctx, a, flops);
@@ -2461,8 +2468,12 @@ int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
 // kernel times of 280 products and convolutions: the projections of GPT-2 at 128-8192 rows and of Swin-B at 2-32
 // images forward, ResNet's 1x1 and 3x3 layers at 1-64 images (forward with batch sums, inference epilogue) for the
 // first table; ResNet's data gradients with the BatchNorm sums, whose epilogue reads two more tensors, for the second.
-// Choosing by them is within 2 % of always taking the fastest tiling; the tile-count thresholds they replace were
-// 8 % off at the sizes they were tuned on, up to 1.9x between.
+// Against the fastest of ALL tilings, each timed alone on 488 such launches: the choice is 2 % slower on average on the
+// projections, forward (worst 1.18) and data gradient (1.19), 2 % on ResNet's data gradients with the sums (1.17), and 5-6 %
+// on its forward convolutions.  Those are worst where the output has 64 channels (stage 1 at 16-64 images: 1.2-1.45, 56 x 56
+// x 256 -> 64 at 20 images 12.3 us as 128 x 128 and 8.5 as 64 x 64): the columns a tile has beyond the output are not priced.
+// Tilings without an entry (3, 6, 7, 11, kSplit64, kSplit64Pair, kSplit64x32Deep: for callers that ask, and for tuners) are
+// the fastest on some launches, by 1 % on average and 9 % at most.
 struct TileCost {
   int cfg, bm, bn;
   float start, round, alone, shared, store;
@@ -2486,18 +2497,24 @@ const TileCost kSumsCost[] = {
     {kSplit32Deep, 32, 32, 4.20f, 0.38f, 0.062f, 0.082f, 5.42f},
     {kSplit64x32, 64, 32, 4.16f, 0.44f, 0.168f, 0.134f, 2.81f}};
 
-// fp32 where the output has too few tiles to fill the chip, and on large grids too: the reduction is split inside the
+// fp32 where the output has fewer than one and a half 128 x 128 tiles per compute unit: the reduction is split inside the
 // workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 multiplies at 1/16 of the bf16 rate, so it
-// gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us; 2048 x 3072 over 768: 100 -> 86).
-// -1: none of them.
+// gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us).  -1: none of them.
+// The lines, with mean times over the layers of the three models in each class (244 launches), the choice = 1:
+//   up to one 32 x 32 tile per CU, K >= 1024 (53): eight wavefronts; four 1.11.  K < 1024 (25): four; eight 1.01
+//   up to two, K < 1536 (38): 32 x 32 on four; eight 1.05, 64 x 32 1.05.  Two such tiles on a CU hide each other's
+//     latencies until the reduction is long enough to do so alone: K >= 1536 (9) 64 x 32 on eight; 32 x 32 on eight 1.02, four 1.05
+//   up to one 64 x 64 tile per CU, K >= 768 (19): kSplit64; 32 x 32 on eight 1.01 (0.89-1.17), kSplit64x32 1.08
+//   up to two, K >= 512 (42): kSplit64x32; kSplit64Pair 1.01 (0.91-1.12), 32 x 32 1.03
+//   beyond, K >= 256 (48): kSplit64Pair; igemm_kernel 64 x 64 0.97 (0.82-1.1), kSplit64x32 0.98: no line here is sharp
+// From one and a half 128 x 128 tiles per CU on igemm_kernel takes 128 x 128 (33): 64 x 64 takes 0.91 of that on average
+// (8192 x 768 over 3072: 383 us as 128 x 128, 294 as kSplit64Pair; 8192 x 3072 over 768: 287 and 330).
 // (bf16 with channels that are no whole 64-element step: the two smallest forms only.)
 int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps) {
   if (!split_tile_fits(dtype, in_c, taps)) return -1;
   const int64_t t32 = tiles_for(gemm_m, gemm_n, 32, 32), t64 = tiles_for(gemm_m, gemm_n, 64, 64);
   if (t32 <= 256) return gemm_k >= 1024 ? kSplit32Deep : kSplit32;
   if (dtype == kBF16) return t32 <= 512 ? kSplit32 : -1;
-  // up to two 32 x 32 tiles per CU: they hide each other's latencies until the reduction is long enough to do so alone
-  // (3136 x 128 over 1152 with the batch sums: 17.4 us as 64 x 32, 16.2 as 32 x 32; 640 x 768 over 3072: 32.4 and 33.9)
   if (t32 <= 512) return gemm_k >= 1536 ? kSplit64x32Deep : kSplit32;
   if (t64 <= 256 && gemm_k >= 768) return kSplit64;
   if (t64 <= 512 && gemm_k >= 512) return kSplit64x32;
@@ -2524,7 +2541,8 @@ int heuristic_tile(int asked, const TileQuery& q) {
   float best_us = INFINITY;
   for (const TileCost& t : q.sums ? kSumsCost : kPlainCost) {
     // one and a half 128 x 128 tiles per compute unit or more, beside a second lane of weight gradients: smaller tiles
-    // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 8 x 1024 12.05 -> 11.76 ms)
+    // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 step of 8 x 1024 tokens 13.34 ms
+    // without this line, 12.19 with it; 3 x 777 tokens and Swin-B of 32 images the same either way)
     if (!q.sums && large && t.bm * t.bn < 128 * 128) continue;
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;

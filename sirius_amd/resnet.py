@@ -69,8 +69,8 @@ class ResNetEngine(EngineBase):
         # wgrad_group_wgs workgroups of equal length, so that a layer is split only where a whole stage would
         # not fill the chip.  Needs the second lane's rule that no dy buffer is handed out twice.  Off by default:
         # measured on ResNet-152 at batch 64, the grouped launches need 2.4 ms of kernel time per step instead of
-        # 6.3 ms (745 against 320 TFLOP/s, no partial filters in stages 3 and 4, 300 launches fewer), but the step
-        # is 16.5-17.1 ms against 16.3 ms: the many short launches run in the gaps of the data-gradient chain,
+        # 4.2 ms (720 against 270-500 TFLOP/s, no partial filters in stages 3 and 4, 147 launches fewer), but the step
+        # is 14.8-15.3 ms against 14.2 ms: the many short launches run in the gaps of the data-gradient chain,
         # which is the critical path, while a launch that fills the chip holds that chain up for as long as it runs
         # (also when it is capped to one workgroup per compute unit).
         # fuse_eval_bn: the forward-only (inference) plan runs convolution + BatchNorm (+ residual) (+ ReLU) as one
@@ -99,31 +99,27 @@ class ResNetEngine(EngineBase):
         # coefficients (its last workgroup per column tile), so that only the apply launch follows.
         # Off by default: measured on MI355X at batch 64, the tail it adds to every convolution (two
         # round trips of device-scope atomics, then a few batches of uncached loads in one workgroup)
-        # costs as much as the finalize launch it saves (20.2 ms per step against 19.3 ms)
+        # costs more than the finalize launch it saves (15.1 ms per step against 14.2 ms)
         self.fuse_bn_finalize = fuse_bn_finalize
         # bn_acc: the convolution epilogues ADD their BatchNorm sums to exact integer accumulators (one pair per
         # channel, zeroed by one launch at the head of the step) instead of leaving them per row tile, and the
         # BatchNorm that follows is ONE launch that derives its coefficients from the two totals: no finalize
         # launch in the large stages, no pass over per-tile partials in the small ones.  bn_acc_max_rows bounds
         # the layers that take this form by their number of rows (0: all of them).
-        # Off by default: measured on MI355X at batch 64 (same box, alternating runs), 20.4 ms per step with every
-        # layer in this form, 17.8 ms with the layers of up to 60 000 rows, 16.8 ms with the 14x14 and 7x7 stages
-        # only, against 15.6 ms without.  The BatchNorm launch gets 1.6 us shorter (12.9 -> 11.3 us) and 77
-        # finalize launches go, but every convolution that adds to the accumulators gets 6-8 us LONGER: the
-        # integer atomics of all row tiles of a channel meet at one address, a device-scope read-modify-write on
-        # one address takes about 70 ns, and the kernel is not done before the last of them is (98 row tiles x 70 ns
-        # = 7 us at 14x14, 1568 tiles at 56x56) -- that with one pair of words per channel, interleaved.  With the
-        # words laid out in planes (512 contiguous bytes per atomic instruction) and the row tiles spread over 4 / 8
-        # copies per channel the 14x14 and 7x7 stages alone cost 15.61 / 15.79 ms against 15.52 ms: still no gain,
-        # what the shorter BatchNorm launch wins the tail of the convolution loses.  Same bits in the loss as the
-        # per-tile form in every variant.
+        # Off by default: no clear gain on MI355X at batch 64 (14.09 ms per step with every layer in this form, 14.18-14.23
+        # without, in one process).  The BatchNorm launch gets 1.6 us shorter (12.9 -> 11.3 us) and 77 finalize launches go, but every
+        # convolution that adds to the accumulators gets longer: the integer atomics of all row tiles of a channel
+        # meet at one address, where read-modify-writes queue up (12-21 ns each with the words in planes of 512 contiguous bytes
+        # and the row tiles spread over bn_acc_copies copies per channel), and the kernel is not done before the last of them is.
+        # Same bits in the loss as the per-tile form.
         self.bn_acc = (os.environ.get("TCH_BN_ACC", "0") != "0") if bn_acc is None else bool(bn_acc)
         self.bn_acc_max_rows = int(os.environ.get("TCH_BN_ACC_MAX_ROWS", "0"))
         self.bn_acc_copies = int(os.environ.get("TCH_BN_ACC_COPIES", "4"))   # row tile t adds to copy t % copies
         # autotune: when a plan is built, time each distinct convolution shape with every tiling and
         # keep the fastest (forward and data gradient separately); off = the library's heuristic
         self.autotune = autotune
-        # tile_margin: see _pick_tiling (measured on the batch-64 step: 0 / 3 / 6 / 10 % -> 15.87 / 15.82 / 15.77 / 15.83 ms)
+        # tile_margin: see _pick_tiling (batch-64 step at 0 / 3 / 5 / 10 %: 14.17-14.22 / 14.24 / 14.16 / 14.30-14.32 ms; the
+        # library's own choice 14.24)
         self.tile_margin = float(os.environ.get("TCH_TILE_MARGIN", "0.05"))
         # retain_gradients: no gradient buffer of a plan is handed out twice, and the plan lists every
         # intermediate tensor of the step by name (plan.tensors): for inspection layer by layer; the launches,
