@@ -613,7 +613,10 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(EmbedArgs p) {
     float acc[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = 0.f;
-    for (int64_t j = tok; j >= 0; j = next_same[j]) {
+    // The links are made long before this launch (beside the forward pass), and a killed batch may have dropped the launch
+    // that makes them: whatever the buffer holds, the walk goes forward only and ends with the tokens.
+    for (int64_t j = tok, to; j >= 0; j = to > j && to < p.tokens ? to : -1) {
+      to = next_same[j];
       Chunk g;
       g.u = static_cast<const uint4*>(p.dy)[j * p.cc + c];
       float v[E];

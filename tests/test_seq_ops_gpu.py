@@ -413,3 +413,31 @@ def test_softmax_ce_lm(ctx, dtype, rows, classes, ld):
     assert torch.all(dl[labels.cuda() < 0][:, :classes] == 0)
     pad = dl[:, (classes + 3) // 4 * 4:]
     assert torch.all(pad == 7.0), "columns beyond the last four-float piece are not touched"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_embedding_backward_walks_forward_whatever_the_links_hold(ctx, dtype):
+    """Links nobody made (the launch that makes them was dropped with a killed batch): a walk goes on only to a later token
+    of the batch, so it stays inside dy and ends."""
+    from sirius_amd import ops
+    B, T, C, vocab = 3, 37, 64, 128
+    n = B * T
+    g = _gen(36)
+    ids = torch.randperm(vocab, generator=g)[:n].view(B, T)      # every token once: no two walks add to one row
+    dy = rnd((B, T, C), dtype, g)
+    links = torch.randint(-2 ** 31, 2 ** 31 - 1, (n,), generator=g).tolist()
+    for i, v in {0: 0, 1: 0, 2: 5, 5: 2, 3: n, 4: n - 1, 6: 2 ** 31 - 1, 7: -2 ** 31, 8: 9, 9: 10, n - 1: n - 1}.items():
+        links[i] = v                                              # to itself, back, a cycle, just past the end, far, a chain
+    chain = torch.tensor(links + [1] * n, dtype=torch.int32, device="cuda")
+    dwte, dwpe = torch.zeros((vocab, C), device="cuda"), torch.zeros((T, C), device="cuda")
+    ops.embedding_bwd(ctx, ids.cuda(), dy.cuda(), dwte, dwpe, chain=chain, chain_ready=True)
+    torch.cuda.synchronize()
+    rows, want = dy.view(n, C).double(), torch.zeros((vocab, C), dtype=torch.float64)
+    for t in range(n):
+        j = t
+        while True:
+            want[ids.view(-1)[t]] += rows[j]
+            if not j < links[j] < n:
+                break
+            j = links[j]
+    close(dwte, want.float(), torch.float32, "dwte", rtol=1e-6)   # at most four fp32 additions of exact values
