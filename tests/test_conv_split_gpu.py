@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import test_ops_gpu as T
+import test_recorded_launches as R
 
 pytestmark = pytest.mark.gpu
 
@@ -40,8 +41,15 @@ def test_batchnorm_sums(ctx, dtype, case, tile_cfg):
 @pytest.mark.parametrize("rows,K,C", [(196, 256, 1024), (196, 512, 2048), (784, 512, 2048), (1024, 256, 1024), (4704, 256, 1024),
                                       (343, 1024, 1024), (2048, 768, 768)])
 def test_library_choice(ctx, dtype, rows, K, C):
-    """One size on each side of the lines of the library's own choice."""
+    """Products of few output tiles, on the library's own choice."""
     T.test_conv_fwd(ctx, dtype, (rows, 1, 1, C, K, 1, 1, 1, 0), -1)
+
+
+@pytest.mark.parametrize("rows,K,C,want", R.F32_CHOICE)
+def test_fp32_choice_on_both_sides_of_its_lines(ctx, rows, K, C, want):
+    """`want` is what runs (held on the CPU by test_recorded_launches.py); here its results, forward and data gradient."""
+    T.test_conv_fwd(ctx, torch.float32, (rows, 1, 1, C, K, 1, 1, 1, 0), -1)
+    T.test_conv_dgrad(ctx, torch.float32, (rows, 1, 1, K, C, 1, 1, 1, 0), -1)
 
 
 @dtypes

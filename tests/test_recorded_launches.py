@@ -200,3 +200,44 @@ def test_floor_table_files_every_convolution_kernel_under_its_direction(rec, dty
                                  tile_cfg, 0, 1))
     wgrad(rec, dtype, tile_cfg, 1)
     assert [family(r[0]) for r in rec.end()] == ["conv forward", "conv data gradient", "conv weight gradient"]
+
+
+# rows, output columns, reduction, and what the library takes for them in fp32: both sides of every line of its choice
+F32_CHOICE = [
+    (196, 256, 1008, "32x32,4way"), (196, 256, 1024, "32x32,8way"), (196, 256, 128, "32x32,4way"),
+    (256, 1024, 1024, "32x32,8way"), (257, 1024, 1024, "32x32,4way"), (257, 1024, 1520, "32x32,4way"), (257, 1024, 1536, "64x32,8way"),
+    (512, 1024, 1024, "32x32,4way"), (513, 1024, 1024, "64x64,8way"), (513, 1024, 768, "64x64,8way"), (513, 1024, 752, "64x32,4way"),
+    (1024, 1024, 1024, "64x64,8way"), (1025, 1024, 1024, "64x32,4way"), (513, 1024, 512, "64x32,4way"), (513, 1024, 496, "64x64,4way"),
+    (2048, 1024, 512, "64x32,4way"), (2049, 1024, 512, "64x64,4way"), (2049, 1024, 256, "64x64,4way"), (2049, 1024, 240, "igemm_kernel<f32,fwd,64x64"),
+    (6016, 1024, 256, "64x64,4way"), (6017, 1024, 256, "igemm_kernel<f32,fwd,128x128"), (6017, 1024, 128, "igemm_kernel<f32,fwd,64x64"),
+]
+
+
+def product(rec, dtype, rows, cols, depth, tile_cfg):
+    rec.begin()
+    check(lib().tch_conv2d_fwd(rec.ctx, dtype, address(0), address(1), address(2), None, None, None, 0, rows, 1, 1, depth, cols, 1, 1,
+                               1, 0, tile_cfg, 0))
+    (name, _, _), = rec.end()
+    return name
+
+
+@pytest.mark.parametrize("rows,cols,depth,want", F32_CHOICE)
+def test_fp32_choice_on_both_sides_of_its_lines(rec, rows, cols, depth, want):
+    assert want in product(rec, F32, rows, cols, depth, -1)
+    assert product(rec, F32, rows, cols, depth, -2).startswith("igemm_kernel<f32,fwd,")
+
+
+def test_bf16_choice_for_large_products_and_in_order(rec):
+    """From 384 tiles of 128 x 128 on a plain product takes no smaller one; with one order of additions asked for neither a
+    split tiling nor the 3x3 patch kernel runs."""
+    assert ",128x128," in product(rec, BF16, 8192, 768, 768, -1) and ",128x128," in product(rec, BF16, 100352, 128, 128, -1)
+    assert ",128x128," not in product(rec, BF16, 8192 - 128, 768, 768, -1)
+    assert product(rec, BF16, 196, 256, 1024, -1).startswith("igemm4_kernel")
+    for rows in (1, 49, 196, 1000, 8192, 300000):
+        for cols, depth in ((64, 256), (256, 1024), (768, 64), (512, 96)):
+            assert not product(rec, BF16, rows, cols, depth, -2).startswith(("igemm3", "igemm4"))
+    for cfg, patch in ((-1, True), (-2, False)):
+        rec.begin()
+        check(lib().tch_conv2d_fwd(rec.ctx, BF16, address(0), address(1), address(2), None, None, None, 0, 64, 14, 14, 256, 256, 3, 3, 1, 1,
+                                   cfg, 0))
+        assert rec.end()[0][0].startswith("igemm3_kernel") == patch
