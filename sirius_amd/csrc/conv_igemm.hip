@@ -319,11 +319,89 @@ __device__ inline void store_floats(float* dst, const float* v) {
 //                  sum(g * xhat), xhat = (bn_x - mean) * invstd: the two reductions of the
 //                  BatchNorm backward.
 // ---------------------------------------------------------------------------
+// What the epilogue reads beside the accumulators: per output chunk (a "visit" of a thread) the addend, and for the
+// BatchNorm sums the BatchNorm's input and the ReLU's output.  Requested for all chunks of a thread at once, or, where the
+// accumulators leave no registers for that, for the chunks of one 32-row band (a data gradient's addend: for one chunk).
+// Bounded by latency: reading each chunk's operands when its turn came cost a trip to memory per chunk (the stores between
+// them keep the compiler from moving the loads up).  Launches in the step, one at a time: inference convolutions with a
+// residual 1-4 us less, data gradients with BatchNorm sums 2-5, with an addend too 5-9; a ResNet-152 request of one image
+// 1104 -> 995 us, of 24 images 2288 -> 2148, training steps of 64, 2 x 16 and 20 images 2-3 % shorter.
+template <typename T, int MODE, int VISITS, int BAND>
+struct EpilogueOperands {
+  static constexpr int kGroup = VISITS <= 8 ? VISITS : BAND;
+  static constexpr int kAddGroup = MODE == kFwd || VISITS <= 4 ? kGroup : 1;
+  static constexpr int E = Elem<T>::kPerChunk;
+  Chunk add[kAddGroup], x[kGroup], relu[kGroup];
+  // of the thread's columns: scale and bias (forward), mean and inverse std (data gradient with BatchNorm sums)
+  float c0[E], c1[E];
+
+  __device__ static inline void request_columns(const float* src, int n, int col, float (&c)[E]) {
+    const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(src, static_cast<uint32_t>(n) * 4);
+#pragma unroll
+    for (int e = 0; e < E; e += 4) {
+      const Chunk v = load_chunk(rsrc, static_cast<uint32_t>(col + e) * 4, col < n);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[e + k] = v.f[k];
+    }
+  }
+
+  // `row`, `col`: of the chunk in the output
+  __device__ inline void request_sums(const IgemmArgs& p, int i, int row, int col, bool ok) {
+    const uint32_t bytes = static_cast<uint32_t>(p.gemm_m) * p.gemm_n * sizeof(T);
+    const uint32_t at = (static_cast<uint32_t>(row) * p.gemm_n + col) * static_cast<uint32_t>(sizeof(T));
+    x[i] = load_chunk(make_rsrc(p.bn_x, bytes), at, ok);
+    if (p.bn_mask) relu[i] = load_chunk(make_rsrc(p.bn_mask, bytes), at, ok);
+  }
+  __device__ inline void request_add(const IgemmArgs& p, int i, int row, int col, bool ok) {
+    const uint32_t bytes = static_cast<uint32_t>(p.gemm_m) * p.gemm_n * sizeof(T);
+    const uint32_t at = (static_cast<uint32_t>(row) * p.gemm_n + col) * static_cast<uint32_t>(sizeof(T));
+    if (MODE == kDgrad && p.add_sub) {   // lives on the even pixels: zeros elsewhere
+      const uint32_t hs = (p.H + 1) >> 1, ws = (p.W + 1) >> 1;
+      uint32_t img, rem, h, w;
+      p.div_plane.divmod(static_cast<uint32_t>(row), img, rem);
+      p.div_width.divmod(rem, h, w);
+      const uint32_t sub = (((img * hs + (h >> 1)) * ws + (w >> 1)) * p.gemm_n + col) * static_cast<uint32_t>(sizeof(T));
+      add[i] = load_chunk(make_rsrc(p.add, static_cast<uint32_t>(p.N) * hs * ws * p.gemm_n * sizeof(T)), sub, ok && ((h | w) & 1u) == 0u);
+    } else {
+      add[i] = load_chunk(make_rsrc(p.add, bytes), at, ok);
+    }
+  }
+
+  // The operands of the group of chunks that starts at `visit`, if one does.  (NT threads store, a chunk column each;
+  // row_of: visit -> row of the tile.)
+  template <int BN, int NT, typename RowOf>
+  __device__ inline void request_group(const IgemmArgs& p, int visit, bool sums, int tid, int m0, int n0, RowOf row_of) {
+    const int col = n0 + (tid % (BN / E)) * E;
+    auto stored = [&](int row) { return tid < NT && row < p.gemm_m && col < p.gemm_n; };
+    if (MODE == kDgrad && sums && visit % kGroup == 0) {
+#pragma unroll
+      for (int v = 0; v < kGroup; ++v) request_sums(p, v, m0 + row_of(visit + v), col, stored(m0 + row_of(visit + v)));
+    }
+    if (p.add && visit % kAddGroup == 0) {
+#pragma unroll
+      for (int v = 0; v < kAddGroup; ++v) request_add(p, v, m0 + row_of(visit + v), col, stored(m0 + row_of(visit + v)));
+    }
+  }
+  // ahead of the walk over the chunks
+  template <int BN, int NT, typename RowOf>
+  __device__ inline void request_first(const IgemmArgs& p, int tid, int m0, int n0, RowOf row_of) {
+    const int col = n0 + (tid % (BN / E)) * E;
+    const bool sums = MODE == kDgrad && (p.stats || p.stat_acc);
+    const float* const p0 = MODE == kFwd ? p.scale : sums ? p.bn_mean : nullptr;
+    const float* const p1 = MODE == kFwd ? p.bias : sums ? p.bn_invstd : nullptr;
+    if (p0) request_columns(p0, p.gemm_n, col, c0);
+    if (p1) request_columns(p1, p.gemm_n, col, c1);
+    request_group<BN, NT>(p, 0, sums, tid, m0, n0, row_of);
+  }
+};
+
 // The accumulators reach it through `walk(fin)`, which calls fin(visit, row of the tile, column of the tile, E values) for
-// every chunk this thread stores (column chunk tid % CH, so `row_of(visit)` alone names it beforehand).
-// NT of the workgroup's BLOCK threads store something; the others only keep the barriers company.
-template <typename T, int MODE, int BN, int NT, int BLOCK, int VISITS, int STAGE_BYTES, typename RowOf, typename Walk>
-__device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, int m0, int n0, int tile_m, RowOf row_of, Walk walk) {
+// every chunk this thread stores (column chunk tid % CH, so `row_of(visit)` alone names it beforehand); `o` holds the operands
+// of its first group of chunks.  NT of the workgroup's BLOCK threads store something; the
+// others only keep the barriers company.
+template <typename T, int MODE, int BN, int NT, int BLOCK, int VISITS, int BAND, int STAGE_BYTES, typename RowOf, typename Walk>
+__device__ inline void finish_walk(const IgemmArgs& p, EpilogueOperands<T, MODE, VISITS, BAND>& o, float* stage, int tid, int m0, int n0,
+                                   int tile_m, RowOf row_of, Walk walk) {
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int CH = BN / E;   // column chunks of the tile; a thread always gets chunk tid % CH
   constexpr int ROWS = NT / CH;
@@ -333,55 +411,23 @@ __device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, in
   float st_sum[E], st_sq[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) st_sum[e] = st_sq[e] = 0.f;
-  // data gradient with BatchNorm sums: the chunks of bn_x and bn_mask this thread will meet are
-  // requested up front, so that their latency overlaps the staging of the accumulators
-  float bn_mu[E], bn_is[E];
-  uint4 pre_x[VISITS], pre_m[VISITS];
-  if (MODE == kDgrad && want_stats) {
-    const int col = n0 + (tid % CH) * E;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      bn_mu[e] = col < p.gemm_n ? p.bn_mean[col + e] : 0.f;
-      bn_is[e] = col < p.gemm_n ? p.bn_invstd[col + e] : 0.f;
-    }
-#pragma unroll
-    for (int visit = 0; visit < VISITS; ++visit) {
-      const int row = m0 + row_of(visit);
-      const bool ok = storing && row < p.gemm_m && col < p.gemm_n;
-      const int64_t idx = static_cast<int64_t>(row) * p.gemm_n + col;
-      pre_x[visit] = ok ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_x) + idx) : make_uint4(0, 0, 0, 0);
-      pre_m[visit] = (ok && p.bn_mask) ? *reinterpret_cast<const uint4*>(static_cast<const T*>(p.bn_mask) + idx)
-                                       : make_uint4(0, 0, 0, 0);
-    }
-  }
-
   walk([&](int visit, int tr, int tc, float* v) {
+    if (visit > 0) o.template request_group<BN, NT>(p, visit, MODE == kDgrad && want_stats, tid, m0, n0, row_of);
     const int row = m0 + tr, col = n0 + tc;
     if (row >= p.gemm_m || col >= p.gemm_n) return;
     const int64_t idx = static_cast<int64_t>(row) * p.gemm_n + col;
+    const int sums_at = visit % o.kGroup, add_at = visit % o.kAddGroup;
     if (MODE == kFwd && p.scale) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) v[e] *= p.scale[col + e];
+      for (int e = 0; e < E; ++e) v[e] *= o.c0[e];
     }
     if (MODE == kFwd && p.bias) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) v[e] += p.bias[col + e];
+      for (int e = 0; e < E; ++e) v[e] += o.c1[e];
     }
-    bool add_here = p.add != nullptr;
-    int64_t add_idx = idx;
-    if (MODE == kDgrad && p.add_sub && add_here) {
-      uint32_t img, rem, h, w;
-      p.div_plane.divmod(static_cast<uint32_t>(row), img, rem);
-      p.div_width.divmod(rem, h, w);
-      add_here = ((h | w) & 1u) == 0u;
-      const int64_t hs = (p.H + 1) >> 1, ws = (p.W + 1) >> 1;
-      add_idx = ((static_cast<int64_t>(img) * hs + (h >> 1)) * ws + (w >> 1)) * p.gemm_n + col;
-    }
-    if (add_here) {
-      Chunk ca;
-      ca.u = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.add) + add_idx);
+    if (p.add) {
       float a[E];
-      chunk_to_float<T>(ca, a);
+      chunk_to_float<T>(o.add[add_at], a);
       if (p.mask) {
         Chunk cm;
         cm.u = *reinterpret_cast<const uint4*>(static_cast<const T*>(p.mask) + idx);
@@ -403,13 +449,9 @@ __device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, in
     } else if (MODE == kDgrad && want_stats) {
       Chunk c = float_to_chunk<T>(v);
       chunk_to_float<T>(c, v);
-      Chunk cx;
-      cx.u = pre_x[visit];
       if (p.bn_mask) {
-        Chunk cm;
-        cm.u = pre_m[visit];
         float m[E];
-        chunk_to_float<T>(cm, m);
+        chunk_to_float<T>(o.relu[sums_at], m);
 #pragma unroll
         for (int e = 0; e < E; ++e)
           if (!(m[e] > 0.f)) v[e] = 0.f;
@@ -417,11 +459,11 @@ __device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, in
       }
       *reinterpret_cast<uint4*>(static_cast<T*>(p.out) + idx) = c.u;
       float x[E];
-      chunk_to_float<T>(cx, x);
+      chunk_to_float<T>(o.x[sums_at], x);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         st_sum[e] += v[e];
-        st_sq[e] += v[e] * ((x[e] - bn_mu[e]) * bn_is[e]);
+        st_sq[e] += v[e] * ((x[e] - o.c0[e]) * o.c1[e]);
       }
     } else {
       const Chunk c = float_to_chunk<T>(v);
@@ -483,22 +525,32 @@ __device__ inline void finish_walk(const IgemmArgs& p, float* stage, int tid, in
   }
 }
 
-// The form for accumulators spread over the wavefronts of a tile, one 32-row band at a time.
-template <typename T, int MODE, int WM, int WN, int TM, int TN>
-__device__ inline void finish_tile(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0,
-                                   int tile_m) {
-  constexpr int BN = WN * TN * 32;
-  constexpr int NT = WM * WN * 64;
-  constexpr int CH = BN / Elem<T>::kPerChunk;
-  constexpr int ITERS = (WM * 32 * CH) / NT;
-  finish_walk<T, MODE, BN, NT, NT, TM * ITERS, WM * 32 * (BN + kStagePad) * 4>(
-      p, stage, tid, m0, n0, tile_m,
-      [&](int visit) {
-        const int r = (tid + (visit % ITERS) * NT) / CH;
-        return ((r >> 5) * TM + visit / ITERS) * 32 + (r & 31);
-      },
-      [&](auto fin) { staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, fin); });
-}
+// The form for accumulators spread over the wavefronts of a tile, one 32-row band at a time.  EARLY: the operands are
+// requested when the kernel starts and wait in registers until the accumulators are done (the kernels that can spare the
+// registers), instead of costing a trip to memory behind the last multiply.
+template <typename T, int MODE, int WM, int WN, int TM, int TN, bool EARLY>
+struct TileEpilogue {
+  static constexpr int BN = WN * TN * 32, NT = WM * WN * 64, CH = BN / Elem<T>::kPerChunk;
+  static constexpr int ITERS = (WM * 32 * CH) / NT, VISITS = TM * ITERS;
+  EpilogueOperands<T, MODE, VISITS, ITERS> operands;
+
+  __device__ static inline int row_of(int tid, int visit) {
+    const int r = (tid + (visit % ITERS) * NT) / CH;
+    return ((r >> 5) * TM + visit / ITERS) * 32 + (r & 31);
+  }
+  __device__ inline void request(const IgemmArgs& p, int tid, int m0, int n0) {
+    operands.template request_first<BN, NT>(p, tid, m0, n0, [&](int visit) { return row_of(tid, visit); });
+  }
+  __device__ inline void start(const IgemmArgs& p, int tid, int m0, int n0) {
+    if constexpr (EARLY) request(p, tid, m0, n0);
+  }
+  __device__ inline void finish(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0, int tile_m) {
+    if constexpr (!EARLY) request(p, tid, m0, n0);
+    finish_walk<T, MODE, BN, NT, NT, VISITS, ITERS, WM * 32 * (BN + kStagePad) * 4>(
+        p, operands, stage, tid, m0, n0, tile_m, [&](int visit) { return row_of(tid, visit); },
+        [&](auto fin) { staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, fin); });
+  }
+};
 
 // ---------------------------------------------------------------------------
 // forward / data gradient
@@ -671,7 +723,8 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
     load_tiles(kt + 4, ra0, rb0);
   }
 
-  finish_tile<T, MODE, WM, WN, TM, TN>(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
+  TileEpilogue<T, MODE, WM, WN, TM, TN, false> epilogue;
+  epilogue.finish(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
@@ -1272,6 +1325,14 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
 constexpr int kStep2 = 64;                  // reduction elements per step
 constexpr int kRowBytes2 = kStep2 * 2;      // 128
 
+// Whether a kernel can keep the epilogue's operands in registers from its start: by what LDS leaves of the registers (512
+// per lane of a SIMD, shared by the wavefronts on it).
+template <int MODE, int WAVES, int FRAGS, int RING_BYTES>
+constexpr bool igemm2_early() {
+  constexpr int per_simd = 163840 / RING_BYTES * WAVES / 4, registers = 512 / per_simd;
+  return FRAGS <= (MODE == kFwd ? 3 : 2) && registers >= (MODE == kFwd ? 80 : 160);
+}
+
 template <int MODE, int WM, int WN, int TM, int TN, int NBUF, int ROT = 0, int KS = kStep2>
 __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
   using T = bf16;
@@ -1318,6 +1379,8 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     tile_n = id - tile_m * p.tiles_n;
   }
   const int m0 = tile_m * BM, n0 = tile_n * BN;
+  TileEpilogue<T, MODE, WM, WN, TM, TN, igemm2_early<MODE, WM * WN, TM * TN, NBUF * BUF_BYTES>()> epilogue;
+  epilogue.start(p, tid, m0, n0);
 
   const int in_h = (MODE == kFwd) ? p.H : p.Ho;
   const int in_w = (MODE == kFwd) ? p.W : p.Wo;
@@ -1586,7 +1649,7 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
       if (kt0 + u < nk) step(kt0 + u, u);
   }
 
-  finish_tile<T, MODE, WM, WN, TM, TN>(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
+  epilogue.finish(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
 }
 
 // ---------------------------------------------------------------------------
@@ -1634,6 +1697,9 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
   const int slow = id / run, fast = id - slow * run;
   const int tile_m = p.group_rows ? fast : slow, tile_n = p.group_rows ? slow : fast;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
+  auto row_of = [&](int visit) { return (tid + visit * NT) / CH; };
+  EpilogueOperands<T, MODE, VISITS, VISITS> operands;
+  operands.template request_first<BN, NTE>(p, tid, m0, n0, row_of);
 
   const int in_h = (MODE == kFwd) ? p.H : p.Ho;
   const int in_w = (MODE == kFwd) ? p.W : p.Wo;
@@ -1796,9 +1862,8 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
 
   // ---- the partial tiles meet: [wave][BM][LD] fp32, over the rings ----
   float* red = reinterpret_cast<float*>(lds);
-  finish_walk<T, MODE, BN, NTE, NT, VISITS, LDS_BYTES>(
-      p, red, tid, m0, n0, tile_m, [&](int visit) { return (tid + visit * NT) / CH; },
-      [&](auto fin) {
+  finish_walk<T, MODE, BN, NTE, NT, VISITS, VISITS, LDS_BYTES>(
+      p, operands, red, tid, m0, n0, tile_m, row_of, [&](auto fin) {
         __syncthreads();   // every wavefront is done with its ring
         float* mine = red + wave * (BM * LD);
 #pragma unroll
@@ -1866,6 +1931,8 @@ __global__ __launch_bounds__(256) void igemm3_kernel(IgemmArgs p) {
   const int tile_m = id / p.tiles_n;
   const int tile_n = id - tile_m * p.tiles_n;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
+  TileEpilogue<T, MODE, WM, WN, TM, TN, true> epilogue;
+  epilogue.start(p, tid, m0, n0);
 
   const int in_c = (MODE == kFwd) ? p.C : p.K;
   const int cblocks = in_c / kStep2;
@@ -2021,7 +2088,7 @@ __global__ __launch_bounds__(256) void igemm3_kernel(IgemmArgs p) {
     }
   }
 
-  finish_tile<T, MODE, WM, WN, TM, TN>(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
+  epilogue.finish(p, acc, reinterpret_cast<float*>(lds), tid, m0, n0, tile_m);
 }
 
 __device__ __forceinline__ void splitk_reduce_body(const ReduceArgs& p, uint32_t block) {
