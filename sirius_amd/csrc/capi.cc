@@ -124,7 +124,9 @@ int tch_program_end_record(tch_context* ctx) {
     if (rc == 0) rc = conv2d_wgrad_flush(&c);
     c.trailing_reduce.valid = c.trailing_col_sum.valid = false;
   }
+  const Program& done = *c.recording;
   c.recording = nullptr;
+  c.prepare_lanes(done);
   return rc;
 }
 

@@ -124,7 +124,7 @@ class Context {
   explicit Context(hipStream_t s) : stream(s) {}
   ~Context();
   hipStream_t stream;
-  // second stream (default priority) for lane-1 launches of a replayed program; made on first use
+  // second stream (default priority) for lane-1 launches of a replayed program; made when one is recorded, or on first use
   hipStream_t side = nullptr;
   // Compute-unit share: with a limit in force the launches go to a pair of streams whose CU mask keeps
   // the highest-numbered `cu_limit` compute units (made once per limit, kept for the process); 0 = no
@@ -140,6 +140,14 @@ class Context {
   // at such a point it is made to wait for lane 1, and lane 0 waits for it at the next one.
   hipStream_t relay = nullptr;
   bool relay_dirty = false;  // the relay waits for lane-1 work that lane 0 has not waited for
+  // A stream whose launches run beside those of `stream`.  A process has four hardware queues (HIP's default) and its streams
+  // are dealt out to them in turn, so one stream in a few shares the main lane's queue: as a second lane it overlaps
+  // nothing, as a relay its waits hold the main lane up.  Two engines' worth of streams later the same engine has read 6.4
+  // for 4.8 ms (Swin-B, 7 images), 5.6 for 4.45 (GPT-2, 8 x 256), 12.7 for 11.9 (8 x 1024).  Which queue a stream has
+  // cannot be asked, so two small kernels find out whether they meet; 0.1 ms for a stream that is turned down.
+  hipStream_t stream_beside_main();
+  // makes the streams a recorded program will use, so that the first replay need not
+  void prepare_lanes(const Program& prog);
   // recording state: the lane new launches are stamped with, and whether the next lane-1 launch
   // has to wait for lane 0
   int lane = 0;
