@@ -160,8 +160,9 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * 15 - 20 split the reduction over the wavefronts of a workgroup, for outputs of few tiles: 15 / 16 = 32x32 over four /
  * eight wavefronts, 17 / 20 = 64x32 over four / eight, 18 / 19 = 64x64 with one / two workgroups per CU (input channels a
  * multiple of 64 bytes; anything else runs tiling 2 for them).  Partial sums are added in the order of the wavefronts.
- * 21 / 22 = 64x64 and 128x64 (eight wavefronts) with the operand reads pipelined over the reduction steps (bf16, input
- * channels a multiple of 64; anything else runs tilings 2 / 1 for them; same bits as those).
+ * 21 = 64x64 with the operand reads pipelined over the reduction steps, 22 / 23 / 24 = 128x64, 128x128 and 128x192 with
+ * reads, loads and multiplies interleaved on eight wavefronts, as tiling 0 has them (bf16, input channels a multiple of 64;
+ * anything else runs tilings 2, 1, 0 and 0 for them; same bits as those).
  * c_logical: input channels that carry data when C is zero-padded to a chunk (0 = C); it only enters the
  * algorithmic-work figure the profiler reports, never the arithmetic. */
 int tch_conv2d_fwd(tch_context* ctx, int dtype, const void* x, const void* w, void* y, const void* add,

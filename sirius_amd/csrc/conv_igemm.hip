@@ -37,6 +37,7 @@
 #include "col_sum.h"
 #include "kernels.h"
 #include <algorithm>
+#include <iterator>
 #include <vector>
 
 #include "context.h"
@@ -172,9 +173,12 @@ struct TapWalker {
 // whose result the publishing thread waits for before the barrier that precedes the counter bump,
 // and the finishing workgroup reads them with device-scope atomic loads.  Atomics execute at the
 // point all slices share.
-template <int MODE, int BN, int NT>
+// (Its flag lies in the last word of the staging tile, behind the sums: a variable of its own would cost every kernel 4 bytes
+// of LDS, and two workgroups of 80 KB their place on one CU.)
+template <int MODE, int BN, int NT, int STAGE_BYTES>
 __device__ inline void finalize_column_tile(const IgemmArgs& p, float* stage, int tid, int n0) {
-  __shared__ int last_arrival;
+  static_assert(NT * 16 + 4 <= STAGE_BYTES, "sums and flag fit the staging tile");
+  int& last_arrival = reinterpret_cast<int*>(stage)[STAGE_BYTES / 4 - 1];
   __syncthreads();
   if (tid == 0) {
     int* counter = p.fin_counters + n0 / BN;
@@ -254,6 +258,15 @@ __device__ inline void finalize_column_tile(const IgemmArgs& p, float* stage, in
   }
 }
 
+// Threads of a workgroup that store a tile BN columns wide: whole rows of chunks per visit, a power of two of them (all
+// threads, unless the tile is 96 or 192 columns wide).
+template <int E, int BN, int NT>
+constexpr int storing_threads() {
+  int rows = 1;
+  while (2 * rows * (BN / E) <= NT) rows *= 2;
+  return rows * (BN / E);
+}
+
 // The accumulators of one workgroup tile, one 32-row band (index tm) at a time:
 // lanes write float4 groups into the staging tile [WM*32][BN + pad], then every
 // thread takes E consecutive columns of one row and hands them to `fin` together with the
@@ -265,8 +278,9 @@ __device__ inline void staged_epilogue(f32x16_t (&acc)[TM][TN], float* stage, in
   constexpr int NT = WM * WN * 64;
   constexpr int LD = BN + kStagePad;
   constexpr int CH = BN / E;
-  constexpr int ITERS = (WM * 32 * CH) / NT;
-  static_assert((WM * 32 * CH) % NT == 0, "epilogue mapping");
+  constexpr int NTE = storing_threads<E, BN, NT>();
+  constexpr int ITERS = (WM * 32 * CH) / NTE;
+  static_assert((WM * 32 * CH) % NTE == 0, "epilogue mapping");
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
 #pragma unroll
@@ -284,9 +298,10 @@ __device__ inline void staged_epilogue(f32x16_t (&acc)[TM][TN], float* stage, in
       }
     }
     __syncthreads();
+    if (NTE < NT && tid >= NTE) continue;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-      const int q = tid + it * NT;
+      const int q = tid + it * NTE;
       const int r = q / CH, cc = q - r * CH;
       float v[E];
 #pragma unroll
@@ -521,7 +536,7 @@ __device__ inline void finish_walk(const IgemmArgs& p, EpilogueOperands<T, MODE,
         }
       }
     }
-    if (p.fin_counters) finalize_column_tile<MODE, BN, NT>(p, stage, tid, n0);
+    if (p.fin_counters) finalize_column_tile<MODE, BN, NT, STAGE_BYTES>(p, stage, tid, n0);
   }
 }
 
@@ -531,22 +546,23 @@ __device__ inline void finish_walk(const IgemmArgs& p, EpilogueOperands<T, MODE,
 template <typename T, int MODE, int WM, int WN, int TM, int TN, bool EARLY>
 struct TileEpilogue {
   static constexpr int BN = WN * TN * 32, NT = WM * WN * 64, CH = BN / Elem<T>::kPerChunk;
-  static constexpr int ITERS = (WM * 32 * CH) / NT, VISITS = TM * ITERS;
+  static constexpr int NTE = storing_threads<Elem<T>::kPerChunk, BN, NT>();
+  static constexpr int ITERS = (WM * 32 * CH) / NTE, VISITS = TM * ITERS;
   EpilogueOperands<T, MODE, VISITS, ITERS> operands;
 
   __device__ static inline int row_of(int tid, int visit) {
-    const int r = (tid + (visit % ITERS) * NT) / CH;
+    const int r = (tid + (visit % ITERS) * NTE) / CH;
     return ((r >> 5) * TM + visit / ITERS) * 32 + (r & 31);
   }
   __device__ inline void request(const IgemmArgs& p, int tid, int m0, int n0) {
-    operands.template request_first<BN, NT>(p, tid, m0, n0, [&](int visit) { return row_of(tid, visit); });
+    operands.template request_first<BN, NTE>(p, tid, m0, n0, [&](int visit) { return row_of(tid, visit); });
   }
   __device__ inline void start(const IgemmArgs& p, int tid, int m0, int n0) {
     if constexpr (EARLY) request(p, tid, m0, n0);
   }
   __device__ inline void finish(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0, int tile_m) {
     if constexpr (!EARLY) request(p, tid, m0, n0);
-    finish_walk<T, MODE, BN, NT, NT, VISITS, ITERS, WM * 32 * (BN + kStagePad) * 4>(
+    finish_walk<T, MODE, BN, NTE, NT, VISITS, ITERS, WM * 32 * (BN + kStagePad) * 4>(
         p, operands, stage, tid, m0, n0, tile_m, [&](int visit) { return row_of(tid, visit); },
         [&](auto fin) { staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, fin); });
   }
@@ -1312,9 +1328,12 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
 //   * a step never straddles a filter tap (channels % 64 == 0), so the tap walk is scalar:
 //     a lane keeps one byte offset and one validity bit per tap for each row it loads;
 //   * NBUF tiles in LDS, one barrier per step: one is multiplied, one is being requested, and NBUF - 2 are in flight
-//     across the barrier (none with two, where the other workgroups of the CU fill the trip to memory: 8192 x 768 over
-//     3072 takes 45.2 us as 128 x 128 with two 64-element tiles, 61 with three, 51.5 with three of 32; 8192 x 2304
-//     over 768 44.8, 53.5 and 43.2);
+//     across the barrier (none with two, where the other workgroups of the CU fill the trip to memory);
+//   * ROT = 1 is the rotated, interleaved loop (see there) with eight wavefronts per tile: two on every SIMD, one multiplies
+//     while the other waits.  What bounds a tile then is the operand path of the CU (direct loads reach 135 B/ns, LDS reads
+//     600; the loop alone 1.65 PFLOP/s at 128 x 192, MFMA alone 1.84 where 2.5 is the peak).  8192 x 768 over 3072: 43.7 us
+//     as 128 x 128 on four wavefronts without it, 37.2 as 128 x 192; 8192 x 2304 over 768 44.8 and 41.1 (128 x 128),
+//     2048 x 2304 15.3 and 12.3 (128 x 192); 12 544 x 256 over 1024 with batch sums 14.6 and 12.3 (128 x 128, three tiles);
 //   * ROT = 2 reads the operands of the next step into a second register set while this step is multiplied: the barrier
 //     hands over a tile one step before it is needed and the LDS latency passes behind the multiplies.  What bounds
 //     the small tiles then is LDS itself (a 64 x 64 tile: 32 KB read, 16 KB written per step).  1024 x 768 over 3072:
@@ -1439,7 +1458,8 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 
   // scalar walk over (tap, channel block)
   int ld_r = 0, ld_s = 0, ld_cb = 0, ld_t = 0, ld_kt = 0;
-  auto issue_loads = [&](int buf) {
+  // direct load j (of the A_LD + B_LD) of the tile the walk stands at
+  auto issue_load = [&](int buf, int j) {
     // element offset of this tap relative to tap (0,0), then bytes
     const int tap_elems = (MODE == kFwd) ? (ld_r * in_w + ld_s) * in_c : -((ld_r >> sl) * in_w + (ld_s >> sl)) * in_c;
     const int a_step = (tap_elems + ld_cb * KS) * 2;
@@ -1447,17 +1467,15 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     // a tile behind the last one: every offset out of range, so zeros land and memory is not asked
     const uint32_t tap_bit = ld_kt < nk ? 1u << ld_t : 0u;
     const int beyond = ld_kt < nk ? 0 : static_cast<int>(kOutOfRange);
-    unsigned char* dst_a = lds + buf * BUF_BYTES + wave * A_LD * 1024;
-    unsigned char* dst_b = lds + buf * BUF_BYTES + A_BYTES + wave * B_LD * 1024;
-#pragma unroll
-    for (int j = 0; j < A_LD; ++j) {
+    if (j < A_LD) {
       const bool ok = (a_taps[j] & tap_bit) != 0;
       const int off = ok ? a_off[j] + a_step : static_cast<int>(kOutOfRange);
-      load_to_lds(rsrc_a, dst_a + j * 1024, off, 0);
+      load_to_lds(rsrc_a, lds + buf * BUF_BYTES + (wave * A_LD + j) * 1024, off, 0);
+    } else {
+      load_to_lds(rsrc_b, lds + buf * BUF_BYTES + A_BYTES + (wave * B_LD + j - A_LD) * 1024, b_off[j - A_LD] | beyond, b_step);
     }
-#pragma unroll
-    for (int j = 0; j < B_LD; ++j)
-      load_to_lds(rsrc_b, dst_b + j * 1024, b_off[j] | beyond, b_step);
+  };
+  auto next_tile = [&] {
     ++ld_kt;
     // selects, not branches: no block boundary while operand reads are in flight
     const int next_tap = ++ld_cb == cblocks ? 1 : 0;
@@ -1467,6 +1485,11 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     const int next_row = ld_s == p.S ? 1 : 0;
     ld_s = next_row ? 0 : ld_s;
     ld_r += next_row;
+  };
+  auto issue_loads = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < A_LD + B_LD; ++j) issue_load(buf, j);
+    next_tile();
   };
 
   f32x16_t acc[TM][TN];
@@ -1598,43 +1621,79 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     });
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile: the epilogue uses their place
   } else if constexpr (ROT == 1) {
-    // Rotated loop for the large tiles, whose workgroup has a compute unit to itself (nobody else fills the
-    // gap a barrier leaves): the barrier that hands over tile kt+1 sits BEFORE the last quarter of tile kt's
-    // multiplies, whose operands are in registers by then, and the first operand reads of tile kt+1 are issued
-    // in front of that quarter.  The matrix pipeline therefore has a quarter's multiplies to chew on while the
-    // barrier, the reads' latency and the issue of the next tile's loads pass.  Every wait stands behind a
-    // quarter's multiplies that were issued after the reads it waits for, and nothing is in flight at the loop
-    // edge.  Order of additions per accumulator: as in the plain loop (same results bit for bit).
-    static_assert(NBUF == 2 && KS == 64, "the rotated loop keeps two 64-element tiles in LDS");
-    uint4_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
-    issue_loads(0);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    if (1 < nk) issue_loads(1);
-    read_frags(0, 0, fa0, fb0);
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    auto body = [&](int kt, int u) {
-      read_frags(u, 1, fa1, fb1);
-      multiply(fa0, fb0);
-      asm volatile("s_waitcnt lgkmcnt(0)");
-      read_frags(u, 2, fa0, fb0);
-      multiply(fa1, fb1);
-      asm volatile("s_waitcnt lgkmcnt(0)");
-      read_frags(u, 3, fa1, fb1);
-      multiply(fa0, fb0);
-      // all of tile kt is in registers; tile kt+1 (the only loads outstanding) must have landed
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (kt + 1 < nk) read_frags(u ^ 1, 0, fa0, fb0);
-      multiply(fa1, fb1);
-      if (kt + 2 < nk) issue_loads(u);
-      asm volatile("s_waitcnt lgkmcnt(0)");
-    };
-    int kt0 = 0;
-    for (; kt0 + 2 <= nk; kt0 += 2) {
-      body(kt0, 0);
-      body(kt0 + 1, 1);
+    // Rotated and interleaved: while the 16-element slice s of a tile is multiplied, slice s+1 is read into the other register set and
+    // a part of the direct loads goes out, an instruction or two behind every MFMA, so that nothing but the barrier
+    // leaves the matrix pipe without work.  The barrier that hands over tile kt+1 stands in front of tile kt's last slice,
+    // which is in registers by then, as is everything else of tile kt: its buffer takes tile kt+NBUF from there on.
+    constexpr int SL = KS / 16;
+    uint4_t fa[2][TM], fb[2][TN];
+    uint32_t a_sl[SL], b_sl[SL];
+#pragma unroll
+    for (int kk = 0; kk < SL; ++kk) {
+      a_sl[kk] = a_rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16);
+      b_sl[kk] = b_rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16);
     }
-    if (kt0 < nk) body(kt0, 0);
-    __syncthreads();   // the epilogue stages through the operand buffers: every wave is done reading them
+    auto read_one = [&](int buf, int kk, int set, int i) {   // operand i (of the TM + TN) of slice kk
+      const uint32_t at = buf * BUF_BYTES;
+      if (i < TM)
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][i]) : "v"(a_sl[kk] + at), "n"(i * 32 * RB));
+      else
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][i - TM]) : "v"(b_sl[kk] + at), "n"((i - TM) * 32 * RB));
+    };
+    auto hold_set = [&](int set) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(fa[set][i]));
+#pragma unroll
+      for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(fb[set][i]));
+    };
+    // multiplies the slice in `set`; meanwhile slice kk of the tile in `buf` is read into the other set and part `q` of the
+    // loads goes to `ld_buf`
+    auto slice = [&](auto set_c, auto buf_c, auto kk_c, auto q_c, auto ld_buf_c) {
+      constexpr int set = decltype(set_c)::value, buf = decltype(buf_c)::value, kk = decltype(kk_c)::value;
+      constexpr int q = decltype(q_c)::value, ld_buf = decltype(ld_buf_c)::value;
+      constexpr int READS = TM + TN, FIRST = q * LOADS / SL, AUX = READS + (q + 1) * LOADS / SL - FIRST, MF = TM * TN;
+      constexpr int PER = (AUX + MF - 1) / MF > 2 ? (AUX + MF - 1) / MF : 2;
+      unrolled<MF>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value, tm = m / TN, tn = m % TN;
+        acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fb[set][tn]),
+                                                              __builtin_bit_cast(bf16x8_t, fa[set][tm]), acc[tm][tn], 0, 0, 0);
+        unrolled<PER>([&](auto a_c) {
+          constexpr int a = m * PER + decltype(a_c)::value;
+          if constexpr (a < READS) read_one(buf, kk, set ^ 1, a);
+          else if constexpr (a < AUX) issue_load(ld_buf, FIRST + a - READS);
+        });
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      if constexpr (q == SL - 1) next_tile();
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      hold_set(set ^ 1);
+    };
+    auto istep = [&](auto u_c) {
+      constexpr int u = decltype(u_c)::value, before = (u + NBUF - 1) % NBUF;
+      unrolled<SL - 1>([&](auto s_c) {
+        constexpr int s = decltype(s_c)::value;
+        slice(std::integral_constant<int, (s & 1)>{}, u_c, std::integral_constant<int, s + 1>{}, std::integral_constant<int, s + 1>{},
+              std::integral_constant<int, before>{});
+      });
+      wait_and_meet<AHEAD>();
+      slice(std::integral_constant<int, ((SL - 1) & 1)>{}, std::integral_constant<int, (u + 1) % NBUF>{}, std::integral_constant<int, 0>{},
+            std::integral_constant<int, 0>{}, u_c);
+    };
+#pragma unroll
+    for (int s = 0; s < NBUF - 1; ++s) issue_loads(s);
+#pragma unroll
+    for (int j = 0; j < LOADS / SL; ++j) issue_load(NBUF - 1, j);
+    wait_and_meet<AHEAD + LOADS / SL>();
+#pragma unroll
+    for (int i = 0; i < TM + TN; ++i) read_one(0, 0, 0, i);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_set(0);
+    int kt0 = 0;
+    for (; kt0 + NBUF <= nk; kt0 += NBUF) unrolled<NBUF>(istep);
+    unrolled<NBUF - 1>([&](auto u_c) {
+      if (kt0 + decltype(u_c)::value < nk) istep(u_c);
+    });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile: the epilogue uses their place
   } else {
 #pragma unroll
     for (int s = 0; s < NBUF - 1; ++s)
@@ -2339,12 +2398,14 @@ enum SplitTile : int {
 
 // Tilings of igemm2_kernel with pipelined operand reads
 enum PipeTile : int {
-  kPipe64 = 21,       // 64 x 64
-  kPipe128x64 = 22,   // 128 x 64, eight wavefronts
+  kPipe64 = 21,       // 64 x 64, operand reads pipelined over the steps, four LDS tiles
+  kMix128x64 = 22,    // interleaved, eight wavefronts: 128 x 64, four LDS tiles
+  kMix128 = 23,       // 128 x 128, three (tiling 0 has two, and a second workgroup beside it on its CU)
+  kMix128x192 = 24,   // 128 x 192, three
 };
 
 // the tiling of the same shape that runs where a pipelined one does not exist
-int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : 1; }
+int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : tile_cfg == kMix128x64 ? 1 : 0; }
 
 // The weight-gradient kernel's tile (0 = 128 x 128, 1 = 128 x 64, 2 = 64 x 64) for a tiling number: the same shape where
 // there is one.  How the other kernels walk a tile (steps, LDS tiles, reductions split over wavefronts, the 3x3 patch) has
@@ -2356,12 +2417,14 @@ int wgrad_tile(int tile_cfg) {
     case 10:
     case 11:
     case 12:
+    case kMix128:
+    case kMix128x192:
       return 0;
     case 1:
     case 5:
     case 6:
     case 13:
-    case kPipe128x64:
+    case kMix128x64:
       return 1;
     default:
       return 2;
@@ -2409,8 +2472,8 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
       tile_cfg = 1;
     }
     // 9 / 10: 256 x 256 on eight wavefronts (128 x 64 each), two LDS tiles, plain / rotated loop: for products with a
-    // thousand such tiles or more (65 536 x 4096 x 4096: 1.22 PFLOP/s both, 1.04 for 128 x 128; 8192 x 3072 over 768: 50 us
-    // rotated, 53 plain, 52 for 128 x 128; slower than 128 x 128 on the other layers of the three models, by up to 1.7x)
+    // thousand such tiles or more (65 536 x 4096 x 4096: 1.17 and 1.23 PFLOP/s, 1.03 for 128 x 128; slower than 128 x 128 on
+    // the other layers of the three models, by up to 1.7x)
     if (tile_cfg == 9 || tile_cfg == 10) {
       if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32)
         return tile_cfg == 9 ? launch_cfg2<MODE, 2, 4, 4, 2, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 4, 4, 2, 2, 1>(ctx, a, flops);
@@ -2434,16 +2497,16 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
         return tile_cfg == 6 ? launch_cfg2<MODE, 2, 2, 2, 1, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 1, 1, 2>(ctx, a, flops);
       tile_cfg -= 5;
     }
-    // 21 / 22: operand reads pipelined over the reduction steps (see igemm2_kernel), four tiles in LDS: 64 x 64, and
-    // 128 x 64 on eight wavefronts.  (128 x 128 with two tiles, 229 registers: 43.2 us for 8192 x 768 over 3072 alone
-    // against 50.6, but the GPT-2 step is 0.2 ms slower with it, beside the weight gradients: not built.)
+    // 21: operand reads pipelined over the steps, 22 - 24: interleaved on eight wavefronts (as tiling 0; see igemm2_kernel)
     if (tile_cfg >= kPipe64 && setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32) {
       if (tile_cfg == kPipe64) return launch_cfg2<MODE, 2, 2, 1, 1, 4, 2>(ctx, a, flops);
-      return launch_cfg2<MODE, 4, 2, 1, 1, 4, 2>(ctx, a, flops);
+      if (tile_cfg == kMix128) return launch_cfg2<MODE, 4, 2, 1, 2, 3, 1>(ctx, a, flops);
+      if (tile_cfg == kMix128x192) return launch_cfg2<MODE, 4, 2, 1, 3, 3, 1>(ctx, a, flops);
+      return launch_cfg2<MODE, 4, 2, 1, 1, 4, 1>(ctx, a, flops);
     }
     if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32 && tile_cfg >= 0 && tile_cfg <= 2) {
       if (tile_cfg == 0)
-        return setting == 3 ? launch_cfg2<MODE, 2, 2, 2, 2, 3>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 2, 2, 2>(ctx, a, flops);
+        return setting == 3 ? launch_cfg2<MODE, 4, 2, 1, 2, 3, 1>(ctx, a, flops) : launch_cfg2<MODE, 4, 2, 1, 2, 2, 1>(ctx, a, flops);
       if (tile_cfg == 1)
         return setting == 2 ? launch_cfg2<MODE, 2, 2, 2, 1, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 2, 1, 3>(ctx, a, flops);
       return setting == 2 ? launch_cfg2<MODE, 2, 2, 1, 1, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 2, 1, 1, 3>(ctx, a, flops);
@@ -2474,7 +2537,7 @@ double conv_flops(const ConvShape& s, int Ho, int Wo) {
 // rows of the workgroup tile of a tiling number (5 = the 3x3 patch kernel, or tiling 1 where it does not fit)
 int tile_rows(int tile_cfg) {
   if (tile_cfg == 9 || tile_cfg == 10) return 256;
-  if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 ? 64 : 128;
+    if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 ? 64 : 128;
   if (tile_cfg >= kSplit32) return tile_cfg <= kSplit32Deep ? 32 : 64;
   if (tile_cfg >= 11 && tile_cfg <= 14) return tile_cfg == 14 ? 64 : 128;
   return (tile_cfg == 5 || tile_cfg == 6) ? 128 : tile_cfg >= 2 ? 64 : 128;
@@ -2531,14 +2594,12 @@ int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
 //   start + round * r + steps * max(alone, shared * r) + store * (outputs / 10^6)
 // with r = workgroups per compute unit, rounded up, and steps = 64-element reduction steps.  `alone` is a step of one
 // workgroup on a CU (a chain of latencies), `shared` what a step costs each of several that share the CU's operand
-// path; `round` is the epilogue, which those take in turn.  The constants are least-squares fits (mean error 3-7 %) to
-// kernel times of 280 products and convolutions: the projections of GPT-2 at 128-8192 rows and of Swin-B at 2-32
-// images forward, ResNet's 1x1 and 3x3 layers at 1-64 images (forward with batch sums, inference epilogue) for the
-// first table; ResNet's data gradients with the BatchNorm sums, whose epilogue reads two more tensors, for the second.
-// Against the fastest of ALL tilings, each timed alone on 488 such launches: the choice is 2 % slower on average on the
-// projections, forward (worst 1.18) and data gradient (1.19), 2 % on ResNet's data gradients with the sums (1.17), and 5-6 %
-// on its forward convolutions.  Those are worst where the output has 64 channels (stage 1 at 16-64 images: 1.2-1.45, 56 x 56
-// x 256 -> 64 at 20 images 12.3 us as 128 x 128 and 8.5 as 64 x 64): the columns a tile has beyond the output are not priced.
+// path; `round` is the epilogue, which those take in turn.  The constants are least-squares fits (mean error 3-8 %) to
+// 556 different convolutions where they stand in a step or request, one launch at a time (operands as cold or warm as their
+// producers leave them; 3 us of event among it), each with every tiling: ResNet-152 at 1-64 images, GPT-2 at 512-8192
+// tokens, Swin-B at 3-32 images; the second table for ResNet's data gradients with the BatchNorm sums, whose epilogue
+// reads two more tensors.  (Fits to launches repeated on warm operands prefer large tiles: a request of 24 images took
+// 2437 us with them, 2098 with these.)  Against the fastest of all tilings per launch, summed over a step or request: 1-2 %, one image 3.
 // Tilings without an entry (3, 6, 7, 11, kSplit64, kSplit64Pair, kSplit64x32Deep: for callers that ask, and for tuners) are
 // the fastest on some launches, by 1 % on average and 9 % at most.
 struct TileCost {
@@ -2546,24 +2607,21 @@ struct TileCost {
   float start, round, alone, shared, store;
 };
 const TileCost kPlainCost[] = {
-    {0, 128, 128, 3.72f, 2.39f, 0.596f, 0.377f, 0.05f},  {1, 128, 64, 3.69f, 1.28f, 0.377f, 0.243f, 0.24f},
-    {2, 64, 64, 3.51f, 0.64f, 0.261f, 0.158f, 0.14f},    {5, 128, 64, 0.93f, 4.74f, 0.267f, 0.067f, 0.47f},
-    {12, 128, 128, 4.48f, 0.88f, 0.798f, 0.474f, 0.20f}, {13, 128, 64, 4.47f, 0.15f, 0.495f, 0.347f, 0.35f},
-    {14, 64, 64, 3.72f, 0.00f, 0.391f, 0.235f, 0.40f},   {kPipe64, 64, 64, 3.43f, 1.05f, 0.199f, 0.145f, 0.40f},
-    {kPipe128x64, 128, 64, 2.75f, 2.21f, 0.108f, 0.262f, 0.48f},
-    {kSplit32, 32, 32, 3.28f, 0.21f, 0.092f, 0.079f, 2.14f},
-    {kSplit32Deep, 32, 32, 3.47f, 0.07f, 0.075f, 0.082f, 3.11f},
-    {kSplit64x32, 64, 32, 3.46f, 0.19f, 0.147f, 0.127f, 1.27f}};
+    {0, 128, 128, 6.49f, 0.18f, 0.893f, 0.491f, 0.61f}, {1, 128, 64, 6.69f, 0.03f, 0.419f, 0.308f, 0.88f},
+    {2, 64, 64, 6.39f, 0.00f, 0.343f, 0.209f, 0.68f}, {5, 128, 64, 4.96f, 1.67f, 0.313f, 0.133f, 1.40f},
+    {12, 128, 128, 7.89f, 0.00f, 1.073f, 0.602f, 0.37f}, {13, 128, 64, 6.82f, 0.00f, 0.640f, 0.407f, 0.44f},
+    {14, 64, 64, 6.44f, 0.00f, 0.598f, 0.265f, 0.41f}, {kSplit32, 32, 32, 6.13f, 0.00f, 0.108f, 0.114f, 2.05f},
+    {kSplit32Deep, 32, 32, 5.70f, 0.00f, 0.148f, 0.117f, 3.12f}, {kSplit64x32, 64, 32, 6.05f, 0.00f, 0.208f, 0.160f, 1.53f},
+    {kPipe64, 64, 64, 6.24f, 0.00f, 0.264f, 0.194f, 1.40f}, {kMix128x64, 128, 64, 5.60f, 1.22f, 0.336f, 0.340f, 0.83f},
+    {kMix128, 128, 128, 5.74f, 1.31f, 0.542f, 0.493f, 0.72f}, {kMix128x192, 128, 192, 5.38f, 3.00f, 0.677f, 0.639f, 0.53f}};
 const TileCost kSumsCost[] = {
-    {0, 128, 128, 5.71f, 2.89f, 0.629f, 0.424f, 0.40f},  {1, 128, 64, 4.73f, 2.32f, 0.413f, 0.280f, 0.26f},
-    {2, 64, 64, 4.58f, 1.30f, 0.285f, 0.184f, 0.25f},    {5, 128, 64, 1.28f, 6.10f, 0.266f, 0.067f, 0.55f},
-    {12, 128, 128, 6.18f, 1.64f, 0.818f, 0.501f, 0.55f}, {13, 128, 64, 5.57f, 1.10f, 0.528f, 0.363f, 0.31f},
-    {14, 64, 64, 4.79f, 0.70f, 0.408f, 0.242f, 0.47f},   {kPipe64, 64, 64, 4.09f, 1.97f, 0.225f, 0.148f, 0.55f},
-    {kPipe128x64, 128, 64, 2.69f, 5.40f, 0.272f, 0.291f, 0.57f},
-    {kSplit32, 32, 32, 3.44f, 0.48f, 0.108f, 0.087f, 3.96f},
-    {kSplit32Deep, 32, 32, 4.20f, 0.38f, 0.062f, 0.082f, 5.42f},
-    {kSplit64x32, 64, 32, 4.16f, 0.44f, 0.168f, 0.134f, 2.81f}};
-
+    {0, 128, 128, 6.87f, 3.59f, 0.830f, 0.404f, 0.69f}, {1, 128, 64, 6.60f, 1.70f, 0.430f, 0.290f, 0.65f},
+    {2, 64, 64, 6.41f, 0.85f, 0.364f, 0.188f, 0.53f}, {5, 128, 64, 4.70f, 4.68f, 0.294f, 0.088f, 0.58f},
+    {12, 128, 128, 8.06f, 4.67f, 0.904f, 0.420f, 0.31f}, {13, 128, 64, 8.07f, 0.95f, 0.638f, 0.287f, 0.79f},
+    {14, 64, 64, 7.33f, 0.10f, 0.585f, 0.210f, 1.13f}, {kSplit32, 32, 32, 6.35f, 0.00f, 0.134f, 0.099f, 4.42f},
+    {kSplit32Deep, 32, 32, 5.72f, 1.24f, 0.180f, 0.109f, 0.25f}, {kSplit64x32, 64, 32, 6.71f, 0.26f, 0.213f, 0.150f, 2.36f},
+    {kPipe64, 64, 64, 5.75f, 1.60f, 0.276f, 0.163f, 0.68f}, {kMix128x64, 128, 64, 4.52f, 4.11f, 0.256f, 0.316f, 0.74f},
+    {kMix128, 128, 128, 3.63f, 5.89f, 0.446f, 0.382f, 0.83f}};
 // fp32 where the output has fewer than one and a half 128 x 128 tiles per compute unit: the reduction is split inside the
 // workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 multiplies at 1/16 of the bf16 rate, so it
 // gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us).  -1: none of them.
@@ -2596,6 +2654,7 @@ struct TileQuery {
   int dtype, gemm_m, gemm_n, gemm_k, in_c, taps;
   bool patch;   // the 3x3 patch kernel fits
   bool sums;    // data gradient with the BatchNorm sums in its epilogue
+  bool dgrad;
 };
 int heuristic_tile(int asked, const TileQuery& q) {
   if (!direct_tile_fits(q.dtype, q.in_c, q.taps)) {
@@ -2603,14 +2662,27 @@ int heuristic_tile(int asked, const TileQuery& q) {
     return split >= 0 ? split : pick_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k);
   }
   const float steps = static_cast<float>(q.gemm_k) / 64.f, store = static_cast<float>(q.gemm_m) * q.gemm_n * 1e-6f;
-  const bool large = tiles_for(q.gemm_m, q.gemm_n, 128, 128) >= 384;
+  const bool large = q.gemm_n > 64 && tiles_for(q.gemm_m, q.gemm_n, 128, 128) >= 384;
   int best = 2;
   float best_us = INFINITY;
-  for (const TileCost& t : q.sums ? kSumsCost : kPlainCost) {
+  const TileCost* const costs = q.sums ? kSumsCost : kPlainCost;
+  const size_t entries = q.sums ? std::size(kSumsCost) : std::size(kPlainCost);
+  for (size_t i = 0; i < entries; ++i) {
+    const TileCost& t = costs[i];
     // one and a half 128 x 128 tiles per compute unit or more, beside a second lane of weight gradients: smaller tiles
     // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 step of 8 x 1024 tokens 13.34 ms
     // without this line, 12.19 with it; 3 x 777 tokens and Swin-B of 32 images the same either way)
     if (!q.sums && large && t.bm * t.bn < 128 * 128) continue;
+    // 128 x 192 has a CU to itself: over a short reduction its epilogue and the next tile's first trip to memory are in
+    // nobody's shadow, where the grid has several rounds (8192 x 3072 over 768 54.8 us, 47.5 as 128 x 128; 2048 x 3072 15.7
+    // and 15.9; over 3072, 8192 x 768: 38.4 and 43.6)
+    if (!q.sums && large && t.cfg == kMix128x192 && q.gemm_k < 1024) continue;
+    // A transformer's data gradients run beside weight gradients that hold 64 KB of LDS and half of every SIMD's registers:
+    // there the 128 x 128 tilings on eight wavefronts lose to 128 x 128 and 128 x 64 on four (Swin-B step of 32 images 10.03 ms
+    // with them, 9.92 without; GPT-2 8 x 1024 12.03 and 11.96, 8 x 256 and 3 x 777 the same)
+    if (q.dgrad && !q.sums && (t.cfg == 0 || t.cfg == kMix128)) continue;
+    // at least half of the tile's columns lie in the output (56 x 56 x 256 -> 64, 20 images: 11.0 us as 128 x 128, 9.3 as 128 x 64)
+    if (t.bn >= 2 * q.gemm_n && t.bn > 32) continue;
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
@@ -2727,7 +2799,7 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false});
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false});
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
@@ -2747,7 +2819,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int gemm_m = s.N * Ho * Wo;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false});
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false});
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2755,7 +2827,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
 
 int conv2d_dgrad_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   const int gemm_m = s.N * s.H * s.W;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S, patch_kernel_fits(s, s.K), true});
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.C, s.R * s.S * s.K, s.K, s.R * s.S, patch_kernel_fits(s, s.K), true, true});
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;
@@ -2799,7 +2871,7 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr});
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr, true});
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);

@@ -297,7 +297,7 @@ class ResNetEngine(EngineBase):
         """The fastest tiling, or a larger tile that is within `tile_margin` of it: alone on the chip a small tile
         can win by a few percent and still lose in the step, where it shares L2 bandwidth with the weight gradients
         (a larger tile fetches fewer operand bytes per flop)."""
-        area = lambda cfg: {0: 4, 11: 4, 12: 4, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2, 22: 2, 15: 0.25, 16: 0.25, 17: 0.5, 20: 0.5}.get(cfg, 1)
+        area = lambda cfg: {0: 4, 11: 4, 12: 4, 23: 4, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2, 22: 2, 15: 0.25, 16: 0.25, 17: 0.5, 20: 0.5}.get(cfg, 1)
         best = min(timings.values())
         ok = [cfg for cfg, t in timings.items() if t <= best * (1.0 + self.tile_margin)]
         return min(ok, key=lambda cfg: (-area(cfg), timings[cfg]))
@@ -346,14 +346,14 @@ class ResNetEngine(EngineBase):
         # 6 / 7 = tilings 1 / 2 with two LDS tiles in flight (more workgroups per CU)
         # 11 - 14 = 128 x 128 (three / two LDS tiles), 128 x 64, 64 x 64 with 32-element reduction steps: half the LDS
         # per workgroup, which the wide, shallow products of the first two stages prefer
-        # 21 / 22 = 64 x 64, 128 x 64 with operand reads pipelined over the steps
-        cfgs = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14, 21, 22) if c.cout > 64 else (1, 2, 3, 6, 7, 13, 14, 21, 22)) + patch
+        # 21 = 64 x 64 with operand reads pipelined over the steps, 22 / 23 = 128 x 64, 128 x 128 interleaved
+        cfgs = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14, 21, 22, 23) if c.cout > 64 else (1, 2, 3, 6, 7, 13, 14, 21, 22)) + patch
         # 15 - 20 = the reduction split over the wavefronts of a workgroup: only where a 64 x 64 tiling cannot fill the chip
         few = lambda pixels, channels: (15, 16, 17, 18, 19) if -(-pixels // 64) * -(-channels // 64) <= 512 else ()
         cfgs += few(n * ho * wo, c.cout)
         t_f = {cfg: self._time_program(fwd(cfg)) / reps for cfg in cfgs}
         tf = self._pick_tiling(t_f)
-        cfgs_d = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14, 21, 22) if c.cin_store > 64 else (1, 2, 3, 6, 7, 13, 14, 21, 22)) + patch
+        cfgs_d = ((0, 1, 2, 3, 6, 7, 11, 12, 13, 14, 21, 22, 23) if c.cin_store > 64 else (1, 2, 3, 6, 7, 13, 14, 21, 22)) + patch
         cfgs_d += few(n * h * w, c.cin_store)
         t_d = {cfg: self._time_program(dgrad(cfg)) / reps for cfg in cfgs_d} if c.cin_store >= 64 else {-1: 0.0}
         td = self._pick_tiling(t_d)
