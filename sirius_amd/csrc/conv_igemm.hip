@@ -2893,13 +2893,17 @@ int64_t conv2d_wgrad_workspace_bytes(const ConvShape& s, int dtype, int splits) 
   return static_cast<int64_t>(splits) * (static_cast<int64_t>(s.K) * s.R * s.S * s.C + s.K) * 4;
 }
 
-// tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups
-// (TCH_WGRAD_BIG_TILE_WGS: another count)
-bool wgrad_big_tile(int gemm_m, int gemm_n, int64_t splits) {
-  static const int from = [] {
+// tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups, in fp32 1024
+// (TCH_WGRAD_BIG_TILE_WGS: another count).  An fp32 gradient is bound by the matrix pipes: 144 workgroups of 128 x 128 use
+// those of 144 compute units, and their 36 KB of LDS (64 x 64: 20) keep main-lane workgroups away.  In the step, from 128 /
+// 256 / 512 / 1024 / 2000 on / never: GPT-2 2 x 256 6.48 / 6.39 / 6.22 / 6.22 / 6.19 / 6.25 ms, 1 x 512 7.34 / 6.98 / 6.88 / 6.88 /
+// 6.86 / 6.89, 8 x 512 31.48 / 31.50 / 31.56 / 31.50 / 31.94 / 31.88.
+bool wgrad_big_tile(int dtype, int gemm_m, int gemm_n, int64_t splits) {
+  static const int asked = [] {
     const char* e = getenv("TCH_WGRAD_BIG_TILE_WGS");
-    return e && atoi(e) > 0 ? atoi(e) : 128;
+    return e && atoi(e) > 0 ? atoi(e) : 0;
   }();
+  const int from = asked ? asked : dtype == kF32 ? 1024 : 128;
   return gemm_m >= 128 && gemm_n >= 128 && tiles_for(gemm_m, gemm_n, 128, 128) * splits >= from;
 }
 
@@ -2941,7 +2945,7 @@ int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
     const int64_t steps = ((pixels + want - 1) / want + BK - 1) / BK;
     const int64_t splits = (pixels + steps * BK - 1) / (steps * BK);
     if (splits != want) continue;   // the same as a smaller count
-    const bool big = wgrad_big_tile(gemm_m, gemm_n, splits);
+    const bool big = wgrad_big_tile(dtype, gemm_m, gemm_n, splits);
     const Cost& c = cost[dtype == kBF16][big];
     const int side = big ? 128 : 64;
     const float r = static_cast<float>((tiles_for(gemm_m, gemm_n, side, side) * splits + 255) / 256);
@@ -2992,7 +2996,7 @@ int conv2d_wgrad(Context* ctx, int dtype, const ConvShape& s, const void* x, con
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
   if (tile_cfg < 0) {
-    tile_cfg = wgrad_big_tile(a.gemm_m, a.gemm_n, splits) ? 0 : 2;
+    tile_cfg = wgrad_big_tile(dtype, a.gemm_m, a.gemm_n, splits) ? 0 : 2;
   }
   int rc = dtype == kBF16 ? launch_wgrad<bf16>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo))
                           : launch_wgrad<float>(ctx, a, tile_cfg, conv_flops(s, a.Ho, a.Wo));
