@@ -13,7 +13,7 @@ def test_tile(dtype, K, C, splits, side):
     rec = R.Recorder()
     try:
         rec.begin()
-        check(lib().tch_conv2d_wgrad(rec.ctx, dtype, *[R.address(i) for i in range(4)], splits, 0, 512, 1, 1, C, K, 1, 1, 1, 0, -1, 0))
+        check(lib().tch_conv2d_wgrad(rec.ctx, dtype, *[R.address(i) for i in range(4)], splits, 0, 64 * splits, 1, 1, C, K, 1, 1, 1, 0, -1, 0))
         name, wgs, _ = rec.end()[0]
     finally:
         rec.close()
