@@ -378,8 +378,11 @@ __global__ __launch_bounds__(256) void bn_apply_cols_kernel(ApplyArgs p) {
 // same fixed order, from L2: row_blocks x 512 bytes), then applies.  The workgroups of slab 0 also write the
 // per-channel outputs (saved statistics, running statistics / dgamma, dbeta).
 // At small batches the launch is one chain of latencies, so everything that does not depend on the sums is requested
-// ahead of them (the channel's parameters, the thread's first row): the chain is one trip to memory instead of three
-// (20 images, 14x14 stage: forward 6.1 -> 5.8 us per launch, backward 7.4 -> 6.1).
+// ahead of them (the channel's parameters, the thread's first two rows): the chain is one trip to memory instead of three.
+// Two rows ahead and 64 row blocks per trip of the sums take 82 / 90 registers, which leaves room beside the second lane's
+// weight gradients; steps of 20 / 2 x 16 / 64 images, and 4 in fp32, in ms: one row and 128 row blocks 7.25 / 13.95 / 13.92 / 7.23,
+// two and 128 (126 registers) 7.24 / 13.93 / 14.06 / 7.09, two and 64 7.13 / 13.73 / 13.91 / 6.93, two and 32 7.12 / 13.73 / 13.96 /
+// 6.91, four and 64 (117) 7.20 / 13.84 / 13.89 / 7.03, one and 64 7.11 / 13.81 / 14.21 / 7.04.
 constexpr int kFusedCols = 64;
 constexpr int kFusedMaxRowBlocks = 256;
 
@@ -436,24 +439,30 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
       }
     }
   }
-  // the first row of this thread (a thread beyond the slab fetches the slab's last row and stores nothing)
-  Chunk fa, fb = zero_chunk();
-  {
-    const int64_t r = r0 + ty < r1 ? r0 + ty : r1 - 1;
-    fa.u = static_cast<const uint4*>(p.a)[r * cc + col_chunk];
-    if (has_b) fb.u = static_cast<const uint4*>(p.b)[r * cc + col_chunk];
-  }
+  // the next U rows of this thread (a row beyond the slab stands for the slab's last row and is not stored)
+  constexpr int U = 2;
+  auto request = [&](int64_t r, Chunk (&ca)[U], Chunk (&cb)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t row = r + u * RPP < r1 ? r + u * RPP : r1 - 1;
+      ca[u].u = static_cast<const uint4*>(p.a)[row * cc + col_chunk];
+      cb[u] = zero_chunk();
+      if (has_b) cb[u].u = static_cast<const uint4*>(p.b)[row * cc + col_chunk];
+    }
+  };
+  Chunk fa[U], fb[U];
+  request(r0 + ty, fa, fb);
   {
     const int pr = tid & 31, part = tid >> 5;
     double s0 = 0.0, q0 = 0.0, s1 = 0.0, q1 = 0.0;
-    constexpr int U = 16;   // 128 row blocks per round trip
+    constexpr int B = 8;   // 64 row blocks per round trip
     // uniform base + 32-bit lane offset: one address register per request
     const float* base = p.partial + static_cast<int64_t>(c0) * 2;
     const uint32_t stride = static_cast<uint32_t>(p.C) * 2;   // floats per row block
-    for (int b = part; b < p.row_blocks; b += 8 * U) {
-      float4 v[U];
+    for (int b = part; b < p.row_blocks; b += 8 * B) {
+      float4 v[B];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < B; ++u) {
         // every request is made (a row block past the end repeats the last one and counts as zero): a
         // conditional request would be a branch of its own
         const int bb = b + 8 * u;
@@ -461,10 +470,10 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
         v[u] = *reinterpret_cast<const float4*>(base + off);
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int u = 0; u < B; ++u)
         if (b + 8 * u >= p.row_blocks) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < B; ++u) {
         // keeps the conversions to fp64 next to their additions (hoisted, they would cost 2 registers per value)
         if (u % 4 == 0) __builtin_amdgcn_sched_barrier(0);
         s0 += v[u].x;
@@ -550,21 +559,21 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
     }
     static_cast<uint4*>(p.out)[i] = float_to_chunk<T>(vo).u;
   };
-  if (r0 + ty < r1) finish((r0 + ty) * cc + col_chunk, fa, fb);
-  // the rest two rows per trip: both rows' chunks are requested before either is used
-  for (int64_t r = r0 + ty + RPP; r < r1; r += 2 * RPP) {
-    const int64_t i0 = r * cc + col_chunk, i1 = i0 + RPP * cc;
-    const bool second = r + RPP < r1;
-    Chunk a0, a1, b0 = zero_chunk(), b1 = zero_chunk();
-    a0.u = static_cast<const uint4*>(p.a)[i0];
-    if (has_b) b0.u = static_cast<const uint4*>(p.b)[i0];
-    a1 = a0;
-    if (second) {
-      a1.u = static_cast<const uint4*>(p.a)[i1];
-      if (has_b) b1.u = static_cast<const uint4*>(p.b)[i1];
+  // U rows ahead: the next ones are requested before these are used
+  for (int64_t r = r0 + ty; r < r1; r += U * RPP) {
+    Chunk na[U], nb[U];
+    const bool more = r + U * RPP < r1;
+    if (more) request(r + U * RPP, na, nb);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (r + u * RPP < r1) finish((r + u * RPP) * cc + col_chunk, fa[u], fb[u]);
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        fa[u] = na[u];
+        fb[u] = nb[u];
+      }
     }
-    finish(i0, a0, b0);
-    if (second) finish(i1, a1, b1);
   }
 }
 
