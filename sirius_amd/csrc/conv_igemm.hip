@@ -800,18 +800,24 @@ __device__ inline void wait_and_meet() {
 // 50 176 34 -> 26; reading a step ahead of its multiplication into a second register set (169 instead of 136
 // registers) gained nothing on top.
 // POINTWISE: x is read at dy's pixels (no tap arithmetic).  BIAS: the launch may be asked for the bias gradient.
-template <int WM, int WN, int TM, int TN>
+// Over up to 60 steps 64 x 64 keeps five tiles in LDS instead of eight: the seven requests of the full ring's start are a good
+// part of such a reduction, and 40 KB leave room for a main-lane workgroup.  Steps of 20 images 7.11 -> 7.06 ms, of 2 x 16 13.67 ->
+// 13.49 (28-56 steps per split), GPT-2 3 x 777, Swin-B of 7 and ResNet of 64 images the same; over 64 steps and more the full
+// ring wins (GPT-2 8 x 256 4.50 ms, 4.55 with five tiles; ResNet of 64 images 13.87 and 14.02).  Three tiles up to 48 steps: 20
+// images 7.01, but Swin-B of 7 images 4.89 for 4.75.
+constexpr int kWgradRing = 65536, kWgradShortRing = 40960, kWgradShortSteps = 60;
+template <int WM, int WN, int TM, int TN, int RING>
 constexpr int wgrad_direct_buffers() {
-  return 65536 / (32 * (WM * TM + WN * TN) * 64);
+  return RING / (32 * (WM * TM + WN * TN) * 64);
 }
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, int RING>
 constexpr int wgrad_direct_lds() {
-  constexpr int ring = wgrad_direct_buffers<WM, WN, TM, TN>() * 32 * (WM * TM + WN * TN) * 64, stage = WM * 32 * (WN * TN * 32 + kStagePad) * 4;
+  constexpr int ring = wgrad_direct_buffers<WM, WN, TM, TN, RING>() * 32 * (WM * TM + WN * TN) * 64, stage = WM * 32 * (WN * TN * 32 + kStagePad) * 4;
   return ring > stage ? ring : stage;
 }
-template <int WM, int WN, int TM, int TN, bool POINTWISE, bool BIAS>
+template <int WM, int WN, int TM, int TN, int RING, bool POINTWISE, bool BIAS>
 __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t id, unsigned char* lds) {
-  constexpr int BKP = 32, NBUF = wgrad_direct_buffers<WM, WN, TM, TN>();
+  constexpr int BKP = 32, NBUF = wgrad_direct_buffers<WM, WN, TM, TN, RING>();
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32, NW = WM * WN;
   constexpr int RA = BM * 2, RB = BN * 2;              // bytes of one pixel row
   constexpr int SA = RA / 16, SB = RB / 16;            // 16-byte slots of it
@@ -1280,14 +1286,14 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_f32_kernel(WgradArgs w) {
   wgrad_body_f32<WM, WN, TM, TN>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs));
 }
 
-template <int WM, int WN, int TM, int TN, bool POINTWISE, bool BIAS>
+template <int WM, int WN, int TM, int TN, int RING, bool POINTWISE, bool BIAS>
 __global__ __launch_bounds__(WM* WN * 64) void wgrad_kernel(WgradArgs w) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[wgrad_direct_lds<WM, WN, TM, TN>()];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[wgrad_direct_lds<WM, WN, TM, TN, RING>()];
   if (blockIdx.x >= w.gemm_wgs) {
     wgrad_passenger(w, reinterpret_cast<double*>(lds));
     return;
   }
-  wgrad_body_direct<WM, WN, TM, TN, POINTWISE, BIAS>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs), lds);
+  wgrad_body_direct<WM, WN, TM, TN, RING, POINTWISE, BIAS>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs), lds);
 }
 
 // The weight gradients of several convolutions in one launch.  `table` holds one argument block per convolution,
@@ -1304,14 +1310,14 @@ struct WgradGroupArgs {
 
 template <typename T, int WM, int WN, int TM, int TN>
 __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs g) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[sizeof(T) == 2 ? wgrad_direct_lds<WM, WN, TM, TN>() : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[sizeof(T) == 2 ? wgrad_direct_lds<WM, WN, TM, TN, kWgradRing>() : 16];
   for (uint32_t gid = xcd_remap(blockIdx.x, gridDim.x); gid < g.entries; gid += gridDim.x) {
     const uint2 e = g.map[gid];
     const IgemmArgs p = g.table[__builtin_amdgcn_readfirstlane(e.x)];
     const uint32_t id = __builtin_amdgcn_readfirstlane(e.y);
     if constexpr (sizeof(T) == 4) wgrad_body_f32<WM, WN, TM, TN>(p, id);
-    else if (p.pointwise) wgrad_body_direct<WM, WN, TM, TN, true, true>(p, id, lds);
-    else wgrad_body_direct<WM, WN, TM, TN, false, true>(p, id, lds);
+    else if (p.pointwise) wgrad_body_direct<WM, WN, TM, TN, kWgradRing, true, true>(p, id, lds);
+    else wgrad_body_direct<WM, WN, TM, TN, kWgradRing, false, true>(p, id, lds);
     __syncthreads();   // the next entry's operand tiles overwrite what the epilogue staged in LDS
   }
 }
@@ -2243,6 +2249,12 @@ double conv_bytes(const IgemmArgs& a, int eb) {
   return ((MODE == kFwd ? x : y) + w + out * extra) * eb + out * (a.out_f32 ? 4 : eb);
 }
 
+template <int WM, int WN, int TM, int TN, int RING>
+void (*wgrad_direct_kernel(const IgemmArgs& a))(WgradArgs) {
+  if (a.pointwise) return a.dbias ? wgrad_kernel<WM, WN, TM, TN, RING, true, true> : wgrad_kernel<WM, WN, TM, TN, RING, true, false>;
+  return a.dbias ? wgrad_kernel<WM, WN, TM, TN, RING, false, true> : wgrad_kernel<WM, WN, TM, TN, RING, false, false>;
+}
+
 template <typename T, int MODE, int WM, int WN, int TM, int TN>
 int launch_cfg(Context* ctx, IgemmArgs& a, double flops) {
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
@@ -2279,10 +2291,10 @@ int launch_cfg(Context* ctx, IgemmArgs& a, double flops) {
     void (*kernel)(WgradArgs);
     if constexpr (sizeof(T) == 4)
       kernel = wgrad_f32_kernel<WM, WN, TM, TN>;
-    else if (a.pointwise)
-      kernel = a.dbias ? wgrad_kernel<WM, WN, TM, TN, true, true> : wgrad_kernel<WM, WN, TM, TN, true, false>;
+    else if (TM * TN == 1 && a.k_per_split <= 32 * kWgradShortSteps)
+      kernel = wgrad_direct_kernel<WM, WN, TM, TN, TM * TN == 1 ? kWgradShortRing : kWgradRing>(a);
     else
-      kernel = a.dbias ? wgrad_kernel<WM, WN, TM, TN, false, true> : wgrad_kernel<WM, WN, TM, TN, false, false>;
+      kernel = wgrad_direct_kernel<WM, WN, TM, TN, kWgradRing>(a);
     return launch(ctx, kernel, dim3(blocks), block, w, igemm_name<T, MODE, WM, WN, TM, TN>(), flops, 0, bytes);
   } else
     return launch(ctx, igemm_kernel<T, MODE, WM, WN, TM, TN>, grid, block, a, igemm_name<T, MODE, WM, WN, TM, TN>(),
