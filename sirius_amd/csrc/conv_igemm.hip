@@ -1631,7 +1631,11 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     // a part of the direct loads goes out, an instruction or two behind every MFMA, so that nothing but the barrier
     // leaves the matrix pipe without work.  The barrier that hands over tile kt+1 stands in front of tile kt's last slice,
     // which is in registers by then, as is everything else of tile kt: its buffer takes tile kt+NBUF from there on.
-    constexpr int SL = KS / 16;
+    // With two buffers that tile is waited for SL slices later, and what goes out behind the last slices has no time to
+    // land: it all goes out behind the first half of them (65 536 x 4096 x 4096 as 256 x 256 1808 us when spread over all
+    // four, 1677 over two, 1754 in one; GPT-2's output head at 8192 rows 896, 842, 885; 12 544 x 256 over 1024 as 128 x 128
+    // 14.9, 14.0, 14.5).
+    constexpr int SL = KS / 16, LOAD_SL = NBUF == 2 ? SL / 2 : SL;
     uint4_t fa[2][TM], fb[2][TN];
     uint32_t a_sl[SL], b_sl[SL];
 #pragma unroll
@@ -1657,7 +1661,8 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
     auto slice = [&](auto set_c, auto buf_c, auto kk_c, auto q_c, auto ld_buf_c) {
       constexpr int set = decltype(set_c)::value, buf = decltype(buf_c)::value, kk = decltype(kk_c)::value;
       constexpr int q = decltype(q_c)::value, ld_buf = decltype(ld_buf_c)::value;
-      constexpr int READS = TM + TN, FIRST = q * LOADS / SL, AUX = READS + (q + 1) * LOADS / SL - FIRST, MF = TM * TN;
+      constexpr int READS = TM + TN, FIRST = (q < LOAD_SL ? q : LOAD_SL) * LOADS / LOAD_SL, MF = TM * TN;
+      constexpr int AUX = READS + (q < LOAD_SL ? (q + 1) * LOADS / LOAD_SL - FIRST : 0);
       constexpr int PER = (AUX + MF - 1) / MF > 2 ? (AUX + MF - 1) / MF : 2;
       unrolled<MF>([&](auto m_c) {
         constexpr int m = decltype(m_c)::value, tm = m / TN, tn = m % TN;
@@ -1670,7 +1675,7 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
         });
         __builtin_amdgcn_sched_barrier(0);
       });
-      if constexpr (q == SL - 1) next_tile();
+      if constexpr (q == LOAD_SL - 1) next_tile();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       hold_set(set ^ 1);
     };
@@ -1688,8 +1693,8 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 #pragma unroll
     for (int s = 0; s < NBUF - 1; ++s) issue_loads(s);
 #pragma unroll
-    for (int j = 0; j < LOADS / SL; ++j) issue_load(NBUF - 1, j);
-    wait_and_meet<AHEAD + LOADS / SL>();
+    for (int j = 0; j < LOADS / LOAD_SL; ++j) issue_load(NBUF - 1, j);
+    wait_and_meet<AHEAD + LOADS / LOAD_SL>();
 #pragma unroll
     for (int i = 0; i < TM + TN; ++i) read_one(0, 0, 0, i);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -2549,7 +2554,7 @@ double conv_flops(const ConvShape& s, int Ho, int Wo) {
 // rows of the workgroup tile of a tiling number (5 = the 3x3 patch kernel, or tiling 1 where it does not fit)
 int tile_rows(int tile_cfg) {
   if (tile_cfg == 9 || tile_cfg == 10) return 256;
-    if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 ? 64 : 128;
+  if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 ? 64 : 128;
   if (tile_cfg >= kSplit32) return tile_cfg <= kSplit32Deep ? 32 : 64;
   if (tile_cfg >= 11 && tile_cfg <= 14) return tile_cfg == 14 ? 64 : 128;
   return (tile_cfg == 5 || tile_cfg == 6) ? 128 : tile_cfg >= 2 ? 64 : 128;
