@@ -271,9 +271,8 @@ constexpr int storing_threads() {
 // lanes write float4 groups into the staging tile [WM*32][BN + pad], then every
 // thread takes E consecutive columns of one row and hands them to `fin` together with the
 // number of the visit (tm * ITERS + it, a compile-time constant after unrolling).
-template <typename T, int WM, int WN, int TM, int TN, typename Fin>
+template <int E, int WM, int WN, int TM, int TN, typename Fin>
 __device__ inline void staged_epilogue(f32x16_t (&acc)[TM][TN], float* stage, int tid, Fin fin) {
-  constexpr int E = Elem<T>::kPerChunk;
   constexpr int BN = WN * TN * 32;
   constexpr int NT = WM * WN * 64;
   constexpr int LD = BN + kStagePad;
@@ -561,10 +560,24 @@ struct TileEpilogue {
     if constexpr (EARLY) request(p, tid, m0, n0);
   }
   __device__ inline void finish(const IgemmArgs& p, f32x16_t (&acc)[TM][TN], float* stage, int tid, int m0, int n0, int tile_m) {
+    // Nothing but fp32 outputs of a bf16 product (an output head): four columns per thread instead of the eight of a bf16 chunk,
+    // so that the lanes of a store lie side by side.  Two stores of every other 16 bytes fill each memory line in two
+    // goes (8192 x 50304 over 768, 256 x 256: 842 us with them, 801 so; 2048 rows 234 and 219).
+    // Only for the 256 x 256 tile, which large products get; the kernels of the smaller tiles keep their registers.
+    if constexpr (MODE == kFwd && sizeof(T) == 2 && WM * TM * WN * TN >= 64) {
+      if (p.out_f32 && !p.scale && !p.bias && !p.add && !p.relu_out && !p.stats && !p.stat_acc) {
+        staged_epilogue<4, WM, WN, TM, TN>(acc, stage, tid, [&](int, int tr, int tc, const float* v) {
+          const int row = m0 + tr, col = n0 + tc;
+          if (row < p.gemm_m && col < p.gemm_n)
+            store_floats<4>(static_cast<float*>(p.out) + static_cast<int64_t>(row) * p.gemm_n + col, v);
+        });
+        return;
+      }
+    }
     if constexpr (!EARLY) request(p, tid, m0, n0);
     finish_walk<T, MODE, BN, NTE, NT, VISITS, ITERS, WM * 32 * (BN + kStagePad) * 4>(
         p, operands, stage, tid, m0, n0, tile_m, [&](int visit) { return row_of(tid, visit); },
-        [&](auto fin) { staged_epilogue<T, WM, WN, TM, TN>(acc, stage, tid, fin); });
+        [&](auto fin) { staged_epilogue<Elem<T>::kPerChunk, WM, WN, TM, TN>(acc, stage, tid, fin); });
   }
 };
 
@@ -1039,7 +1052,7 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
   float* out = static_cast<float*>(p.out);
   if (p.splits > 1) out += static_cast<int64_t>(split) * p.gemm_m * p.gemm_n;
   const bool accumulate = p.splits == 1 && p.accumulate;
-  staged_epilogue<bf16, WM, WN, TM, TN>(acc, reinterpret_cast<float*>(lds), tid, [&](int, int tr, int tc, float* v) {
+  staged_epilogue<Elem<bf16>::kPerChunk, WM, WN, TM, TN>(acc, reinterpret_cast<float*>(lds), tid, [&](int, int tr, int tc, float* v) {
     const int row = m0 + tr, col = n0 + tc;
     if (row >= p.gemm_m || col >= p.gemm_n) return;
     float* dst = out + static_cast<int64_t>(row) * p.gemm_n + col;
@@ -1225,7 +1238,7 @@ __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) 
   float* out = static_cast<float*>(p.out);
   if (p.splits > 1) out += static_cast<int64_t>(split) * p.gemm_m * p.gemm_n;
   const bool accumulate = p.splits == 1 && p.accumulate;
-  staged_epilogue<T, WM, WN, TM, TN>(acc, reinterpret_cast<float*>(lds), tid, [&](int, int tr, int tc, float* v) {
+  staged_epilogue<Elem<T>::kPerChunk, WM, WN, TM, TN>(acc, reinterpret_cast<float*>(lds), tid, [&](int, int tr, int tc, float* v) {
     const int row = m0 + tr, col = n0 + tc;
     if (row >= p.gemm_m || col >= p.gemm_n) return;
     float* dst = out + static_cast<int64_t>(row) * p.gemm_n + col;
