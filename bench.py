@@ -33,9 +33,9 @@ HANDOVER_PAGE_MB = 128
 PROFILE_FILE = "profiles/resnet152_bf16_bs64_step_kernel_stats_and_traffic.txt"
 MEASURED_TRAFFIC_MIB = {
     "wgrad_kernel<bf16,64x64>": 64.44 + 5.60,
-    "wgrad_kernel<bf16,128x128>": 34.36 + 17.23,
-    "bn_fin_apply_kernel<bf16,bwd>": 24.40 + 11.91,
-    "bn_fin_apply_kernel<bf16,fwd>": 20.40 + 12.03,
+    "wgrad_kernel<bf16,128x128>": 34.38 + 17.23,
+    "bn_fin_apply_kernel<bf16,bwd>": 24.37 + 11.91,
+    "bn_fin_apply_kernel<bf16,fwd>": 20.39 + 12.03,
 }
 
 
