@@ -12,7 +12,7 @@ using namespace tch;
 
 struct tch_context {
   Context ctx;
-  explicit tch_context(hipStream_t s) : ctx(s) {}
+  explicit tch_context(hipStream_t s) : ctx(s) { ctx.streams_meet = run_at_the_same_time; }
 };
 struct tch_program {
   Program prog;

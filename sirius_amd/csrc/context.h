@@ -119,6 +119,9 @@ struct Program {
   std::vector<LaunchRecord> launches;
 };
 
+// Whether launches on the two streams run at the same time (1) or not (0); -1: cannot tell.  Both are idle when it returns.
+int run_at_the_same_time(hipStream_t a, hipStream_t b);   // lanes.hip
+
 class Context {
  public:
   explicit Context(hipStream_t s) : stream(s) {}
@@ -146,6 +149,8 @@ class Context {
   // for 4.8 ms (Swin-B, 7 images), 5.6 for 4.45 (GPT-2, 8 x 256), 12.7 for 11.9 (8 x 1024).  Which queue a stream has
   // cannot be asked, so two small kernels find out whether they meet; 0.1 ms for a stream that is turned down.
   hipStream_t stream_beside_main();
+  // what it asks about two idle streams: 1 they meet, 0 they do not, -1 cannot tell; any stream will do without it
+  int (*streams_meet)(hipStream_t, hipStream_t) = nullptr;
   // makes the streams a recorded program will use, so that the first replay need not
   void prepare_lanes(const Program& prog);
   // recording state: the lane new launches are stamped with, and whether the next lane-1 launch
