@@ -51,6 +51,23 @@ bool fork_by_stop_event() {
 void set_error(const std::string& msg) { g_error = msg; }
 const char* last_error() { return g_error.c_str(); }
 
+StreamMark::~StreamMark() {
+  if (event) (void)hipEventDestroy(event);
+}
+
+namespace {
+int place_mark(StreamMark* mark, hipStream_t from) {
+  if (!mark->event && hipEventCreateWithFlags(&mark->event, kOrderEvent) != hipSuccess) {
+    mark->event = nullptr;
+    return -5;
+  }
+  return hipEventRecord(mark->event, from) == hipSuccess ? 0 : -5;
+}
+int wait_for_mark(const StreamMark* mark, hipStream_t to) {
+  return mark->event && hipStreamWaitEvent(to, mark->event, 0) == hipSuccess ? 0 : -5;
+}
+}  // namespace
+
 // ---------------------------------------------------------------------------
 // LaunchQueue
 // ---------------------------------------------------------------------------
@@ -90,9 +107,31 @@ void LaunchQueue::submit_dependency(hipStream_t from, hipStream_t to) {
   {
     std::lock_guard<std::mutex> lock(mu_);
     wait_.emplace_back();
-    wait_.back().is_dependency = true;
+    wait_.back().kind = Kind::kDependency;
     wait_.back().on = from;
     wait_.back().to = to;
+  }
+  cv_work_.notify_one();
+}
+
+void LaunchQueue::submit_mark(std::shared_ptr<StreamMark> mark, hipStream_t from) {
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    wait_.emplace_back();
+    wait_.back().kind = Kind::kMark;
+    wait_.back().on = from;
+    wait_.back().mark = std::move(mark);
+  }
+  cv_work_.notify_one();
+}
+
+void LaunchQueue::submit_wait(std::shared_ptr<StreamMark> mark, hipStream_t to) {
+  {
+    std::lock_guard<std::mutex> lock(mu_);
+    wait_.emplace_back();
+    wait_.back().kind = Kind::kWait;
+    wait_.back().to = to;
+    wait_.back().mark = std::move(mark);
   }
   cv_work_.notify_one();
 }
@@ -122,7 +161,7 @@ void LaunchQueue::resume(bool drop_commands) {
   {
     std::lock_guard<std::mutex> lock(mu_);
     if (drop_commands)
-      for (auto it = wait_.begin(); it != wait_.end();) it = (!it->is_sync && !it->is_dependency) ? wait_.erase(it) : it + 1;
+      for (auto it = wait_.begin(); it != wait_.end();) it = it->kind == Kind::kLaunch ? wait_.erase(it) : it + 1;
     suspended_ = false;
     parked_ = false;
   }
@@ -133,7 +172,7 @@ size_t LaunchQueue::clear() {
   std::lock_guard<std::mutex> lock(mu_);
   size_t removed = 0;
   for (auto it = wait_.begin(); it != wait_.end();) {
-    if (!it->is_sync && !it->is_dependency) {
+    if (it->kind == Kind::kLaunch) {
       it = wait_.erase(it);
       ++removed;
     } else {
@@ -148,7 +187,7 @@ int LaunchQueue::synchronize() {
   if (stop_) return 0;
   const uint64_t ticket = next_ticket_++;
   wait_.emplace_back();
-  wait_.back().is_sync = true;
+  wait_.back().kind = Kind::kSync;
   wait_.back().sync_ticket = ticket;
   cv_work_.notify_one();
   cv_done_.wait(lock, [&] { return done_ticket_ >= ticket; });
@@ -161,7 +200,7 @@ size_t LaunchQueue::size() {
   // stream dependencies count: whoever waits for the queue to empty before giving the stream work of
   // its own (copies, read-backs) relies on the trailing dependency of a compute-unit-limited run
   for (auto& it : wait_)
-    if (!it.is_sync) ++n;
+    if (it.kind != Kind::kSync) ++n;
   return n;
 }
 
@@ -288,12 +327,12 @@ void LaunchQueue::worker_loop() {
         if (stop_) break;
         continue;
       }
-      item = wait_.front();
+      item = std::move(wait_.front());
       wait_.pop_front();
-      fork_follows = !item.is_dependency && !item.is_sync && fork_by_stop_event() && !wait_.empty() &&
-                     wait_.front().is_dependency && wait_.front().on == (item.on ? item.on : stream_);
+      fork_follows = item.kind == Kind::kLaunch && fork_by_stop_event() && !wait_.empty() &&
+                     wait_.front().kind == Kind::kDependency && wait_.front().on == (item.on ? item.on : stream_);
     }
-    if (item.is_dependency) {
+    if (item.kind == Kind::kDependency) {
       if (fork_event_ && fork_from_ == item.on && item.to != item.on) {
         // the launch before this entry signals fork_event_ when it ends; as in chain(), the event may be used
         // again once the wait is enqueued
@@ -309,7 +348,12 @@ void LaunchQueue::worker_loop() {
       free_events_.push_back(fork_event_);
       fork_event_ = nullptr;
     }
-    if (item.is_sync) {
+    if (item.kind == Kind::kMark || item.kind == Kind::kWait) {
+      if ((item.kind == Kind::kMark ? place_mark(item.mark.get(), item.on) : wait_for_mark(item.mark.get(), item.to)) != 0)
+        error_.store(static_cast<int>(hipErrorUnknown));
+      continue;
+    }
+    if (item.kind == Kind::kSync) {
       sync_everything();
       {
         std::lock_guard<std::mutex> lock(mu_);
@@ -336,10 +380,6 @@ Context::~Context() {
   if (side) {
     (void)hipStreamSynchronize(side);
     (void)hipStreamDestroy(side);
-  }
-  if (relay) {
-    (void)hipStreamSynchronize(relay);
-    (void)hipStreamDestroy(relay);
   }
   for (hipEvent_t e : events_) (void)hipEventDestroy(e);
 }
@@ -368,14 +408,10 @@ hipStream_t Context::stream_beside_main() {
 }
 
 void Context::prepare_lanes(const Program& prog) {
-  bool second = false, behind = false;
-  for (const LaunchRecord& r : prog.launches) {
-    second = second || (r.fn && r.lane == 1);
-    behind = behind || r.op == kOpJoinBehind;
-  }
+  bool second = false;
+  for (const LaunchRecord& r : prog.launches) second = second || (r.fn && r.lane == 1);
   if (!second || g_reject.load(std::memory_order_acquire)) return;
   if (!side) side = stream_beside_main();
-  if (behind && side && !relay) relay = stream_beside_main();
 }
 
 hipEvent_t Context::next_event() {
@@ -413,6 +449,33 @@ int Context::depend(hipStream_t from, hipStream_t to) {
   return 0;
 }
 
+// lane 0 waits for what lane 1 had been given at the point before, and lane 1 is marked for the next one
+int Context::join_behind() {
+  if (behind_pending) {
+    const auto& mark = behind_marks[behind_turn];
+    if (queue) {
+      queue->submit_wait(mark, main_stream());
+    } else if (wait_for_mark(mark.get(), main_stream()) != 0) {
+      set_error("join behind: hipStreamWaitEvent failed");
+      return -5;
+    }
+    behind_pending = false;
+  }
+  if (!side_dirty) return 0;
+  behind_turn ^= 1;
+  auto& mark = behind_marks[behind_turn];
+  if (!mark) mark = std::make_shared<StreamMark>();
+  hipStream_t lane1 = cu_limit > 0 ? masked_side : side;
+  if (queue) {
+    queue->submit_mark(mark, lane1);
+  } else if (place_mark(mark.get(), lane1) != 0) {
+    set_error("join behind: hipEventRecord failed");
+    return -5;
+  }
+  behind_pending = true;   // side_dirty stays up: lane 0 has not waited for this work yet
+  return 0;
+}
+
 int Context::set_cu_limit(int n_cus) {
   const int total = cu_partition_total();
   if (n_cus <= 0 || (total > 0 && n_cus >= total)) n_cus = 0;
@@ -429,7 +492,7 @@ int Context::set_cu_limit(int n_cus) {
   if (side_dirty && old_side) {
     if (int rc = depend(old_side, new_main)) return rc;
     side_dirty = false;
-    relay_dirty = false;
+    behind_pending = false;
   }
   cu_limit = n_cus;
   main_since_fork_ = true;   // another pair of streams
@@ -456,7 +519,7 @@ int Context::synchronize() {
     return -5;
   }
   side_dirty = false;
-  relay_dirty = false;
+  behind_pending = false;
   return 0;
 }
 
@@ -484,22 +547,7 @@ int Context::dispatch(const LaunchRecord& rec, const LaunchRecord* next) {
     return 0;
   }
   hipStream_t main = main_stream();
-  if (rec.op == kOpJoinBehind) {
-    // depend() makes the event calls here, or queues them in order with the launches behind a launch queue
-    if (relay_dirty) {
-      if (int rc = depend(relay, main)) return rc;
-      relay_dirty = false;
-    }
-    if (side_dirty) {
-      if (!relay && !(relay = stream_beside_main())) {
-        set_error("hipStreamCreateWithFlags failed");
-        return -5;
-      }
-      if (int rc = depend(cu_limit > 0 ? masked_side : side, relay)) return rc;
-      relay_dirty = true;   // side_dirty stays up: lane 0 has not waited for this work yet
-    }
-    return 0;
-  }
+  if (rec.op == kOpJoinBehind) return join_behind();
   if (queue) {
     // behind the preemptible queue the two lanes stay two streams: what would be event calls here are
     // dependencies queued in order with the launches, and the worker makes them when their turn comes
@@ -508,7 +556,7 @@ int Context::dispatch(const LaunchRecord& rec, const LaunchRecord* next) {
         queue->submit_dependency(cu_limit > 0 ? masked_side : side, main);
         side_dirty = false;
       }
-      relay_dirty = false;   // what the relay waits for is older than what lane 0 waits for now
+      behind_pending = false;   // what is marked is older than what lane 0 waits for now
       return 0;
     }
     if (!rec.fn) return 0;
@@ -540,7 +588,7 @@ int Context::dispatch(const LaunchRecord& rec, const LaunchRecord* next) {
       }
       side_dirty = false;
     }
-    relay_dirty = false;
+    behind_pending = false;
     return 0;
   }
   if (rec.lane == 1) {

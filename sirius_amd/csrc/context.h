@@ -26,6 +26,12 @@
 
 namespace tch {
 
+// A point of a stream that another stream is made to wait for at a later time than it is marked.
+struct StreamMark {
+  hipEvent_t event = nullptr;
+  ~StreamMark();
+};
+
 class LaunchQueue {
  public:
   LaunchQueue(hipStream_t stream, int queue_length, int sync_interval);
@@ -40,6 +46,10 @@ class LaunchQueue {
   void submit(const LaunchRecord& rec, hipStream_t on = nullptr);
   // Queued in order with the launches: everything given to `to` afterwards waits for what `from` holds now.
   void submit_dependency(hipStream_t from, hipStream_t to);
+  // The two halves of a dependency, queued in order with the launches like one: `mark` stands for what `from` holds
+  // when its entry's turn comes; everything given to `to` after the other entry waits for that.
+  void submit_mark(std::shared_ptr<StreamMark> mark, hipStream_t from);
+  void submit_wait(std::shared_ptr<StreamMark> mark, hipStream_t to);
   // Erase every launch that has not been handed to the hardware queue yet.
   size_t clear();
   // Wait until everything submitted before this call has finished on the GPU.
@@ -60,12 +70,13 @@ class LaunchQueue {
   uint64_t submitted_total() const { return submitted_total_.load(); }
 
  private:
+  enum class Kind { kLaunch, kSync, kDependency, kMark, kWait };
   struct Item {
-    bool is_sync = false;
-    bool is_dependency = false;
+    Kind kind = Kind::kLaunch;
     uint64_t sync_ticket = 0;
-    hipStream_t on = nullptr;    // launch stream override / dependency source
-    hipStream_t to = nullptr;    // dependency target
+    hipStream_t on = nullptr;    // launch stream override / source of a dependency or a mark
+    hipStream_t to = nullptr;    // target of a dependency or a wait
+    std::shared_ptr<StreamMark> mark;
     LaunchRecord rec;
   };
   struct Logged {
@@ -139,19 +150,24 @@ class Context {
   // everything given to `to` afterwards waits for what `from` holds now (direct or through the queue)
   int depend(hipStream_t from, hipStream_t to);
   bool side_dirty = false;  // lane 1 was given work since the last join
-  // A join one point behind (kOpJoinBehind) goes through a stream of its own that carries nothing but waits:
-  // at such a point it is made to wait for lane 1, and lane 0 waits for it at the next one.
-  hipStream_t relay = nullptr;
-  bool relay_dirty = false;  // the relay waits for lane-1 work that lane 0 has not waited for
+  // A join one point behind (kOpJoinBehind): lane 1 is marked at such a point, and lane 0 waits for the mark at the next
+  // one.  Two marks taken in turn, on lane 1 itself: a third stream that carried the waits from point to point could
+  // share lane 1's hardware queue, where they stood behind every launch lane 1 was given since, and lane 0 waited for
+  // those too (Swin-B, 7 images, nine engines in one process: 4.75-4.81 ms and two at 5.08-5.10; with the marks all nine at 4.67-4.72,
+  // half the event calls of such a point gone).
+  std::shared_ptr<StreamMark> behind_marks[2];
+  int behind_turn = 0;           // the one taken last
+  bool behind_pending = false;   // lane 0 has not waited for it yet
+  int join_behind();
   // A stream whose launches run beside those of `stream`.  A process has four hardware queues (HIP's default) and its streams
   // are dealt out to them in turn, so one stream in a few shares the main lane's queue: as a second lane it overlaps
-  // nothing, as a relay its waits hold the main lane up.  Two engines' worth of streams later the same engine has read 6.4
+  // nothing.  Two engines' worth of streams later the same engine has read 6.4
   // for 4.8 ms (Swin-B, 7 images), 5.6 for 4.45 (GPT-2, 8 x 256), 12.7 for 11.9 (8 x 1024).  Which queue a stream has
   // cannot be asked, so two small kernels find out whether they meet; 0.1 ms for a stream that is turned down.
   hipStream_t stream_beside_main();
   // what it asks about two idle streams: 1 they meet, 0 they do not, -1 cannot tell; any stream will do without it
   int (*streams_meet)(hipStream_t, hipStream_t) = nullptr;
-  // makes the streams a recorded program will use, so that the first replay need not
+  // makes the second lane's stream for a recorded program that will use it, so that the first replay need not
   void prepare_lanes(const Program& prog);
   // recording state: the lane new launches are stamped with, and whether the next lane-1 launch
   // has to wait for lane 0

@@ -1,0 +1,205 @@
+// The two lanes of a program on modelled hardware queues (CPU only; built by tests/test_lanes_model.py with context.cc and the
+// HIP calls below in the place of the runtime).
+//
+// Streams are dealt out to four hardware queues, the least loaded first; a queue runs what its streams hold in the order it
+// was submitted, waits for events included.  Every launch takes the time its argument says, so the moment each one starts
+// is known as soon as it is submitted.
+#include <hip/hip_ext.h>
+#include <hip/hip_runtime.h>
+#include <stdio.h>
+#include <string.h>
+
+#include <algorithm>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "../../sirius_amd/csrc/context.h"
+
+// ---------------------------------------------------------------------------------------------- the modelled runtime
+namespace {
+constexpr int kQueues = 4;
+struct Stream {
+  int queue;
+};
+struct Event {
+  double done = 0.0;   // when the last record of it is reached; one that was never recorded holds nobody up
+};
+struct Span {
+  double start, end;
+};
+struct Launch {        // the argument of every launch
+  int id;
+  double duration;
+};
+std::mutex g_mu;
+double g_time[kQueues];
+int g_load[kQueues];
+std::vector<Span> g_spans;
+int g_streams_alive = 0, g_events_alive = 0;
+
+Stream* as_stream(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
+Event* as_event(hipEvent_t e) { return reinterpret_cast<Event*>(e); }
+
+void reset(const int* load) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  for (int q = 0; q < kQueues; ++q) {
+    g_time[q] = 0.0;
+    g_load[q] = load ? load[q] : 0;
+  }
+  g_spans.clear();
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipStreamCreateWithFlags(hipStream_t* out, unsigned) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  const int q = static_cast<int>(std::min_element(g_load, g_load + kQueues) - g_load);
+  ++g_load[q];
+  ++g_streams_alive;
+  *out = reinterpret_cast<hipStream_t>(new Stream{q});
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  --g_load[as_stream(s)->queue];
+  --g_streams_alive;
+  delete as_stream(s);
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* out, unsigned) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  ++g_events_alive;
+  *out = reinterpret_cast<hipEvent_t>(new Event);
+  return hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* out) { return hipEventCreateWithFlags(out, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  --g_events_alive;
+  delete as_event(e);
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  as_event(e)->done = g_time[as_stream(s)->queue];
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  double& t = g_time[as_stream(s)->queue];
+  t = std::max(t, as_event(e)->done);
+  return hipSuccess;
+}
+hipError_t hipExtLaunchKernel(const void*, dim3, dim3, void** args, size_t, hipStream_t s, hipEvent_t, hipEvent_t stop, int) {
+  std::lock_guard<std::mutex> lock(g_mu);
+  Launch what;
+  memcpy(&what, args[0], sizeof(what));
+  double& t = g_time[as_stream(s)->queue];
+  if (g_spans.size() <= static_cast<size_t>(what.id)) g_spans.resize(static_cast<size_t>(what.id) + 1);
+  g_spans[static_cast<size_t>(what.id)] = Span{t, t + what.duration};
+  t += what.duration;
+  if (stop) as_event(stop)->done = t;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s) {
+  return hipExtLaunchKernel(fn, grid, block, args, lds, s, nullptr, nullptr, 0);
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float*, hipEvent_t, hipEvent_t) { return hipErrorNotSupported; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
+  *st = hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "modelled"; }
+hipError_t hipDeviceGetAttribute(int*, hipDeviceAttribute_t, int) { return hipErrorNotSupported; }
+hipError_t hipExtStreamCreateWithCUMask(hipStream_t* out, uint32_t, const uint32_t*) { return hipStreamCreateWithFlags(out, 0); }
+}  // extern "C"
+
+// ------------------------------------------------------------------------------------------------------- the checks
+namespace {
+using namespace tch;
+int g_failures = 0;
+
+void expect(bool ok, const std::string& what) {
+  if (!ok && ++g_failures <= 20) fprintf(stderr, "FAILED: %s\n", what.c_str());
+}
+
+int on_other_queues(hipStream_t a, hipStream_t b) { return as_stream(a)->queue != as_stream(b)->queue; }
+
+void launch(Context* ctx, int id, double duration) {
+  Launch what{id, duration};
+  submit(ctx, reinterpret_cast<const void*>(&g_failures), dim3(1), dim3(64), &what, sizeof(what), "kernel", 0.0, 1, 0.0);
+}
+
+// Ten sections of a main-lane kernel, a second-lane kernel that waits for it, and another main-lane kernel, with a join one
+// point behind after each: a section starts when the main lane and the second lane's work of the section before the
+// last one have ended -- not before, and not later, whatever streams the process has besides.
+void lanes_one_point_behind(const int* load, bool through_queue) {
+  reset(load);
+  constexpr int kSections = 10;
+  const double side_us[kSections] = {40, 5, 12, 60, 3, 25, 25, 8, 90, 10};
+  hipStream_t main = nullptr;
+  (void)hipStreamCreateWithFlags(&main, 0);
+  {
+    Context ctx(main);
+    ctx.streams_meet = on_other_queues;
+    Program prog;
+    ctx.recording = &prog;
+    for (int k = 0; k < kSections; ++k) {
+      launch(&ctx, 3 * k, 10.0);
+      ctx.lane = 1;
+      ctx.wait_main = true;
+      launch(&ctx, 3 * k + 1, side_us[k]);
+      ctx.lane = 0;
+      ctx.wait_main = false;
+      launch(&ctx, 3 * k + 2, 5.0);
+      ctx.record_join(true);
+    }
+    ctx.record_join();
+    launch(&ctx, 3 * kSections, 1.0);
+    ctx.recording = nullptr;
+    ctx.prepare_lanes(prog);
+    if (through_queue) ctx.queue = std::make_shared<LaunchQueue>(main, 16, 4);
+    char where[96];
+    snprintf(where, sizeof(where), "load %d %d %d %d, %s", load[0], load[1], load[2], load[3], through_queue ? "queue" : "direct");
+    for (int replay = 0; replay < 2; ++replay) {
+      for (size_t i = 0; i < prog.launches.size(); ++i)
+        expect(ctx.dispatch(prog.launches[i], i + 1 < prog.launches.size() ? &prog.launches[i + 1] : nullptr) == 0, where);
+      if (ctx.queue) expect(ctx.queue->synchronize() == 0, where);
+      const std::vector<Span> at = g_spans;
+      expect(at.size() == 3 * kSections + 1, where);
+      for (int k = 0; k < kSections; ++k) {
+        const std::string which = std::string(where) + ", section " + std::to_string(k);
+        expect(at[3 * k + 1].start == std::max(at[3 * k].end, k ? at[3 * k - 2].end : 0.0), which + ": second lane");
+        if (k >= 1)
+          expect(at[3 * k].start == std::max(at[3 * k - 1].end, k >= 2 ? at[3 * (k - 2) + 1].end : 0.0), which + ": main lane");
+      }
+      expect(at[3 * kSections].start == std::max(at[3 * kSections - 1].end, at[3 * kSections - 2].end), std::string(where) + ": join");
+    }
+    ctx.queue.reset();
+  }
+  (void)hipStreamDestroy(main);
+  expect(g_streams_alive == 0 && g_events_alive == 0, "streams or events left behind");
+}
+}  // namespace
+
+int main() {
+  int cases = 0;
+  for (int l = 0; l < 81; ++l) {
+    const int load[kQueues] = {l % 3, l / 3 % 3, l / 9 % 3, l / 27};
+    for (bool through_queue : {false, true}) {
+      lanes_one_point_behind(load, through_queue);
+      ++cases;
+    }
+  }
+  printf("%d cases, %d failures\n", cases, g_failures);
+  return g_failures ? 1 : 0;
+}
