@@ -57,6 +57,10 @@ uint64_t tch_context_take_rejected(tch_context* ctx);
 int tch_context_set_lane(tch_context* ctx, int lane, int wait_main);
 int tch_context_join(tch_context* ctx);
 int tch_context_join_behind(tch_context* ctx);
+/* 1 = launches on lane 1 were seen to run at the same time as launches on lane 0 when its stream was made, 0 = not seen
+ * (another tenant held the chip meanwhile, or the streams could not be asked; the next recordings look again),
+ * -1 = no lane 1 yet. */
+int tch_context_second_lane(tch_context* ctx);
 int tch_context_synchronize(tch_context* ctx); /* both streams of the context */
 
 /* ---- programs: record once, replay every step ---------------------------------- */

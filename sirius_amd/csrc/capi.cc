@@ -72,6 +72,14 @@ int tch_context_join_behind(tch_context* ctx) {
   return ctx->ctx.record_join(true);
 }
 
+int tch_context_second_lane(tch_context* ctx) {
+  if (!ctx) {
+    set_error("tch_context_second_lane: null context");
+    return -22;
+  }
+  return !ctx->ctx.side ? -1 : ctx->ctx.side_shown ? 1 : 0;
+}
+
 int tch_context_synchronize(tch_context* ctx) {
   if (!ctx) {
     set_error("tch_context_synchronize: null context");

@@ -377,41 +377,53 @@ void LaunchQueue::worker_loop() {
 // ---------------------------------------------------------------------------
 
 Context::~Context() {
-  if (side) {
-    (void)hipStreamSynchronize(side);
-    (void)hipStreamDestroy(side);
+  if (side) former_sides_.push_back(side);
+  for (hipStream_t s : former_sides_) {
+    (void)hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
   }
   for (hipEvent_t e : events_) (void)hipEventDestroy(e);
 }
 
-hipStream_t Context::stream_beside_main() {
-  hipStream_t made = nullptr;
-  std::vector<hipStream_t> others;
-  constexpr int kTries = 6;
-  for (int i = 0; i < kTries; ++i) {
+bool Context::choose_side() {
+  if (looks_left > 0) --looks_left;
+  std::vector<hipStream_t> made;   // all kept until the end: a stream given back would be dealt out again
+  int met = 0;
+  for (int i = 0; i < kCandidates && met == 0; ++i) {
     hipStream_t s = nullptr;
     if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
       (void)hipGetLastError();
       break;
     }
-    // the last try is taken as it is, and so is any stream where the streams cannot be asked
+    made.push_back(s);
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    const bool ask = streams_meet && i + 1 < kTries && hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
-    if (!ask || streams_meet(stream, s) != 0) {
-      made = s;
-      break;
-    }
-    others.push_back(s);   // kept until the end: a stream given back would be dealt out again
+    met = streams_meet && hipStreamIsCapturing(stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone ? 0 : -1;
+    for (int k = 0; k < kAsks && met == 0; ++k) met = streams_meet(stream, s);
   }
-  for (hipStream_t s : others) (void)hipStreamDestroy(s);
-  return made;
+  const bool shown = met > 0;
+  if (met != 0) std::swap(made.front(), made.back());
+  hipStream_t chosen = made.empty() || (side && !shown) ? nullptr : made.front();
+  for (hipStream_t s : made)
+    if (s != chosen) (void)hipStreamDestroy(s);
+  if (!chosen) return side != nullptr;
+  if (side) {
+    // the new stream takes over where the old one stands, whose work may still be running or be queued
+    if (depend(side, chosen) != 0) {
+      (void)hipStreamDestroy(chosen);
+      return true;
+    }
+    former_sides_.push_back(side);
+  }
+  side = chosen;
+  side_shown = shown;
+  return true;
 }
 
 void Context::prepare_lanes(const Program& prog) {
   bool second = false;
   for (const LaunchRecord& r : prog.launches) second = second || (r.fn && r.lane == 1);
   if (!second || g_reject.load(std::memory_order_acquire)) return;
-  if (!side) side = stream_beside_main();
+  if (!side || (!side_shown && looks_left > 0)) (void)choose_side();
 }
 
 hipEvent_t Context::next_event() {
@@ -561,7 +573,7 @@ int Context::dispatch(const LaunchRecord& rec, const LaunchRecord* next) {
     }
     if (!rec.fn) return 0;
     if (rec.lane == 1) {
-      if (cu_limit == 0 && !side && !(side = stream_beside_main())) {
+      if (cu_limit == 0 && !side && !choose_side()) {
         set_error("hipStreamCreateWithFlags failed");
         return -5;
       }
@@ -592,7 +604,7 @@ int Context::dispatch(const LaunchRecord& rec, const LaunchRecord* next) {
     return 0;
   }
   if (rec.lane == 1) {
-    if (cu_limit == 0 && !side && !(side = stream_beside_main())) {
+    if (cu_limit == 0 && !side && !choose_side()) {
       set_error("hipStreamCreateWithFlags failed");
       return -5;
     }

@@ -130,7 +130,7 @@ struct Program {
   std::vector<LaunchRecord> launches;
 };
 
-// Whether launches on the two streams run at the same time (1) or not (0); -1: cannot tell.  Both are idle when it returns.
+// Whether launches on the two streams ran at the same time (1) or not (0); -1: cannot tell.  Both are idle when it returns.
 int run_at_the_same_time(hipStream_t a, hipStream_t b);   // lanes.hip
 
 class Context {
@@ -159,15 +159,21 @@ class Context {
   int behind_turn = 0;           // the one taken last
   bool behind_pending = false;   // lane 0 has not waited for it yet
   int join_behind();
-  // A stream whose launches run beside those of `stream`.  A process has four hardware queues (HIP's default) and its streams
-  // are dealt out to them in turn, so one stream in a few shares the main lane's queue: as a second lane it overlaps
-  // nothing.  Two engines' worth of streams later the same engine has read 6.4
-  // for 4.8 ms (Swin-B, 7 images), 5.6 for 4.45 (GPT-2, 8 x 256), 12.7 for 11.9 (8 x 1024).  Which queue a stream has
-  // cannot be asked, so two small kernels find out whether they meet; 0.1 ms for a stream that is turned down.
-  hipStream_t stream_beside_main();
-  // what it asks about two idle streams: 1 they meet, 0 they do not, -1 cannot tell; any stream will do without it
+  // Lane 1's stream has to run beside `stream`.  A process has four hardware queues (HIP's default) and its streams are dealt
+  // out to them in turn, so one stream in a few shares the main lane's queue and overlaps nothing as a second lane: two
+  // engines' worth of streams later the same engine has read 6.4 for 4.8 ms (Swin-B, 7 images), 5.6 for 4.45 (GPT-2, 8 x 256),
+  // 12.7 for 11.9 (8 x 1024).  Which queue a stream has cannot be asked, so two small kernels find out whether they meet.
+  // That they meet proves it; that they do not may also mean that another tenant held the chip meanwhile, so a candidate is
+  // asked kAsks times before it is turned down, and where none of them met the first one serves for now and the
+  // next recordings look again, kLooks times in all.
+  static constexpr int kAsks = 3, kCandidates = 6, kLooks = 4;
+  bool side_shown = false;   // the streams met: lane 1 is known to run beside lane 0
+  int looks_left = kLooks;
+  // side = a stream that runs beside `stream`, or the best there is; false where no stream can be made
+  bool choose_side();
+  // what it asks about two idle streams: 1 they meet, 0 they did not, -1 cannot tell; any stream will do without it
   int (*streams_meet)(hipStream_t, hipStream_t) = nullptr;
-  // makes the second lane's stream for a recorded program that will use it, so that the first replay need not
+  // chooses lane 1's stream for a recorded program that will use it, so that the first replay need not
   void prepare_lanes(const Program& prog);
   // recording state: the lane new launches are stamped with, and whether the next lane-1 launch
   // has to wait for lane 0
@@ -217,6 +223,7 @@ class Context {
   bool main_since_fork_ = true;
   std::vector<hipEvent_t> events_;
   size_t event_next_ = 0;
+  std::vector<hipStream_t> former_sides_;   // a launch queue may still hold entries for them
 };
 
 struct KernelStat {

@@ -1,4 +1,4 @@
-// Whether two streams' launches run side by side: asked when the second lane's streams are made (Context::stream_beside_main).
+// Whether two streams' launches run side by side: asked when the second lane's stream is made (Context::choose_side).
 #include "context.h"
 
 #include <mutex>

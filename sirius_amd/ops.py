@@ -118,6 +118,12 @@ class Context:
         finally:
             check(lib().tch_context_set_lane(self.handle, 0, 0), "tch_context_set_lane")
 
+    def second_lane(self):
+        """True: launches of the second lane were seen to run beside the main lane's when its stream was made; False: not
+        (yet) seen; None: no program with a second lane has been recorded."""
+        got = lib().tch_context_second_lane(self.handle)
+        return None if got < 0 else bool(got)
+
     def join(self, behind=False):
         """While recording: the main lane waits for everything the second lane was given so far.  With `behind`
         it waits for what the second lane had been given at the previous join(behind=True) only, so the second

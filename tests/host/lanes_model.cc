@@ -189,10 +189,69 @@ void lanes_one_point_behind(const int* load, bool through_queue) {
   (void)hipStreamDestroy(main);
   expect(g_streams_alive == 0 && g_events_alive == 0, "streams or events left behind");
 }
+
+// ---- which stream becomes the second lane, with the answers of the streams given
+std::vector<int> g_answers;   // one per ask; the last one for all that follow
+size_t g_asked = 0;
+int scripted(hipStream_t, hipStream_t) { return g_answers[std::min(g_asked++, g_answers.size() - 1)]; }
+
+void record_two_lanes(Context* ctx, Program* prog) {
+  ctx->recording = prog;
+  launch(ctx, 0, 10.0);
+  ctx->lane = 1;
+  ctx->wait_main = true;
+  launch(ctx, 1, 40.0);
+  ctx->lane = 0;
+  ctx->wait_main = false;
+  launch(ctx, 2, 5.0);
+  ctx->recording = nullptr;
+  ctx->prepare_lanes(*prog);
+}
+
+void choice(const char* name, std::vector<int> answers, bool shown, size_t asks, size_t asks_later, bool shown_later) {
+  reset(nullptr);
+  g_answers = answers;
+  g_asked = 0;
+  hipStream_t main = nullptr;
+  (void)hipStreamCreateWithFlags(&main, 0);
+  {
+    Context ctx(main);
+    ctx.streams_meet = scripted;
+    Program first, later;
+    record_two_lanes(&ctx, &first);
+    expect(ctx.side && ctx.side_shown == shown, std::string(name) + ": shown");
+    expect(g_asked == asks, std::string(name) + ": asks " + std::to_string(g_asked));
+    expect(g_streams_alive == 2, std::string(name) + ": refused streams are given back");
+    for (auto& l : first.launches) expect(ctx.dispatch(l) == 0, name);
+    const Span before = g_spans[1];
+    g_asked = asks;
+    for (int i = 0; i < 10; ++i) record_two_lanes(&ctx, &later);   // new plans
+    expect(ctx.side_shown == shown_later, std::string(name) + ": shown later");
+    expect(g_asked == asks_later, std::string(name) + ": asks later " + std::to_string(g_asked));
+    expect(g_streams_alive <= 3, std::string(name) + ": streams");
+    for (auto& l : first.launches) expect(ctx.dispatch(l) == 0, name);
+    expect(g_spans[1].start >= before.end, std::string(name) + ": a new second lane starts where the old one stands");
+  }
+  (void)hipStreamDestroy(main);
+  expect(g_streams_alive == 0 && g_events_alive == 0, std::string(name) + ": left behind");
+}
 }  // namespace
 
 int main() {
   int cases = 0;
+  constexpr int kAsks = Context::kAsks, kAll = Context::kAsks * Context::kCandidates;
+  choice("meets at once", {1}, true, 1, 1, true);
+  choice("missed, but meets when asked again", {0, 0, 1}, true, 3, 3, true);
+  choice("shares the queue, the next one does not", {0, 0, 0, 1}, true, kAsks + 1, kAsks + 1, true);
+  std::vector<int> last(kAll, 0);
+  last[kAll - 1] = 1;
+  choice("only the last one meets", last, true, kAll, kAll, true);
+  choice("none ever meets", {0}, false, kAll, kAll * Context::kLooks, false);
+  std::vector<int> later(kAll, 0);
+  later.push_back(1);
+  choice("chip held by another tenant at first", later, false, kAll, kAll + 1, true);
+  choice("cannot be asked", {-1}, false, 1, Context::kLooks, false);
+  cases += 7;
   for (int l = 0; l < 81; ++l) {
     const int load[kQueues] = {l % 3, l / 3 % 3, l / 9 % 3, l / 27};
     for (bool through_queue : {false, true}) {
