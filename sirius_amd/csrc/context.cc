@@ -385,7 +385,23 @@ Context::~Context() {
   for (hipEvent_t e : events_) (void)hipEventDestroy(e);
 }
 
+namespace {
+// While a thread captures a graph in global mode, calls that could disturb it are errors in every thread that does not say
+// that its own calls have nothing to do with the capture.  Making streams and asking them has nothing to do with one.
+class OutsideCaptures {
+ public:
+  OutsideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  ~OutsideCaptures() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  OutsideCaptures(const OutsideCaptures&) = delete;
+  OutsideCaptures& operator=(const OutsideCaptures&) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+}  // namespace
+
 bool Context::choose_side() {
+  OutsideCaptures here;
   if (looks_left > 0) --looks_left;
   std::vector<hipStream_t> made;   // all kept until the end: a stream given back would be dealt out again
   int met = 0;

@@ -1,5 +1,5 @@
-// The two lanes of a program on modelled hardware queues (CPU only; built by tests/test_lanes_model.py with context.cc and the
-// HIP calls below in the place of the runtime).
+// The two lanes of a program on modelled hardware queues (CPU only; built by tests/test_lanes_model.py with context.cc, lanes.hip
+// and the HIP calls below in the place of the runtime).
 //
 // Streams are dealt out to four hardware queues, the least loaded first; a queue runs what its streams hold in the order it
 // was submitted, waits for events included.  Every launch takes the time its argument says, so the moment each one starts
@@ -7,6 +7,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -41,6 +42,37 @@ int g_streams_alive = 0, g_events_alive = 0;
 Stream* as_stream(hipStream_t s) { return reinterpret_cast<Stream*>(s); }
 Event* as_event(hipEvent_t e) { return reinterpret_cast<Event*>(e); }
 
+// another thread captures a graph in global mode: calls that may disturb a capture are refused unless the calling thread
+// has taken itself out of it, and the null stream may not be touched at all
+bool g_captured_elsewhere = false;
+thread_local hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;
+std::string g_disturbed;
+hipError_t unsafe(const char* call, bool null_stream = false) {
+  if (!g_captured_elsewhere || (g_mode == hipStreamCaptureModeRelaxed && !null_stream)) return hipSuccess;
+  g_disturbed = call;
+  return hipErrorStreamCaptureUnsupported;
+}
+
+// the two kernels of a question (lanes.hip): they meet if they were given to different queues
+const void* g_handshake_kernel = nullptr;
+unsigned* g_answer = nullptr;
+hipStream_t g_asked_first = nullptr;
+void handshake(void** args, hipStream_t s) {
+  unsigned token;
+  int polls;
+  memcpy(&token, args[3], sizeof(token));
+  memcpy(&polls, args[4], sizeof(polls));
+  if (polls == 0) return;
+  if (!g_asked_first) {
+    g_asked_first = s;
+    return;
+  }
+  const bool met = as_stream(s)->queue != as_stream(g_asked_first)->queue;
+  g_asked_first = nullptr;
+  if (g_answer) g_answer[0] = met ? token : 0, g_answer[1] = token;   // the one that comes second sees the other's flag either way
+}
+
+
 void reset(const int* load) {
   std::lock_guard<std::mutex> lock(g_mu);
   for (int q = 0; q < kQueues; ++q) {
@@ -53,6 +85,7 @@ void reset(const int* load) {
 
 extern "C" {
 hipError_t hipStreamCreateWithFlags(hipStream_t* out, unsigned) {
+  if (unsafe("hipStreamCreateWithFlags") != hipSuccess) return hipErrorStreamCaptureUnsupported;
   std::lock_guard<std::mutex> lock(g_mu);
   const int q = static_cast<int>(std::min_element(g_load, g_load + kQueues) - g_load);
   ++g_load[q];
@@ -103,6 +136,10 @@ hipError_t hipExtLaunchKernel(const void*, dim3, dim3, void** args, size_t, hipS
   return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* fn, dim3 grid, dim3 block, void** args, size_t lds, hipStream_t s) {
+  if (fn == g_handshake_kernel) {
+    handshake(args, s);
+    return hipSuccess;
+  }
   return hipExtLaunchKernel(fn, grid, block, args, lds, s, nullptr, nullptr, 0);
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
@@ -120,6 +157,53 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "modelled"; }
 hipError_t hipDeviceGetAttribute(int*, hipDeviceAttribute_t, int) { return hipErrorNotSupported; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* mode) {
+  std::swap(*mode, g_mode);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (unsafe("hipHostMalloc") != hipSuccess) return hipErrorStreamCaptureUnsupported;
+  *p = g_answer = static_cast<unsigned*>(calloc(1, n));
+  return hipSuccess;
+}
+hipError_t hipHostGetDevicePointer(void** out, void* p, unsigned) {
+  *out = p;
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) {
+  static unsigned flags[4];
+  *p = flags;
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void*, const void*, size_t, hipMemcpyKind) { return unsafe("hipMemcpy", true); }
+// what the compiler emits for a file with kernels
+void** __hipRegisterFatBinary(const void*) {
+  static void* handle;
+  return &handle;
+}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
+  if (strstr(name, "handshake_kernel")) g_handshake_kernel = host;
+}
+void __hipRegisterVar(void**, void*, char*, const char*, int, size_t, int, int) {}
+void __hipUnregisterFatBinary(void**) {}
+namespace {
+struct {
+  dim3 grid, block;
+  size_t lds;
+  hipStream_t stream;
+} g_call;
+}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t s) {
+  g_call = {grid, block, lds, s};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipStream_t* s) {
+  *grid = g_call.grid;
+  *block = g_call.block;
+  *lds = g_call.lds;
+  *s = g_call.stream;
+  return hipSuccess;
+}
 hipError_t hipExtStreamCreateWithCUMask(hipStream_t* out, uint32_t, const uint32_t*) { return hipStreamCreateWithFlags(out, 0); }
 }  // extern "C"
 
@@ -235,6 +319,26 @@ void choice(const char* name, std::vector<int> answers, bool shown, size_t asks,
   (void)hipStreamDestroy(main);
   expect(g_streams_alive == 0 && g_events_alive == 0, std::string(name) + ": left behind");
 }
+
+// A recording that ends while another thread captures a graph: the second lane is chosen as ever, and no call disturbs the capture.
+void beside_a_capture(const int* load) {
+  reset(load);
+  hipStream_t main = nullptr;
+  (void)hipStreamCreateWithFlags(&main, 0);
+  {
+    Context ctx(main);
+    ctx.streams_meet = run_at_the_same_time;
+    Program prog;
+    g_captured_elsewhere = true;
+    g_disturbed.clear();
+    record_two_lanes(&ctx, &prog);
+    g_captured_elsewhere = false;
+    expect(g_disturbed.empty(), "a capture in another thread is disturbed by " + g_disturbed);
+    expect(g_mode == hipStreamCaptureModeGlobal, "the thread's capture mode is put back");
+    expect(ctx.side && ctx.side_shown && on_other_queues(main, ctx.side), "second lane beside a capture");
+  }
+  (void)hipStreamDestroy(main);
+}
 }  // namespace
 
 int main() {
@@ -258,6 +362,8 @@ int main() {
       lanes_one_point_behind(load, through_queue);
       ++cases;
     }
+    beside_a_capture(load);
+    ++cases;
   }
   printf("%d cases, %d failures\n", cases, g_failures);
   return g_failures ? 1 : 0;

@@ -34,3 +34,48 @@ def test_second_lane_of_an_idle_chip_is_shown_to_run_beside_the_first(operands, 
         torch.cuda.synchronize()
         kept += [record(ctx, *operands), ctx, torch.cuda.Stream()]
         assert ctx.second_lane() is True
+
+
+def test_a_recording_leaves_another_threads_capture_alone(operands):
+    """A graph is captured in global mode while the recording of a two-lane program ends in another thread, for the first time
+    (a stream is made and asked about) and again: the graph is whole, replays right, and the program runs right."""
+    import threading
+
+    from sirius_amd import ops
+    x, w, ys = operands
+    a, b = torch.zeros(4096, device="cuda"), torch.zeros(4096, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    got, errors = [], []
+    mains = [torch.cuda.Stream() for _ in range(2)]
+
+    def other():
+        try:
+            for main in mains:
+                ctx = ops.Context(main)
+                got.append((ctx, record(ctx, x, w, ys)))
+        except Exception as e:      # noqa: BLE001  (told to the main thread)
+            errors.append(e)
+
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, capture_error_mode="global"):
+        torch.mul(a, 2.0, out=b)
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+        b.add_(1.0)
+    assert not errors, errors
+    for i in range(3):
+        a.fill_(float(i))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(b, torch.full_like(b, 2 * i + 1.0))
+    want = (x.view(32, 64).float() @ w.view(64, 64).float().t())
+    for ctx, prog in got:
+        assert ctx.second_lane() is True
+        for y in ys:
+            y.zero_()
+        torch.cuda.synchronize()
+        ctx.run(prog)
+        ctx.synchronize()
+        for y in ys:
+            assert (y.view(32, 64).float() - want).abs().max() <= 1e-2 * want.abs().max()
