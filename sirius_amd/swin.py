@@ -409,7 +409,7 @@ class SwinEngine(EngineBase):
             R0, C0 = st0["R"], st0["C"]
             e0 = act(rows0, C0)
             ops.conv2d_fwd(ctx, x0, self._w("features.0.0.weight"), e0.view(B, R0, R0, C0), P, 0,
-                           bias=self._view(self.params, "features.0.0.bias"), c_logical=3)
+                           bias=self._view(self.params, "features.0.0.bias"), c_logical=3, tile_cfg=order)
             x = act(rows0, C0)
             embed_stats = new_ln(rows0)
             ln_fwd("features.0.2", e0, x, embed_stats)
@@ -512,7 +512,7 @@ class SwinEngine(EngineBase):
             ops.avgpool_fwd(ctx, hf.view(B, stL["R"], stL["R"], CL), pooled)
             logits = act(B, self.num_classes, dtype=torch.float32)
             ops.conv2d_fwd(ctx, pooled.view(B, 1, 1, CL), self._w("head.weight"), logits.view(B, 1, 1, self.num_classes), 1, 0,
-                           bias=self._view(self.params, "head.bias"))
+                           bias=self._view(self.params, "head.bias"), tile_cfg=order)
             dlogits = act(B, self.num_classes)
             ops.softmax_ce_fwd_bwd(ctx, logits, plan.labels, plan.loss_rows, plan.loss, dlogits, loss_scale=loss_scale)
             plan.n_forward = len(prog)
