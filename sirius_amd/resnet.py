@@ -859,12 +859,14 @@ class ResNetEngine(EngineBase):
         return plan
 
     def eval_plan(self, batch):
+        # eval_in_order and fuse_eval_bn may be set between requests: each has its own program
         plans = self.__dict__.setdefault("_eval_plans", {})
-        if batch not in plans:
+        key = (batch, bool(self.eval_in_order), bool(self.fuse_eval_bn))
+        if key not in plans:
             if getattr(self, "_eval_coef", None) is None:
                 self.prepare_eval()
-            plans[batch] = self._build_eval_plan(batch)
-        return plans[batch]
+            plans[key] = self._build_eval_plan(batch)
+        return plans[key]
 
     def forward_eval(self, x):
         """x [B,3,S,S] fp32 on the GPU -> the plan whose `logits` [B, classes] (fp32) the launches fill.  The
