@@ -2708,9 +2708,12 @@ int heuristic_tile(int asked, const TileQuery& q) {
     // and 15.9; over 3072, 8192 x 768: 38.4 and 43.6)
     if (!q.sums && large && t.cfg == kMix128x192 && q.gemm_k < 1024) continue;
     // A transformer's data gradients run beside weight gradients that hold 64 KB of LDS and half of every SIMD's registers:
-    // there the 128 x 128 tilings on eight wavefronts lose to 128 x 128 and 128 x 64 on four (Swin-B step of 32 images 10.03 ms
-    // with them, 9.92 without; GPT-2 8 x 1024 12.03 and 11.96, 8 x 256 and 3 x 777 the same)
-    if (q.dgrad && !q.sums && (t.cfg == 0 || t.cfg == kMix128)) continue;
+    // there the 128 x 128 tilings on eight wavefronts lose in the step (Swin-B of 32 images 9.85 ms without them, 9.91 with
+    // both; of 24 images 8.30 and 8.38; GPT-2 2 x 512 3.70 and 3.75).  Not so over long reductions, where the table's next choice is
+    // 64 x 64 at twice the operand bytes per flop: with three LDS tiles from 2048 on, GPT-2 takes 7.53 ms on 4 x 1024 (8.20
+    // without), 8.46 on 5 x 1024 (8.88), 6.47 on 3 x 1024 (6.81), 5.85 on 12 x 256 (6.21); other GPT-2 sizes and Swin-B of 4-32
+    // images, whose longest are 3072 and 4096, are the same.
+    if (q.dgrad && !q.sums && (t.cfg == 0 || (t.cfg == kMix128 && q.gemm_k <= 2048))) continue;
     // at least half of the tile's columns lie in the output (56 x 56 x 256 -> 64, 20 images: 11.0 us as 128 x 128, 9.3 as 128 x 64)
     if (t.bn >= 2 * q.gemm_n && t.bn > 32) continue;
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
