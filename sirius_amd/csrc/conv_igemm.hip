@@ -813,12 +813,17 @@ __device__ inline void wait_and_meet() {
 // 50 176 34 -> 26; reading a step ahead of its multiplication into a second register set (169 instead of 136
 // registers) gained nothing on top.
 // POINTWISE: x is read at dy's pixels (no tap arithmetic).  BIAS: the launch may be asked for the bias gradient.
-// Over up to 60 steps 64 x 64 keeps five tiles in LDS instead of eight: the seven requests of the full ring's start are a good
-// part of such a reduction, and 40 KB leave room for a main-lane workgroup.  Steps of 20 images 7.11 -> 7.06 ms, of 2 x 16 13.67 ->
-// 13.49 (28-56 steps per split), GPT-2 3 x 777, Swin-B of 7 and ResNet of 64 images the same; over 64 steps and more the full
-// ring wins (GPT-2 8 x 256 4.50 ms, 4.55 with five tiles; ResNet of 64 images 13.87 and 14.02).  Three tiles up to 48 steps: 20
-// images 7.01, but Swin-B of 7 images 4.89 for 4.75.
-constexpr int kWgradRing = 65536, kWgradShortRing = 40960, kWgradShortSteps = 60;
+// 64 x 64 keeps five tiles in LDS instead of eight where the launch has more than one workgroup per compute unit, or few
+// steps, or leaves compute units free (short_wgrad_ring): the seven requests of the full ring's start are a good part of a short
+// reduction, and 40 KB leave room for another workgroup.  ResNet steps in ms with the full ring / five tiles up to 60 steps / this
+// rule: of 16 images 6.80 / 6.72 / 6.72, 2 x 16 13.73 / 13.57 / 13.58, 21 7.77 / 7.92 / 7.77, 24 8.13 / 8.27 / 8.13, 28 8.61 / 8.59 /
+// 8.55, 32 9.08 / 9.24 / 9.11; of 6-15, 17-20, 40, 48 and 64 images, GPT-2 and Swin-B the same within 0.5 % with all.  Its weight gradients of the third
+// stage, 72 of 155: 3 x 3 as 432 workgroups of 33-66 steps are as fast or faster with five tiles, 1 x 1 as 192 of 33 (16
+// images) faster, as 256 of 31 (20) the same and of 33-49 (21-32) slower: one workgroup on every compute unit lives off its
+// own requests.  With several on each, 60 or 100 steps make no difference.  (Three tiles up to 48 steps: 20 images 7.01 for 7.06,
+// but Swin-B of 7 images 4.89 for 4.75.)
+constexpr int kWgradRing = 65536, kWgradShortRing = 40960;
+inline bool short_wgrad_ring(int64_t workgroups, int steps) { return steps <= (workgroups > 192 && workgroups <= 256 ? 32 : 60); }
 template <int WM, int WN, int TM, int TN, int RING>
 constexpr int wgrad_direct_buffers() {
   return RING / (32 * (WM * TM + WN * TN) * 64);
@@ -2309,7 +2314,7 @@ int launch_cfg(Context* ctx, IgemmArgs& a, double flops) {
     void (*kernel)(WgradArgs);
     if constexpr (sizeof(T) == 4)
       kernel = wgrad_f32_kernel<WM, WN, TM, TN>;
-    else if (TM * TN == 1 && a.k_per_split <= 32 * kWgradShortSteps)
+    else if (TM * TN == 1 && short_wgrad_ring(wgs, (a.k_per_split + 31) / 32))
       kernel = wgrad_direct_kernel<WM, WN, TM, TN, TM * TN == 1 ? kWgradShortRing : kWgradRing>(a);
     else
       kernel = wgrad_direct_kernel<WM, WN, TM, TN, kWgradRing>(a);
