@@ -2629,7 +2629,9 @@ int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
 //   start + round * r + steps * max(alone, shared * r) + store * (outputs / 10^6)
 // with r = workgroups per compute unit, rounded up, and steps = 64-element reduction steps.  `alone` is a step of one
 // workgroup on a CU (a chain of latencies), `shared` what a step costs each of several that share the CU's operand
-// path; `round` is the epilogue, which those take in turn.  The constants are least-squares fits (mean error 3-8 %) to
+// path; `round` is what each further one adds to the epilogue: for eight of the plain tilings the fit leaves it at 0, and the
+// epilogue is then in `start`, which also holds the 3 us of event, and in `store`.  How many workgroups fit on a CU at a time
+// is not in the price; the exceptions below are what that costs.  The constants are least-squares fits (mean error 3-8 %) to
 // 556 different convolutions where they stand in a step or request, one launch at a time (operands as cold or warm as their
 // producers leave them; 3 us of event among it), each with every tiling: ResNet-152 at 1-64 images, GPT-2 at 512-8192
 // tokens, Swin-B at 3-32 images; the second table for ResNet's data gradients with the BatchNorm sums, whose epilogue
@@ -2704,13 +2706,17 @@ int heuristic_tile(int asked, const TileQuery& q) {
   const size_t entries = q.sums ? std::size(kSumsCost) : std::size(kPlainCost);
   for (size_t i = 0; i < entries; ++i) {
     const TileCost& t = costs[i];
-    // one and a half 128 x 128 tiles per compute unit or more, beside a second lane of weight gradients: smaller tiles
-    // fetch more operand bytes per flop and lose in the step what they win alone (GPT-2 step of 8 x 1024 tokens 13.34 ms
-    // without this line, 12.19 with it; 3 x 777 tokens and Swin-B of 32 images the same either way)
+    // From one and a half 128 x 128 tiles per compute unit on the table prices smaller tiles, which fetch more operand bytes per
+    // flop, lower than they come out in a step.  GPT-2 8 x 1024 11.81 ms with this line, 11.91 without;
+    // 1-6 x 1024, 3 x 777, Swin-B of 7-32 images, ResNet of 64 and requests of 24 and 64 the same.  From 256 tiles on 6 x 1024
+    // takes 9.49 for 9.43 and 8 x 256 4.65 for 4.61; from 512 on 2 x 1024 5.26 for 5.16 and 8 x 256 4.71.  (384 tiles are
+    // 8192 x 768 and 2048 x 3072, the products those sizes hang on; nothing measured lies closer on either side.)
     if (!q.sums && large && t.bm * t.bn < 128 * 128) continue;
     // 128 x 192 has a CU to itself: over a short reduction its epilogue and the next tile's first trip to memory are in
-    // nobody's shadow, where the grid has several rounds (8192 x 3072 over 768 54.8 us, 47.5 as 128 x 128; 2048 x 3072 15.7
-    // and 15.9; over 3072, 8192 x 768: 38.4 and 43.6)
+    // nobody's shadow, where the grid has several rounds, and the price knows rounds only as their number (8192 x 3072 over 768
+    // alone 54.8 us, 47.5 as 128 x 128; 2048 x 3072 15.7 and 15.9; over 3072, 8192 x 768: 38.4 and 43.6).  In the steps: GPT-2 4 x
+    // 1024 8.27 ms with this line, 8.35 without, 2 x 1024 5.16 and 5.28, 8 x 256 4.61 and 4.70, 3 x 1024 6.81 and 6.88; 8 x 1024 11.81
+    // and 11.74, the one that it costs something.  Such grids were measured over 768 and from 2304 on; the line is in between.
     if (!q.sums && large && t.cfg == kMix128x192 && q.gemm_k < 1024) continue;
     // A transformer's data gradients run beside weight gradients that hold 64 KB of LDS and half of every SIMD's registers:
     // there the 128 x 128 tilings on eight wavefronts lose in the step (Swin-B of 32 images 9.85 ms without them, 9.91 with
