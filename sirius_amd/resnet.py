@@ -78,8 +78,8 @@ class ResNetEngine(EngineBase):
         self.fuse_eval_bn = True
         # eval_in_order: every sum of the forward-only plan is taken front to back, so that an image's logits are the same
         # bits whatever images are batched with it.  Off by default: the tilings that split a reduction over wavefronts,
-        # which few rows call for, are then left out, and they are what a small request gains from (ResNet-152, 1 / 4 / 16 /
-        # 24 / 64 images: 0.87 / 1.16 / 2.01 / 2.29 / 3.73 ms without, 1.24 / 1.46 / 2.04 / 2.29 / 3.89 with).  Without it bf16
+        # which few rows call for, are then left out, and they are what a small request gains from (ResNet-152, 1 / 4 /
+        # 24 / 64 images: 0.83 / 1.02 / 2.11 / 3.38 ms without, 1.25 / 1.34 / 2.14 / 3.50 with).  Without it bf16
         # logits of one image differ by about 2e-3 between batch sizes; at one batch size they are the same bits every time.
         self.eval_in_order = bool(eval_in_order)
         # compact_downsample_dgrad: the data gradient of a stride-2 downsample convolution stays on the small grid
