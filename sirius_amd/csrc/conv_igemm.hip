@@ -2700,7 +2700,9 @@ int heuristic_tile(int asked, const TileQuery& q) {
   }
   const float steps = static_cast<float>(q.gemm_k) / 64.f, store = static_cast<float>(q.gemm_m) * q.gemm_n * 1e-6f;
   const bool large = q.gemm_n > 64 && tiles_for(q.gemm_m, q.gemm_n, 128, 128) >= 384;
-  int best = 2;
+  // what runs where the rules below leave nothing: data gradients on large grids over less than 1024, whose one tiling is 12,
+  // with TCH_IGEMM_K32=0 (128 x 128 there too), and front-to-back products of up to 32 columns
+  int best = large && !q.sums ? 0 : 2;
   float best_us = INFINITY;
   const TileCost* const costs = q.sums ? kSumsCost : kPlainCost;
   const size_t entries = q.sums ? std::size(kSumsCost) : std::size(kPlainCost);
