@@ -2507,7 +2507,7 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
       tile_cfg = 1;
     }
     // 9 / 10: 256 x 256 on eight wavefronts (128 x 64 each), two LDS tiles, plain / rotated loop: for products with a
-    // thousand such tiles or more (65 536 x 4096 x 4096: 1.17 and 1.23 PFLOP/s, 1.03 for 128 x 128; slower than 128 x 128 on
+    // thousand such tiles or more (65 536 x 4096 x 4096: 1.18 and 1.31 PFLOP/s, 1.03 for 128 x 128; slower than 128 x 128 on
     // the other layers of the three models, by up to 1.7x)
     if (tile_cfg == 9 || tile_cfg == 10) {
       if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32)
@@ -2727,7 +2727,7 @@ int heuristic_tile(int asked, const TileQuery& q) {
     // without), 8.46 on 5 x 1024 (8.88), 6.47 on 3 x 1024 (6.81), 5.85 on 12 x 256 (6.21); other GPT-2 sizes and Swin-B of 4-32
     // images, whose longest are 3072 and 4096, are the same.
     if (q.dgrad && !q.sums && (t.cfg == 0 || (t.cfg == kMix128 && q.gemm_k <= 2048))) continue;
-    // at least half of the tile's columns lie in the output (56 x 56 x 256 -> 64, 20 images: 11.0 us as 128 x 128, 9.3 as 128 x 64)
+    // more than half of the tile's columns lie in the output (56 x 56 x 256 -> 64, 20 images: 11.0 us as 128 x 128, 9.3 as 128 x 64)
     if (t.bn >= 2 * q.gemm_n && t.bn > 32) continue;
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;

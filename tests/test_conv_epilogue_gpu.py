@@ -8,7 +8,7 @@ import test_ops_gpu as T
 from oracle import nn_ops as O
 
 pytestmark = pytest.mark.gpu
-TILES = [0, 1, 2, 3, 5, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22]
+TILES = [0, 1, 2, 3, 5, 9, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 21, 22, 23, 24]
 # one row, rows and columns beyond a tile's edge, a band more than a tile
 CASES = [(1, 1, 1, 64, 8, 1, 1, 1, 0), (3, 7, 13, 64, 200, 1, 1, 1, 0), (1, 17, 17, 128, 136, 3, 3, 1, 1)]
 

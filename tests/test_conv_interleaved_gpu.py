@@ -9,6 +9,9 @@ import test_ops_gpu as T
 gpu = pytest.mark.gpu
 TILES = [0, 10, 22, 23, 24]
 STEPS = [(130, 1, 1, 64 * k, 200, 1, 1, 1, 0) for k in range(1, 6)]     # up to three tiles in flight; 200 columns: a ragged tile
+# the same for data gradients, whose reduction runs over K and the taps
+DGRAD_STEPS = ([(130, 1, 1, 200, 64 * k, 1, 1, 1, 0) for k in range(1, 8)] +
+               [(3, 9, 7, 136, 64, 3, 3, 1, 1), (2, 9, 11, 200, 128, 3, 3, 1, 1), (3, 9, 7, 136, 64, 3, 3, 2, 1), (2, 13, 10, 200, 192, 3, 3, 2, 1)])
 
 
 @gpu
@@ -16,6 +19,13 @@ STEPS = [(130, 1, 1, 64 * k, 200, 1, 1, 1, 0) for k in range(1, 6)]     # up to 
 @pytest.mark.parametrize("case", P.CASES + STEPS)
 def test_forward_and_data_gradient(ctx, case, tile_cfg):
     T.test_conv_fwd(ctx, torch.bfloat16, case, tile_cfg)
+    T.test_conv_dgrad(ctx, torch.bfloat16, case, tile_cfg)
+
+
+@gpu
+@pytest.mark.parametrize("tile_cfg", TILES)
+@pytest.mark.parametrize("case", DGRAD_STEPS)
+def test_data_gradient_steps(ctx, case, tile_cfg):
     T.test_conv_dgrad(ctx, torch.bfloat16, case, tile_cfg)
 
 
@@ -28,9 +38,11 @@ def test_batchnorm_sums(ctx, case, tile_cfg):
 
 
 @gpu
-@pytest.mark.parametrize("case", [(1000, 1, 1, 832, 520, 1, 1, 1, 0), (3, 15, 13, 128, 200, 3, 3, 1, 1), (2, 16, 16, 64, 392, 3, 3, 2, 1)])
+@pytest.mark.parametrize("case", [(1000, 1, 1, 832, 520, 1, 1, 1, 0), (3, 15, 13, 128, 200, 3, 3, 1, 1), (2, 16, 16, 64, 392, 3, 3, 2, 1),
+                                  (1000, 1, 1, 448, 320, 1, 1, 1, 0), (3, 15, 13, 320, 192, 3, 3, 1, 1), (2, 16, 16, 192, 448, 3, 3, 2, 1)])
 def test_every_interleaved_tiling_adds_in_the_same_order(ctx, case):
-    """Tiling 9 is the plain loop."""
+    """Tiling 9 is the plain loop.  Forward in every case, the data gradient in those whose K is whole steps (another kernel runs
+    in the others)."""
     from sirius_amd import ops
     N, H, W, C, K, R, S, st, pad = case
     g = T._gen(51)
@@ -44,11 +56,10 @@ def test_every_interleaved_tiling_adds_in_the_same_order(ctx, case):
         ops.conv2d_fwd(ctx, x, w, y, st, pad, tile_cfg=tile_cfg)
         if K % 64 == 0:
             ops.conv2d_dgrad(ctx, dy, wt, dx, st, pad, tile_cfg=tile_cfg)
-        else:
-            dx.zero_()
         torch.cuda.synchronize()
         want = want or (y, dx)
-        assert torch.equal(y, want[0]) and torch.equal(dx, want[1]), tile_cfg
+        assert torch.equal(y, want[0]), tile_cfg
+        assert K % 64 or torch.equal(dx, want[1]), tile_cfg
 
 
 @pytest.mark.parametrize("dtype", [0, 1], ids=["f32", "bf16"])

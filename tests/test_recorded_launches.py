@@ -68,10 +68,10 @@ def wgrad(rec, dtype, tile_cfg, splits, trailing=False):
 
 
 @dtypes
-@pytest.mark.parametrize("tile_cfg", range(23))
+@pytest.mark.parametrize("tile_cfg", range(25))
 def test_every_tiling_number_of_a_weight_gradient_runs_its_kernel(rec, dtype, tile_cfg):
     """The tilings of the other directions stand for a shape; none of their kernels may get a weight gradient's operands."""
-    side = {0: (128, 128), 1: (128, 64)}.get({9: 0, 10: 0, 11: 0, 12: 0, 5: 1, 6: 1, 13: 1, 22: 1}.get(tile_cfg, tile_cfg), (64, 64))
+    side = {0: (128, 128), 1: (128, 64)}.get({9: 0, 10: 0, 11: 0, 12: 0, 23: 0, 24: 0, 5: 1, 6: 1, 13: 1, 22: 1}.get(tile_cfg, tile_cfg), (64, 64))
     tiles = (K // side[0]) * (-(-C // side[1]))
     for splits in (1, 4):
         rec.begin()
@@ -170,7 +170,7 @@ def test_row_tiles_of_the_statistics_are_those_of_the_kernel(dtype, setting):
     many row tiles, for every tiling and setting of TCH_IGEMM2.  0: igemm_kernel whatever tiling is asked for."""
     got = in_own_process("""
 dtype, staged, L = %d, %r, T.lib()
-for cfg in [-2, -1] + list(range(23)):
+for cfg in [-2, -1] + list(range(25)):
     for shape in ((2, 14, 14, 128, 256, 3, 3, 1, 1), (1, 56, 56, 64, 128, 1, 1, 2, 0), (3, 9, 7, 24, 40, 3, 3, 1, 1),
                   (64, 56, 56, 256, 64, 1, 1, 1, 0), (1, 7, 7, 32, 512, 1, 1, 1, 0)):
         rec.begin()
@@ -190,7 +190,7 @@ print("ok", end="")
 
 
 @dtypes
-@pytest.mark.parametrize("tile_cfg", range(23))
+@pytest.mark.parametrize("tile_cfg", range(25))
 def test_floor_table_files_every_convolution_kernel_under_its_direction(rec, dtype, tile_cfg):
     from sirius_amd.floor_table import family
     rec.begin()
