@@ -813,8 +813,8 @@ __device__ inline void wait_and_meet() {
 // 50 176 34 -> 26; reading a step ahead of its multiplication into a second register set (169 instead of 136
 // registers) gained nothing on top.
 // POINTWISE: x is read at dy's pixels (no tap arithmetic).  BIAS: the launch may be asked for the bias gradient.
-// 64 x 64 keeps five tiles in LDS instead of eight where the launch has more than one workgroup per compute unit, or few
-// steps, or leaves compute units free (short_wgrad_ring): the seven requests of the full ring's start are a good part of a short
+// 64 x 64 keeps five tiles in LDS instead of eight over up to 60 steps, and over up to 32 where the launch is about one
+// workgroup on every compute unit (short_wgrad_ring): the seven requests of the full ring's start are a good part of a short
 // reduction, and 40 KB leave room for another workgroup.  ResNet steps in ms with the full ring / five tiles up to 60 steps / this
 // rule: of 16 images 6.80 / 6.72 / 6.72, 2 x 16 13.73 / 13.57 / 13.58, 21 7.77 / 7.92 / 7.77, 24 8.13 / 8.27 / 8.13, 28 8.61 / 8.59 /
 // 8.55, 32 9.08 / 9.24 / 9.11; of 6-15, 17-20, 40, 48 and 64 images, GPT-2 and Swin-B the same within 0.5 % with all.  Its weight gradients of the third
