@@ -1,7 +1,7 @@
 // Implicit-GEMM convolution for gfx950: forward, data gradient and weight
 // gradient over NHWC activations and KRSC filters, on the 32x32 MFMA tiles
-// (v_mfma_f32_32x32x16_bf16 for bf16 storage, v_mfma_f32_32x32x2_f32 for fp32),
-// fp32 accumulation, operands staged through LDS in 16-byte chunks.
+// (v_mfma_f32_32x32x16_bf16; fp32 storage in three bf16 parts, fp32_split.h, or on
+// v_mfma_f32_32x32x2_f32), fp32 accumulation, operands staged through LDS in 16-byte chunks.
 //
 // The reference has no convolution code of its own: its training scripts call
 // torchvision's ResNet (train/resnet152.py:22) and the arithmetic is
@@ -35,6 +35,7 @@
 // output columns: the epilogue moves them through LDS as 16-byte vectors and
 // writes (and reads the residual / mask) as full 16-byte chunks per lane.
 #include "col_sum.h"
+#include "fp32_split.h"
 #include "kernels.h"
 #include <algorithm>
 #include <iterator>
@@ -54,6 +55,11 @@ namespace {
 constexpr int kLdsStride = 5;  // FWD/DGRAD: chunks per LDS tile row: 4 data + 1 pad
 constexpr int kRowPad = 4;     // WGRAD, fp32: chunks of padding per [pixel] row (64 bytes)
 constexpr int kStagePad = 4;   // epilogue staging: floats of padding per row
+
+// fp32 products over longer reductions run on the bf16 pipes (fp32_split.h), shorter ones in fp32: up to here they are launch,
+// epilogue and latency, and the parts only add instructions (784 x 256 over 128: 3.7 us in fp32, 4.0 in parts; 12 544 x 64 over
+// 256: 9.6 and 9.2)
+constexpr int kShortReduction = 128;
 
 enum Mode : int { kFwd = 0, kDgrad = 1, kWgrad = 2 };
 
@@ -97,6 +103,7 @@ struct IgemmArgs {
   int group_rows;   // FWD/DGRAD direct-to-LDS kernel: row tiles per group of the tile order (0 / 1: row-major)
   int k_per_split;  // multiple of BK
   int out_f32;      // FWD/DGRAD: store fp32 instead of T
+  int in_fp32;      // fp32, igemm_kernel: no parts (fp32_split.h), so that every tile adds up the same bits
   int accumulate;   // WGRAD with splits == 1: out += result
   int take_pending; // WGRAD, read by the launcher only: the context's pending split reduction rides this launch
   int pointwise;    // 1x1, stride 1, pad 0
@@ -623,7 +630,6 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
   int a_base[A_PT], a_h0[A_PT], a_w0[A_PT];
   bool a_row_ok[A_PT];
   TapWalker walk;
-  walk.init(chunk_col * E, in_c, p.S);
 #pragma unroll
   for (int i = 0; i < A_PT; ++i) {
     const int row = m0 + ((tid + i * NT) >> 2);
@@ -707,49 +713,84 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
   };
 
   f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
   const int frag_row = lane & 31;
   const int frag_half = lane >> 5;
-  auto compute = [&](int buf) {
-    const uint4* la = lds_a + buf * BM * kLdsStride;
-    const uint4* lb = lds_b + buf * BN * kLdsStride;
+  // the sums of the tile, in `acc`; split_c: in fp32, on the bf16 pipes, small products in `low`
+  auto reduce = [&](auto split_c, f32x16_t (&low)[TM][TN]) {
+    constexpr bool SPLIT = decltype(split_c)::value;
+    clear(acc);
+    if constexpr (SPLIT) clear(low);
+    walk.init(chunk_col * E, in_c, p.S);
+    auto compute = [&](int buf) {
+      const uint4* la = lds_a + buf * BM * kLdsStride;
+      const uint4* lb = lds_b + buf * BN * kLdsStride;
+      auto a_chunk = [&](int tm, int j) {
+        Chunk c;
+        c.u = la[((wm * TM + tm) * 32 + frag_row) * kLdsStride + 2 * j + frag_half];
+        return c;
+      };
+      auto b_chunk = [&](int tn, int j) {
+        Chunk c;
+        c.u = lb[((wn * TN + tn) * 32 + frag_row) * kLdsStride + 2 * j + frag_half];
+        return c;
+      };
+      if constexpr (SPLIT) {
+        Split8 fb[TN];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      Chunk fa[TM], fb[TN];
+        for (int tn = 0; tn < TN; ++tn) fb[tn] = split8(b_chunk(tn, 0), b_chunk(tn, 1));
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) fa[tm].u = la[((wm * TM + tm) * 32 + frag_row) * kLdsStride + 2 * j + frag_half];
+        for (int tm = 0; tm < TM; ++tm) {
+          const Split8 fa = split8(a_chunk(tm, 0), a_chunk(tm, 1));
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) fb[tn].u = lb[((wn * TN + tn) * 32 + frag_row) * kLdsStride + 2 * j + frag_half];
+          for (int tn = 0; tn < TN; ++tn) mma_split(fb[tn], fa, acc[tm][tn], low[tm][tn]);
+        }
+      } else {
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+        for (int j = 0; j < 2; ++j) {
+          Chunk fa[TM], fb[TN];
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) mma<T>(fb[tn], fa[tm], acc[tm][tn]);
-    }
-  };
+          for (int tm = 0; tm < TM; ++tm) fa[tm] = a_chunk(tm, j);
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) fb[tn] = b_chunk(tn, j);
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn) mma<T>(fb[tn], fa[tm], acc[tm][tn]);
+        }
+      }
+    };
 
-  // Register set 0 carries the even tiles, set 1 the odd ones.  The loop has no
-  // conditionals: tiles past the end of the reduction load as zeros (out-of-range
-  // buffer offsets) and multiply to nothing, so an odd tile count costs one empty step.
-  load_tiles(0, ra0, rb0);
-  load_tiles(1, ra1, rb1);
-  store_tiles(0, ra0, rb0);
-  __syncthreads();
-  load_tiles(2, ra0, rb0);
-  for (int kt = 0; kt < nk; kt += 2) {
-    compute(0);  // tile kt
-    store_tiles(1, ra1, rb1);
-    __syncthreads();
-    load_tiles(kt + 3, ra1, rb1);
-    compute(1);  // tile kt + 1
+    // Register set 0 carries the even tiles, set 1 the odd ones.  The loop has no
+    // conditionals: tiles past the end of the reduction load as zeros (out-of-range
+    // buffer offsets) and multiply to nothing, so an odd tile count costs one empty step.
+    load_tiles(0, ra0, rb0);
+    load_tiles(1, ra1, rb1);
     store_tiles(0, ra0, rb0);
     __syncthreads();
-    load_tiles(kt + 4, ra0, rb0);
+    load_tiles(2, ra0, rb0);
+    for (int kt = 0; kt < nk; kt += 2) {
+      compute(0);  // tile kt
+      store_tiles(1, ra1, rb1);
+      __syncthreads();
+      load_tiles(kt + 3, ra1, rb1);
+      compute(1);  // tile kt + 1
+      store_tiles(0, ra0, rb0);
+      __syncthreads();
+      load_tiles(kt + 4, ra0, rb0);
+    }
+  };
+  // 64 x 64 stays with fp32 multiplies: a wavefront would take two operands apart for every one of its 32 x 32 products
+  // (512 x 768 over 768 21.8 us in fp32, 23.9 in parts, as 128 x 128 57.4 and 50.2)
+  if constexpr (EB == 4 && TM * TN > 1) {
+    f32x16_t low[TM][TN];
+    bool plain = p.gemm_k <= kShortReduction || p.in_fp32;
+    if (!plain) {
+      reduce(std::true_type{}, low);
+      plain = __syncthreads_or(join_split(acc, low));
+    }
+    if (plain) reduce(std::false_type{}, low);
+  } else {
+    reduce(std::false_type{}, acc);
   }
 
   TileEpilogue<T, MODE, WM, WN, TM, TN, false> epilogue;
@@ -1098,7 +1139,12 @@ __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) 
   static_assert(NT % CA == 0 && NT % CB == 0, "a thread keeps one chunk column");
   constexpr int OPER_BYTES = 2 * BKP * (LDA + LDB) * 16;
   constexpr int STAGE_BYTES = WM * 32 * (BN + kStagePad) * 4;
-  constexpr int LDS_BYTES = OPER_BYTES > STAGE_BYTES ? OPER_BYTES : STAGE_BYTES;
+  // three parts of bf16 per value: [buffer][dy, x][part][pixel][channel], rows unpadded, 16-byte slots XOR-ed by the row as
+  // in wgrad_body_direct
+  constexpr int RA = BM * 2, RB = BN * 2;
+  constexpr int A_PART = BKP * RA, B_PART = BKP * RB, PARTS_BYTES = 3 * (A_PART + B_PART);
+  static_assert((RA == 256 || RA == 128) && (RB == 256 || RB == 128), "row swizzle");
+  constexpr int LDS_BYTES = std::max({OPER_BYTES, STAGE_BYTES, 2 * PARTS_BYTES});
 
   __shared__ uint4 lds[LDS_BYTES / 16];
   uint4* lds_a = lds;                      // [2][BKP][LDA]
@@ -1172,73 +1218,125 @@ __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) 
   // up the dy chunks they stage anyway (every pixel of the split passes through exactly once).
   const bool sum_dy = p.dbias != nullptr && tile_n == 0;
   float bsum[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) bsum[e] = 0.f;
 
-  auto store_tiles = [&](int buf, const Chunk* ra, const Chunk* rb) {
+  auto swz = [](int row_bytes, int row) { return row_bytes == 256 ? (row & 3) << 2 : ((row >> 1) & 1) << 2; };
+  unsigned char* const parts = reinterpret_cast<unsigned char*>(lds);
+  // four channels of one pixel into the three parts of their operand
+  auto store_parts = [&](unsigned char* tile, int part_bytes, int row_bytes, int row, int cc, const Chunk& c) {
+    uint2 w[3];
+    split4(c, w);
+    unsigned char* dst = tile + row * row_bytes + ((cc >> 1) ^ swz(row_bytes, row)) * 16 + (cc & 1) * 8;
 #pragma unroll
-    for (int i = 0; i < A_PT; ++i) lds_a[(buf * BKP + a_prow + i * (NT / CA)) * LDA + a_cc] = ra[i].u;
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<uint2*>(dst + k * part_bytes) = w[k];
+  };
+  // transposing reads: see wgrad_body_direct
+  const int grp = lane >> 4, q16 = lane & 15;
+  const int tr_pix = 8 * (grp >> 1) + (q16 >> 2);
+  auto band = [&](int row_bytes, int w_band) {
+    return tr_pix * row_bytes + ((w_band * 4) ^ swz(row_bytes, tr_pix)) * 16 + (16 * (grp & 1) + 4 * (q16 & 3)) * 2;
+  };
+  auto read_parts = [&](const unsigned char* tile, int part_bytes, int row_bytes, int w_band) {
+    Split8 f;
 #pragma unroll
-    for (int i = 0; i < B_PT; ++i) lds_b[(buf * BKP + b_prow + i * (NT / CB)) * LDB + b_cc] = rb[i].u;
-    if (sum_dy) {
-#pragma unroll
-      for (int i = 0; i < A_PT; ++i) {
-        float v[E];
-        chunk_to_float<T>(ra[i], v);
-#pragma unroll
-        for (int e = 0; e < E; ++e) bsum[e] += v[e];
-      }
+    for (int k = 0; k < 3; ++k) {
+      const unsigned char* src = tile + k * part_bytes + band(row_bytes, w_band);
+      f.part[k] = read_transposed(src, src + 4 * row_bytes);
     }
+    return f;
   };
 
   f32x16_t acc[TM][TN];
+  // the sums of the tile, in `acc`; split_c: on the bf16 pipes, small products in `low`
+  auto reduce = [&](auto split_c, f32x16_t (&low)[TM][TN]) {
+    constexpr bool SPLIT = decltype(split_c)::value;
+    clear(acc);
+    if constexpr (SPLIT) clear(low);
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int e = 0; e < E; ++e) bsum[e] = 0.f;
 
+    auto store_tiles = [&](int buf, const Chunk* ra, const Chunk* rb) {
+      if constexpr (SPLIT) {
+        unsigned char* a_tile = parts + buf * PARTS_BYTES;
+#pragma unroll
+        for (int i = 0; i < A_PT; ++i) store_parts(a_tile, A_PART, RA, a_prow + i * (NT / CA), a_cc, ra[i]);
+#pragma unroll
+        for (int i = 0; i < B_PT; ++i) store_parts(a_tile + 3 * A_PART, B_PART, RB, b_prow + i * (NT / CB), b_cc, rb[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < A_PT; ++i) lds_a[(buf * BKP + a_prow + i * (NT / CA)) * LDA + a_cc] = ra[i].u;
+#pragma unroll
+        for (int i = 0; i < B_PT; ++i) lds_b[(buf * BKP + b_prow + i * (NT / CB)) * LDB + b_cc] = rb[i].u;
+      }
+      if (sum_dy) {
+#pragma unroll
+        for (int i = 0; i < A_PT; ++i) {
+          float v[E];
+          chunk_to_float<T>(ra[i], v);
+#pragma unroll
+          for (int e = 0; e < E; ++e) bsum[e] += v[e];
+        }
+      }
+    };
 
-  auto compute = [&](int buf) {
-    // fp32: one reduction element per lane and MFMA, no transposition needed
-    const float* la = reinterpret_cast<const float*>(lds_a + buf * BKP * LDA);
-    const float* lb = reinterpret_cast<const float*>(lds_b + buf * BKP * LDB);
+    auto compute = [&](int buf) {
+      if constexpr (SPLIT) {
+        const unsigned char* a_tile = parts + buf * PARTS_BYTES;
+        Split8 fb[TN];
 #pragma unroll
-    for (int ks = 0; ks < BKP / 2; ++ks) {
-      const int prow = ks * 2 + (lane >> 5);
-      float fa[TM], fb[TN];
+        for (int tn = 0; tn < TN; ++tn) fb[tn] = read_parts(a_tile + 3 * A_PART, B_PART, RB, wn * TN + tn);
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) fa[tm] = la[prow * (LDA * 4) + (wm * TM + tm) * 32 + (lane & 31)];
+        for (int tm = 0; tm < TM; ++tm) {
+          const Split8 fa = read_parts(a_tile, A_PART, RA, wm * TM + tm);
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) fb[tn] = lb[prow * (LDB * 4) + (wn * TN + tn) * 32 + (lane & 31)];
+          for (int tn = 0; tn < TN; ++tn) mma_split(fb[tn], fa, acc[tm][tn], low[tm][tn]);
+        }
+      } else {
+        // one reduction element per lane and MFMA, no transposition needed
+        const float* la = reinterpret_cast<const float*>(lds_a + buf * BKP * LDA);
+        const float* lb = reinterpret_cast<const float*>(lds_b + buf * BKP * LDB);
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+        for (int ks = 0; ks < BKP / 2; ++ks) {
+          const int prow = ks * 2 + (lane >> 5);
+          float fa[TM], fb[TN];
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-          acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[tn], fa[tm], acc[tm][tn], 0, 0, 0);
-    }
-  };
+          for (int tm = 0; tm < TM; ++tm) fa[tm] = la[prow * (LDA * 4) + (wm * TM + tm) * 32 + (lane & 31)];
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) fb[tn] = lb[prow * (LDB * 4) + (wn * TN + tn) * 32 + (lane & 31)];
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn)
+              acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[tn], fa[tm], acc[tm][tn], 0, 0, 0);
+        }
+      }
+    };
 
-  // Register set 0 carries the even tiles, set 1 the odd ones.  The loop has no
-  // conditionals: tiles past the end of the reduction load as zeros (out-of-range
-  // buffer offsets) and multiply to nothing, so an odd tile count costs one empty step.
-  load_tiles(0, ra0, rb0);
-  load_tiles(1, ra1, rb1);
-  store_tiles(0, ra0, rb0);
-  __syncthreads();
-  load_tiles(2, ra0, rb0);
-  for (int kt = 0; kt < nk; kt += 2) {
-    compute(0);  // tile kt
-    store_tiles(1, ra1, rb1);
-    __syncthreads();
-    load_tiles(kt + 3, ra1, rb1);
-    compute(1);  // tile kt + 1
+    // Register set 0 carries the even tiles, set 1 the odd ones.  The loop has no
+    // conditionals: tiles past the end of the reduction load as zeros (out-of-range
+    // buffer offsets) and multiply to nothing, so an odd tile count costs one empty step.
+    load_tiles(0, ra0, rb0);
+    load_tiles(1, ra1, rb1);
     store_tiles(0, ra0, rb0);
     __syncthreads();
-    load_tiles(kt + 4, ra0, rb0);
+    load_tiles(2, ra0, rb0);
+    for (int kt = 0; kt < nk; kt += 2) {
+      compute(0);  // tile kt
+      store_tiles(1, ra1, rb1);
+      __syncthreads();
+      load_tiles(kt + 3, ra1, rb1);
+      compute(1);  // tile kt + 1
+      store_tiles(0, ra0, rb0);
+      __syncthreads();
+      load_tiles(kt + 4, ra0, rb0);
+    }
+  };
+  f32x16_t low[TM][TN];
+  bool plain = p.k_per_split <= kShortReduction;
+  if (!plain) {
+    reduce(std::true_type{}, low);
+    plain = __syncthreads_or(join_split(acc, low));
   }
-
+  if (plain) reduce(std::false_type{}, low);
 
   float* out = static_cast<float*>(p.out);
   if (p.splits > 1) out += static_cast<int64_t>(split) * p.gemm_m * p.gemm_n;
@@ -1755,7 +1853,7 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 // A step is one 64-byte LDS row per GEMM row (32 bf16 or 16 fp32 elements), laid out as in igemm2_kernel with
 // 32-element steps; in_c must be a multiple of the step.
 template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
-__global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
+__global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int EB = sizeof(T);
   constexpr int BM = TM * 32, BN = TN * 32;
@@ -1854,9 +1952,14 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
 
   // ---- this wavefront's steps: wave, wave + KG, ... as a scalar walk over (tap, channel block) ----
   const int my_steps = nk > wave ? (nk - wave + KG - 1) / KG : 0;
-  int ld_kt = wave, ld_t = wave / cblocks;
-  int ld_cb = wave - ld_t * cblocks;
-  int ld_r = ld_t / p.S, ld_s = ld_t - (ld_t / p.S) * p.S;
+  int ld_kt, ld_t, ld_cb, ld_r, ld_s;
+  auto rewind = [&] {
+    ld_kt = wave;
+    ld_t = wave / cblocks;
+    ld_cb = wave - ld_t * cblocks;
+    ld_r = ld_t / p.S;
+    ld_s = ld_t - ld_r * p.S;
+  };
   unsigned char* ring = lds + wave * (NBUF * BUF_BYTES);
   auto issue_loads = [&](int buf) {
     const int tap_elems = (MODE == kFwd) ? (ld_r * in_w + ld_s) * in_c : -((ld_r >> sl) * in_w + (ld_s >> sl)) * in_c;
@@ -1883,13 +1986,6 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
   };
 
   f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
   const int frag_row = lane & 31, frag_half = lane >> 5;
   const int swz = (frag_row >> 2) & 3;
   const uint32_t ring_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
@@ -1902,51 +1998,87 @@ __global__ __launch_bounds__(KG * 64) void igemm4_kernel(IgemmArgs p) {
     for (int tn = 0; tn < TN; ++tn)
       asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[tn]) : "v"(pa), "n"(A_BYTES + tn * 32 * RB));
   };
-  auto multiply = [&](uint4_t* fa, uint4_t* fb) {
+  auto hold_frags = [&](uint4_t* fa, uint4_t* fb) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(fa[tm]));
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(fb[tn]));
+  };
+  auto chunk = [](const uint4_t& v) {
+    Chunk c;
+    c.h = __builtin_bit_cast(bf16x8_t, v);
+    return c;
+  };
+  auto multiply = [&](uint4_t* fa, uint4_t* fb) {
+    hold_frags(fa, fb);
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        Chunk a, b;
-        a.h = __builtin_bit_cast(bf16x8_t, fa[tm]);
-        b.h = __builtin_bit_cast(bf16x8_t, fb[tn]);
-        mma<T>(b, a, acc[tm][tn]);
-      }
+      for (int tn = 0; tn < TN; ++tn) mma<T>(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
   };
 
   // The tile of step i lands when at most the NBUF-2 tiles requested behind it are outstanding (near the end fewer
   // follow: wait for everything).  The reads of step i-1 were waited for before its multiplies, so its buffer is free.
   constexpr int AHEAD = (NBUF - 2) * (A_LD + B_LD);
   static_assert(AHEAD < 64, "vmcnt range");
-  auto step = [&](int i, int buf) {
-    if (i + NBUF - 1 <= my_steps)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (i + NBUF - 1 < my_steps) issue_loads((buf + NBUF - 1) % NBUF);
-    uint4_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
-    read_frags(buf, 0, fa0, fb0);
-    read_frags(buf, 1, fa1, fb1);
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN) : "memory");
-    multiply(fa0, fb0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    multiply(fa1, fb1);
+  // this wavefront's share of the sums, in `acc`; split_c: in fp32, on the bf16 pipes, small products in `low`
+  auto reduce = [&](auto split_c, f32x16_t (&low)[TM][TN]) {
+    constexpr bool SPLIT = decltype(split_c)::value;
+    rewind();
+    clear(acc);
+    if constexpr (SPLIT) clear(low);
+    auto step = [&](int i, int buf) {
+      if (i + NBUF - 1 <= my_steps)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (i + NBUF - 1 < my_steps) issue_loads((buf + NBUF - 1) % NBUF);
+      uint4_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+      read_frags(buf, 0, fa0, fb0);
+      read_frags(buf, 1, fa1, fb1);
+      if constexpr (SPLIT) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        hold_frags(fa0, fb0);
+        hold_frags(fa1, fb1);
+        Split8 sb[TN];
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) sb[tn] = split8(chunk(fb0[tn]), chunk(fb1[tn]));
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const Split8 sa = split8(chunk(fa0[tm]), chunk(fa1[tm]));
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) mma_split(sb[tn], sa, acc[tm][tn], low[tm][tn]);
+        }
+      } else {
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN) : "memory");
+        multiply(fa0, fb0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        multiply(fa1, fb1);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < NBUF - 1; ++i)
+      if (i < my_steps) issue_loads(i);
+    int i0 = 0;
+    for (; i0 + NBUF <= my_steps; i0 += NBUF) {
+#pragma unroll
+      for (int u = 0; u < NBUF; ++u) step(i0 + u, u);
+    }
+#pragma unroll
+    for (int u = 0; u < NBUF - 1; ++u)
+      if (i0 + u < my_steps) step(i0 + u, u);
   };
-#pragma unroll
-  for (int i = 0; i < NBUF - 1; ++i)
-    if (i < my_steps) issue_loads(i);
-  int i0 = 0;
-  for (; i0 + NBUF <= my_steps; i0 += NBUF) {
-#pragma unroll
-    for (int u = 0; u < NBUF; ++u) step(i0 + u, u);
+  if constexpr (sizeof(T) == 4) {
+    f32x16_t low[TM][TN];
+    bool plain = p.gemm_k <= kShortReduction;
+    if (!plain) {
+      reduce(std::true_type{}, low);
+      plain = __any(join_split(acc, low));
+    }
+    if (plain) reduce(std::false_type{}, low);
+  } else {
+    reduce(std::false_type{}, acc);
   }
-#pragma unroll
-  for (int u = 0; u < NBUF - 1; ++u)
-    if (i0 + u < my_steps) step(i0 + u, u);
 
   // ---- the partial tiles meet: [wave][BM][LD] fp32, over the rings ----
   float* red = reinterpret_cast<float*>(lds);
@@ -2660,9 +2792,9 @@ const TileCost kSumsCost[] = {
     {kPipe64, 64, 64, 5.75f, 1.60f, 0.276f, 0.163f, 0.68f}, {kMix128x64, 128, 64, 4.52f, 4.11f, 0.256f, 0.316f, 0.74f},
     {kMix128, 128, 128, 3.63f, 5.89f, 0.446f, 0.382f, 0.83f}};
 // fp32 where the output has fewer than one and a half 128 x 128 tiles per compute unit: the reduction is split inside the
-// workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 multiplies at 1/16 of the bf16 rate, so it
-// gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us).  -1: none of them.
-// The lines, with mean times over the layers of the three models in each class (244 launches), the choice = 1:
+// workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 takes at least six times the multiplies of bf16, so it
+// gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us, with fp32 multiplies).  -1: none of them.
+// The lines, with mean times over the layers of the three models in each class (244 launches, fp32 multiplies), the choice = 1:
 //   up to one 32 x 32 tile per CU, K >= 1024 (53): eight wavefronts; four 1.11.  K < 1024 (25): four; eight 1.01
 //   up to two, K < 1536 (38): 32 x 32 on four; eight 1.05, 64 x 32 1.05.  Two such tiles on a CU hide each other's
 //     latencies until the reduction is long enough to do so alone: K >= 1536 (9) 64 x 32 on eight; 32 x 32 on eight 1.02, four 1.05
@@ -2844,6 +2976,7 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.k_per_split = (a.gemm_k + 31) / 32 * 32;
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
+  a.in_fp32 = tile_cfg == kAutoInOrder ? 1 : 0;
   if (tile_cfg < 0) {
     tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false});
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
@@ -2940,8 +3073,8 @@ int64_t conv2d_wgrad_workspace_bytes(const ConvShape& s, int dtype, int splits) 
 }
 
 // tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups, in fp32 1024
-// (TCH_WGRAD_BIG_TILE_WGS: another count).  An fp32 gradient is bound by the matrix pipes: 144 workgroups of 128 x 128 use
-// those of 144 compute units, and their 36 KB of LDS (64 x 64: 20) keep main-lane workgroups away.  In the step, from 128 /
+// (TCH_WGRAD_BIG_TILE_WGS: another count).  An fp32 gradient takes its operands apart for six multiplies: 144 workgroups of 128 x 128 use
+// those of 144 compute units, and their 52 KB of LDS (64 x 64: 28) keep main-lane workgroups away.  In the step (fp32 multiplies), from 128 /
 // 256 / 512 / 1024 / 2000 on / never: GPT-2 2 x 256 6.48 / 6.39 / 6.22 / 6.22 / 6.19 / 6.25 ms, 1 x 512 7.34 / 6.98 / 6.88 / 6.88 /
 // 6.86 / 6.89, 8 x 512 31.48 / 31.50 / 31.56 / 31.50 / 31.94 / 31.88.
 bool wgrad_big_tile(int dtype, int gemm_m, int gemm_n, int64_t splits) {

@@ -1,0 +1,115 @@
+// fp32 products on the bf16 matrix pipes.
+//
+// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of mantissa): x = x0 + x1 + x2 with x0 = x rounded to
+// bf16, x1 = the rest rounded to bf16, x2 = what is left.  Of the nine products of two such sums the three smallest
+// (x1 y2, x2 y1, x2 y2, below 2^-26 of the product) are left out; the other six go through v_mfma_f32_32x32x16_bf16, which
+// accumulates in fp32: 192 cycles for a 32 x 32 x 16 product instead of the 512 of eight v_mfma_f32_32x32x2_f32.
+//
+// Error: the five small products have an accumulator of their own, 2^-8 of the size of the other, so that the large one is
+// rounded once per 16 reduction elements (fp32 MFMA: once per element).  Norm of the error against 64 bits over the norm of the
+// result, one wavefront, in units of 1e-7, with fp32 MFMA and in parts (in parts with one accumulator):
+//   normal x normal over 64 / 768 / 4608:  1.4 / 4.9 / 12.2   and 0.5 / 1.6 / 4.2 (1.1 / 4.2 / 10.6)
+//   ReLU'd x normal:                       1.0 / 3.5 / 8.6    and 0.4 / 1.2 / 3.5 (1.1 / 4.0 / 9.9)
+// Rounding the parts matters: cut off instead, they leave out products of one sign (uniform x uniform over 4608: 116 for 6.3).
+// Time: taking a pair of values apart is 11 vector instructions, which pass behind the multiplies; what is left of a small product is
+// its operands' way to the CU (the same 21 us of 26 without the split and five of the six multiplies).
+// Alone, before and after: 512 x 768 over 3072 31.0 -> 25.6 us, 512 x 3072 over 768 25.3 -> 22.1, weight gradient 768 x 3072 over 512
+// 29.7 -> 24.0, output head 512 x 50304 over 768 334 -> 275; GPT-2 2 x 256 6.14 -> 5.39 ms, ResNet-152 of 4 images 7.11 -> 6.60.
+// Range: bf16 has the exponents of fp32, so nothing overflows that fp32 holds except values that round to 2^128 (see below), and
+// below 2^-110 (7.7e-34) the last parts of a value are bf16 denormals: such an operand keeps an absolute error of up to 2^-134.
+// Infinities, NaN and values that round to 2^128 come out as NaN (inf - inf): a kernel that finds a NaN among its sums adds
+// them up again with fp32 MFMA, whose result counts then.
+#pragma once
+
+#include "kernels.h"
+
+namespace tch {
+
+struct Split8 {
+  bf16x8_t part[3];
+};
+
+// a pair of values into the bits of its parts
+__device__ inline void split_pair(float v0, float v1, uint32_t (&w)[3]) {
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const f32x2_t v = {v0, v1};
+    w[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+    if (k < 2) {   // exact
+      v0 -= __uint_as_float(w[k] << 16);
+      v1 -= __uint_as_float(w[k] & 0xffff0000u);
+    }
+  }
+}
+
+__device__ inline void split4(const Chunk& c, uint2 (&w)[3]) {
+  uint32_t a[3], b[3];
+  split_pair(c.f[0], c.f[1], a);
+  split_pair(c.f[2], c.f[3], b);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) w[k] = make_uint2(a[k], b[k]);
+}
+
+// eight reduction elements of one operand row: `lo` and `hi` are two chunks of four
+__device__ inline Split8 split8(const Chunk& lo, const Chunk& hi) {
+  Split8 s;
+  uint2 a[3], b[3];
+  split4(lo, a);
+  split4(hi, b);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    Chunk c;
+    c.u = make_uint4(a[k].x, a[k].y, b[k].x, b[k].y);
+    s.part[k] = c.h;
+  }
+  return s;
+}
+
+// Eight reduction elements of one column of bf16 values that lie [reduction][column] in LDS: ds_read_b64_tr_b16 hands a lane
+// four of them, from the addresses of its group of 16 lanes.
+__device__ inline bf16x8_t read_transposed(const unsigned char* first, const unsigned char* second) {
+  typedef short s16x4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4_t* lds_ptr;
+  const s16x4_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)first), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)second);
+  return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// large += x0 y0; small += the five products next in size
+__device__ inline void mma_split(const Split8& x, const Split8& y, f32x16_t& large, f32x16_t& small) {
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[0], y.part[2], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[2], y.part[0], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[1], small, 0, 0, 0);
+  large = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[0], y.part[0], large, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[0], y.part[1], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[0], small, 0, 0, 0);
+}
+
+// large += small; whether any sum of this lane is NaN
+template <int TM, int TN>
+__device__ inline bool join_split(f32x16_t (&large)[TM][TN], const f32x16_t (&small)[TM][TN]) {
+  bool nan = false;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        large[i][j][e] += small[i][j][e];
+        nan |= large[i][j][e] != large[i][j][e];
+      }
+  return nan;
+}
+
+template <int TM, int TN>
+__device__ inline void clear(f32x16_t (&acc)[TM][TN]) {
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+}
+
+}  // namespace tch

@@ -1,0 +1,65 @@
+"""fp32 products in bf16 parts: as accurate as fp32, on every kernel that takes them, and with infinities, NaN and values next
+to the largest one what fp32 makes of them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TILINGS = [-1, 0, 1, 2, 15, 16, 17, 18, 19, 20]
+
+
+def product(op, rows, cols, depth, tile_cfg, a, b):
+    """a [rows, depth] times b [cols, depth] transposed, through the forward convolution, the data or the weight gradient"""
+    from sirius_amd import ops
+    ctx = ops.Context()
+    if op == "fwd":
+        y = torch.empty(rows, 1, 1, cols, device="cuda")
+        ops.conv2d_fwd(ctx, a.view(rows, 1, 1, depth), b.view(cols, 1, 1, depth), y, 1, 0, tile_cfg=tile_cfg)
+    elif op == "dgrad":
+        y = torch.empty(rows, 1, 1, cols, device="cuda")
+        ops.conv2d_dgrad(ctx, a.view(rows, 1, 1, depth), b.view(cols, 1, 1, depth), y, 1, 0, tile_cfg=tile_cfg)
+    else:
+        y = torch.empty(rows, 1, 1, cols, device="cuda")
+        ops.conv2d_wgrad(ctx, b.t().contiguous().view(depth, 1, 1, cols), a.t().contiguous().view(depth, 1, 1, rows), y, 1, 0, splits=1,
+                         tile_cfg=tile_cfg)
+    torch.cuda.synchronize()
+    return y.view(rows, cols)
+
+
+# depths on both sides of the line, with and without a remainder for the steps, the wavefronts and the LDS tiles
+CASES = [(op, rows, cols, depth) for op in ("fwd", "dgrad", "wgrad")
+         for rows, cols, depth in ((36, 40, 128), (36, 40, 144), (132, 200, 272), (64, 64, 1024), (260, 132, 656))]
+
+
+@pytest.mark.parametrize("tile_cfg", TILINGS)
+@pytest.mark.parametrize("op,rows,cols,depth", CASES)
+def test_error_is_that_of_fp32(op, rows, cols, depth, tile_cfg):
+    """Per value: every one of at most `depth` additions rounds by 2^-24 of a partial sum, which the sum of |a b| bounds, the
+    parts leave out at most 2^-25 of every product and their own sum is 2^-8 as large."""
+    g = torch.Generator().manual_seed(depth + rows)
+    a = torch.randn(rows, depth, generator=g).mul_(torch.exp(2 * torch.randn(rows, depth, generator=g)))
+    b = torch.randn(cols, depth, generator=g)
+    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).double().cpu()
+    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
+    # and over the whole result what sums of independent roundings have, not what the bound above allows
+    assert (got - want).norm() <= 4 * 2.0 ** -24 * max(1, depth / 64) ** 0.5 * want.norm()
+
+
+@pytest.mark.parametrize("tile_cfg", TILINGS)
+@pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
+def test_infinities_nan_and_the_largest_values(op, tile_cfg):
+    rows, cols, depth = 68, 72, 272
+    g = torch.Generator().manual_seed(1)
+    a, b = torch.randn(rows, depth, generator=g), torch.randn(cols, depth, generator=g)
+    inf, largest = float("inf"), torch.finfo(torch.float32).max
+    a[3, 17], a[9, 200], a[33, 5], a[40, 271] = inf, float("nan"), largest, -largest
+    a[50, 3], a[50, 100] = inf, -inf
+    b[20, 17], b[21, 5], b[:, 271] = 0.0, 0.5, b[:, 271].clamp(-0.9, 0.9)
+    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).cpu()
+    want = a.double() @ b.double().t()
+    want = torch.where(want.abs() > largest, torch.sign(want) * inf, want)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[got.isinf()].double(), want[want.isinf()])
+    ok = want.isfinite()
+    size = (torch.where(a.isfinite(), a, 0).double().abs() @ b.double().abs().t())[ok]
+    assert ((got.double() - want)[ok].abs() <= (depth + 2) * 2.0 ** -24 * size).all()
