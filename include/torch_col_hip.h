@@ -155,7 +155,8 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * out_f32 != 0 stores y as fp32 whatever dtype is.  tile_cfg: -1 auto: the choice, and with it the order a reduction is
  * added up in, follows the number of rows, so a sample's result may differ in rounding with the samples batched beside it
  * (bf16 ResNet-152 logits by about 2e-3).  -2 auto among the tilings that add up a reduction front to back (a row's result
- * does not depend on the number of rows).  0 = 128x128, 1 = 128x64, 2 = 64x64,
+ * does not depend on the number of rows).  -3 and -4: the same two for the linear layers of a transformer, which leave the
+ * choice the persistent kernel as well (25 - 27; front to back).  0 = 128x128, 1 = 128x64, 2 = 64x64,
  * 3 = 64x64 on the register-staged kernel even where the direct-to-LDS kernel applies, 5 = 128x64 with the
  * activation side of all nine taps of a channel block held in LDS as one patch (bf16, 3x3, stride 1, pad 1,
  * channels a multiple of 64, rows of at most 63 pixels; any other convolution runs tiling 1 for it).  The patch
@@ -167,6 +168,9 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * 21 = 64x64 with the operand reads pipelined over the reduction steps, 22 / 23 / 24 = 128x64, 128x128 and 128x192 with
  * reads, loads and multiplies interleaved on eight wavefronts, as tiling 0 has them (bf16, input channels a multiple of 64;
  * anything else runs tilings 2, 1, 0 and 0 for them; same bits as those).
+ * 25 / 26 / 27 = 128x192, 128x128 and 256x128 on a persistent grid of at most one workgroup per CU, the tiles of a workgroup one
+ * sequence of reduction steps (bf16, 1x1 stride 1, input channels a multiple of 64, bias and add as the only operands beside x and
+ * w, output in bf16; anything else runs tilings 24, 23 and 23 for them; same bits as those).
  * c_logical: input channels that carry data when C is zero-padded to a chunk (0 = C); it only enters the
  * algorithmic-work figure the profiler reports, never the arithmetic. */
 int tch_conv2d_fwd(tch_context* ctx, int dtype, const void* x, const void* w, void* y, const void* add,

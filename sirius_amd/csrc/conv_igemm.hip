@@ -130,6 +130,7 @@ __device__ inline void mma<float>(const Chunk& first, const Chunk& second, f32x1
 // returns zeros, so padding, ragged edges and the tail of the reduction need neither a
 // branch nor a select, and the loads stay in flight across the multiply of earlier tiles.
 typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
 constexpr uint32_t kOutOfRange = 0x80000000u;
 
 __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
@@ -1003,7 +1004,6 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
   for (int t = 0; t < TM; ++t) rd_a[t] = lds_base + band(RA, wm * TM + t, swz_a(tr_pix));
 #pragma unroll
   for (int t = 0; t < TN; ++t) rd_b[t] = lds_base + A_BYTES + band(RB, wn * TN + t, swz_b(tr_pix));
-  typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
   constexpr int SL = BKP / 16;
   uint2_t fa[SL][TM][2], fb[SL][TN][2];
   // rows + 16 and + 4 keep the row's swizzle (a multiple of four rows)
@@ -1839,6 +1839,262 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm2_kernel(IgemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+// forward / data gradient of a 1x1 layer, bf16, on a persistent grid: a workgroup walks several output tiles
+// ---------------------------------------------------------------------------
+// igemm2_kernel's interleaved loop (ROT = 1) with the tiles of a workgroup as ONE sequence of reduction steps: the loads of the
+// next tile's first steps go out during this tile's last ones, its first operands are read behind this tile's last multiplies,
+// and the output leaves straight from the accumulators, so that between two tiles there is neither a trip to memory nor a barrier
+// nor LDS taken from the operands.  Over 768 reduction elements (12 steps) that used to be 4 us of a tile's 12.
+// Alone, the fastest of the other tilings and 128 x 192 here: 8192 x 2304 over 768 38.4 -> 32.1 us, 8192 x 3072 46.3 -> 40.7 (256 x 128 the
+// same), 8192 x 768 13.8 -> 12.5, over 3072 36.4 -> 34.9; 25088 x 768 over 256 20.3 -> 18.7, 6272 x 1536 over 512 18.4 -> 15.9.
+// GPT-2 8 x 1024 11.72 -> 11.26 ms, 4 x 1024 7.40 -> 6.90, Swin-B of 32 images 9.85 -> 9.74.
+// What bounds it now is power: on operands that are all zeros 8192 x 768 over 3072 takes 28 us, on random ones 38 on the same
+// machine.  A fourth LDS tile gained nothing.  fp32 outputs lose here (an output head 790 us as 256 x 256, 842 so).
+template <int WM, int WN, int TM, int TN, int NBUF>
+__global__ __launch_bounds__(WM* WN * 64) void igemm5_kernel(IgemmArgs p) {
+  constexpr int E = 8, KS = kStep2, RB = kRowBytes2, SL = KS / 16;
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32, NW = WM * WN;
+  constexpr int A_LD = BM / 8 / NW, B_LD = BN / 8 / NW, LOADS = A_LD + B_LD;   // direct loads (eight rows each) per wave and step
+  static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile/loader mismatch");
+  constexpr int A_BYTES = BM * RB, BUF_BYTES = A_BYTES + BN * RB;
+  // The bias of a wavefront's columns travels with the operands: requested with the first step of a tile, which is up to NBUF
+  // tiles ahead of the epilogue that adds it.
+  constexpr int BIAS_BYTES = TN * 32 * 4, BIAS_OFF = NBUF * BUF_BYTES;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[BIAS_OFF + NW * (NBUF + 1) * BIAS_BYTES];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int frag_row = lane & 31, frag_half = lane >> 5;
+  const int nk = p.gemm_k / KS;
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int first = static_cast<int>(xcd_remap(blockIdx.x, gridDim.x));
+
+  auto locate = [&](int id, int& m0, int& n0) {   // the order of igemm2_kernel, within every round of workgroups
+    int tile_m, tile_n;
+    if (p.group_rows > 1) {
+      const int per_group = p.group_rows * p.tiles_n;
+      const int grp = id / per_group, local = id - grp * per_group, row0 = grp * p.group_rows;
+      const int rows = min(p.group_rows, p.tiles_m - row0);
+      tile_n = local / rows;
+      tile_m = row0 + (local - tile_n * rows);
+    } else {
+      tile_m = id / p.tiles_n;
+      tile_n = id - tile_m * p.tiles_n;
+    }
+    m0 = tile_m * BM;
+    n0 = tile_n * BN;
+  };
+
+  const __amdgpu_buffer_rsrc_t rsrc_a = make_rsrc(p.a_src, p.a_bytes);
+  const __amdgpu_buffer_rsrc_t rsrc_b = make_rsrc(p.b_src, p.b_bytes);
+  const __amdgpu_buffer_rsrc_t rsrc_bias = make_rsrc(p.bias, p.bias ? static_cast<uint32_t>(p.gemm_n) * 4u : 0u);
+
+  // ---- the walk of the loads: the lane's rows of tile ld_id, step ld_kt; behind the last tile every offset is out of range ----
+  const int sub_row = lane >> 3, slot = lane & 7;
+  int a_off[A_LD], b_off[B_LD];
+  int ld_id = first, ld_kt = 0, ld_bias = 0;
+  auto enter_tile = [&] {
+    int m0 = 0, n0 = 0;
+    const bool any = ld_id < tiles;
+    if (any) locate(ld_id, m0, n0);
+#pragma unroll
+    for (int j = 0; j < A_LD; ++j) {
+      const int trow = (wave * A_LD + j) * 8 + sub_row, row = m0 + trow;
+      a_off[j] = any && row < p.gemm_m ? (row * p.gemm_k + (slot ^ ((trow >> 1) & 7)) * E) * 2 : static_cast<int>(kOutOfRange);
+    }
+#pragma unroll
+    for (int j = 0; j < B_LD; ++j) {
+      const int trow = (wave * B_LD + j) * 8 + sub_row, row = n0 + trow;
+      b_off[j] = any && row < p.gemm_n ? (row * p.gemm_k + (slot ^ ((trow >> 1) & 7)) * E) * 2 : static_cast<int>(kOutOfRange);
+    }
+    if (p.bias) {
+      unsigned char* dst = lds + BIAS_OFF + (wave * (NBUF + 1) + ld_bias) * BIAS_BYTES;
+      const int col = n0 + wn * TN * 32 + lane * 4;
+      if (lane < TN * 8) load_to_lds(rsrc_bias, dst, any && col < p.gemm_n ? col * 4 : static_cast<int>(kOutOfRange), 0);
+      ld_bias = ld_bias == NBUF ? 0 : ld_bias + 1;
+    }
+  };
+  auto issue_load = [&](uint32_t buf, int j) {   // direct load j of the step the walk stands at
+    if (j < A_LD)
+      load_to_lds(rsrc_a, lds + buf + (wave * A_LD + j) * 1024, a_off[j], ld_kt * RB);
+    else
+      load_to_lds(rsrc_b, lds + buf + A_BYTES + (wave * B_LD + j - A_LD) * 1024, b_off[j - A_LD], ld_kt * RB);
+  };
+  auto next_step = [&] {
+    if (++ld_kt == nk) {
+      ld_kt = 0;
+      ld_id += gridDim.x;
+      enter_tile();
+    }
+  };
+
+  f32x16_t acc[TM][TN];
+  clear(acc);
+  const int swz = (frag_row >> 1) & 7;
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+  const uint32_t a_rd = lds_base + (wm * TM * 32 + frag_row) * RB + swz * 16;
+  const uint32_t b_rd = lds_base + A_BYTES + (wn * TN * 32 + frag_row) * RB + swz * 16;
+  uint4_t fa[2][TM], fb[2][TN];
+  auto read_one = [&](uint32_t pa, uint32_t pb, int set, int i) {   // operand i (of the TM + TN) of a slice
+    if (i < TM)
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][i]) : "v"(pa), "n"(i * 32 * RB));
+    else
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][i - TM]) : "v"(pb), "n"((i - TM) * 32 * RB));
+  };
+  auto hold_set = [&](int set) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(fa[set][i]));
+#pragma unroll
+    for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(fb[set][i]));
+  };
+  // as in igemm2_kernel: multiplies the slice in `set`; meanwhile slice kk of the step in `buf` is read into the other set and
+  // part `q` of the loads goes to `ld_buf`
+  auto slice = [&](auto set_c, uint32_t buf, auto kk_c, auto q_c, uint32_t ld_buf) {
+    constexpr int set = decltype(set_c)::value, kk = decltype(kk_c)::value, q = decltype(q_c)::value;
+    constexpr int READS = TM + TN, FIRST = q * LOADS / SL, MF = TM * TN;
+    constexpr int AUX = READS + (q + 1) * LOADS / SL - FIRST;
+    constexpr int PER = (AUX + MF - 1) / MF > 2 ? (AUX + MF - 1) / MF : 2;
+    const uint32_t pa = (a_rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16)) + buf;
+    const uint32_t pb = (b_rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16)) + buf;
+    unrolled<MF>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value, tm = m / TN, tn = m % TN;
+      acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, fb[set][tn]),
+                                                            __builtin_bit_cast(bf16x8_t, fa[set][tm]), acc[tm][tn], 0, 0, 0);
+      unrolled<PER>([&](auto a_c) {
+        constexpr int a = m * PER + decltype(a_c)::value;
+        if constexpr (a < READS) read_one(pa, pb, set ^ 1, a);
+        else if constexpr (a < AUX) issue_load(ld_buf, FIRST + a - READS);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_set(set ^ 1);
+  };
+
+  // ---- the output: a lane's accumulators are four consecutive columns of one row at a time; two lanes 32 apart exchange every
+  // second group so that each stores 16 bytes of bf16 ----
+  // The addend of a tile is requested a whole tile ahead (a request behind the last multiply cost 4 us a tile).
+  uint2_t add[TM][TN][4];
+  const __amdgpu_buffer_rsrc_t rsrc_add = make_rsrc(p.add, static_cast<uint32_t>(p.gemm_m) * p.gemm_n * 2u);
+  auto request_add = [&](int id) {
+    if (!p.add || id >= tiles) return;
+    int m0, n0;
+    locate(id, m0, n0);
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int row = m0 + (wm * TM + tm) * 32 + frag_row, col = n0 + (wn * TN + tn) * 32 + 8 * j + 4 * frag_half;
+          add[tm][tn][j] = __builtin_amdgcn_raw_buffer_load_b64(
+              rsrc_add, row < p.gemm_m && col < p.gemm_n ? (row * p.gemm_n + col) * 2 : static_cast<int>(kOutOfRange), 0, 0);
+        }
+  };
+  int bias_at = 0;
+  auto epilogue = [&](int id) {
+    int m0, n0;
+    locate(id, m0, n0);
+    const int col0 = n0 + wn * TN * 32;
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      float bias[16];
+      if (p.bias) {
+        uint4_t b[4];
+        const uint32_t at = lds_base + BIAS_OFF + (wave * (NBUF + 1) + bias_at) * BIAS_BYTES + tn * 128 + frag_half * 16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b[j]) : "v"(at), "n"(j * 32));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          asm volatile("" : "+v"(b[j]));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) bias[4 * j + i] = __uint_as_float(b[j][i]);
+        }
+      }
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm) {
+        const int row = m0 + (wm * TM + tm) * 32 + frag_row;
+        float v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          v[e] = acc[tm][tn][e];
+          acc[tm][tn][e] = 0.f;
+        }
+        if (p.bias) {
+#pragma unroll
+          for (int e = 0; e < 16; ++e) v[e] += bias[e];
+        }
+        const int64_t at = static_cast<int64_t>(row) * p.gemm_n + col0 + tn * 32;
+        if (p.add) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint2_t u = add[tm][tn][j];
+            v[4 * j] += __uint_as_float(u[0] << 16);
+            v[4 * j + 1] += __uint_as_float(u[0] & 0xffff0000u);
+            v[4 * j + 2] += __uint_as_float(u[1] << 16);
+            v[4 * j + 3] += __uint_as_float(u[1] & 0xffff0000u);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j += 2) {
+          const Chunk c = float_to_chunk<bf16>(v + 4 * j);   // words 0, 1: group j; 2, 3: group j + 1
+          const auto x = __builtin_amdgcn_permlane32_swap(c.w[0], c.w[2], false, false);
+          const auto y = __builtin_amdgcn_permlane32_swap(c.w[1], c.w[3], false, false);
+          const int cc = 8 * (j + frag_half);
+          if (row < p.gemm_m && col0 + tn * 32 + cc < p.gemm_n)
+            *reinterpret_cast<uint4*>(static_cast<bf16*>(p.out) + at + cc) = make_uint4(x[0], y[0], x[1], y[1]);
+        }
+      }
+    }
+    bias_at = bias_at == NBUF ? 0 : bias_at + 1;
+    return m0 + BM <= p.gemm_m && n0 + BN <= p.gemm_n;   // every lane stored everything
+  };
+
+  constexpr int AHEAD = (NBUF - 2) * LOADS;
+  constexpr int STORES = TM * TN * 2;   // of a bf16 epilogue, at least
+  request_add(first);
+  enter_tile();
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) issue_load(s * BUF_BYTES, j);
+    next_step();
+  }
+#pragma unroll
+  for (int j = 0; j < LOADS / SL; ++j) issue_load((NBUF - 1) * BUF_BYTES, j);
+  wait_and_meet<AHEAD + LOADS / SL>();
+#pragma unroll
+  for (int i = 0; i < TM + TN; ++i) read_one(a_rd ^ static_cast<uint32_t>(frag_half * 16), b_rd ^ static_cast<uint32_t>(frag_half * 16), 0, i);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  hold_set(0);
+  uint32_t buf = 0, before = (NBUF - 1) * BUF_BYTES;
+  bool stored = false;
+  for (int id = first; id < tiles; id += gridDim.x) {
+    for (int kt = 0; kt < nk; ++kt) {
+      unrolled<SL - 1>([&](auto s_c) {
+        constexpr int s = decltype(s_c)::value;
+        slice(std::integral_constant<int, (s & 1)>{}, buf, std::integral_constant<int, s + 1>{}, std::integral_constant<int, s + 1>{}, before);
+      });
+      next_step();
+      // behind an epilogue its stores are among the newest requests
+      if (stored && kt == 0)
+        wait_and_meet<AHEAD + STORES>();
+      else
+        wait_and_meet<AHEAD>();
+      before = buf;
+      buf = buf == (NBUF - 1) * BUF_BYTES ? 0 : buf + BUF_BYTES;
+      slice(std::integral_constant<int, ((SL - 1) & 1)>{}, buf, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, before);
+    }
+    stored = epilogue(id);
+    request_add(id + gridDim.x);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the zeros behind the last tile land before the LDS goes
+}
+
+// ---------------------------------------------------------------------------
 // forward / data gradient where the grid of output tiles cannot fill the chip (fp32: where it has fewer than one and a
 // half 128 x 128 tiles per compute unit): the reduction is dealt out to the KG wavefronts of a workgroup
 // ---------------------------------------------------------------------------
@@ -2478,6 +2734,23 @@ int launch_cfg2(Context* ctx, IgemmArgs& a, double flops) {
                 name.c_str(), flops, 0, conv_bytes<MODE>(a, 2));
 }
 
+template <int MODE, int WM, int WN, int TM, int TN, int NBUF>
+int launch_cfg5(Context* ctx, IgemmArgs& a, double flops) {
+  constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
+  static const std::string name = std::string("igemm5_kernel<bf16,") + (MODE == kFwd ? "fwd," : "dgrad,") + std::to_string(BM) + "x" +
+                                  std::to_string(BN) + "," + std::to_string(NBUF) + "buf,persistent>";
+  a.tiles_m = (a.gemm_m + BM - 1) / BM;
+  a.tiles_n = (a.gemm_n + BN - 1) / BN;
+  a.group_rows = a.tiles_n > 8 ? 4 : 0;
+  const int64_t tiles = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
+  if (tiles <= 0 || tiles > 0x3fffffff) {
+    set_error("igemm: grid out of range");
+    return -22;
+  }
+  return launch(ctx, igemm5_kernel<WM, WN, TM, TN, NBUF>, dim3(static_cast<unsigned>(std::min<int64_t>(tiles, 256))), dim3(WM * WN * 64), a,
+                name.c_str(), flops, 0, conv_bytes<MODE>(a, 2));
+}
+
 template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
 int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
   constexpr int BM = TM * 32, BN = TN * 32;
@@ -2571,6 +2844,18 @@ enum PipeTile : int {
   kMix128x192 = 24,   // 128 x 192, three
 };
 
+// Tilings of igemm5_kernel (persistent grid, interleaved, eight wavefronts, three LDS tiles).  What the kernel does not take
+// runs as kMix128x192 or kMix128, which have the same row tiles (no statistics are taken by kWalk256x128).
+enum WalkTile : int {
+  kWalk128x192 = 25,
+  kWalk128 = 26,       // 128 x 128
+  kWalk256x128 = 27,
+};
+bool walk_tile_fits(const IgemmArgs& a) {
+  return igemm2_setting() != 0 && a.pointwise && a.gemm_k % kStep2 == 0 && !a.out_f32 && !a.scale && !a.relu_out && !a.mask && !a.add_sub &&
+         !a.stats && !a.stat_acc;
+}
+
 // the tiling of the same shape that runs where a pipelined one does not exist
 int pipe_stand_in(int tile_cfg) { return tile_cfg == kPipe64 ? 2 : tile_cfg == kMix128x64 ? 1 : 0; }
 
@@ -2586,6 +2871,9 @@ int wgrad_tile(int tile_cfg) {
     case 12:
     case kMix128:
     case kMix128x192:
+    case kWalk128x192:
+    case kWalk128:
+    case kWalk256x128:
       return 0;
     case 1:
     case 5:
@@ -2641,6 +2929,14 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
     // 9 / 10: 256 x 256 on eight wavefronts (128 x 64 each), two LDS tiles, plain / rotated loop: for products with a
     // thousand such tiles or more (65 536 x 4096 x 4096: 1.18 and 1.31 PFLOP/s, 1.03 for 128 x 128; slower than 128 x 128 on
     // the other layers of the three models, by up to 1.7x)
+    if (tile_cfg >= kWalk128x192) {
+      if (walk_tile_fits(a)) {
+        if (tile_cfg == kWalk128x192) return launch_cfg5<MODE, 4, 2, 1, 3, 3>(ctx, a, flops);
+        if (tile_cfg == kWalk128) return launch_cfg5<MODE, 4, 2, 1, 2, 3>(ctx, a, flops);
+        return launch_cfg5<MODE, 4, 2, 2, 2, 3>(ctx, a, flops);
+      }
+      tile_cfg = tile_cfg == kWalk128x192 ? kMix128x192 : kMix128;
+    }
     if (tile_cfg == 9 || tile_cfg == 10) {
       if (setting != 0 && in_c % kStep2 == 0 && a.R * a.S <= 32)
         return tile_cfg == 9 ? launch_cfg2<MODE, 2, 4, 4, 2, 2>(ctx, a, flops) : launch_cfg2<MODE, 2, 4, 4, 2, 2, 1>(ctx, a, flops);
@@ -2818,14 +3114,29 @@ int split_tile(int dtype, int gemm_m, int gemm_n, int gemm_k, int in_c, int taps
 // The tiling the library takes by itself.  kAutoInOrder: one that adds up every reduction front to back, as all but the
 // split ones do, so that a row's result is the same bits whatever the number of rows.  (The patch kernel, tiling 5, has
 // an order of its own: never with kAutoInOrder.)
-constexpr int kAutoInOrder = -2;
+// kAutoLinear, kAutoLinearInOrder: for the linear layers of a transformer, the same two and igemm5_kernel, whose
+// order of additions is front to back.
+constexpr int kAutoInOrder = -2, kAutoLinear = -3, kAutoLinearInOrder = -4;
+bool asks_in_order(int asked) { return asked == kAutoInOrder || asked == kAutoLinearInOrder; }
 struct TileQuery {
   int dtype, gemm_m, gemm_n, gemm_k, in_c, taps;
   bool patch;   // the 3x3 patch kernel fits
   bool sums;    // data gradient with the BatchNorm sums in its epilogue
   bool dgrad;
+  bool walk = false;   // igemm5_kernel takes it
 };
+// igemm5_kernel's tilings, priced as kPlainCost (r = tiles of a workgroup, one of them on a CU).  Fits to the linear layers of GPT-2 at 1024-
+// 8192 tokens and of Swin-B at 4-32 images where they stand, 220 different ones with each tiling (mean error 5-8 %): first
+// the forward ones, which add a bias and often a residual, then the data gradients.  Of 18.2 ms of forward launches with the tilings
+// above 17.2 are left with this choice (17.1 with the fastest of every launch), of 20.8 ms of data gradients 19.3 (19.3).
+const TileCost kWalkCost[2][3] = {
+    {{kWalk128x192, 128, 192, 7.58f, 0.39f, 0.730f, 0.696f, 0.32f}, {kWalk128, 128, 128, 7.42f, 0.00f, 0.541f, 0.510f, 0.42f},
+     {kWalk256x128, 256, 128, 7.44f, 0.42f, 0.734f, 0.734f, 0.46f}},
+    {{kWalk128x192, 128, 192, 7.14f, 0.52f, 0.693f, 0.693f, 0.23f}, {kWalk128, 128, 128, 6.81f, 0.07f, 0.538f, 0.538f, 0.36f},
+     {kWalk256x128, 256, 128, 6.97f, 0.47f, 0.733f, 0.733f, 0.43f}}};
 int heuristic_tile(int asked, const TileQuery& q) {
+  const bool linear = asked == kAutoLinear || asked == kAutoLinearInOrder;
+  asked = asks_in_order(asked) ? kAutoInOrder : -1;
   if (!direct_tile_fits(q.dtype, q.in_c, q.taps)) {
     const int split = asked == kAutoInOrder ? -1 : split_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k, q.in_c, q.taps);
     return split >= 0 ? split : pick_tile(q.dtype, q.gemm_m, q.gemm_n, q.gemm_k);
@@ -2838,6 +3149,14 @@ int heuristic_tile(int asked, const TileQuery& q) {
   float best_us = INFINITY;
   const TileCost* const costs = q.sums ? kSumsCost : kPlainCost;
   const size_t entries = q.sums ? std::size(kSumsCost) : std::size(kPlainCost);
+  auto take = [&](const TileCost& t) {
+    const float r = static_cast<float>((tiles_for(q.gemm_m, q.gemm_n, t.bm, t.bn) + 255) / 256);
+    const float us = t.start + t.round * r + steps * fmaxf(t.alone, t.shared * r) + t.store * store;
+    if (us < best_us) {
+      best_us = us;
+      best = t.cfg;
+    }
+  };
   for (size_t i = 0; i < entries; ++i) {
     const TileCost& t = costs[i];
     // From one and a half 128 x 128 tiles per compute unit on the table prices smaller tiles, which fetch more operand bytes per
@@ -2864,13 +3183,15 @@ int heuristic_tile(int asked, const TileQuery& q) {
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (t.cfg == 5 && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
-    const float r = static_cast<float>((tiles_for(q.gemm_m, q.gemm_n, t.bm, t.bn) + 255) / 256);
-    const float us = t.start + t.round * r + steps * fmaxf(t.alone, t.shared * r) + t.store * store;
-    if (us < best_us) {
-      best_us = us;
-      best = t.cfg;
-    }
+    take(t);
   }
+  // Data gradients run beside weight gradients, whose LDS has no room on a compute unit that igemm5_kernel holds; from about 2560
+  // rows on that costs less than it gains.  Step with igemm5_kernel for forward products only / for data gradients from 2560 rows on /
+  // for all: GPT-2 of 8 x 256 4.60 / 4.60 / 4.63 ms, 3 x 777 5.33 / 5.33 / 5.42, 2 x 1024 5.16 / 5.16 / 5.20, 3 x 1024 6.25 / 6.20, 4 x 1024 7.37 /
+  // 7.18, 5 x 1024 7.90 / 7.88, 8 x 1024 11.52 / 11.29, Swin-B of 24 images 8.26 / 8.22, of 28 9.00 / 8.98, of 12-20 the same.
+  if (linear && q.walk && (!q.dgrad || q.gemm_m >= 2560))
+    for (const TileCost& t : kWalkCost[q.dgrad])
+      if (t.bn < 2 * q.gemm_n) take(t);
   return best;
 }
 
@@ -2976,9 +3297,9 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.k_per_split = (a.gemm_k + 31) / 32 * 32;
   a.div_plane = FastDiv(a.Ho * a.Wo);
   a.div_width = FastDiv(a.Wo);
-  a.in_fp32 = tile_cfg == kAutoInOrder ? 1 : 0;
+  a.in_fp32 = asks_in_order(tile_cfg) ? 1 : 0;
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false});
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false, walk_tile_fits(a)});
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
@@ -3050,7 +3371,7 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr, true});
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr, true, walk_tile_fits(a)});
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;
   }
   tile_cfg = effective_tile(tile_cfg, dtype, s.K, s.R * s.S);

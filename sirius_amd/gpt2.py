@@ -271,7 +271,7 @@ class GPT2Engine(EngineBase):
 
         # No sample depends on another here, so no sample's bf16 roundings should depend on how many others the
         # batch has: forward products in one order of additions.  (fp32: the order is below the tolerance of any use.)
-        order = ops.IN_ORDER if self.dtype == torch.bfloat16 else -1
+        order = ops.LINEAR_IN_ORDER if self.dtype == torch.bfloat16 else -1
 
         def lin_fwd(name, x, y, add=None):
             ops.conv2d_fwd(ctx, as4(x), self._w(name + ".weight"), as4(y), 1, 0,
@@ -284,7 +284,7 @@ class GPT2Engine(EngineBase):
             """dW, db from (x, dy); dx = dy W"""
             with side():
                 wgrad(as4(x), as4(dy), self._view(self.grads, name + ".weight"), self._view(self.grads, name + ".bias"))
-            ops.conv2d_dgrad(ctx, as4(dy), self._wt(name + ".weight"), as4(dx), 1, 0)
+            ops.conv2d_dgrad(ctx, as4(dy), self._wt(name + ".weight"), as4(dx), 1, 0, tile_cfg=ops.LINEAR)
 
         # strides / batch offsets of head h of sample b inside the packed projection and the score tensor
         qkv_row, qkv_b = 3 * C, (T * 3 * C, D)
@@ -366,7 +366,7 @@ class GPT2Engine(EngineBase):
             d_hf, g = g_c[0], g_c[1]
             with side():
                 wgrad(as4(hf), as4(dlogits), self._view(self.grads, "transformer.wte.weight"))
-            ops.conv2d_dgrad(ctx, as4(dlogits), self._wt("transformer.wte.weight"), as4(d_hf), 1, 0)
+            ops.conv2d_dgrad(ctx, as4(dlogits), self._wt("transformer.wte.weight"), as4(d_hf), 1, 0, tile_cfg=ops.LINEAR)
             ln_bwd("transformer.ln_f", 2 * L, d_hf, h, g)
             mark("bwd", "ln_f")
             for i in range(L - 1, -1, -1):

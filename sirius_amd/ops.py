@@ -184,6 +184,8 @@ def conv_out_hw(H, W, R, S, stride, pad):
 
 
 IN_ORDER = -2   # tile_cfg: the library's choice among tilings whose rounding does not depend on the number of rows
+# tile_cfg for the linear layers of a transformer: as -1 and as IN_ORDER, and the persistent kernel as well
+LINEAR, LINEAR_IN_ORDER = -3, -4
 
 
 def conv2d_fwd(ctx, x, w, y, stride, pad, add=None, mask=None, bias=None, tile_cfg=-1, c_logical=0):

@@ -319,7 +319,7 @@ class SwinEngine(EngineBase):
 
         # No sample depends on another here, so no sample's bf16 roundings should depend on how many others the
         # batch has: forward products in one order of additions.  (fp32: the order is below the tolerance of any use.)
-        order = ops.IN_ORDER if self.dtype == torch.bfloat16 else -1
+        order = ops.LINEAR_IN_ORDER if self.dtype == torch.bfloat16 else -1
 
         def lin_fwd(name, x, y, add=None, bias=True):
             ops.conv2d_fwd(ctx, as4(x), self._w(name + ".weight"), as4(y), 1, 0,
@@ -334,7 +334,7 @@ class SwinEngine(EngineBase):
                 wgrad(as4(x), as4(dy), self._view(self.grads, name + ".weight"),
                       dbias=self._view(self.grads, name + ".bias") if bias else None)
             if dx is not None:
-                ops.conv2d_dgrad(ctx, as4(dy), self._wt(name + ".weight"), as4(dx), 1, 0)
+                ops.conv2d_dgrad(ctx, as4(dy), self._wt(name + ".weight"), as4(dx), 1, 0, tile_cfg=ops.LINEAR)
 
         # scratch the blocks share (program order is the only hazard: one lane)
         def flat(n):
@@ -551,7 +551,7 @@ class SwinEngine(EngineBase):
                     d_nm = v2(g_4c_a, mrows, 4 * C)
                     with side():
                         wgrad(as4(nm), as4(g), self._view(self.grads, pre + "reduction.weight"))
-                    ops.conv2d_dgrad(ctx, as4(g), self._wt(pre + "reduction.weight"), as4(d_nm), 1, 0)
+                    ops.conv2d_dgrad(ctx, as4(g), self._wt(pre + "reduction.weight"), as4(d_nm), 1, 0, tile_cfg=ops.LINEAR)
                     d_xm = v2(g_4c_sets[section % n_sets], mrows, 4 * C)
                     ln_bwd(pre + "norm", d_nm, xm, d_xm, mstats)
                     g = v2(g_ring[section % len(g_ring)], rows, C)
