@@ -110,10 +110,22 @@ __global__ __launch_bounds__(256) void col_reduce_kernel(ColReduceArgs p) {
   }
 }
 
+// The number of rows as the coefficients need it.  An fp64 division is a chain of twenty instructions between a BatchNorm's sums and its
+// first output: the backward pass and the running variance multiply by a reciprocal.  (The forward statistics keep the rounded
+// quotients: their variance is a difference.)  With the parameters of the finalize kernels requested ahead of their sums as well
+// ResNet-152 of 64 images takes 13.79 instead of 13.86 ms, 2 x 16 13.18 instead of 13.25.
+struct RowCount {
+  int64_t n;
+  double inv, unbiased;   // 1 / n, n / (n - 1)
+  RowCount() = default;
+  RowCount(int64_t rows)
+      : n(rows), inv(1.0 / static_cast<double>(rows)), unbiased(rows > 1 ? static_cast<double>(rows) / static_cast<double>(rows - 1) : 1.0) {}
+};
+
 struct FwdFinalizeArgs {
   const float* partial;
   int row_blocks, C;
-  int64_t rows;
+  RowCount rows;
   const float* gamma;
   const float* beta;
   float* running_mean;
@@ -179,29 +191,38 @@ __device__ inline bool finalize_sums(const float* partial, int row_blocks, int C
 
 __global__ __launch_bounds__(kFinalizeThreads) void bn_fwd_finalize_kernel(FwdFinalizeArgs p) {
   const int c = blockIdx.x * 8 + (threadIdx.x & 7);
+  // the channel's parameters are requested ahead of the sums
+  float gamma = 0.f, beta = 0.f, running_mean = 0.f, running_var = 0.f;
+  if (threadIdx.x < 8 && c < p.C) {
+    gamma = p.gamma[c];
+    beta = p.beta[c];
+    if (p.running_mean) {
+      running_mean = p.running_mean[c];
+      running_var = p.running_var[c];
+    }
+  }
   double s, q;
   if (!finalize_sums(p.partial, p.row_blocks, p.C, c, threadIdx.x >> 3, &s, &q)) return;
-  const double n = static_cast<double>(p.rows);
-  const double mean = s / n;
-  double var = q / n - mean * mean;
+  const double mean = s / static_cast<double>(p.rows.n);
+  double var = q / static_cast<double>(p.rows.n) - mean * mean;
   if (var < 0.0) var = 0.0;
   const float invstd = 1.0f / sqrtf(static_cast<float>(var) + p.eps);
   p.save_mean[c] = static_cast<float>(mean);
   p.save_invstd[c] = invstd;
   if (p.running_mean) {
-    const double unbiased = p.rows > 1 ? var * n / (n - 1.0) : var;
-    p.running_mean[c] = (1.f - p.momentum) * p.running_mean[c] + p.momentum * static_cast<float>(mean);
-    p.running_var[c] = (1.f - p.momentum) * p.running_var[c] + p.momentum * static_cast<float>(unbiased);
+    const double unbiased = var * p.rows.unbiased;
+    p.running_mean[c] = (1.f - p.momentum) * running_mean + p.momentum * static_cast<float>(mean);
+    p.running_var[c] = (1.f - p.momentum) * running_var + p.momentum * static_cast<float>(unbiased);
   }
-  const float sc = p.gamma[c] * invstd;
+  const float sc = gamma * invstd;
   p.scale[c] = sc;
-  p.shift[c] = p.beta[c] - static_cast<float>(mean) * sc;
+  p.shift[c] = beta - static_cast<float>(mean) * sc;
 }
 
 struct BwdFinalizeArgs {
   const float* partial;
   int row_blocks, C;
-  int64_t rows;
+  RowCount rows;
   const float* gamma;
   const float* mean;
   const float* invstd;
@@ -213,15 +234,20 @@ struct BwdFinalizeArgs {
 
 __global__ __launch_bounds__(kFinalizeThreads) void bn_bwd_finalize_kernel(BwdFinalizeArgs p) {
   const int c = blockIdx.x * 8 + (threadIdx.x & 7);
+  float gamma = 0.f, saved_mean = 0.f, saved_invstd = 0.f;
+  if (threadIdx.x < 8 && c < p.C) {
+    gamma = p.gamma[c];
+    saved_mean = p.mean[c];
+    saved_invstd = p.invstd[c];
+  }
   double s1, s2;
   if (!finalize_sums(p.partial, p.row_blocks, p.C, c, threadIdx.x >> 3, &s1, &s2)) return;
   const float db = static_cast<float>(s1), dg = static_cast<float>(s2);
   p.dbeta[c] = p.accumulate ? p.dbeta[c] + db : db;
   p.dgamma[c] = p.accumulate ? p.dgamma[c] + dg : dg;
-  const double n = static_cast<double>(p.rows);
-  const double scale = static_cast<double>(p.gamma[c]) * p.invstd[c];
-  const double cb = -scale * p.invstd[c] * (s2 / n);
-  const double c0 = -scale * (s1 / n) - cb * p.mean[c];
+  const double scale = static_cast<double>(gamma) * saved_invstd;
+  const double cb = -scale * saved_invstd * (s2 * p.rows.inv);
+  const double c0 = -scale * (s1 * p.rows.inv) - cb * saved_mean;
   p.coef[c] = static_cast<float>(scale);
   p.coef[p.C + c] = static_cast<float>(cb);
   p.coef[2 * p.C + c] = static_cast<float>(c0);
@@ -389,7 +415,7 @@ constexpr int kFusedMaxRowBlocks = 256;
 struct FinApplyArgs {
   const float* partial;
   int row_blocks, C;
-  int64_t rows;
+  RowCount rows;
   const float* gamma;
   const float* beta;      // forward
   float* running_mean;    // forward (may be null)
@@ -422,7 +448,7 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
   const int64_t col_chunk = c0 / E + tx;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * p.rows_per_slab;
   int64_t r1 = r0 + p.rows_per_slab;
-  if (r1 > p.rows) r1 = p.rows;
+  if (r1 > p.rows.n) r1 = p.rows.n;
   const bool has_b = BWD || p.b != nullptr;
   float par0 = 0.f, par1 = 0.f, par2 = 0.f, par3 = 0.f;   // gamma; beta or saved mean; saved 1/std or the running pair
   if (tid < kFusedCols) {
@@ -496,10 +522,9 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
       s += red[k][tid >> 1][(tid & 1) * 2];
       q += red[k][tid >> 1][(tid & 1) * 2 + 1];
     }
-    const double n = static_cast<double>(p.rows);
     if (!BWD) {
-      const double mean = s / n;
-      double var = q / n - mean * mean;
+      const double mean = s / static_cast<double>(p.rows.n);
+      double var = q / static_cast<double>(p.rows.n) - mean * mean;
       if (var < 0.0) var = 0.0;
       const float invstd = 1.0f / sqrtf(static_cast<float>(var) + p.eps);
       const float sc = par0 * invstd;
@@ -509,7 +534,7 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
         p.save_mean[c] = static_cast<float>(mean);
         p.save_invstd[c] = invstd;
         if (p.running_mean) {
-          const double unbiased = p.rows > 1 ? var * n / (n - 1.0) : var;
+          const double unbiased = var * p.rows.unbiased;
           p.running_mean[c] = (1.f - p.momentum) * par2 + p.momentum * static_cast<float>(mean);
           p.running_var[c] = (1.f - p.momentum) * par3 + p.momentum * static_cast<float>(unbiased);
         }
@@ -517,8 +542,8 @@ __global__ __launch_bounds__(256) void bn_fin_apply_kernel(FinApplyArgs p) {
     } else {
       const double invstd = par2;
       const double scale = static_cast<double>(par0) * invstd;
-      const double cb = -scale * invstd * (q / n);
-      const double cz = -scale * (s / n) - cb * par1;
+      const double cb = -scale * invstd * (q * p.rows.inv);
+      const double cz = -scale * (s * p.rows.inv) - cb * par1;
       coef[0][tid] = static_cast<float>(scale);
       coef[1][tid] = static_cast<float>(cb);
       coef[2][tid] = static_cast<float>(cz);
@@ -587,7 +612,7 @@ struct AccApplyArgs {
   const long long* acc;   // [copies][4][C]: forward sum x, sum x^2; backward sum g, sum g * xhat
   int acc_copies;
   int C;
-  int64_t rows;
+  RowCount rows;
   const float* gamma;
   const float* beta;      // forward
   float* running_mean;    // forward (may be null)
@@ -620,11 +645,10 @@ __global__ __launch_bounds__(256) void bn_acc_apply_kernel(AccApplyArgs p) {
     const int c = c0 + tid;
     double s, q;
     acc_totals(p.acc, p.C, p.acc_copies, c, &s, &q);
-    const double n = static_cast<double>(p.rows);
-    const bool writer = blockIdx.y == 0;
+      const bool writer = blockIdx.y == 0;
     if (!BWD) {
-      const double mean = s / n;
-      double var = q / n - mean * mean;
+      const double mean = s / static_cast<double>(p.rows.n);
+      double var = q / static_cast<double>(p.rows.n) - mean * mean;
       if (var < 0.0) var = 0.0;
       const float invstd = 1.0f / sqrtf(static_cast<float>(var) + p.eps);
       const float sc = p.gamma[c] * invstd;
@@ -634,7 +658,7 @@ __global__ __launch_bounds__(256) void bn_acc_apply_kernel(AccApplyArgs p) {
         p.save_mean[c] = static_cast<float>(mean);
         p.save_invstd[c] = invstd;
         if (p.running_mean) {
-          const double unbiased = p.rows > 1 ? var * n / (n - 1.0) : var;
+          const double unbiased = var * p.rows.unbiased;
           p.running_mean[c] = (1.f - p.momentum) * p.running_mean[c] + p.momentum * static_cast<float>(mean);
           p.running_var[c] = (1.f - p.momentum) * p.running_var[c] + p.momentum * static_cast<float>(unbiased);
         }
@@ -642,8 +666,8 @@ __global__ __launch_bounds__(256) void bn_acc_apply_kernel(AccApplyArgs p) {
     } else {
       const double invstd = p.save_invstd[c];
       const double scale = static_cast<double>(p.gamma[c]) * invstd;
-      const double cb = -scale * invstd * (q / n);
-      const double cz = -scale * (s / n) - cb * p.save_mean[c];
+      const double cb = -scale * invstd * (q * p.rows.inv);
+      const double cz = -scale * (s * p.rows.inv) - cb * p.save_mean[c];
       coef[0][tid] = static_cast<float>(scale);
       coef[1][tid] = static_cast<float>(cb);
       coef[2][tid] = static_cast<float>(cz);
@@ -668,7 +692,7 @@ __global__ __launch_bounds__(256) void bn_acc_apply_kernel(AccApplyArgs p) {
   const int64_t col_chunk = static_cast<int64_t>(blockIdx.x) * CPR + tx;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * p.rows_per_slab;
   int64_t r1 = r0 + p.rows_per_slab;
-  if (r1 > p.rows) r1 = p.rows;
+  if (r1 > p.rows.n) r1 = p.rows.n;
   const bool has_b = BWD || p.b != nullptr;
   for (int64_t r = r0 + ty; r < r1; r += U * RPP) {
     Chunk ca[U], cb[U];
@@ -729,11 +753,11 @@ int launch_acc_apply(Context* ctx, AccApplyArgs& a, const char* name, double byt
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int trip = 4 * (256 / CPR);
   const int64_t col_blocks = a.C / (CPR * E);
-  const double tensor_mb = static_cast<double>(a.rows) * a.C * sizeof(T) / 1e6;
+  const double tensor_mb = static_cast<double>(a.rows.n) * a.C * sizeof(T) / 1e6;
   const int target = tensor_mb > 40.0 ? target_large : target_small;
   int64_t slabs = target / col_blocks;
   if (slabs < 1) slabs = 1;
-  int64_t rps = (a.rows + slabs - 1) / slabs;
+  int64_t rps = (a.rows.n + slabs - 1) / slabs;
   rps = (rps + trip - 1) / trip * trip;
   a.rows_per_slab = static_cast<int>(rps);
   static const int nt = [] {
@@ -741,7 +765,7 @@ int launch_acc_apply(Context* ctx, AccApplyArgs& a, const char* name, double byt
     return e ? atoi(e) : 1;
   }();
   a.nt = (nt && tensor_mb > 40.0) ? 1 : 0;   // small tensors were just written and sit in the caches
-  const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>((a.rows + rps - 1) / rps));
+  const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>((a.rows.n + rps - 1) / rps));
   return launch(ctx, bn_acc_apply_kernel<T, BWD, CPR>, grid, dim3(256), a, name, bytes, 1);
 }
 
