@@ -138,7 +138,7 @@ struct FastDiv {
       shr = p - 32;
     }
   }
-  __device__ inline uint32_t div(uint32_t n) const { return d == 1 ? n : (__umulhi(n, mul) >> shr); }
+  __device__ inline uint32_t div(uint32_t n) const { return mul == 0 ? n : __umulhi(n, mul) >> shr; }   // (0: d is 1)
   __device__ inline void divmod(uint32_t n, uint32_t& q, uint32_t& r) const {
     q = div(n);
     r = n - q * d;
@@ -266,7 +266,7 @@ struct LaunchRecord {
   //                   (nothing at the first one), and lane 1's work up to here is what the next one waits for
   int lane;
   int op;
-  alignas(16) unsigned char args[448];
+  alignas(16) unsigned char args[512];
 };
 enum LaunchOp : int { kOpLaunch = 0, kOpLaunchAfter = 1, kOpJoin = 2, kOpJoinBehind = 3 };
 

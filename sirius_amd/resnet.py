@@ -297,7 +297,7 @@ class ResNetEngine(EngineBase):
         """The fastest tiling, or a larger tile that is within `tile_margin` of it: alone on the chip a small tile
         can win by a few percent and still lose in the step, where it shares L2 bandwidth with the weight gradients
         (a larger tile fetches fewer operand bytes per flop)."""
-        area = lambda cfg: {0: 4, 11: 4, 12: 4, 23: 4, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2, 22: 2, 15: 0.25, 16: 0.25, 17: 0.5, 20: 0.5}.get(cfg, 1)
+        area = lambda cfg: {0: 4, 11: 4, 12: 4, 23: 4, 28: 4, 31: 2, 9: 16, 10: 16, 1: 2, 5: 2, 6: 2, 13: 2, 22: 2, 15: 0.25, 16: 0.25, 17: 0.5, 20: 0.5}.get(cfg, 1)
         best = min(timings.values())
         ok = [cfg for cfg, t in timings.items() if t <= best * (1.0 + self.tile_margin)]
         return min(ok, key=lambda cfg: (-area(cfg), timings[cfg]))
@@ -341,8 +341,8 @@ class ResNetEngine(EngineBase):
                     else:
                         ops.conv2d_dgrad(ctx, z, wt, x, c.stride, c.pad, tile_cfg=cfg, c_logical=c.cin)
             return rec
-        # 5 = the 3x3 patch kernel (stride-1 3x3 layers; elsewhere the library runs tiling 1 for it)
-        patch = (5,) if (c.k == 3 and c.stride == 1 and c.pad == 1) else ()
+        # 5, 28 - 31 = the 3x3 patch kernel (stride-1 3x3 layers; elsewhere the library runs other kernels for them)
+        patch = (5, 28, 29, 30, 31) if (c.k == 3 and c.stride == 1 and c.pad == 1) else ()
         # 6 / 7 = tilings 1 / 2 with two LDS tiles in flight (more workgroups per CU)
         # 11 - 14 = 128 x 128 (three / two LDS tiles), 128 x 64, 64 x 64 with 32-element reduction steps: half the LDS
         # per workgroup, which the wide, shallow products of the first two stages prefer
