@@ -61,6 +61,13 @@ __device__ inline Chunk pack_slab(const float* p) {
   return c;
 }
 
+__device__ inline Chunk pack_half(const f32x16_t& acc, int s) {
+  Chunk c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) c.w[i] = pack_bf16(acc[8 * s + 2 * i], acc[8 * s + 2 * i + 1]);
+  return c;
+}
+
 __device__ inline void zero_acc(f32x16_t& a) {
 #pragma unroll
   for (int e = 0; e < 16; ++e) a[e] = 0.f;

@@ -18,6 +18,13 @@
 // {16s + 8t + 4(lane/32) + i}, which is a permutation of the 16 reduction indices of one MFMA step; the other
 // operand is read from LDS with the same permutation (transposing reads, ds_read_b64_tr_b16).
 //
+// A step stores its tiles to one of two buffers, so that one barrier a step is enough; a mask is applied behind a branch of the
+// whole wavefront instead of in every score.  The key kernel has KG = 1 or 2 walk groups of four wavefronts: group g walks the
+// tiles g, g + KG, .. for the same fixed rows, staged in LDS of its own, and the groups' accumulators are added at the end.
+// What bounds them: with several workgroups on a CU the exponentials and what surrounds them, 960 of the 1470 cycles that a
+// forward step's instructions take (96 heads of 1024: forward 32.9 -> 29.3 us, backward 82 -> 76); with one, the chain of steps (36
+// heads of 777: 20.8 -> 15.7 and 46.8 -> 38.2).
+//
 // RAGGED (a sequence length that is no multiple of 128): the last fixed block and the last walked tile reach past the
 // sequence.  Loads of rows beyond it fetch the last row again (no branch, always a finite value), and nothing is
 // stored for them.  A walked key beyond the end is masked like a future key (a causal mask covers it already); a walked
@@ -101,8 +108,7 @@ __device__ inline void load_fixed(const bf16* base, int64_t rs, int first, int T
 }
 
 // acc[ct] holds the transposed result: column 32 ct + 8 (r / 4) + 4 (lane / 32) + r % 4 of fixed row lane % 32.
-// Goes through this wave's LDS patch so that a row leaves as 16-byte pieces.
-template <bool RAGGED>
+// Goes through this wave's LDS patch so that a row leaves as 16-byte pieces.  T = 0: a wave that stores nothing.
 __device__ inline void store_fixed(f32x16_t (&acc)[2], float mul, unsigned char* patch, bf16* base, int64_t rs, int first,
                                    int T, int lane) {
 #pragma unroll
@@ -119,24 +125,27 @@ __device__ inline void store_fixed(f32x16_t (&acc)[2], float mul, unsigned char*
   for (int i = 0; i < 4; ++i) {
     const int q = lane + 64 * i;
     const uint4 v = *reinterpret_cast<const uint4*>(patch + (q >> 3) * kRowB + (q & 7) * 16);
-    if (!RAGGED || first + (q >> 3) < T)
+    if (first + (q >> 3) < T)
       *reinterpret_cast<uint4*>(base + static_cast<int64_t>(first + (q >> 3)) * rs + (q & 7) * 8) = v;
   }
+}
+
+// the workgroup's tiles: two buffers of one pair of tiles per walk group, later what join_groups hands over (32 KB)
+template <int KG>
+constexpr int flash_lds() {
+  return 2 * KG * 2 * kTileB;
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // forward (DQ = false) and the dQ half of the backward (DQ = true): fixed queries, walked keys
 // ---------------------------------------------------------------------------------------------------------
 template <bool CAUSAL, bool DQ, bool RAGGED>
-__global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kTileB];
-  unsigned char* kt = lds;
-  unsigned char* vt = lds + kTileB;
+__global__ __launch_bounds__(256, 3) void flash_query_kernel(FlashArgs p) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[flash_lds<1>()];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
-  // Workgroup ids go to the XCDs round-robin and all of them are resident at once, so the order is the
+  // Workgroup ids go to the XCDs round-robin and most of them are resident at once, so the order is the
   // placement: the blocks of one head keep one residue of the id modulo 8 (one XCD, one L2 for its keys and
-  // values), and the long blocks of a causal problem come first so that each compute unit's share of
-  // consecutive ids mixes long and short ones.
+  // values), and the long blocks of a causal problem come first, so that the short ones fill what they leave.
   const int blocks = RAGGED ? (p.T + kFixed - 1) / kFixed : p.T / kFixed;
   const int nbh = gridDim.x / blocks;
   const int qb = blocks - 1 - blockIdx.x / nbh;
@@ -147,6 +156,19 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
   const int query = qw0 + (lane & 31);
   const bool real = !RAGGED || query < p.T;
   const int64_t stat_at = static_cast<int64_t>(bh) * p.T + (real ? query : p.T - 1);
+
+  const int tiles = RAGGED ? (p.T + kWalk - 1) / kWalk : p.T / kWalk;
+  const int seen = (q0 + kFixed) / kWalk;   // tiles a causal block of queries sees
+  const int steps = CAUSAL ? (RAGGED && seen > tiles ? tiles : seen) : tiles;
+  const bf16* kbase = p.k + qkv_off;
+  const bf16* vbase = p.v + qkv_off;
+  TileRegs rk, rv;
+  auto fetch = [&](int kb) {   // behind the last tile the last one again: no branch around the loads
+    const int row = (kb < steps ? kb : steps - 1) * kWalk;
+    rk = tile_load_at<RAGGED>(kbase, p.qkv_rs, row, p.T, tid);
+    rv = tile_load_at<RAGGED>(vbase, p.qkv_rs, row, p.T, tid);
+  };
+  fetch(0);
 
   Chunk qf[4], dof[4];
   load_fixed<RAGGED>(p.q + qkv_off, p.qkv_rs, qw0, p.T, lane, qf);
@@ -168,14 +190,6 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
     lse2 = p.lse[stat_at] * kLog2e;
   }
 
-  const int tiles = RAGGED ? (p.T + kWalk - 1) / kWalk : p.T / kWalk;
-  const int seen = (q0 + kFixed) / kWalk;   // tiles a causal block of queries sees
-  const int steps = CAUSAL ? (RAGGED && seen > tiles ? tiles : seen) : tiles;
-  const bf16* kbase = p.k + qkv_off;
-  const bf16* vbase = p.v + qkv_off;
-  TileRegs rk = tile_load_at<RAGGED>(kbase, p.qkv_rs, 0, p.T, tid);
-  TileRegs rv = tile_load_at<RAGGED>(vbase, p.qkv_rs, 0, p.T, tid);
-
   f32x16_t acc[2];
   zero_acc(acc[0]);
   zero_acc(acc[1]);
@@ -183,48 +197,41 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
   float m = -INFINITY, l = 0.f;
 
   for (int kb = 0; kb < steps; ++kb) {
-    __syncthreads();
+    unsigned char* kt = lds + (kb & 1) * 2 * kTileB;
+    unsigned char* vt = kt + kTileB;
     tile_store(kt, tid, rk);
     tile_store(vt, tid, rv);
+    // the one barrier of a step: whoever stores to the other buffer next has seen everyone through the step that read it
     __syncthreads();
-    {
-      // the last step fetches its own tile again rather than branching around the loads
-      const int next = (kb + 1 < steps ? kb + 1 : kb) * kWalk;
-      rk = tile_load_at<RAGGED>(kbase, p.qkv_rs, next, p.T, tid);
-      rv = tile_load_at<RAGGED>(vbase, p.qkv_rs, next, p.T, tid);
-    }
+    fetch(kb + 1);
     const int k0 = kb * kWalk;
     if (CAUSAL && k0 > qw0 + 31) continue;   // nothing of this tile is visible to this wave's queries
 
-    f32x16_t s[2], dp[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      zero_acc(s[t]);
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) s[t] = mma16(frag_rows<kRowB>(kt, 32 * t, ks, lane), qf[ks], s[t]);
-      if (DQ) {
-        zero_acc(dp[t]);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) dp[t] = mma16(frag_rows<kRowB>(vt, 32 * t, ks, lane), dof[ks], dp[t]);
-      }
-    }
     // some key of the tile lies beyond some query, or beyond the sequence
     const bool diagonal = CAUSAL ? k0 + kWalk - 1 > qw0 : RAGGED && k0 + kWalk > p.T;
-    const int last = CAUSAL ? query : p.T - 1;   // the last key this lane's query sees
-    float pr[2][16];
-    if (!DQ) {
+    const int last = (CAUSAL ? query : p.T - 1) - k0 - 4 * half;   // the last key this lane's query sees, from the lane's first
+    if constexpr (!DQ) {
+      f32x16_t s[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        zero_acc(s[t]);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) s[t] = mma16(frag_rows<kRowB>(kt, 32 * t, ks, lane), qf[ks], s[t]);
+      }
+      if (diagonal) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (32 * t + 8 * (r >> 2) + (r & 3) > last) s[t][r] = -INFINITY;
+      }
       // running maximum on the raw scores (the scale is positive), then exp2(s * c - m * c) as one fused
       // multiply-add and one exponential per score
       float bmax = -INFINITY;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float v = s[t][r];
-          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > last) v = -INFINITY;
-          pr[t][r] = v;
-          bmax = fmaxf(bmax, v);
-        }
+        for (int r = 0; r < 16; ++r) bmax = fmaxf(bmax, s[t][r]);
       bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
       const float m_new = fmaxf(m, bmax);
       const bool moved = m_new != m;
@@ -236,8 +243,8 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          pr[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(pr[t][r], c, -mc));
-          sum += pr[t][r];
+          s[t][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], c, -mc));
+          sum += s[t][r];
         }
       l = l * alpha + sum;
       // after the first tiles the maxima seldom move: the accumulators are rescaled only when one in the wave did
@@ -247,25 +254,42 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
 #pragma unroll
           for (int e = 0; e < 16; ++e) acc[ct][e] *= alpha;
       }
-    } else {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float pv = __builtin_amdgcn_exp2f(s[t][r] * c - lse2);
-          if (diagonal && k0 + 32 * t + 8 * (r >> 2) + 4 * half + (r & 3) > last) pv = 0.f;
-          pr[t][r] = pv * (dp[t][r] - delta);
+        for (int sl = 0; sl < 2; ++sl) {
+          const Chunk pc = pack_half(s[t], sl);
+#pragma unroll
+          for (int ct = 0; ct < 2; ++ct) acc[ct] = mma16(frag_cols<kRowB>(vt, 32 * t + 16 * sl, ct, lane), pc, acc[ct]);
         }
-    }
-    const unsigned char* second = DQ ? kt : vt;
+    } else {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < 2; ++t) {
+        f32x16_t s, dp;
+        zero_acc(s);
+        zero_acc(dp);
 #pragma unroll
-      for (int sl = 0; sl < 2; ++sl) {
-        const Chunk pc = pack_slab(&pr[t][8 * sl]);
+        for (int ks = 0; ks < 4; ++ks) {
+          s = mma16(frag_rows<kRowB>(kt, 32 * t, ks, lane), qf[ks], s);
+          dp = mma16(frag_rows<kRowB>(vt, 32 * t, ks, lane), dof[ks], dp);
+        }
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct) acc[ct] = mma16(frag_cols<kRowB>(second, 32 * t + 16 * sl, ct, lane), pc, acc[ct]);
+        for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r] * c - lse2);
+        if (diagonal) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            if (32 * t + 8 * (r >> 2) + (r & 3) > last) s[r] = 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] *= dp[r] - delta;
+#pragma unroll
+        for (int sl = 0; sl < 2; ++sl) {
+          const Chunk pc = pack_half(s, sl);
+#pragma unroll
+          for (int ct = 0; ct < 2; ++ct) acc[ct] = mma16(frag_cols<kRowB>(kt, 32 * t + 16 * sl, ct, lane), pc, acc[ct]);
+        }
       }
+    }
   }
 
   float mul = p.scale;
@@ -274,21 +298,44 @@ __global__ __launch_bounds__(256) void flash_query_kernel(FlashArgs p) {
     mul = 1.f / l;
     if (half == 0 && real) p.lse[stat_at] = m * p.scale + __builtin_amdgcn_logf(l) * kLn2;
   }
-  __syncthreads();   // every wave is done with the tiles: the space becomes four output patches
-  store_fixed<RAGGED>(acc, mul, lds + wave * 32 * kRowB, p.out + (DQ ? qkv_off : o_off), DQ ? p.qkv_rs : p.o_rs, qw0, p.T,
+  __syncthreads();   // every wave is done with the space: it becomes four output patches
+  store_fixed(acc, mul, lds + wave * 32 * kRowB, p.out + (DQ ? qkv_off : o_off), DQ ? p.qkv_rs : p.o_rs, qw0, p.T,
                       lane);
 }
 
 // ---------------------------------------------------------------------------------------------------------
 // dK and dV: fixed keys, walked queries
 // ---------------------------------------------------------------------------------------------------------
-template <bool CAUSAL, bool RAGGED>
-__global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kTileB];
-  __shared__ __attribute__((aligned(16))) float stat[2][kWalk];   // log-sum-exp (base 2) and delta of the staged queries
-  unsigned char* qt = lds;
-  unsigned char* dot = lds + kTileB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
+// Adds the accumulators of walk group 1 to those of group 0.  Uses the LDS of the tiles; every wave calls it.
+__device__ inline void join_groups(f32x16_t (&acc)[2], unsigned char* lds, int group, int wave, int lane) {
+  float4* place = reinterpret_cast<float4*>(lds) + wave * 512 + lane;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const f32x16_t& v = acc[j >> 2];
+    const int e = 4 * (j & 3);
+    if (group == 1) place[64 * j] = make_float4(v[e], v[e + 1], v[e + 2], v[e + 3]);
+  }
+  __syncthreads();
+  if (group == 1) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float4 v = place[64 * j];
+    f32x16_t& to = acc[j >> 2];
+    const int e = 4 * (j & 3);
+    to[e] += v.x;
+    to[e + 1] += v.y;
+    to[e + 2] += v.z;
+    to[e + 3] += v.w;
+  }
+}
+
+template <bool CAUSAL, bool RAGGED, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void flash_key_kernel(FlashArgs p) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[flash_lds<KG>()];
+  __shared__ __attribute__((aligned(16))) float stat[2][KG][2][kWalk];   // log-sum-exp (base 2) and delta of the staged queries
+  const int lane = threadIdx.x & 63, tid = threadIdx.x & 255, wave = tid >> 6, half = lane >> 5;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int nbh = gridDim.x / (RAGGED ? (p.T + kFixed - 1) / kFixed : p.T / kFixed);   // placement as in flash_query_kernel: early keys see most queries
   const int kblk = blockIdx.x / nbh;
   const int bh = blockIdx.x % nbh;
@@ -296,10 +343,6 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   const int64_t qkv_off = b * p.qkv_bs + h * kHd, o_off = b * p.o_bs + h * kHd;
   const int k0 = kblk * kFixed, kw0 = k0 + 32 * wave;
   const int key = kw0 + (lane & 31);
-
-  Chunk kf[4], vf[4];
-  load_fixed<RAGGED>(p.k + qkv_off, p.qkv_rs, kw0, p.T, lane, kf);
-  load_fixed<RAGGED>(p.v + qkv_off, p.qkv_rs, kw0, p.T, lane, vf);
 
   const int first = CAUSAL ? k0 / kWalk : 0;   // queries before the first key see none of these keys
   const int steps = RAGGED ? (p.T + kWalk - 1) / kWalk : p.T / kWalk;
@@ -309,7 +352,8 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   const float* dlt = p.delta + static_cast<int64_t>(bh) * p.T;
   TileRegs rq, rd;
   float rstat = 0.f;
-  auto fetch = [&](int qb) {
+  auto fetch = [&](int at_tile) {   // behind the last tile the last one again: no branch around the loads
+    const int qb = at_tile < steps ? at_tile : steps - 1;
     rq = tile_load_at<RAGGED>(qbase, p.qkv_rs, qb * kWalk, p.T, tid);
     rd = tile_load_at<RAGGED>(dobase, p.o_rs, qb * kWalk, p.T, tid);
     const int row = qb * kWalk + (tid & (kWalk - 1));
@@ -318,7 +362,11 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
     if (tid < kWalk) rstat = real ? lse[at] * kLog2e : INFINITY;
     else if (tid < 2 * kWalk) rstat = dlt[at];
   };
-  fetch(first);
+  fetch(first + group);
+
+  Chunk kf[4], vf[4];
+  load_fixed<RAGGED>(p.k + qkv_off, p.qkv_rs, kw0, p.T, lane, kf);
+  load_fixed<RAGGED>(p.v + qkv_off, p.qkv_rs, kw0, p.T, lane, vf);
 
   f32x16_t dk[2], dv[2];
   zero_acc(dk[0]);
@@ -327,64 +375,72 @@ __global__ __launch_bounds__(256) void flash_key_kernel(FlashArgs p) {
   zero_acc(dv[1]);
   const float c = p.scale * kLog2e;
 
-  for (int qb = first; qb < steps; ++qb) {
-    __syncthreads();
+  for (int qb0 = first, turn = 0; qb0 < steps; qb0 += KG, turn ^= 1) {
+    const int qb = qb0 + group;
+    unsigned char* qt = lds + (turn * KG + group) * 2 * kTileB;
+    unsigned char* dot = qt + kTileB;
+    float(&st)[2][kWalk] = stat[turn][group];
     tile_store(qt, tid, rq);
     tile_store(dot, tid, rd);
-    if (tid < 2 * kWalk) stat[tid >> 6][tid & 63] = rstat;
-    __syncthreads();
-    fetch(qb + 1 < steps ? qb + 1 : qb);   // the last step fetches its own tile again: no branch around the loads
+    if (tid < 2 * kWalk) st[tid >> 6][tid & 63] = rstat;
+    __syncthreads();   // the one of a step, as in flash_query_kernel
+    fetch(qb + KG);
     const int q0 = qb * kWalk;
-    if (CAUSAL && q0 + kWalk - 1 < kw0) continue;   // every staged query lies before this wave's keys
+    if (qb >= steps || (CAUSAL && q0 + kWalk - 1 < kw0)) continue;   // no (more) staged query sees this wave's keys
 
-    f32x16_t s[2], dp[2];
+    const bool diagonal = CAUSAL && q0 < kw0 + 31;   // some staged query lies before some key of this wave
+    const int before = key - q0 - 4 * half;          // the lane's queries below this one lie before its key
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      zero_acc(s[t]);
-      zero_acc(dp[t]);
+      f32x16_t s, dp;
+      zero_acc(s);
+      zero_acc(dp);
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        s[t] = mma16(frag_rows<kRowB>(qt, 32 * t, ks, lane), kf[ks], s[t]);
-        dp[t] = mma16(frag_rows<kRowB>(dot, 32 * t, ks, lane), vf[ks], dp[t]);
+        s = mma16(frag_rows<kRowB>(qt, 32 * t, ks, lane), kf[ks], s);
+        dp = mma16(frag_rows<kRowB>(dot, 32 * t, ks, lane), vf[ks], dp);
       }
-    }
-    const bool diagonal = CAUSAL && q0 < kw0 + 31;   // some staged query lies before some key of this wave
-    float pr[2][16], ds[2][16];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int row = 32 * t + 8 * j + 4 * half;
-        const float4 l4 = *reinterpret_cast<const float4*>(&stat[0][row]);
-        const float4 d4 = *reinterpret_cast<const float4*>(&stat[1][row]);
-        const float ls[4] = {l4.x, l4.y, l4.z, l4.w}, dl[4] = {d4.x, d4.y, d4.z, d4.w};
+        const float4 l4 = *reinterpret_cast<const float4*>(&st[0][32 * t + 8 * j + 4 * half]);
+        const float ls[4] = {l4.x, l4.y, l4.z, l4.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * j + i;
-          float pv = __builtin_amdgcn_exp2f(s[t][r] * c - ls[i]);
-          if (diagonal && key > q0 + row + i) pv = 0.f;
-          pr[t][r] = pv;
-          ds[t][r] = pv * (dp[t][r] - dl[i]);
-        }
+        for (int i = 0; i < 4; ++i) s[4 * j + i] = __builtin_amdgcn_exp2f(s[4 * j + i] * c - ls[i]);
+      }
+      if (diagonal) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * t + 8 * (r >> 2) + (r & 3) < before) s[r] = 0.f;
       }
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+      for (int j = 0; j < 4; ++j) {
+        const float4 d4 = *reinterpret_cast<const float4*>(&st[1][32 * t + 8 * j + 4 * half]);
+        const float dl[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dp[4 * j + i] = s[4 * j + i] * (dp[4 * j + i] - dl[i]);
+      }
 #pragma unroll
       for (int sl = 0; sl < 2; ++sl) {
-        const Chunk pc = pack_slab(&pr[t][8 * sl]);
-        const Chunk dc = pack_slab(&ds[t][8 * sl]);
+        const Chunk pc = pack_half(s, sl);
+        const Chunk dc = pack_half(dp, sl);
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) {
           dv[ct] = mma16(frag_cols<kRowB>(dot, 32 * t + 16 * sl, ct, lane), pc, dv[ct]);
           dk[ct] = mma16(frag_cols<kRowB>(qt, 32 * t + 16 * sl, ct, lane), dc, dk[ct]);
         }
       }
+    }
+  }
+  if (KG == 2) {
+    join_groups(dv, lds, group, wave, lane);
+    join_groups(dk, lds, group, wave, lane);
   }
   __syncthreads();
-  unsigned char* patch = lds + wave * 32 * kRowB;
-  store_fixed<RAGGED>(dv, 1.f, patch, p.dv + qkv_off, p.qkv_rs, kw0, p.T, lane);
+  unsigned char* patch = lds + (4 * group + wave) * 32 * kRowB;
+  const int rows = group == 0 ? p.T : 0;
+  store_fixed(dv, 1.f, patch, p.dv + qkv_off, p.qkv_rs, kw0, rows, lane);
   __syncthreads();
-  store_fixed<RAGGED>(dk, p.scale, patch, p.dk + qkv_off, p.qkv_rs, kw0, p.T, lane);
+  store_fixed(dk, p.scale, patch, p.dk + qkv_off, p.qkv_rs, kw0, rows, lane);
 }
 
 int check_geometry(const char* who, int dtype, int B, int H, int T, int64_t qkv_rs, int64_t qkv_bs, int64_t o_rs,
@@ -400,6 +456,23 @@ int check_geometry(const char* who, int dtype, int B, int H, int T, int64_t qkv_
   TCH_CHECK_ARG(qkv_rs % 8 == 0 && qkv_bs % 8 == 0 && o_rs % 8 == 0 && o_bs % 8 == 0,
                 w + ": strides must keep 16-byte alignment");
   return 0;
+}
+
+// Workgroups that share one CU hide each other's latencies; one that is alone on it lives off its own wavefronts, and two groups
+// halve its chain of steps.  dK and dV with one group / two, in us more or less than one: 36 heads of 777 (252 workgroups) -4, 12
+// of 1024 (96) -5, 24 of 512 (96) -2, 96 of 256 (192) 0; 96 of 512 (384) +5, 96 of 1024 (768) +6.  (The two query kernels gain less:
+// groups of 36 heads of 777 dQ -1.3, forward -2 with three of them; and with one their results are those they always were.)
+bool split_walk(const dim3& grid, int T) { return grid.x <= 256 && T > 5 * kWalk; }
+
+template <bool DQ>
+void (*query_kernel(bool causal, bool ragged))(FlashArgs) {
+  return causal ? (ragged ? flash_query_kernel<true, DQ, true> : flash_query_kernel<true, DQ, false>)
+                : (ragged ? flash_query_kernel<false, DQ, true> : flash_query_kernel<false, DQ, false>);
+}
+template <int KG>
+void (*key_kernel(bool causal, bool ragged))(FlashArgs) {
+  return causal ? (ragged ? flash_key_kernel<true, true, KG> : flash_key_kernel<true, false, KG>)
+                : (ragged ? flash_key_kernel<false, true, KG> : flash_key_kernel<false, false, KG>);
 }
 
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
@@ -428,10 +501,8 @@ int flash_attn_fwd(Context* ctx, int dtype, const void* q, const void* k, const 
   const dim3 grid(static_cast<unsigned>((T + kFixed - 1) / kFixed) * B * H);
   const double flops = 4.0 * B * H * static_cast<double>(T) * T * kHd * (causal ? 0.5 : 1.0);
   const bool ragged = T % kFixed != 0;
-  void (*const kernel)(FlashArgs) =
-      causal ? (ragged ? flash_query_kernel<true, false, true> : flash_query_kernel<true, false, false>)
-             : (ragged ? flash_query_kernel<false, false, true> : flash_query_kernel<false, false, false>);
-  return launch(ctx, kernel, grid, dim3(256), a, causal ? "flash_attn_fwd<causal>" : "flash_attn_fwd<full>", flops, 0);
+  return launch(ctx, query_kernel<false>(causal, ragged), grid, dim3(256), a, causal ? "flash_attn_fwd<causal>" : "flash_attn_fwd<full>",
+                flops, 0);
 }
 
 int flash_attn_bwd(Context* ctx, int dtype, const void* q, const void* k, const void* v, const void* o, const void* dout,
@@ -464,14 +535,12 @@ int flash_attn_bwd(Context* ctx, int dtype, const void* q, const void* k, const 
   const double pair = 2.0 * B * H * static_cast<double>(T) * T * kHd * (causal ? 0.5 : 1.0);   // one T x T x 64 product
   // the dQ launch leaves delta for the dK / dV launch
   const bool ragged = T % kFixed != 0;
-  void (*const dq_kernel)(FlashArgs) =
-      causal ? (ragged ? flash_query_kernel<true, true, true> : flash_query_kernel<true, true, false>)
-             : (ragged ? flash_query_kernel<false, true, true> : flash_query_kernel<false, true, false>);
-  void (*const dkv_kernel)(FlashArgs) = causal ? (ragged ? flash_key_kernel<true, true> : flash_key_kernel<true, false>)
-                                               : (ragged ? flash_key_kernel<false, true> : flash_key_kernel<false, false>);
-  if (int rc = launch(ctx, dq_kernel, grid, dim3(256), a, causal ? "flash_attn_dq<causal>" : "flash_attn_dq<full>", 3.0 * pair, 0))
+  const bool split = split_walk(grid, T);
+  if (int rc = launch(ctx, query_kernel<true>(causal, ragged), grid, dim3(256), a,
+                      causal ? "flash_attn_dq<causal>" : "flash_attn_dq<full>", 3.0 * pair, 0))
     return rc;
-  return launch(ctx, dkv_kernel, grid, dim3(256), a, causal ? "flash_attn_dkv<causal>" : "flash_attn_dkv<full>", 4.0 * pair, 0);
+  return launch(ctx, split ? key_kernel<2>(causal, ragged) : key_kernel<1>(causal, ragged), grid, dim3(split ? 512 : 256), a,
+                causal ? "flash_attn_dkv<causal>" : "flash_attn_dkv<full>", 4.0 * pair, 0);
 }
 
 }  // namespace tch

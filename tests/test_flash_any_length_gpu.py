@@ -52,3 +52,11 @@ def test_any_length(ctx, B, H, T, causal):
         assert torch.all(t[:guard] == 7) and torch.all(t[guard + n:] == 7)
     for t in (lse, delta):
         assert torch.all(t[B * H * T:] == 7)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 320), (1, 2, 321), (2, 3, 384), (1, 1, 449), (65, 4, 64), (44, 6, 128), (86, 1, 330)])
+def test_walk_groups(ctx, B, H, T, causal):
+    """Up to 256 workgroups two groups of wavefronts walk the tiles of dK and dV, from six tiles of 64 on: both sides of the line
+    (one of seven tiles: a group has a last turn without one), whole and ragged lengths, more workgroups than compute units."""
+    test_any_length(ctx, B, H, T, causal)
