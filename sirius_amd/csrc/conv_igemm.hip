@@ -859,8 +859,8 @@ __device__ inline void wait_and_meet() {
 // divided by the tiles in flight until the operand path of the CU is full (64 x 64, 147 / 75 / 53 us with two / three /
 // four tiles where eight steps' worth of splits are missing).  Against the form that staged tiles in registers (two in
 // flight, LDS stores of its own): 256 x 2304 over 12 544 pixels 44 -> 31 us, 3072 x 768 over 8192 62 -> 47, 128 x 1152 over
-// 50 176 34 -> 26; reading a step ahead of its multiplication into a second register set (169 instead of 136
-// registers) gained nothing on top.
+// 50 176 34 -> 26; reading a whole step ahead of its multiplication into a second register set (169 instead of 136
+// registers) gained nothing on top, a slice ahead does (128 x 128, below).
 // POINTWISE: x is read at dy's pixels (no tap arithmetic).  BIAS: the launch may be asked for the bias gradient.
 // 64 x 64 keeps five tiles in LDS instead of eight over up to 60 steps, and over up to 32 where the launch is about one
 // workgroup on every compute unit (short_wgrad_ring): the seven requests of the full ring's start are a good part of a short
@@ -927,9 +927,12 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
     a_off[i] = (a_pix[i] * p.K + a_ch) * 2;
   }
   const int a_step = BKP * p.K * 2;
-  // not pointwise: the lane's tap and channel, and every load's place in the image, moved on by 32 pixels per step
+  // Not pointwise: the lane's tap and channel, and every load's place in the input image, moved on by 32 output pixels per step.
+  // Row, column and offset move by constants and by others where a row or an image ends: 18 instructions a load, none of them
+  // an integer multiplication, which takes the time of four (with seven of those: 256 x 2304 over 12 544 pixels unsplit 65.6 us
+  // for 64.1, over 3136 20.4 for 19.5).
   int b_c = b_n, b_h = 0, b_w = 0;
-  uint32_t b_img[B_LD], b_oh[B_LD], b_ow[B_LD];
+  int b_hi[B_LD], b_wi[B_LD];
   uint32_t step_img = 0, step_oh = 0, step_ow = 0;
   if (!POINTWISE) {
     const int tap = p.div_c.div(b_n);
@@ -940,50 +943,54 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
     p.div_plane.divmod(BKP, step_img, step_oh);
     p.div_width.divmod(step_oh, step_oh, step_ow);
   }
+  const int in_rows = p.Ho * p.stride, in_cols = p.Wo * p.stride;   // what a wrap takes off
+  const int h_end = b_h + in_rows, w_end = b_w + in_cols;
+  const int step_hi = step_oh * p.stride, step_wi = step_ow * p.stride;
+  const int off_step = ((static_cast<int>(step_img) * p.H + step_hi) * p.W + step_wi) * p.C * 2;
+  const int off_row = off_step + p.stride * (p.W - p.Wo) * p.C * 2, off_img = (p.H - in_rows) * p.W * p.C * 2;
 #pragma unroll
   for (int i = 0; i < B_LD; ++i) {
     b_pix[i] = k_begin + (wave * B_LD + i) * (64 / SB) + b_row;
     b_off[i] = (b_pix[i] * p.C + b_c) * 2;
-    b_img[i] = b_oh[i] = b_ow[i] = 0;
+    b_hi[i] = b_wi[i] = 0;
     if (!POINTWISE) {
-      uint32_t rem;
-      p.div_plane.divmod(static_cast<uint32_t>(b_pix[i]), b_img[i], rem);
-      p.div_width.divmod(rem, b_oh[i], b_ow[i]);
+      uint32_t img, rem, oh, ow;
+      p.div_plane.divmod(static_cast<uint32_t>(b_pix[i]), img, rem);
+      p.div_width.divmod(rem, oh, ow);
+      b_hi[i] = static_cast<int>(oh) * p.stride + b_h;
+      b_wi[i] = static_cast<int>(ow) * p.stride + b_w;
+      b_off[i] = (((static_cast<int>(img) * p.H + b_hi[i]) * p.W + b_wi[i]) * p.C + b_c) * 2;
     }
   }
   const int b_step = BKP * p.C * 2;
   // Every lane issues every load whatever it asks for (the counted waits rely on it): an offset out of range where
   // there is no pixel, a tap outside the image, or a tile behind the last one.
-  auto issue_loads = [&](int buf) {
-    unsigned char* dst_a = lds + buf * BUF_BYTES + wave * A_LD * 1024;
-    unsigned char* dst_b = lds + buf * BUF_BYTES + A_BYTES + wave * B_LD * 1024;
-#pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      load_to_lds(rsrc_a, dst_a + i * 1024, a_pix[i] < a_end ? a_off[i] : static_cast<int>(kOutOfRange), 0);
-      a_pix[i] += BKP;
-      a_off[i] += a_step;
+  constexpr int LOADS = A_LD + B_LD;
+  auto issue_load = [&](int buf, int j) {
+    if (j < A_LD) {
+      load_to_lds(rsrc_a, lds + buf * BUF_BYTES + (wave * A_LD + j) * 1024, a_pix[j] < a_end ? a_off[j] : static_cast<int>(kOutOfRange), 0);
+      a_pix[j] += BKP;
+      a_off[j] += a_step;
+      return;
     }
-#pragma unroll
-    for (int i = 0; i < B_LD; ++i) {
-      int off = b_off[i];
-      bool ok = b_pix[i] < b_end;
-      if (POINTWISE) {
-        b_off[i] += b_step;
-      } else {
-        const int hi = static_cast<int>(b_oh[i]) * p.stride + b_h, wi = static_cast<int>(b_ow[i]) * p.stride + b_w;
-        ok = ok & (static_cast<unsigned>(hi) < static_cast<unsigned>(p.H)) & (static_cast<unsigned>(wi) < static_cast<unsigned>(p.W));
-        off = (((static_cast<int>(b_img[i]) * p.H + hi) * p.W + wi) * p.C + b_c) * 2;
-        b_ow[i] += step_ow;
-        const uint32_t row = b_ow[i] >= static_cast<uint32_t>(p.Wo) ? 1u : 0u;
-        b_ow[i] -= row * p.Wo;
-        b_oh[i] += step_oh + row;
-        const uint32_t img = b_oh[i] >= static_cast<uint32_t>(p.Ho) ? 1u : 0u;
-        b_oh[i] -= img * p.Ho;
-        b_img[i] += step_img + img;
-      }
-      load_to_lds(rsrc_b, dst_b + i * 1024, ok ? off : static_cast<int>(kOutOfRange), 0);
-      b_pix[i] += BKP;
+    const int i = j - A_LD;
+    const int off = b_off[i];
+    bool ok = b_pix[i] < b_end;
+    if (POINTWISE) {
+      b_off[i] += b_step;
+    } else {
+      ok = ok & (static_cast<unsigned>(b_hi[i]) < static_cast<unsigned>(p.H)) & (static_cast<unsigned>(b_wi[i]) < static_cast<unsigned>(p.W));
+      b_wi[i] += step_wi;
+      const bool row = b_wi[i] >= w_end;
+      b_wi[i] -= row ? in_cols : 0;
+      b_hi[i] += row ? step_hi + p.stride : step_hi;
+      const bool img = b_hi[i] >= h_end;
+      b_hi[i] -= img ? in_rows : 0;
+      b_off[i] += row ? off_row : off_step;
+      b_off[i] += img ? off_img : 0;
     }
+    load_to_lds(rsrc_b, lds + buf * BUF_BYTES + A_BYTES + (wave * B_LD + i) * 1024, ok ? off : static_cast<int>(kOutOfRange), 0);
+    b_pix[i] += BKP;
   };
 
   f32x16_t acc[TM][TN];
@@ -1009,39 +1016,30 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
   for (int t = 0; t < TM; ++t) rd_a[t] = lds_base + band(RA, wm * TM + t, swz_a(tr_pix));
 #pragma unroll
   for (int t = 0; t < TN; ++t) rd_b[t] = lds_base + A_BYTES + band(RB, wn * TN + t, swz_b(tr_pix));
-  constexpr int SL = BKP / 16;
+  constexpr int SL = BKP / 16, READS = 2 * (TM + TN);
   uint2_t fa[SL][TM][2], fb[SL][TN][2];
-  // rows + 16 and + 4 keep the row's swizzle (a multiple of four rows)
-  auto read_tile = [&](auto buf_c) {
-    constexpr int AT = decltype(buf_c)::value * BUF_BYTES;
+  // read i of slice ks of the tile in buffer `buf` (rows + 16 and + 4 keep the row's swizzle, a multiple of four rows)
+  auto read_one = [&](auto buf_c, auto ks_c, auto i_c) {
+    constexpr int ks = decltype(ks_c)::value, i = decltype(i_c)::value, t = i & 1, j = i >> 1;
+    constexpr int AT = decltype(buf_c)::value * BUF_BYTES, ROW = ks * 16 + 4 * t;
     auto &ra = fa;
     auto &rb = fb;
-#pragma unroll
-    for (int ks = 0; ks < SL; ++ks)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const uint32_t at = rd_a[tm];
-          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(ra[ks][tm][t]) : "v"(at), "n"(AT + (ks * 16 + 4 * t) * RA));
-        }
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          const uint32_t at = rd_b[tn];
-          asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(rb[ks][tn][t]) : "v"(at), "n"(AT + (ks * 16 + 4 * t) * RB));
-        }
-      }
+    if constexpr (j < TM) {
+      const uint32_t at = rd_a[j];
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(ra[ks][j][t]) : "v"(at), "n"(AT + ROW * RA));
+    } else {
+      const uint32_t at = rd_b[j - TM];
+      asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(rb[ks][j - TM][t]) : "v"(at), "n"(AT + ROW * RB));
+    }
   };
-  auto hold_tile = [&] {
+  auto hold_slice = [&](int ks) {
 #pragma unroll
-    for (int ks = 0; ks < SL; ++ks)
+    for (int t = 0; t < 2; ++t) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(fa[ks][tm][t]));
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) asm volatile("" : "+v"(fa[ks][tm][t]));
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(fb[ks][tn][t]));
-      }
+      for (int tn = 0; tn < TN; ++tn) asm volatile("" : "+v"(fb[ks][tn][t]));
+    }
   };
   auto chunk = [](const uint2_t (&v)[2]) {
     Chunk c;
@@ -1059,40 +1057,86 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm) bsum[tm] = 0.f;
 
-  constexpr int LOADS = A_LD + B_LD;
   constexpr int AHEAD = (NBUF - 2) * LOADS;
+  typedef std::integral_constant<int, 0> first_t;
+  typedef std::integral_constant<int, 1> second_t;
+  static_assert(SL == 2, "two slices a step");
+  // multiplies slice ks; `behind(m)` stands behind its m-th MFMA
+  auto multiply = [&](int ks, auto behind) {
+    Chunk ca[TM], cb[TN];
 #pragma unroll
-  for (int s = 0; s < NBUF - 1; ++s) issue_loads(s);
-  auto step = [&](auto u_c) {
-    constexpr int u = decltype(u_c)::value;
-    wait_and_meet<AHEAD>();
-    read_tile(u_c);
-    issue_loads((u + NBUF - 1) % NBUF);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    hold_tile();
+    for (int tm = 0; tm < TM; ++tm) ca[tm] = chunk(fa[ks][tm]);
 #pragma unroll
-    for (int ks = 0; ks < SL; ++ks) {
-      Chunk ca[TM], cb[TN];
+    for (int tn = 0; tn < TN; ++tn) cb[tn] = chunk(fb[ks][tn]);
+    unrolled<TM * TN>([&](auto m_c) {
+      constexpr int m = decltype(m_c)::value, tm = m / TN, tn = m % TN;
+      mma<bf16>(cb[tn], ca[tm], acc[tm][tn]);
+      behind(m_c);
+    });
+    if (sum_dy) {
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) ca[tm] = chunk(fa[ks][tm]);
+      for (int tm = 0; tm < TM; ++tm) {
+        float v[8];
+        chunk_to_float<bf16>(ca[tm], v);
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) cb[tn] = chunk(fb[ks][tn]);
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) mma<bf16>(cb[tn], ca[tm], acc[tm][tn]);
-      if (sum_dy) {
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          float v[8];
-          chunk_to_float<bf16>(ca[tm], v);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) bsum[tm] += v[e];
-        }
+        for (int e = 0; e < 8; ++e) bsum[tm] += v[e];
       }
     }
-    __builtin_amdgcn_sched_barrier(0);   // the next step's addresses stay in the next step (36 registers less)
   };
+  // 64 x 64: all reads of a step, then its multiplies; others as in igemm2_kernel's interleaved tilings: while slice ks is
+  // multiplied, the slice behind it is read into the other registers and a half of the direct loads goes out.  The barrier that
+  // hands over the next tile stands in front of a tile's last slice, which is in registers by then: the buffer takes another
+  // tile from there on.  128 x 128 alone on a CU: 0.249 -> 0.203 us a step (3072 x 768 over 8192
+  // rows unsplit 71 -> 59.5).  What bounds it with two workgroups on a CU is LDS, 24 KB in and out per 16 pixels: 0.179 both ways.  (64 x 64 has one MFMA to put four reads and a
+  // load behind: 1 x 1 the same, 3 x 3 66 -> 78 us.)
+  constexpr bool INTERLEAVED = TM * TN > 1;
+  constexpr int EARLY = INTERLEAVED ? LOADS / 2 : 0;   // of a tile's loads, behind the second slice; the others behind the next first one
+  auto slice = [&](auto ks_c, auto buf_c, auto ld_buf_c) {   // multiplies slice ks; reads the other one from `buf`
+    constexpr int ks = decltype(ks_c)::value, FROM = ks == 1 ? 0 : EARLY, AUX = READS + (ks == 1 ? EARLY : LOADS - EARLY);
+    constexpr int PER = (AUX + TM * TN - 1) / (TM * TN);
+    multiply(ks, [&](auto m_c) {
+      unrolled<PER>([&](auto a_c) {
+        constexpr int a = decltype(m_c)::value * PER + decltype(a_c)::value;
+        if constexpr (a < READS) read_one(buf_c, std::integral_constant<int, ks ^ 1>{}, std::integral_constant<int, a>{});
+        else if constexpr (a < AUX) issue_load(decltype(ld_buf_c)::value, FROM + a - READS);
+      });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_slice(ks ^ 1);
+  };
+  auto step = [&](auto u_c) {
+    constexpr int u = decltype(u_c)::value, before = (u + NBUF - 1) % NBUF;
+    if constexpr (INTERLEAVED) {
+      slice(first_t{}, u_c, std::integral_constant<int, before>{});
+      wait_and_meet<AHEAD>();
+      slice(second_t{}, std::integral_constant<int, (u + 1) % NBUF>{}, u_c);
+    } else {
+      wait_and_meet<AHEAD>();
+      unrolled<READS>([&](auto i_c) { read_one(u_c, first_t{}, i_c); });
+      unrolled<READS>([&](auto i_c) { read_one(u_c, second_t{}, i_c); });
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) issue_load(before, j);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      hold_slice(0);
+      hold_slice(1);
+      multiply(0, [](auto) {});
+      multiply(1, [](auto) {});
+      __builtin_amdgcn_sched_barrier(0);   // the next step's addresses stay in the next step (36 registers less)
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s)
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) issue_load(s, j);
+  if constexpr (INTERLEAVED) {
+#pragma unroll
+    for (int j = 0; j < EARLY; ++j) issue_load(NBUF - 1, j);
+    wait_and_meet<AHEAD + EARLY>();
+    unrolled<READS>([&](auto i_c) { read_one(first_t{}, first_t{}, i_c); });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    hold_slice(0);
+  }
   int kt = 0;
   for (; kt + NBUF <= nk; kt += NBUF) unrolled<NBUF>(step);
   unrolled<NBUF - 1>([&](auto u_c) {
@@ -3459,8 +3503,9 @@ int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
   }
   // The split count with the shortest start + steps * max(alone, shared * r) + store * (10^6 results written), r =
   // workgroups per compute unit, rounded up: least-squares fits (6-8 % mean error) to 1 500 launches of every split count
-  // on the layers of the three models at 128-8192 rows and 1-64 images, per dtype for 128 x 128 and 64 x 64 tiles.  A
-  // partial filter is read again by the reduction that rides the next launch: kReread on top of what it
+  // on the layers of the three models at 128-8192 rows and 1-64 images, per dtype for 128 x 128 and 64 x 64 tiles
+  // (128 x 128 in bf16 alone on a CU measured again since: 0.249 -> 0.203, GPT-2 8 x 1024 11.20 -> 11.14 ms, ResNet of 32 images 8.94 ->
+  // 8.73).  A partial filter is read again by the reduction that rides the next launch: kReread on top of what it
   // costs to write.  (Aiming at 192-384 workgroups instead split short reductions that were launch latency and
   // partial filters already: 1024 -> 3072 over 343 rows 17.8 us with two splits, 10.1 with one; 256 -> 768 over 5488
   // rows 15.6 with 16, 10.8 with 4.)
@@ -3468,7 +3513,7 @@ int conv2d_wgrad_pick_splits(const ConvShape& s, int dtype) {
     float start, alone, shared, store;
   };
   static const Cost cost[2][2] = {{{3.39f, 0.229f, 0.383f, 1.55f}, {8.56f, 0.371f, 0.912f, 0.71f}},     // fp32: 64, 128
-                                  {{3.08f, 0.109f, 0.089f, 2.33f}, {6.37f, 0.249f, 0.179f, 0.94f}}};   // bf16
+                                  {{3.08f, 0.109f, 0.089f, 2.33f}, {6.37f, 0.203f, 0.179f, 0.94f}}};   // bf16
   constexpr float kReread = 1.f;   // microseconds per 10^6 results; 0 - 2 in the steps: within 1 %, 1 the best of most
   int best = 1;
   float best_us = INFINITY;
