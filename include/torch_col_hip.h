@@ -173,6 +173,7 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * w, output in bf16; anything else runs tilings 24, 23 and 23 for them; same bits as those).
  * 28 / 29 = tiling 5 with 128x128 and 64x64, 30 / 31 = 64x64 and 128x64 with nine filter tiles in LDS instead of three (what tiling 5
  * does not take runs tilings 23, 21, 21 and 22 for them; 5 and 28 - 31 give the same bits).
+ * 32 = 16x16 with the reduction split over eight wavefronts, as 15 - 20 (bf16; fp32 runs tiling 16 for it).
  * c_logical: input channels that carry data when C is zero-padded to a chunk (0 = C); it only enters the
  * algorithmic-work figure the profiler reports, never the arithmetic. */
 int tch_conv2d_fwd(tch_context* ctx, int dtype, const void* x, const void* w, void* y, const void* add,

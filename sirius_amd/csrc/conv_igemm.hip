@@ -2160,6 +2160,10 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm5_kernel(IgemmArgs p) {
 // What bounds it: the trip to memory behind every launch boundary and the chain of steps behind it.  196 x 256 over 2304 (a
 // 3x3 layer of one image) 13.2 -> 6.1 us, 784 x 512 over 4608 36.9 -> 14.8, fp32 784 x 256 over 2304 77.6 -> 14.8 against
 // 64 x 64 tiles of igemm2_kernel / igemm_kernel; the 151 launches of a ResNet-152 request take 4.4-6.9 us each.
+__device__ inline void multiply_add(const Chunk& first, const Chunk& second, f32x4_t& acc) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(first.h, second.h, acc, 0, 0, 0);
+}
+
 // Every wavefront owns the WHOLE TM*32 x TN*32 tile for every KG-th reduction step and has a ring of NBUF operand
 // tiles of its own in LDS, filled with direct loads: nothing is shared before the end, so the main loop has no
 // barrier and a wavefront waits for its own loads only.  The partial tiles meet in LDS once and are added in the
@@ -2167,11 +2171,16 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm5_kernel(IgemmArgs p) {
 // compute unit and a serial chain of nk / KG steps instead of nk.
 // A step is one 64-byte LDS row per GEMM row (32 bf16 or 16 fp32 elements), laid out as in igemm2_kernel with
 // 32-element steps; in_c must be a multiple of the step.
-template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
+// FS = 16 (bf16): tiles of 16 x 16 per MFMA, a whole step each.  What bounds a launch that leaves compute units without a workgroup is
+// the 77 bytes / ns that direct loads bring into the LDS of one: four times the workgroups load half as many bytes each.
+// In a request of one image, 196 rows and 256 channels over 1024 and over 2304: 6.2 us on average on 56 workgroups of 32 x 32, 4.9 on 208;
+// 1024 channels over 256, where 224 fill the chip, 4.0 and 6.6 on 832.
+template <typename T, int MODE, int TM, int TN, int KG, int NBUF, int FS = 32>
 __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int EB = sizeof(T);
-  constexpr int BM = TM * 32, BN = TN * 32;
+  static_assert(FS == 32 || (FS == 16 && sizeof(T) == 2 && TM == 1 && TN == 1), "the shapes of the multiplies below");
+  constexpr int BM = TM * FS, BN = TN * FS;
   constexpr int RB = 64;                 // bytes of one LDS row
   constexpr int KS = RB / EB;            // reduction elements per step
   constexpr int A_LD = BM / 16, B_LD = BN / 16;   // direct loads (sixteen rows each) per step
@@ -2268,18 +2277,19 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
     }
   };
 
-  f32x16_t acc[TM][TN];
-  const int frag_row = lane & 31, frag_half = lane >> 5;
+  typedef std::conditional_t<FS == 32, f32x16_t, f32x4_t> acc_t;
+  acc_t acc[TM][TN];
+  const int frag_row = lane & (FS - 1), frag_half = lane / FS;   // which chunk of a row's slice
   const int swz = (frag_row >> 2) & 3;
   const uint32_t ring_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(ring));
   const uint32_t rd = ring_base + frag_row * RB + swz * 16;
   auto read_frags = [&](int buf, int kk, uint4_t* fa, uint4_t* fb) {
     const uint32_t pa = (rd ^ static_cast<uint32_t>((2 * kk + frag_half) * 16)) + buf * BUF_BYTES;
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[tm]) : "v"(pa), "n"(tm * 32 * RB));
+    for (int tm = 0; tm < TM; ++tm) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[tm]) : "v"(pa), "n"(tm * FS * RB));
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn)
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[tn]) : "v"(pa), "n"(A_BYTES + tn * 32 * RB));
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[tn]) : "v"(pa), "n"(A_BYTES + tn * FS * RB));
   };
   auto hold_frags = [&](uint4_t* fa, uint4_t* fb) {
 #pragma unroll
@@ -2297,7 +2307,8 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) mma<T>(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
+      for (int tn = 0; tn < TN; ++tn) if constexpr (FS == 32) mma<T>(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
+        else multiply_add(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
   };
 
   // The tile of step i lands when at most the NBUF-2 tiles requested behind it are outstanding (near the end fewer
@@ -2305,11 +2316,15 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   constexpr int AHEAD = (NBUF - 2) * (A_LD + B_LD);
   static_assert(AHEAD < 64, "vmcnt range");
   // this wavefront's share of the sums, in `acc`; split_c: in fp32, on the bf16 pipes, small products in `low`
-  auto reduce = [&](auto split_c, f32x16_t (&low)[TM][TN], bool first) {
+  auto reduce = [&](auto split_c, acc_t (&low)[TM][TN], bool first) {
     constexpr bool SPLIT = decltype(split_c)::value;
     rewind();
-    clear(acc);
-    if constexpr (SPLIT) clear(low);
+    if constexpr (FS == 16) {
+      acc[0][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    } else {
+      clear(acc);
+      if constexpr (SPLIT) clear(low);
+    }
     auto step = [&](int i, int buf) {
       if (i + NBUF - 1 <= my_steps)
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AHEAD) : "memory");
@@ -2318,25 +2333,30 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
       if (i + NBUF - 1 < my_steps) issue_loads((buf + NBUF - 1) % NBUF);
       uint4_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
       read_frags(buf, 0, fa0, fb0);
-      read_frags(buf, 1, fa1, fb1);
-      if constexpr (SPLIT) {
+      if constexpr (FS == 16) {   // the whole step is one operand
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        hold_frags(fa0, fb0);
-        hold_frags(fa1, fb1);
-        Split8 sb[TN];
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) sb[tn] = split8(chunk(fb0[tn]), chunk(fb1[tn]));
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) {
-          const Split8 sa = split8(chunk(fa0[tm]), chunk(fa1[tm]));
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn) mma_split(sb[tn], sa, acc[tm][tn], low[tm][tn]);
-        }
-      } else {
-        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN) : "memory");
         multiply(fa0, fb0);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        multiply(fa1, fb1);
+      } else {
+        read_frags(buf, 1, fa1, fb1);
+        if constexpr (SPLIT) {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          hold_frags(fa0, fb0);
+          hold_frags(fa1, fb1);
+          Split8 sb[TN];
+  #pragma unroll
+          for (int tn = 0; tn < TN; ++tn) sb[tn] = split8(chunk(fb0[tn]), chunk(fb1[tn]));
+  #pragma unroll
+          for (int tm = 0; tm < TM; ++tm) {
+            const Split8 sa = split8(chunk(fa0[tm]), chunk(fa1[tm]));
+  #pragma unroll
+            for (int tn = 0; tn < TN; ++tn) mma_split(sb[tn], sa, acc[tm][tn], low[tm][tn]);
+          }
+        } else {
+          asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TM + TN) : "memory");
+          multiply(fa0, fb0);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          multiply(fa1, fb1);
+        }
       }
     };
 #pragma unroll
@@ -2375,8 +2395,8 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
 #pragma unroll
           for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              *reinterpret_cast<float4*>(mine + (tm * 32 + frag_row) * LD + tn * 32 + 8 * j + 4 * frag_half) =
+            for (int j = 0; j < (FS == 32 ? 4 : 1); ++j)
+              *reinterpret_cast<float4*>(mine + (tm * FS + frag_row) * LD + tn * FS + 8 * j + 4 * frag_half) =
                   make_float4(acc[tm][tn][4 * j], acc[tm][tn][4 * j + 1], acc[tm][tn][4 * j + 2], acc[tm][tn][4 * j + 3]);
         __syncthreads();
         if (NTE < NT && tid >= NTE) return;
@@ -2800,9 +2820,9 @@ int launch_cfg5(Context* ctx, IgemmArgs& a, double flops) {
                 name.c_str(), flops, 0, conv_bytes<MODE>(a, 2));
 }
 
-template <typename T, int MODE, int TM, int TN, int KG, int NBUF>
+template <typename T, int MODE, int TM, int TN, int KG, int NBUF, int FS = 32>
 int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
-  constexpr int BM = TM * 32, BN = TN * 32;
+  constexpr int BM = TM * FS, BN = TN * FS;
   static const std::string name = std::string("igemm4_kernel<") + (sizeof(T) == 2 ? "bf16," : "f32,") +
                                   (MODE == kFwd ? "fwd," : "dgrad,") + std::to_string(BM) + "x" + std::to_string(BN) + "," +
                                   std::to_string(KG) + "way," + std::to_string(NBUF) + "buf>";
@@ -2816,7 +2836,7 @@ int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
   // the larger operand is the one an XCD should fetch once
   a.group_rows = static_cast<int64_t>(a.gemm_n) * a.gemm_k > static_cast<int64_t>(a.a_bytes / sizeof(T)) ? 1 : 0;
   bind_divisions(a, a.group_rows ? a.tiles_m : a.tiles_n);
-  return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF>, dim3(static_cast<unsigned>(wgs)), dim3(KG * 64), a, name.c_str(),
+  return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF, FS>, dim3(static_cast<unsigned>(wgs)), dim3(KG * 64), a, name.c_str(),
                 flops, 0, conv_bytes<MODE>(a, sizeof(T)));
 }
 
@@ -2886,6 +2906,7 @@ enum SplitTile : int {
   kSplit64 = 18,         // 64 x 64, 4, 4 (fp32: 8, 2)
   kSplit64Pair = 19,     // 64 x 64, 4, 2
   kSplit64x32Deep = 20,  // 64 x 32, 8, 3
+  kSplit16 = 32,         // 16 x 16, 8, 4 (bf16)
 };
 
 // Tilings of igemm2_kernel with pipelined operand reads
@@ -2916,7 +2937,7 @@ enum PatchTile : int {
   kPatch64Deep = 30,       // the same with nine filter tiles in LDS instead of three
   kPatch128x64Deep = 31,   // 5 with nine
 };
-bool patch_tile(int tile_cfg) { return tile_cfg == 5 || tile_cfg >= kPatch128; }
+bool patch_tile(int tile_cfg) { return tile_cfg == 5 || (tile_cfg >= kPatch128 && tile_cfg <= kPatch128x64Deep); }
 bool patch_64_rows(int tile_cfg) { return tile_cfg == kPatch64 || tile_cfg == kPatch64Deep; }
 
 // the tiling of the same shape that runs where a pipelined one does not exist
@@ -2968,6 +2989,9 @@ template <typename T, int MODE>
 int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
   static_assert(MODE == kFwd || MODE == kDgrad, "weight gradients go through launch_wgrad");
   switch (tile_cfg) {
+    case kSplit16:
+      if constexpr (sizeof(T) == 2) return launch_cfg4<T, MODE, 1, 1, 8, 4, 16>(ctx, a, flops);
+      return launch_cfg4<T, MODE, 1, 1, 8, 2>(ctx, a, flops);   // not reached: effective_tile
     case kSplit32:
       return launch_cfg4<T, MODE, 1, 1, 4, 4>(ctx, a, flops);
     case kSplit32Deep:
@@ -3070,6 +3094,7 @@ double conv_flops(const ConvShape& s, int Ho, int Wo) {
 // rows of the workgroup tile of a tiling number (5 = the 3x3 patch kernel, or tiling 1 where it does not fit)
 int tile_rows(int tile_cfg) {
   if (tile_cfg == 9 || tile_cfg == 10) return 256;
+  if (tile_cfg == kSplit16) return 16;
   if (tile_cfg >= kPipe64) return tile_cfg == kPipe64 || patch_64_rows(tile_cfg) ? 64 : 128;
   if (tile_cfg >= kSplit32) return tile_cfg <= kSplit32Deep ? 32 : 64;
   if (tile_cfg >= 11 && tile_cfg <= 14) return tile_cfg == 14 ? 64 : 128;
@@ -3078,7 +3103,7 @@ int tile_rows(int tile_cfg) {
 
 // column tiles of 32: callers of the in-kernel finalize provide a counter per 64 columns
 bool narrow_tile(int tile_cfg) {
-  return tile_cfg == kSplit32 || tile_cfg == kSplit32Deep || tile_cfg == kSplit64x32 || tile_cfg == kSplit64x32Deep;
+  return tile_cfg == kSplit16 || tile_cfg == kSplit32 || tile_cfg == kSplit32Deep || tile_cfg == kSplit64x32 || tile_cfg == kSplit64x32Deep;
 }
 
 int64_t tiles_for(int m, int n, int bm, int bn) {
@@ -3107,6 +3132,7 @@ bool direct_tile_fits(int dtype, int in_c, int taps) {
 int effective_tile(int tile_cfg, int dtype, int in_c, int taps) {
   if ((tile_cfg == 9 || tile_cfg == 10) && !(dtype == kBF16 && in_c % 64 == 0 && taps <= 32 && igemm2_setting() != 0))
     return 0;
+  if (tile_cfg == kSplit16) return !split_tile_fits(dtype, in_c, taps) ? 2 : dtype == kBF16 ? tile_cfg : kSplit32Deep;
   if (tile_cfg >= kPipe64) return direct_tile_fits(dtype, in_c, taps) ? tile_cfg : pipe_stand_in(tile_cfg);
   if (tile_cfg >= kSplit32 && !split_tile_fits(dtype, in_c, taps)) return 2;
   return tile_cfg;
@@ -3133,7 +3159,7 @@ int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
 // 556 different convolutions where they stand in a step or request, one launch at a time (operands as cold or warm as their
 // producers leave them; 3 us of event among it), each with every tiling: ResNet-152 at 1-64 images, GPT-2 at 512-8192
 // tokens, Swin-B at 3-32 images; the second table for ResNet's data gradients with the BatchNorm sums, whose epilogue
-// reads two more tensors.  (The patch tilings, 5 and 28-31, were fitted in the same way to ResNet-152's 3x3 convolutions alone:
+// reads two more tensors.  (kSplit16: two points of requests of one image, 208 and 832 workgroups, see igemm4_kernel.  The patch tilings, 5 and 28-31, were fitted in the same way to ResNet-152's 3x3 convolutions alone:
 // one round of workgroups is fastest with nine filter tiles, several with three, of which two workgroups fit on a CU.)  (Fits to launches repeated on warm operands prefer large tiles: a request of 24 images took
 // 2437 us with them, 2098 with these.)  Against the fastest of all tilings per launch, summed over a step or request: 1-2 %, one image 3.
 // Tilings without an entry (3, 6, 7, 11, kSplit64, kSplit64Pair, kSplit64x32Deep: for callers that ask, and for tuners) are
@@ -3151,7 +3177,7 @@ const TileCost kPlainCost[] = {
     {kPipe64, 64, 64, 6.24f, 0.00f, 0.264f, 0.194f, 1.40f}, {kMix128x64, 128, 64, 5.60f, 1.22f, 0.336f, 0.340f, 0.83f},
     {kMix128, 128, 128, 5.74f, 1.31f, 0.542f, 0.493f, 0.72f}, {kMix128x192, 128, 192, 5.38f, 3.00f, 0.677f, 0.639f, 0.53f},
     {kPatch128, 128, 128, 6.02f, 0.53f, 0.404f, 0.404f, 0.71f}, {kPatch64, 64, 64, 5.37f, 0.00f, 0.303f, 0.134f, 1.64f},
-    {kPatch64Deep, 64, 64, 5.30f, 1.53f, 0.142f, 0.161f, 1.62f}, {kPatch128x64Deep, 128, 64, 5.63f, 1.04f, 0.188f, 0.206f, 1.56f}};
+    {kSplit16, 16, 16, 4.00f, 1.20f, 0.055f, 0.060f, 3.00f}, {kPatch64Deep, 64, 64, 5.30f, 1.53f, 0.142f, 0.161f, 1.62f}, {kPatch128x64Deep, 128, 64, 5.63f, 1.04f, 0.188f, 0.206f, 1.56f}};
 const TileCost kSumsCost[] = {
     {0, 128, 128, 6.87f, 3.59f, 0.830f, 0.404f, 0.69f}, {1, 128, 64, 6.60f, 1.70f, 0.430f, 0.290f, 0.65f},
     {2, 64, 64, 6.41f, 0.85f, 0.364f, 0.188f, 0.53f}, {5, 128, 64, 3.36f, 5.47f, 0.295f, 0.010f, 0.64f},
@@ -3257,7 +3283,7 @@ int heuristic_tile(int asked, const TileQuery& q) {
     if (t.bn >= 2 * q.gemm_n && t.bn > 32) continue;
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (patch_tile(t.cfg) && (!q.patch || asked == kAutoInOrder)) continue;
-    if (t.cfg >= kSplit32 && t.cfg <= kSplit64x32Deep && asked == kAutoInOrder) continue;
+    if (t.bm * t.bn <= 64 * 32 && asked == kAutoInOrder) continue;   // igemm4_kernel's
     take(t);
   }
   // Data gradients run beside weight gradients, whose LDS has no room on a compute unit that igemm5_kernel holds; from about 2560

@@ -66,6 +66,7 @@ struct Elem<bf16> {
 // A 16-byte chunk as it travels global -> register -> LDS -> MFMA operand.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16_t;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 
 union Chunk {
   uint4 u;
