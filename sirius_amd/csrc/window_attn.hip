@@ -15,6 +15,11 @@
 //              dS goes to memory (its sum over windows is the bias gradient) and, with P, to LDS as [query][key]
 //              phase 2 (lane = key):   dV^T = dO^T P, dK^T = Q^T dS, both operands read by transposing loads
 //
+// What bounds them is memory: a problem reads and writes 19 KB (backward 34) and multiplies next to nothing.  Every load of a workgroup is
+// requested before the first is waited for, and the probabilities and dS go through LDS rows to memory, 16 bytes a lane, both
+// ways (in the accumulators' layout a load or store touches 32 rows with 16 bytes each).  Warm, 2048 windows x 4 heads: forward 44
+// -> 35.5 us, backward 80 -> 52.5 (4.3 and 5.4 TB/s); 128 x 16 13.2 -> 11.4 and 19.9 -> 16.1; Swin-B of 32 images 9.73 -> 9.34 ms.
+//
 // The bias arrives gathered per head as [heads][64][64] fp32 with -inf in the key columns beyond the window's
 // tokens (that is what masks the padding); the shift mask as [windows per image][64][64] fp32.
 #include "attn_frag.h"
@@ -32,6 +37,7 @@ constexpr int kRowP = 144;           // LDS bytes per [query][64 keys] row
 constexpr int kTileS = kTok * kRowS; // 5120
 constexpr int kTileP = kTok * kRowP; // 9216
 constexpr int kPatch = 32 * kRowS;   // 2560: one wave's output rows on their way to memory
+constexpr int kPatchP = 32 * kRowP;  // 4608: one wave's probabilities
 
 struct WinAttnArgs {
   const bf16* qkv;     // [windows * N][3C]
@@ -46,16 +52,39 @@ struct WinAttnArgs {
   float scale;
 };
 
-// rows [0, N) of one head's [N][32] slice (row stride `rs` elements) into a zero-padded [64][32] LDS tile, by the
-// 128 threads of a wave pair
-__device__ inline void stage_rows(const bf16* base, int64_t rs, int N, unsigned char* tile, int t2) {
+// rows [0, N) of one head's [N][32] slice (row stride `rs` elements), by the 128 threads of a wave pair, and the zero-padded
+// [64][32] LDS tile they become.  (Apart, so that a kernel asks for everything before it waits for anything.)
+struct HeadRows {
+  uint4 lo, hi;   // rows t2 / 4 and 32 + t2 / 4, slot t2 % 4
+};
+__device__ inline HeadRows load_rows(const bf16* base, int64_t rs, int N, int t2) {
+  const int row = t2 >> 2, slot = t2 & 3;
+  HeadRows r;
+  r.lo = r.hi = make_uint4(0u, 0u, 0u, 0u);
+  if (row < N) r.lo = *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(row) * rs + slot * 8);
+  if (row + 32 < N) r.hi = *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(row + 32) * rs + slot * 8);
+  return r;
+}
+__device__ inline void stage_rows(const HeadRows& r, unsigned char* tile, int t2) {
+  unsigned char* dst = tile + (t2 >> 2) * kRowS + (t2 & 3) * 16;
+  *reinterpret_cast<uint4*>(dst) = r.lo;
+  *reinterpret_cast<uint4*>(dst + 32 * kRowS) = r.hi;
+}
+
+// what one lane of a wave wrote to LDS is there for its other lanes (a wave's LDS accesses stay in order)
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// 32 rows of a [N][64] bf16 matrix that is contiguous in memory, from row `first` on: LDS rows of kRowP bytes -> memory, 16 bytes
+// a lane of one wave.  (Written from the accumulators' layout instead, a store touches 32 rows with 16 bytes each.)
+__device__ inline void copy_rows_out(const unsigned char* tile, bf16* to, int N, int first, int lane) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = t2 + 128 * i;
-    const int row = c >> 2, slot = c & 3;
-    uint4 v = make_uint4(0u, 0u, 0u, 0u);
-    if (row < N) v = *reinterpret_cast<const uint4*>(base + static_cast<int64_t>(row) * rs + slot * 8);
-    *reinterpret_cast<uint4*>(tile + row * kRowS + slot * 16) = v;
+  for (int i = 0; i < 4; ++i) {
+    const int row = (lane >> 3) + 8 * i, slot = lane & 7;
+    if (first + row < N)
+      *reinterpret_cast<uint4*>(to + (first + row) * kTok + slot * 8) = *reinterpret_cast<const uint4*>(tile + row * kRowP + slot * 16);
   }
 }
 
@@ -63,6 +92,7 @@ __device__ inline void stage_rows(const bf16* base, int64_t rs, int N, unsigned 
 // those below N exist, 32 columns, row stride rs
 __device__ inline void store_rows(const f32x16_t& acc, float mul, unsigned char* patch, bf16* base, int64_t rs, int first,
                                   int N, int lane) {
+  wave_sync();   // the patch may hold what the wave stored last
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     uint2 w;
@@ -70,7 +100,7 @@ __device__ inline void store_rows(const f32x16_t& acc, float mul, unsigned char*
     w.y = pack_bf16(acc[4 * j + 2] * mul, acc[4 * j + 3] * mul);
     *reinterpret_cast<uint2*>(patch + (lane & 31) * kRowS + (8 * j + 4 * (lane >> 5)) * 2) = w;
   }
-  __syncthreads();
+  wave_sync();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int q = lane + 64 * i;
@@ -82,19 +112,17 @@ __device__ inline void store_rows(const f32x16_t& acc, float mul, unsigned char*
 }
 
 __global__ __launch_bounds__(256) void window_attn_fwd_kernel(WinAttnArgs p) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 2 * kTileS + 4 * kPatch];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * 2 * kTileS + 4 * kPatchP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5;
   const int pair = wave >> 1, wp = wave & 1;
   const int pidx = blockIdx.x * 2 + pair;
   const int win = pidx / p.heads, h = pidx - win * p.heads;
   unsigned char* kt = lds + pair * 2 * kTileS;
   unsigned char* vt = kt + kTileS;
-  unsigned char* patch = lds + 4 * kTileS + wave * kPatch;
+  unsigned char* patch = lds + 4 * kTileS + wave * kPatchP;   // the wave's probabilities, then its output rows
   const int64_t rs = 3 * static_cast<int64_t>(p.C);
   const bf16* qbase = p.qkv + static_cast<int64_t>(win) * p.N * rs + h * kHd;
-  stage_rows(qbase + p.C, rs, p.N, kt, tid & 127);
-  stage_rows(qbase + 2 * p.C, rs, p.N, vt, tid & 127);
-
+  const HeadRows kr = load_rows(qbase + p.C, rs, p.N, tid & 127), vr = load_rows(qbase + 2 * p.C, rs, p.N, tid & 127);
   const int query = 32 * wp + (lane & 31);
   const bool live = query < p.N;
   Chunk qf[2];
@@ -103,6 +131,8 @@ __global__ __launch_bounds__(256) void window_attn_fwd_kernel(WinAttnArgs p) {
     qf[ks] = zero_chunk();
     if (live) qf[ks].u = *reinterpret_cast<const uint4*>(qbase + static_cast<int64_t>(query) * rs + ks * 16 + 8 * half);
   }
+  stage_rows(kr, kt, tid & 127);
+  stage_rows(vr, vt, tid & 127);
   __syncthreads();
 
   f32x16_t s[2];
@@ -147,7 +177,6 @@ __global__ __launch_bounds__(256) void window_attn_fwd_kernel(WinAttnArgs p) {
     }
   sum += __shfl_xor(sum, 32, 64);
   const float inv = 1.f / sum;
-  bf16* prow = p.probs + (static_cast<int64_t>(pidx) * p.N + query) * kTok;
   f32x16_t acc;
   zero_acc(acc);
 #pragma unroll
@@ -157,13 +186,14 @@ __global__ __launch_bounds__(256) void window_attn_fwd_kernel(WinAttnArgs p) {
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
       const Chunk pc = pack_slab(&pr[t][8 * sl]);
-      if (live) {
-        *reinterpret_cast<uint2*>(prow + 32 * t + 16 * sl + 4 * half) = make_uint2(pc.w[0], pc.w[1]);
-        *reinterpret_cast<uint2*>(prow + 32 * t + 16 * sl + 8 + 4 * half) = make_uint2(pc.w[2], pc.w[3]);
-      }
+      unsigned char* to = patch + (lane & 31) * kRowP + (32 * t + 16 * sl + 4 * half) * 2;
+      *reinterpret_cast<uint2*>(to) = make_uint2(pc.w[0], pc.w[1]);
+      *reinterpret_cast<uint2*>(to + 16) = make_uint2(pc.w[2], pc.w[3]);
       acc = mma16(frag_cols<kRowS>(vt, 32 * t + 16 * sl, 0, lane), pc, acc);
     }
   }
+  wave_sync();
+  copy_rows_out(patch, p.probs + static_cast<int64_t>(pidx) * p.N * kTok, p.N, 32 * wp, lane);
   store_rows(acc, 1.f, patch, p.o + static_cast<int64_t>(win) * p.N * p.C + h * kHd, p.C, 32 * wp, p.N, lane);
 }
 
@@ -185,30 +215,39 @@ __global__ __launch_bounds__(256) void window_attn_bwd_kernel(WinAttnArgs p) {
   const int64_t row0 = static_cast<int64_t>(win) * p.N;
   const bf16* qbase = p.qkv + row0 * rs + h * kHd;
   const bf16* dobase = p.dout + row0 * p.C + h * kHd;
-  stage_rows(qbase, rs, p.N, qt, tid & 127);
-  stage_rows(qbase + p.C, rs, p.N, kt, tid & 127);
-  stage_rows(qbase + 2 * p.C, rs, p.N, vt, tid & 127);
-  stage_rows(dobase, p.C, p.N, dot, tid & 127);
+  const int t2 = tid & 127;
+  {
+    const bf16* probs = p.probs + static_cast<int64_t>(pidx) * p.N * kTok;
+    const HeadRows vr = load_rows(qbase + 2 * p.C, rs, p.N, t2), dr = load_rows(dobase, p.C, p.N, t2);
+    uint4 pr4[4];   // rows t2 / 8 + 16 i: zeros beyond the window's tokens
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pr4[i] = make_uint4(0u, 0u, 0u, 0u);
+      if ((t2 >> 3) + 16 * i < p.N) pr4[i] = *reinterpret_cast<const uint4*>(probs + t2 * 8 + 16 * i * kTok);
+    }
+    const HeadRows kr = load_rows(qbase + p.C, rs, p.N, t2), qr = load_rows(qbase, rs, p.N, t2);
+    stage_rows(vr, vt, t2);
+    stage_rows(dr, dot, t2);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(pt + ((t2 >> 3) + 16 * i) * kRowP + (t2 & 7) * 16) = pr4[i];
+    stage_rows(kr, kt, t2);
+    stage_rows(qr, qt, t2);
+  }
+  __syncthreads();
 
   // ---- phase 1: this wave's 32 queries ----
   const int query = 32 * wp + (lane & 31);
-  const bool live = query < p.N;
   float pr[2][16];
-  {
-    const bf16* prow = p.probs + (static_cast<int64_t>(pidx) * p.N + query) * kTok;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        uint2 w = make_uint2(0u, 0u);
-        if (live) w = *reinterpret_cast<const uint2*>(prow + 32 * t + 8 * j + 4 * half);
-        pr[t][4 * j] = __uint_as_float(w.x << 16);
-        pr[t][4 * j + 1] = __uint_as_float(w.x & 0xffff0000u);
-        pr[t][4 * j + 2] = __uint_as_float(w.y << 16);
-        pr[t][4 * j + 3] = __uint_as_float(w.y & 0xffff0000u);
-      }
-  }
-  __syncthreads();
+    for (int j = 0; j < 4; ++j) {
+      const uint2 w = *reinterpret_cast<const uint2*>(pt + query * kRowP + (32 * t + 8 * j + 4 * half) * 2);
+      pr[t][4 * j] = __uint_as_float(w.x << 16);
+      pr[t][4 * j + 1] = __uint_as_float(w.x & 0xffff0000u);
+      pr[t][4 * j + 2] = __uint_as_float(w.y << 16);
+      pr[t][4 * j + 3] = __uint_as_float(w.y & 0xffff0000u);
+    }
   f32x16_t dp[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
@@ -223,7 +262,6 @@ __global__ __launch_bounds__(256) void window_attn_bwd_kernel(WinAttnArgs p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) delta += pr[t][r] * dp[t][r];
   delta += __shfl_xor(delta, 32, 64);
-  bf16* dsrow = p.ds + (static_cast<int64_t>(pidx) * p.N + query) * kTok;
   f32x16_t dq;
   zero_acc(dq);
 #pragma unroll
@@ -233,21 +271,15 @@ __global__ __launch_bounds__(256) void window_attn_bwd_kernel(WinAttnArgs p) {
     for (int r = 0; r < 16; ++r) ds[r] = pr[t][r] * (dp[t][r] - delta);
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
-      const Chunk pc = pack_slab(&pr[t][8 * sl]);
       const Chunk dc = pack_slab(&ds[8 * sl]);
       const int col = 32 * t + 16 * sl + 4 * half;
-      if (live) {
-        *reinterpret_cast<uint2*>(dsrow + col) = make_uint2(dc.w[0], dc.w[1]);
-        *reinterpret_cast<uint2*>(dsrow + col + 8) = make_uint2(dc.w[2], dc.w[3]);
-      }
-      *reinterpret_cast<uint2*>(pt + query * kRowP + col * 2) = make_uint2(pc.w[0], pc.w[1]);
-      *reinterpret_cast<uint2*>(pt + query * kRowP + (col + 8) * 2) = make_uint2(pc.w[2], pc.w[3]);
       *reinterpret_cast<uint2*>(dst + query * kRowP + col * 2) = make_uint2(dc.w[0], dc.w[1]);
       *reinterpret_cast<uint2*>(dst + query * kRowP + (col + 8) * 2) = make_uint2(dc.w[2], dc.w[3]);
       dq = mma16(frag_cols<kRowS>(kt, 32 * t + 16 * sl, 0, lane), dc, dq);
     }
   }
-  __syncthreads();   // P and dS of all 64 queries are in LDS; K and V are no longer read
+  __syncthreads();   // dS of all 64 queries is in LDS; K and V are no longer read
+  copy_rows_out(dst + 32 * wp * kRowP, p.ds + static_cast<int64_t>(pidx) * p.N * kTok, p.N, 32 * wp, lane);
   store_rows(dq, p.scale, patch, p.dqkv + row0 * rs + h * kHd, rs, 32 * wp, p.N, lane);
 
   // ---- phase 2: this wave's 32 keys ----
