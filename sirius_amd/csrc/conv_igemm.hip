@@ -2441,11 +2441,12 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
 // multiplies.  Warm, 7x7 of 64 images, 512 channels: 27.0 -> 20.5 us; in place, 14x14 of 16 images, 256
 // channels: forward 16.4 -> 14.1, data gradient with sums 17.7 -> 14.6.
 // ---------------------------------------------------------------------------
-// of the `steps` steps up to the one with tap `tap`, how many request a load of the next patch
+// Of the `steps` steps up to the one with tap `tap`, how many request a load of the next patch in this channel block.  (Those of the
+// block before do not count: the first block has none before it, whose patch is older than every filter.)
 template <int P_LD>
 constexpr int patch_loads_among(int tap, int steps) {
   int n = 0;
-  for (int i = 0; i < steps; ++i) n += (tap + 9 - i) % 9 < P_LD ? 1 : 0;
+  for (int i = 0; i < steps && i <= tap; ++i) n += tap - i < P_LD ? 1 : 0;
   return n;
 }
 
@@ -2610,7 +2611,7 @@ __global__ __launch_bounds__(WM * 128) void igemm3_kernel(IgemmArgs p) {
       });
       slice(integral_constant<int, 0>{}, row, integral_constant<int, u>{}, integral_constant<int, 3>{}, [&] {});
       // Filter kt + 1 has landed when only what was requested behind it is outstanding: filters kt + 2 .. kt + NBUF-1 and the loads
-      // of patches in this step and the NBUF-2 before it.  In front of the next channel block its patch has to be there as well,
+      // of the next patch in this step and the NBUF-2 before it.  In front of the next channel block its patch has to be there as well,
       // whose last load has the filter loads of 9 - P_LD steps behind it.
       constexpr int newer = (NBUF - 2) * B_LD + patch_loads_among<P_LD>(tap, NBUF - 1);
       wait_and_meet<tap == 8 ? std::min(newer, (9 - P_LD) * B_LD) : newer>();

@@ -68,3 +68,29 @@ def test_tilings_give_the_same_bits():
         ops.conv2d_fwd(ctx, x, wt, out[-1], 1, 1, tile_cfg=cfg)
     torch.cuda.synchronize()
     assert all(torch.equal(out[0], o) for o in out[1:])
+
+
+@pytest.mark.parametrize("shape", [(64, 56, 56, 64, 64), (32, 28, 28, 128, 128)])
+@pytest.mark.parametrize("tile_cfg", [5, 28, 29, 30, 31])
+def test_first_filters_are_waited_for(tile_cfg, shape):
+    """With nine filter tiles in LDS the first channel block has fewer loads in flight than the later ones: a count that takes
+    the next patch's loads of a block before it for granted lets a step read its filter early.  Beside another stream's work."""
+    from sirius_amd import ops
+    n, h, w, c, k = shape
+    beside = torch.cuda.Stream()
+    ctx, other = ops.Context(torch.cuda.current_stream()), ops.Context(beside)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    x, wt, ox, ody = rand(n, h, w, c), rand(k, 3, 3, c), rand(64, 14, 14, 256), rand(64, 14, 14, 1024)
+    odw = torch.zeros(1024, 1, 1, 256, device="cuda")
+    ref = torch.empty(n, h, w, k, device="cuda", dtype=torch.bfloat16)
+    ops.conv2d_fwd(ctx, x, wt, ref, 1, 1, tile_cfg=5)
+    torch.cuda.synchronize()
+    for i in range(30):
+        y = torch.full_like(ref, float("nan"))
+        torch.cuda.synchronize()
+        for _ in range(i % 3):
+            ops.conv2d_wgrad(other, ox, ody, odw, 1, 0)
+        ops.conv2d_fwd(ctx, x, wt, y, 1, 1, tile_cfg=tile_cfg)
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref), i
