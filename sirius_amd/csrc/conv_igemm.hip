@@ -103,7 +103,7 @@ struct IgemmArgs {
   int group_rows;   // FWD/DGRAD direct-to-LDS kernel: row tiles per group of the tile order (0 / 1: row-major)
   int k_per_split;  // multiple of BK
   int out_f32;      // FWD/DGRAD: store fp32 instead of T
-  int in_fp32;      // fp32, igemm_kernel: no parts (fp32_split.h), so that every tile adds up the same bits
+  int in_fp32;      // fp32: no parts (fp32_split.h), see split_products()
   int accumulate;   // WGRAD with splits == 1: out += result
   int take_pending; // WGRAD, read by the launcher only: the context's pending split reduction rides this launch
   int pointwise;    // 1x1, stride 1, pad 0
@@ -597,6 +597,16 @@ struct TileEpilogue {
   }
 };
 
+// Whether an fp32 product runs on the bf16 pipes.  Not one that was asked for front to back, where every tile adds up the same
+// bits, and not a convolution whose output a training BatchNorm takes: behind it stands a ReLU, and whichever of two equally
+// good roundings a pre-activation gets near zero, another one opens or closes gates, each of which moves a gradient by more than all
+// other rounding does (ResNet-152 of 4 images, the gradients against those of fp32 multiplies: 2e-7 relative without a gate, 7.5e-5
+// with two).  Data and weight gradients are smooth.
+template <int MODE>
+__device__ inline bool split_products(const IgemmArgs& p) {
+  return p.gemm_k > kShortReduction && !p.in_fp32 && !(MODE == kFwd && (p.stats || p.stat_acc));
+}
+
 // ---------------------------------------------------------------------------
 // forward / data gradient
 // ---------------------------------------------------------------------------
@@ -791,7 +801,7 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
   // (512 x 768 over 768 21.8 us in fp32, 23.9 in parts, as 128 x 128 57.4 and 50.2)
   if constexpr (EB == 4 && TM * TN > 1) {
     f32x16_t low[TM][TN];
-    bool plain = p.gemm_k <= kShortReduction || p.in_fp32;
+    bool plain = !split_products<MODE>(p);
     if (!plain) {
       reduce(std::true_type{}, low);
       plain = __syncthreads_or(join_split(acc, low));
@@ -2374,12 +2384,12 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   };
   if constexpr (sizeof(T) == 4) {
     f32x16_t low[TM][TN];
-    bool plain = p.gemm_k <= kShortReduction;
+    bool plain = !split_products<MODE>(p);
     if (!plain) {
       reduce(std::true_type{}, low, true);
       plain = __any(join_split(acc, low));
     }
-    if (plain) reduce(std::false_type{}, low, p.gemm_k <= kShortReduction);
+    if (plain) reduce(std::false_type{}, low, !split_products<MODE>(p));
   } else {
     reduce(std::false_type{}, acc, true);
   }
