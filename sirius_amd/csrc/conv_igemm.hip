@@ -3236,6 +3236,7 @@ struct TileQuery {
   bool sums;    // data gradient with the BatchNorm sums in its epilogue
   bool dgrad;
   bool walk = false;   // igemm5_kernel takes it
+  bool counted = false;   // a forward product whose row tiles leave sums: callers size those for row tiles of 32 at the least
 };
 // igemm5_kernel's tilings, priced as kPlainCost (r = tiles of a workgroup, one of them on a CU).  Fits to the linear layers of GPT-2 at 1024-
 // 8192 tokens and of Swin-B at 4-32 images where they stand, 220 different ones with each tiling (mean error 5-8 %): first
@@ -3295,6 +3296,7 @@ int heuristic_tile(int asked, const TileQuery& q) {
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (patch_tile(t.cfg) && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.bm * t.bn <= 64 * 32 && asked == kAutoInOrder) continue;   // igemm4_kernel's
+    if (t.bm < 32 && q.counted) continue;
     take(t);
   }
   // Data gradients run beside weight gradients, whose LDS has no room on a compute unit that igemm5_kernel holds; from about 2560
@@ -3411,7 +3413,8 @@ int conv2d_fwd(Context* ctx, int dtype, const ConvShape& s, const void* x, const
   a.div_width = FastDiv(a.Wo);
   a.in_fp32 = asks_in_order(tile_cfg) ? 1 : 0;
   if (tile_cfg < 0) {
-    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false, walk_tile_fits(a)});
+    tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false, walk_tile_fits(a),
+                                         bn_partial || bn_acc});
     // statistics are sized by the caller for the heuristic's row tiles: leave those launches alone
     if (!bn_partial && !bn_acc && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.C, s.R * s.S)) tile_cfg = 10;
   }
@@ -3431,7 +3434,7 @@ int conv2d_fwd_stat_rows(const ConvShape& s, int dtype, int tile_cfg) {
   int Ho, Wo;
   conv_output_hw(s, &Ho, &Wo);
   const int gemm_m = s.N * Ho * Wo;
-  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false});
+  if (tile_cfg < 0) tile_cfg = heuristic_tile(tile_cfg, {dtype, gemm_m, s.K, s.R * s.S * s.C, s.C, s.R * s.S, patch_kernel_fits(s, s.C), false, false, false, true});
   tile_cfg = effective_tile(tile_cfg, dtype, s.C, s.R * s.S);
   const int bm = tile_rows(tile_cfg);
   return (gemm_m + bm - 1) / bm;

@@ -37,3 +37,11 @@ def test_forward_and_data_gradient(ctx, dtype, case):
 def test_batchnorm_sums(ctx, dtype, case):
     T.test_conv_with_bn_statistics(ctx, dtype, case, 32)
     T.test_conv_dgrad_with_bn_backward_sums(ctx, dtype, case, 32, True)
+
+
+def test_statistics_keep_row_tiles_of_32():
+    """Callers size the sums of a forward product for the row tiles of tiling 15, the smallest that the choice made for one."""
+    from sirius_amd import ops
+    for n, h, c, k, r in [(1, 14, 1024, 256, 1), (1, 14, 256, 256, 3), (1, 7, 512, 512, 3), (2, 7, 2048, 512, 1)]:
+        x = torch.empty(n, h, h, c, dtype=torch.bfloat16, device="meta")
+        assert ops.conv2d_fwd_stat_rows(x, k, r, r, 1, r // 2) <= ops.conv2d_fwd_stat_rows(x, k, r, r, 1, r // 2, 15)
