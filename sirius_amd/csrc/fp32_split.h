@@ -15,13 +15,16 @@
 // its operands' way to the CU (the same 21 us of 26 without the split and five of the six multiplies).
 // Alone, before and after: 512 x 768 over 3072 31.0 -> 25.6 us, 512 x 3072 over 768 25.3 -> 22.1, weight gradient 768 x 3072 over 512
 // 29.7 -> 24.0, output head 512 x 50304 over 768 334 -> 275; GPT-2 2 x 256 6.14 -> 5.39 ms, ResNet-152 of 4 images 7.11 -> 6.60.
-// Range: bf16 has the exponents of fp32, so nothing overflows that fp32 holds except values that round to 2^128 (see below), and
-// below 2^-110 (7.7e-34) the last parts of a value are bf16 denormals: such an operand keeps an absolute error of up to 2^-134.
-// Infinities, NaN and values that round to 2^128 come out as NaN (inf - inf): a kernel that finds a NaN among its sums adds
-// them up again with fp32 MFMA, whose result counts then.
+// Range: bf16 has the exponents of fp32, but a first part may be larger than its value (by 2^-9 of it), and with it a first product or
+// a sum of them: these overflow up to 0.8 % below the largest fp32 value, and a value that rounds to 2^128 is an infinity in its
+// first part.  Infinities and NaN among the operands come out as NaN (inf - inf).  So a kernel that finds a sum that is not finite,
+// infinity or NaN, adds all of them up again with fp32 MFMA, whose result counts then: where fp32 has infinities too that costs
+// the second pass only.
+// Below 2^-110 (7.7e-34) the last parts of a value are bf16 denormals: such an operand keeps an absolute error of up to 2^-134.
 #pragma once
 
 #include "kernels.h"
+#include <cfloat>
 
 namespace tch {
 
@@ -86,10 +89,10 @@ __device__ inline void mma_split(const Split8& x, const Split8& y, f32x16_t& lar
   small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[0], small, 0, 0, 0);
 }
 
-// large += small; whether any sum of this lane is NaN
+// large += small; whether any sum of this lane is not finite
 template <int TM, int TN>
 __device__ inline bool join_split(f32x16_t (&large)[TM][TN], const f32x16_t (&small)[TM][TN]) {
-  bool nan = false;
+  bool beyond = false;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -97,9 +100,9 @@ __device__ inline bool join_split(f32x16_t (&large)[TM][TN], const f32x16_t (&sm
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         large[i][j][e] += small[i][j][e];
-        nan |= large[i][j][e] != large[i][j][e];
+        beyond |= !(fabsf(large[i][j][e]) <= FLT_MAX);
       }
-  return nan;
+  return beyond;
 }
 
 template <int TM, int TN>

@@ -63,3 +63,23 @@ def test_infinities_nan_and_the_largest_values(op, tile_cfg):
     ok = want.isfinite()
     size = (torch.where(a.isfinite(), a, 0).double().abs() @ b.double().abs().t())[ok]
     assert ((got.double() - want)[ok].abs() <= (depth + 2) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("tile_cfg", TILINGS)
+@pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
+def test_results_next_to_the_largest_value_are_finite(op, tile_cfg):
+    """The first part of a value may be larger than the value.  Products of first parts, and sums of such products, overflow then
+    where the result does not: 1.999 * 2^127, and 253 times 1.0040^2 * 2^120 (0.996 * 2^128; 1.0078^2 in first parts)."""
+    rows, cols, depth = 68, 72, 272
+    g = torch.Generator().manual_seed(2)
+    a, b = torch.randn(rows, depth, generator=g), torch.randn(cols, depth, generator=g)
+    for row, col, sign in ((5, 7, 1.0), (40, 50, -1.0)):
+        a[row, 17], b[col, 17] = sign * 1.999 * 2.0 ** 63, 2.0 ** 64
+    for row, col, sign in ((9, 11, 1.0), (66, 70, -1.0)):
+        a[row, :253], b[col, :253] = sign * 1.0040 * 2.0 ** 62, 1.0040 * 2.0 ** 58
+        a[row, 17] = b[col, 17] = 0.0     # leaves the others' large values alone
+        a[row, 253], b[col, 253] = a[row, 0], b[col, 0]
+    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).double().cpu()
+    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    assert want.abs().max() < torch.finfo(torch.float32).max and (want.abs() > 2.0 ** 127).sum() >= 4
+    assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
