@@ -3485,6 +3485,7 @@ int conv2d_dgrad(Context* ctx, int dtype, const ConvShape& s, const void* dy, co
   // 1x1 stride 1: dy is a dense [pixels][K] matrix in the same pixel order as dx
   a.div_plane = FastDiv(s.H * s.W);
   a.div_width = FastDiv(s.W);
+  a.in_fp32 = asks_in_order(tile_cfg) ? 1 : 0;
   if (tile_cfg < 0) {
     tile_cfg = heuristic_tile(tile_cfg, {dtype, a.gemm_m, a.gemm_n, a.gemm_k, s.K, s.R * s.S, patch_kernel_fits(s, s.K), bn != nullptr, true, walk_tile_fits(a)});
     if (!bn && wants_huge_tile(dtype, a.gemm_m, a.gemm_n, s.K, s.R * s.S)) tile_cfg = 10;

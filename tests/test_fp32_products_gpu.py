@@ -83,3 +83,14 @@ def test_results_next_to_the_largest_value_are_finite(op, tile_cfg):
     want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     assert want.abs().max() < torch.finfo(torch.float32).max and (want.abs() > 2.0 ** 127).sum() >= 4
     assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("op", ["fwd", "dgrad"])
+def test_in_order_rows_are_the_same_bits_at_every_number_of_rows(op):
+    """tile_cfg = IN_ORDER: 64 x 64 tiles, which multiply in fp32 anyway, up to 384 tiles of 128 x 64; those; and 128 x 128."""
+    from sirius_amd import ops
+    cols, depth = 128, 144
+    g = torch.Generator("cuda").manual_seed(3)
+    a, b = (torch.randn(n, depth, device="cuda", generator=g) for n in (49280, cols))
+    first, *others = [product(op, rows, cols, depth, ops.IN_ORDER, a[:rows], b)[:66] for rows in (66, 24700, 49280)]
+    assert all(torch.equal(first, o) for o in others)
