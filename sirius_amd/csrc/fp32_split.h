@@ -1,20 +1,19 @@
 // fp32 products on the bf16 matrix pipes.
 //
 // An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of mantissa): x = x0 + x1 + x2 with x0 = x rounded to
-// bf16, x1 = the rest rounded to bf16, x2 = what is left.  Of the nine products of two such sums the three smallest
-// (x1 y2, x2 y1, x2 y2, below 2^-26 of the product) are left out; the other six go through v_mfma_f32_32x32x16_bf16, which
-// accumulates in fp32: 192 cycles for a 32 x 32 x 16 product instead of the 512 of eight v_mfma_f32_32x32x2_f32.
+// bf16, x1 = the rest rounded to bf16, x2 = what is left.  Of the nine products of two such sums eight go through
+// v_mfma_f32_32x32x16_bf16, which accumulates in fp32: 256 cycles for a 32 x 32 x 16 product instead of the 512 of eight
+// v_mfma_f32_32x32x2_f32.  The ninth, x2 y2, is below 2^-36 of the product, less than what the sum of the small products is rounded by.
 //
-// Error: the five small products have an accumulator of their own, 2^-8 of the size of the other, so that the large one is
-// rounded once per 16 reduction elements (fp32 MFMA: once per element).  Norm of the error against 64 bits over the norm of the
-// result, one wavefront, in units of 1e-7, with fp32 MFMA and in parts (in parts with one accumulator):
-//   normal x normal over 64 / 768 / 4608:  1.4 / 4.9 / 12.2   and 0.5 / 1.6 / 4.2 (1.1 / 4.2 / 10.6)
-//   ReLU'd x normal:                       1.0 / 3.5 / 8.6    and 0.4 / 1.2 / 3.5 (1.1 / 4.0 / 9.9)
+// Error: the seven small products have an accumulator of their own, 2^-8 of the size of the other, so that the large one is
+// rounded once per 16 reduction elements (fp32 MFMA: once per element), and a sum of one product is rounded as fp32 rounds it.  Norm of
+// the error against 64 bits over the norm of the result, 128 x 128 tiles, in units of 1e-7, with fp32 MFMA and in parts:
+//   normal x normal over 136 / 768 / 4608:   2.1 / 4.9 / 12.2   and 0.7 / 1.6 / 4.2
+//   ReLU'd x normal:                         1.5 / 3.5 / 8.6    and 0.5 / 1.2 / 3.5
+// (In one accumulator 4.2 over 768.)  Without x1 y2 and x2 y1 a sum of one product is off by 0.62 units in the last place instead of 0.5.
 // Rounding the parts matters: cut off instead, they leave out products of one sign (uniform x uniform over 4608: 116 for 6.3).
 // Time: taking a pair of values apart is 11 vector instructions, which pass behind the multiplies; what is left of a small product is
-// its operands' way to the CU (the same 21 us of 26 without the split and five of the six multiplies).
-// Alone, before and after: 512 x 768 over 3072 31.0 -> 25.6 us, 512 x 3072 over 768 25.3 -> 22.1, weight gradient 768 x 3072 over 512
-// 29.7 -> 24.0, output head 512 x 50304 over 768 334 -> 275; GPT-2 2 x 256 6.14 -> 5.39 ms, ResNet-152 of 4 images 7.11 -> 6.60.
+// its operands' way to the CU.
 // Range: bf16 has the exponents of fp32, but a first part may be larger than its value (by 2^-9 of it), and with it a first product or
 // a sum of them: these overflow up to 0.8 % below the largest fp32 value, and a value that rounds to 2^128 is an infinity in its
 // first part.  Infinities and NaN among the operands come out as NaN (inf - inf).  So a kernel that finds a sum that is not finite,
@@ -79,8 +78,10 @@ __device__ inline bf16x8_t read_transposed(const unsigned char* first, const uns
   return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// large += x0 y0; small += the five products next in size
+// large += x0 y0; small += the seven products next in size
 __device__ inline void mma_split(const Split8& x, const Split8& y, f32x16_t& large, f32x16_t& small) {
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[2], small, 0, 0, 0);
+  small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[2], y.part[1], small, 0, 0, 0);
   small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[0], y.part[2], small, 0, 0, 0);
   small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[2], y.part[0], small, 0, 0, 0);
   small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[1], small, 0, 0, 0);

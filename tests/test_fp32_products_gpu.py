@@ -34,7 +34,7 @@ CASES = [(op, rows, cols, depth) for op in ("fwd", "dgrad", "wgrad")
 @pytest.mark.parametrize("op,rows,cols,depth", CASES)
 def test_error_is_that_of_fp32(op, rows, cols, depth, tile_cfg):
     """Per value: every one of at most `depth` additions rounds by 2^-24 of a partial sum, which the sum of |a b| bounds, the
-    parts leave out at most 2^-25 of every product and their own sum is 2^-8 as large."""
+    parts leave out at most 2^-36 of every product and their own sum is 2^-8 as large."""
     g = torch.Generator().manual_seed(depth + rows)
     a = torch.randn(rows, depth, generator=g).mul_(torch.exp(2 * torch.randn(rows, depth, generator=g)))
     b = torch.randn(cols, depth, generator=g)
@@ -43,6 +43,67 @@ def test_error_is_that_of_fp32(op, rows, cols, depth, tile_cfg):
     assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
     # and over the whole result what sums of independent roundings have, not what the bound above allows
     assert (got - want).norm() <= 4 * 2.0 ** -24 * max(1, depth / 64) ** 0.5 * want.norm()
+
+
+def fp32_multiplies(a, b, groups):
+    """What v_mfma_f32_32x32x2_f32 gives: one rounding to fp32 per reduction element, steps of 16 elements dealt out to `groups`
+    wavefronts, whose sums are added in their order.  (With fp64 inside: a product of two fp32 values is exact there.)"""
+    total, a, b = None, a.double(), b.double()
+    for group in range(groups):
+        acc = torch.zeros(a.shape[0], b.shape[0], device=a.device)
+        for k in range(a.shape[1]):
+            if k // 16 % groups == group:
+                acc = torch.addr(acc.double(), a[:, k], b[:, k]).float()
+        total = acc if total is None else total + acc
+    return total
+
+
+# a value's distribution over a row; "wide": a few products of a sum dominate it, and its error is that of single products
+DISTRIBUTIONS = {
+    "normal": lambda shape, g: torch.randn(shape, device="cuda", generator=g),
+    "relu": lambda shape, g: torch.randn(shape, device="cuda", generator=g).clamp_(min=0),
+    "uniform": lambda shape, g: torch.rand(shape, device="cuda", generator=g),
+    "wide": lambda shape, g: torch.randn(shape, device="cuda", generator=g) * torch.exp(3 * torch.randn(shape, device="cuda", generator=g)),
+}
+# tiling: wavefronts that share the reduction of a forward product or data gradient.  2 multiplies in fp32 there.
+GROUPS = {0: 1, 1: 1, 2: 1, 15: 4, 16: 8, 17: 4, 18: 8, 19: 4, 20: 8}
+PAIRS = [("normal", "normal"), ("relu", "normal"), ("uniform", "uniform"), ("wide", "normal"), ("wide", "wide")]
+
+
+@pytest.mark.parametrize("depth", [144, 656])
+@pytest.mark.parametrize("first,second", PAIRS)
+def test_error_is_no_larger_than_with_fp32_multiplies(first, second, depth):
+    """Against 64 bits, over a whole result, next to fp32 multiplies in the same order; every value counts by the sum of |a b|.  What is
+    left out of a product is 2^-36 of it and the small products' sum rounds by 2^-32 of the result, so the parts can be off by
+    2^-8 more where one product is all of a sum; elsewhere they round less often.  The allowance of 3 % is that and what two sets of
+    34 320 roundings differ by (1 %)."""
+    g = torch.Generator("cuda").manual_seed(depth)
+    a, b = DISTRIBUTIONS[first]((260, depth), g), DISTRIBUTIONS[second]((132, depth), g)
+    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    error = lambda y: ((y.double() - want) / size).norm().item()
+    off = {groups: error(fp32_multiplies(a, b, groups)) for groups in (1, 4, 8)}
+    for op in ("fwd", "dgrad", "wgrad"):
+        for tile_cfg in (0, 2) if op == "wgrad" else GROUPS:
+            groups = 1 if op == "wgrad" else GROUPS[tile_cfg]
+            ratio = error(product(op, 260, 132, depth, tile_cfg, a, b)) / off[groups]
+            print(f"{first} x {second} over {depth}, {op} tiling {tile_cfg}: {ratio:.3f}")
+            assert ratio <= 1.03, (op, tile_cfg, ratio)
+            if tile_cfg == 2 and op != "wgrad":   # fp32 multiplies: the reference is what they give
+                assert ratio >= 0.97, (op, ratio)
+
+
+@pytest.mark.parametrize("tile_cfg", TILINGS)
+@pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
+def test_single_products_are_rounded_once(op, tile_cfg):
+    """Sums of one product and zeros: half a unit in the last place, as a product in fp32, and what the small products' sum rounds (seven
+    times half a unit of a 2^-8 as large value) and leaves out: 2^-7 of a unit."""
+    g = torch.Generator("cuda").manual_seed(4)
+    rows, cols, depth = 260, 132, 144
+    a, b = torch.zeros(rows, depth, device="cuda"), torch.randn(cols, depth, device="cuda", generator=g)
+    a[torch.arange(rows), torch.arange(rows) % depth] = torch.randn(rows, device="cuda", generator=g)
+    got, want = product(op, rows, cols, depth, tile_cfg, a, b).double(), a.double() @ b.double().t()
+    unit = torch.exp2(torch.floor(torch.log2(want.abs())) - 23)
+    assert ((got - want).abs() <= (0.5 + 2.0 ** -7) * unit).all()
 
 
 @pytest.mark.parametrize("tile_cfg", TILINGS)
