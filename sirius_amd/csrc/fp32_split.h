@@ -1,25 +1,27 @@
 // fp32 products on the bf16 matrix pipes.
 //
-// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of mantissa): x = x0 + x1 + x2 with x0 = x rounded to
-// bf16, x1 = the rest rounded to bf16, x2 = what is left.  Of the nine products of two such sums eight go through
+// An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 bits of mantissa): x = x0 + x1 + x2 with x0 = the upper half of
+// the bits of x, x1 = the upper half of the bits of what is left, x2 = the rest.  Of the nine products of two such sums eight go through
 // v_mfma_f32_32x32x16_bf16, which accumulates in fp32: 256 cycles for a 32 x 32 x 16 product instead of the 512 of eight
-// v_mfma_f32_32x32x2_f32.  The ninth, x2 y2, is below 2^-36 of the product, less than what the sum of the small products is rounded by.
+// v_mfma_f32_32x32x2_f32.  The ninth, x2 y2, is below 2^-30 of the product, 2^-7 of a unit in the last place.
 //
-// Error: the seven small products have an accumulator of their own, 2^-8 of the size of the other, so that the large one is
+// Error: the seven small products have an accumulator of their own, 2^-5 of the size of the other at most, so that the large one is
 // rounded once per 16 reduction elements (fp32 MFMA: once per element), and a sum of one product is rounded as fp32 rounds it.  Norm of
 // the error against 64 bits over the norm of the result, 128 x 128 tiles, in units of 1e-7, with fp32 MFMA and in parts:
 //   normal x normal over 136 / 768 / 4608:   2.1 / 4.9 / 12.2   and 0.7 / 1.6 / 4.2
 //   ReLU'd x normal:                         1.5 / 3.5 / 8.6    and 0.5 / 1.2 / 3.5
-// (In one accumulator 4.2 over 768.)  Without x1 y2 and x2 y1 a sum of one product is off by 0.62 units in the last place instead of 0.5.
-// Rounding the parts matters: cut off instead, they leave out products of one sign (uniform x uniform over 4608: 116 for 6.3).
-// Time: taking a pair of values apart is 11 vector instructions, which pass behind the multiplies; what is left of a small product is
-// its operands' way to the CU.
-// Range: bf16 has the exponents of fp32, but a first part may be larger than its value (by 2^-9 of it), and with it a first product or
-// a sum of them: these overflow up to 0.8 % below the largest fp32 value, and a value that rounds to 2^128 is an infinity in its
-// first part.  Infinities and NaN among the operands come out as NaN (inf - inf).  So a kernel that finds a sum that is not finite,
-// infinity or NaN, adds all of them up again with fp32 MFMA, whose result counts then: where fp32 has infinities too that costs
-// the second pass only.
-// Below 2^-110 (7.7e-34) the last parts of a value are bf16 denormals: such an operand keeps an absolute error of up to 2^-134.
+//   uniform x uniform:                       1.7 / 4.2 / 10.1   and 0.7 / 1.5 / 3.6
+// (In one accumulator 4.2 for normal x normal over 768.)
+//
+// Range: operands are taken apart times 2^24, and the sums multiplied by 2^-48 at the end.  The last bit of the smallest values is then a
+// normal bf16 number, so that parts lose no bit of any value.  (Without the factor the last parts of values below 2^-110 are bf16
+// denormals and cut off at 2^-134.)  At the other end parts overflow, from operands of 2^104 or sums of 2^80 on; they come out as
+// infinity, or as NaN where infinities cancel.  A kernel that finds a sum that is not finite adds all of them up again
+// with fp32 MFMA, whose result counts then: what fp32 makes of infinities, NaN and the largest values.
+//
+// Time: taking a pair of values apart is 13 vector instructions, which are what bounds small products.  Rounded parts (v_cvt_pk_bf16_f32
+// instead of v_perm_b32, a shift for one of two masks) took 4 % longer over the forward products of the three models; rests by
+// v_dot2_f32_bf16, 9 instructions, as long as those, and weight gradients 6 % longer.
 #pragma once
 
 #include "kernels.h"
@@ -27,21 +29,22 @@
 
 namespace tch {
 
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
+
 struct Split8 {
   bf16x8_t part[3];
 };
 
-// a pair of values into the bits of its parts
+// A pair of values, times kSplitScale, into the bits of its parts.
 __device__ inline void split_pair(float v0, float v1, uint32_t (&w)[3]) {
-  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  v0 *= kSplitScale;
+  v1 *= kSplitScale;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const f32x2_t v = {v0, v1};
-    w[k] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-    if (k < 2) {   // exact
-      v0 -= __uint_as_float(w[k] << 16);
-      v1 -= __uint_as_float(w[k] & 0xffff0000u);
+    w[k] = __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u);
+    if (k < 2) {
+      v0 -= __uint_as_float(__float_as_uint(v0) & 0xffff0000u);
+      v1 -= __uint_as_float(__float_as_uint(v1) & 0xffff0000u);
     }
   }
 }
@@ -90,7 +93,7 @@ __device__ inline void mma_split(const Split8& x, const Split8& y, f32x16_t& lar
   small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x.part[1], y.part[0], small, 0, 0, 0);
 }
 
-// large += small; whether any sum of this lane is not finite
+// large = (large + small) * kSplitUnscale; whether any sum of this lane is not finite
 template <int TM, int TN>
 __device__ inline bool join_split(f32x16_t (&large)[TM][TN], const f32x16_t (&small)[TM][TN]) {
   bool beyond = false;
@@ -102,6 +105,7 @@ __device__ inline bool join_split(f32x16_t (&large)[TM][TN], const f32x16_t (&sm
       for (int e = 0; e < 16; ++e) {
         large[i][j][e] += small[i][j][e];
         beyond |= !(fabsf(large[i][j][e]) <= FLT_MAX);
+        large[i][j][e] *= kSplitUnscale;
       }
   return beyond;
 }
