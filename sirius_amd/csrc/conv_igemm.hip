@@ -38,6 +38,7 @@
 #include "fp32_split.h"
 #include "kernels.h"
 #include <algorithm>
+#include <climits>
 #include <iterator>
 #include <vector>
 
@@ -55,11 +56,6 @@ namespace {
 constexpr int kLdsStride = 5;  // FWD/DGRAD: chunks per LDS tile row: 4 data + 1 pad
 constexpr int kRowPad = 4;     // WGRAD, fp32: chunks of padding per [pixel] row (64 bytes)
 constexpr int kStagePad = 4;   // epilogue staging: floats of padding per row
-
-// fp32 products over longer reductions run on the bf16 pipes (fp32_split.h), shorter ones in fp32: up to here they are launch,
-// epilogue and latency, and the parts only add instructions (784 x 256 over 128: 3.7 us in fp32, 4.0 in parts; 12 544 x 64 over
-// 256: 9.6 and 9.2)
-constexpr int kShortReduction = 128;
 
 enum Mode : int { kFwd = 0, kDgrad = 1, kWgrad = 2 };
 
@@ -103,7 +99,7 @@ struct IgemmArgs {
   int group_rows;   // FWD/DGRAD direct-to-LDS kernel: row tiles per group of the tile order (0 / 1: row-major)
   int k_per_split;  // multiple of BK
   int out_f32;      // FWD/DGRAD: store fp32 instead of T
-  int in_fp32;      // fp32: no parts (fp32_split.h), see split_products()
+  int in_fp32;      // fp32, read by the launcher only: no parts (fp32_split.h)
   int accumulate;   // WGRAD with splits == 1: out += result
   int take_pending; // WGRAD, read by the launcher only: the context's pending split reduction rides this launch
   int pointwise;    // 1x1, stride 1, pad 0
@@ -597,21 +593,11 @@ struct TileEpilogue {
   }
 };
 
-// Whether an fp32 product runs on the bf16 pipes.  Not one that was asked for front to back, where every tile adds up the same
-// bits, and not a convolution whose output a training BatchNorm takes: behind it stands a ReLU, and whichever of two equally
-// good roundings a pre-activation gets near zero, another one opens or closes gates, each of which moves a gradient by more than all
-// other rounding does (ResNet-152 of 4 images, the gradients against those of fp32 multiplies: 2e-7 relative without a gate, 7.5e-5
-// with two).  Data and weight gradients are smooth.
-template <int MODE>
-__device__ inline bool split_products(const IgemmArgs& p) {
-  return p.gemm_k > kShortReduction && !p.in_fp32 && !(MODE == kFwd && (p.stats || p.stat_acc));
-}
-
 // ---------------------------------------------------------------------------
-// forward / data gradient
+// forward / data gradient.  PARTS: an fp32 product on the bf16 pipes (fp32_split.h)
 // ---------------------------------------------------------------------------
-template <typename T, int MODE, int WM, int WN, int TM, int TN>
-__global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
+template <typename T, int MODE, int WM, int WN, int TM, int TN, bool PARTS = false>
+__global__ __launch_bounds__(WM* WN * 64, PARTS ? 2 : 1) void igemm_kernel(IgemmArgs p) {
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int BK = 4 * E;
   constexpr int BM = WM * TM * 32;
@@ -797,16 +783,10 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm_kernel(IgemmArgs p) {
       load_tiles(kt + 4, ra0, rb0);
     }
   };
-  // 64 x 64 stays with fp32 multiplies: a wavefront would take two operands apart for every one of its 32 x 32 products
-  // (512 x 768 over 768 21.8 us in fp32, 23.9 in parts, as 128 x 128 57.4 and 50.2)
-  if constexpr (EB == 4 && TM * TN > 1) {
+  if constexpr (PARTS) {
     f32x16_t low[TM][TN];
-    bool plain = !split_products<MODE>(p);
-    if (!plain) {
-      reduce(std::true_type{}, low);
-      plain = __syncthreads_or(join_split(acc, low));
-    }
-    if (plain) reduce(std::false_type{}, low);
+    reduce(std::true_type{}, low);
+    if (__syncthreads_or(join_split(acc, low))) reduce(std::false_type{}, low);
   } else {
     reduce(std::false_type{}, acc);
   }
@@ -1181,7 +1161,7 @@ __device__ __forceinline__ void wgrad_body_direct(const IgemmArgs& p, uint32_t i
 }
 
 // `id`: the workgroup's place among the tiles_m * tiles_n * splits workgroups of this weight gradient
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, bool PARTS>
 __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) {
   typedef float T;
   constexpr int E = Elem<T>::kPerChunk;
@@ -1203,7 +1183,7 @@ __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) 
   constexpr int RA = BM * 2, RB = BN * 2;
   constexpr int A_PART = BKP * RA, B_PART = BKP * RB, PARTS_BYTES = 3 * (A_PART + B_PART);
   static_assert((RA == 256 || RA == 128) && (RB == 256 || RB == 128), "row swizzle");
-  constexpr int LDS_BYTES = std::max({OPER_BYTES, STAGE_BYTES, 2 * PARTS_BYTES});
+  constexpr int LDS_BYTES = std::max({OPER_BYTES, STAGE_BYTES, PARTS ? 2 * PARTS_BYTES : 0});
 
   __shared__ uint4 lds[LDS_BYTES / 16];
   uint4* lds_a = lds;                      // [2][BKP][LDA]
@@ -1387,13 +1367,13 @@ __device__ __forceinline__ void wgrad_body_f32(const IgemmArgs& p, uint32_t id) 
       load_tiles(kt + 4, ra0, rb0);
     }
   };
-  f32x16_t low[TM][TN];
-  bool plain = p.k_per_split <= kShortReduction;
-  if (!plain) {
+  if constexpr (PARTS) {
+    f32x16_t low[TM][TN];
     reduce(std::true_type{}, low);
-    plain = __syncthreads_or(join_split(acc, low));
+    if (__syncthreads_or(join_split(acc, low))) reduce(std::false_type{}, low);
+  } else {
+    reduce(std::false_type{}, acc);
   }
-  if (plain) reduce(std::false_type{}, low);
 
   float* out = static_cast<float*>(p.out);
   if (p.splits > 1) out += static_cast<int64_t>(split) * p.gemm_m * p.gemm_n;
@@ -1449,14 +1429,14 @@ __device__ __forceinline__ void wgrad_passenger(const WgradArgs& w, double* lds)
     col_sum_body(w.cols, id - w.red_blocks, lds);
 }
 
-template <int WM, int WN, int TM, int TN>
+template <int WM, int WN, int TM, int TN, bool PARTS>
 __global__ __launch_bounds__(WM* WN * 64) void wgrad_f32_kernel(WgradArgs w) {
   if (blockIdx.x >= w.gemm_wgs) {
     __shared__ double red[kColSumLds];
     wgrad_passenger(w, red);
     return;
   }
-  wgrad_body_f32<WM, WN, TM, TN>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs));
+  wgrad_body_f32<WM, WN, TM, TN, PARTS>(w.a, xcd_remap(blockIdx.x, w.gemm_wgs));
 }
 
 template <int WM, int WN, int TM, int TN, int RING, bool POINTWISE, bool BIAS>
@@ -1488,7 +1468,7 @@ __global__ __launch_bounds__(WM* WN * 64) void wgrad_group_kernel(WgradGroupArgs
     const uint2 e = g.map[gid];
     const IgemmArgs p = g.table[__builtin_amdgcn_readfirstlane(e.x)];
     const uint32_t id = __builtin_amdgcn_readfirstlane(e.y);
-    if constexpr (sizeof(T) == 4) wgrad_body_f32<WM, WN, TM, TN>(p, id);
+    if constexpr (sizeof(T) == 4) wgrad_body_f32<WM, WN, TM, TN, false>(p, id);
     else if (p.pointwise) wgrad_body_direct<WM, WN, TM, TN, kWgradRing, true, true>(p, id, lds);
     else wgrad_body_direct<WM, WN, TM, TN, kWgradRing, false, true>(p, id, lds);
     __syncthreads();   // the next entry's operand tiles overwrite what the epilogue staged in LDS
@@ -2170,10 +2150,6 @@ __global__ __launch_bounds__(WM* WN * 64) void igemm5_kernel(IgemmArgs p) {
 // What bounds it: the trip to memory behind every launch boundary and the chain of steps behind it.  196 x 256 over 2304 (a
 // 3x3 layer of one image) 13.2 -> 6.1 us, 784 x 512 over 4608 36.9 -> 14.8, fp32 784 x 256 over 2304 77.6 -> 14.8 against
 // 64 x 64 tiles of igemm2_kernel / igemm_kernel; the 151 launches of a ResNet-152 request take 4.4-6.9 us each.
-__device__ inline void multiply_add(const Chunk& first, const Chunk& second, f32x4_t& acc) {
-  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(first.h, second.h, acc, 0, 0, 0);
-}
-
 // Every wavefront owns the WHOLE TM*32 x TN*32 tile for every KG-th reduction step and has a ring of NBUF operand
 // tiles of its own in LDS, filled with direct loads: nothing is shared before the end, so the main loop has no
 // barrier and a wavefront waits for its own loads only.  The partial tiles meet in LDS once and are added in the
@@ -2185,7 +2161,8 @@ __device__ inline void multiply_add(const Chunk& first, const Chunk& second, f32
 // the 77 bytes / ns that direct loads bring into the LDS of one: four times the workgroups load half as many bytes each.
 // In a request of one image, 196 rows and 256 channels over 1024 and over 2304: 6.2 us on average on 56 workgroups of 32 x 32, 4.9 on 208;
 // 1024 channels over 256, where 224 fill the chip, 4.0 and 6.6 on 832.
-template <typename T, int MODE, int TM, int TN, int KG, int NBUF, int FS = 32>
+// PARTS: an fp32 product on the bf16 pipes (fp32_split.h).
+template <typename T, int MODE, int TM, int TN, int KG, int NBUF, int FS = 32, bool PARTS = false>
 __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   constexpr int E = Elem<T>::kPerChunk;
   constexpr int EB = sizeof(T);
@@ -2317,8 +2294,13 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) if constexpr (FS == 32) mma<T>(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
-        else multiply_add(chunk(fb[tn]), chunk(fa[tm]), acc[tm][tn]);
+      for (int tn = 0; tn < TN; ++tn) {
+        const Chunk a = chunk(fa[tm]), b = chunk(fb[tn]);
+        if constexpr (FS == 32)
+          mma<T>(b, a, acc[tm][tn]);
+        else
+          acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b.h, a.h, acc[tm][tn], 0, 0, 0);
+      }
   };
 
   // The tile of step i lands when at most the NBUF-2 tiles requested behind it are outstanding (near the end fewer
@@ -2326,7 +2308,11 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
   constexpr int AHEAD = (NBUF - 2) * (A_LD + B_LD);
   static_assert(AHEAD < 64, "vmcnt range");
   // this wavefront's share of the sums, in `acc`; split_c: in fp32, on the bf16 pipes, small products in `low`
-  auto reduce = [&](auto split_c, acc_t (&low)[TM][TN], bool first) {
+  // The epilogue's operands are requested behind the first loads, except beside the 128 accumulators of a 64 x 64 tile in parts, where there
+  // are no registers for them.
+  constexpr bool EARLY = !(PARTS && TM * TN == 4);
+  auto request_operands = [&] { operands.template request_first<BN, NTE>(p, tid, m0, n0, row_of); };
+  auto reduce = [&](auto split_c, acc_t (&low)[TM][TN], bool request) {
     constexpr bool SPLIT = decltype(split_c)::value;
     rewind();
     if constexpr (FS == 16) {
@@ -2353,12 +2339,12 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
           hold_frags(fa0, fb0);
           hold_frags(fa1, fb1);
           Split8 sb[TN];
-  #pragma unroll
+#pragma unroll
           for (int tn = 0; tn < TN; ++tn) sb[tn] = split8(chunk(fb0[tn]), chunk(fb1[tn]));
-  #pragma unroll
+#pragma unroll
           for (int tm = 0; tm < TM; ++tm) {
             const Split8 sa = split8(chunk(fa0[tm]), chunk(fa1[tm]));
-  #pragma unroll
+#pragma unroll
             for (int tn = 0; tn < TN; ++tn) mma_split(sb[tn], sa, acc[tm][tn], low[tm][tn]);
           }
         } else {
@@ -2372,7 +2358,7 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
 #pragma unroll
     for (int i = 0; i < NBUF - 1; ++i)
       if (i < my_steps) issue_loads(i);
-    if (first) operands.template request_first<BN, NTE>(p, tid, m0, n0, row_of);
+    if (request) request_operands();
     int i0 = 0;
     for (; i0 + NBUF <= my_steps; i0 += NBUF) {
 #pragma unroll
@@ -2382,14 +2368,11 @@ __global__ __launch_bounds__(KG * 64, 2) void igemm4_kernel(IgemmArgs p) {
     for (int u = 0; u < NBUF - 1; ++u)
       if (i0 + u < my_steps) step(i0 + u, u);
   };
-  if constexpr (sizeof(T) == 4) {
+  if constexpr (PARTS) {
     f32x16_t low[TM][TN];
-    bool plain = !split_products<MODE>(p);
-    if (!plain) {
-      reduce(std::true_type{}, low, true);
-      plain = __any(join_split(acc, low));
-    }
-    if (plain) reduce(std::false_type{}, low, !split_products<MODE>(p));
+    reduce(std::true_type{}, low, EARLY);
+    if (__any(join_split(acc, low))) reduce(std::false_type{}, low, false);
+    if constexpr (!EARLY) request_operands();
   } else {
     reduce(std::false_type{}, acc, true);
   }
@@ -2705,12 +2688,12 @@ int ilog2_exact(int v) {
   return ((1 << l) == v) ? l : -1;
 }
 
-template <typename T, int MODE, int WM, int WN, int TM, int TN>
+template <typename T, int MODE, int WM, int WN, int TM, int TN, bool PARTS = false>
 const char* igemm_name() {
   static const std::string name = std::string(MODE == kWgrad ? "wgrad_kernel<" : "igemm_kernel<") +
                                   (sizeof(T) == 2 ? "bf16" : "f32") + "," +
                                   (MODE == kFwd ? "fwd," : MODE == kDgrad ? "dgrad," : "") +
-                                  std::to_string(WM * TM * 32) + "x" + std::to_string(WN * TN * 32) + ">";
+                                  std::to_string(WM * TM * 32) + "x" + std::to_string(WN * TN * 32) + (PARTS ? ",parts>" : ">");
   return name.c_str();
 }
 
@@ -2735,6 +2718,35 @@ void bind_divisions(IgemmArgs& a, int run) {
   a.div_c = FastDiv(a.C);
   a.div_s = FastDiv(a.S);
 }
+
+// Which fp32 products go through the bf16 pipes (fp32_split.h); the others are multiplied in fp32 by kernels that hold nothing else.
+// What decides is whether a SIMD has a second wavefront: taking operands apart does not pass behind a wavefront's own
+// multiplies, but behind those of another one.  Then, how many of its instructions a multiply costs.  Times alone in parts as shares of those
+// in fp32, over the layers of the three models at 64-8192 rows and 1-32 images (244 forward products and data gradients, 122 weight
+// gradients):
+//   128 x 128 tiles 0.84-1.00, 128 x 64 0.88-0.98, 64 x 64 split over wavefronts 0.74-0.91 (one wavefront on a SIMD: 1.05-1.10)
+//   64 x 32 over 512 - 8192: 0.85-1.00.  Over 16384 and more 0.97-1.07 (2331 x 768: 1.01, over 50304 1.07; 2048 x 768 over that 0.87)
+//   32 x 32 over eight wavefronts, K >= 1024: 0.94-1.00 (1.04 once); over four, less than 512 1.00-1.03, one wavefront on a SIMD 1.00-1.20
+//   weight gradients: 128 x 128, which have four workgroups on a CU, 0.80-0.90; 64 x 64 with more than one 0.89-1.00, up to four reduction
+//   steps 1.01-1.07; else 0.97-1.09
+// Data gradients run beside weight gradients, whose work fills what a second wavefront leaves.  Steps with tiles below 64 x 64 in parts
+// for both / for forward products only: ResNet-152 of 16 images 17.40 / 17.05 ms, Swin-B of 2 images 6.34 / 6.24 (fp32 multiplies 17.2, 6.26),
+// the other steps the same; 32 x 32 tiles over four wavefronts forward: GPT-2 of 2 x 256 5.97 / 5.89 without.
+// Never: what was asked for front to back (every tile adds up the same bits), and a convolution whose output a training BatchNorm takes.  Behind
+// it stands a ReLU, and whichever of two equally good roundings a pre-activation gets near zero, another one opens or closes gates, each
+// of which moves a gradient by more than all other rounding does (ResNet-152 of 4 images, the gradients against those of fp32
+// multiplies: 2e-7 relative without a gate, 7.5e-5 with two).  Data and weight gradients are smooth.
+template <typename T, int MODE, int BM, int BN, int KG>
+constexpr bool parts_tile() {   // KG: wavefronts a reduction is split over (1: igemm_kernel, whose 64 x 64 tiles take two operands apart per product)
+  return sizeof(T) == 4 && (BM * BN > 64 * 64 || (KG > 1 && (BM * BN == 64 * 64 || (MODE == kFwd && (BM > 32 || KG == 8)))));
+}
+template <int MODE, int BM, int BN>
+bool product_in_parts(const IgemmArgs& a, int64_t wavefronts) {
+  if (a.in_fp32 || (MODE == kFwd && (a.stats || a.stat_acc))) return false;
+  const int from = BM * BN == 32 * 32 ? 1024 : 256, to = BM * BN == 64 * 32 ? 16384 : INT_MAX;
+  return wavefronts > 4 * 256 && a.gemm_k >= from && a.gemm_k < to;
+}
+bool wgrad_in_parts(const IgemmArgs& a, int64_t workgroups) { return workgroups > 256 && a.k_per_split > 4 * 16; }
 
 template <int WM, int WN, int TM, int TN, int RING>
 void (*wgrad_direct_kernel(const IgemmArgs& a))(WgradArgs) {
@@ -2778,16 +2790,24 @@ int launch_cfg(Context* ctx, IgemmArgs& a, double flops) {
       cs.valid = false;
     }
     void (*kernel)(WgradArgs);
-    if constexpr (sizeof(T) == 4)
-      kernel = wgrad_f32_kernel<WM, WN, TM, TN>;
-    else if (TM * TN == 1 && short_wgrad_ring(wgs, (a.k_per_split + 31) / 32))
+    const char* name = igemm_name<T, MODE, WM, WN, TM, TN>();
+    if constexpr (sizeof(T) == 4) {
+      const bool parts = wgrad_in_parts(a, wgs);
+      kernel = parts ? wgrad_f32_kernel<WM, WN, TM, TN, true> : wgrad_f32_kernel<WM, WN, TM, TN, false>;
+      if (parts) name = igemm_name<T, MODE, WM, WN, TM, TN, true>();
+    } else if (TM * TN == 1 && short_wgrad_ring(wgs, (a.k_per_split + 31) / 32))
       kernel = wgrad_direct_kernel<WM, WN, TM, TN, TM * TN == 1 ? kWgradShortRing : kWgradRing>(a);
     else
       kernel = wgrad_direct_kernel<WM, WN, TM, TN, kWgradRing>(a);
-    return launch(ctx, kernel, dim3(blocks), block, w, igemm_name<T, MODE, WM, WN, TM, TN>(), flops, 0, bytes);
-  } else
-    return launch(ctx, igemm_kernel<T, MODE, WM, WN, TM, TN>, grid, block, a, igemm_name<T, MODE, WM, WN, TM, TN>(),
-                  flops, 0, conv_bytes<MODE>(a, sizeof(T)));
+    return launch(ctx, kernel, dim3(blocks), block, w, name, flops, 0, bytes);
+  } else {
+    const char* name = igemm_name<T, MODE, WM, WN, TM, TN>();
+    const double bytes = conv_bytes<MODE>(a, sizeof(T));
+    if constexpr (parts_tile<T, MODE, BM, BN, 1>())
+      if (product_in_parts<MODE, BM, BN>(a, wgs * 4))
+        return launch(ctx, igemm_kernel<T, MODE, WM, WN, TM, TN, true>, grid, block, a, igemm_name<T, MODE, WM, WN, TM, TN, true>(), flops, 0, bytes);
+    return launch(ctx, igemm_kernel<T, MODE, WM, WN, TM, TN>, grid, block, a, name, flops, 0, bytes);
+  }
 }
 
 template <int MODE, int WM, int WN, int TM, int TN, int NBUF, int ROT = 0, int KS = kStep2>
@@ -2837,6 +2857,7 @@ int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
   static const std::string name = std::string("igemm4_kernel<") + (sizeof(T) == 2 ? "bf16," : "f32,") +
                                   (MODE == kFwd ? "fwd," : "dgrad,") + std::to_string(BM) + "x" + std::to_string(BN) + "," +
                                   std::to_string(KG) + "way," + std::to_string(NBUF) + "buf>";
+  static const std::string parts_name = name.substr(0, name.size() - 1) + ",parts>";
   a.tiles_m = (a.gemm_m + BM - 1) / BM;
   a.tiles_n = (a.gemm_n + BN - 1) / BN;
   const int64_t wgs = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
@@ -2847,8 +2868,12 @@ int launch_cfg4(Context* ctx, IgemmArgs& a, double flops) {
   // the larger operand is the one an XCD should fetch once
   a.group_rows = static_cast<int64_t>(a.gemm_n) * a.gemm_k > static_cast<int64_t>(a.a_bytes / sizeof(T)) ? 1 : 0;
   bind_divisions(a, a.group_rows ? a.tiles_m : a.tiles_n);
-  return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF, FS>, dim3(static_cast<unsigned>(wgs)), dim3(KG * 64), a, name.c_str(),
-                flops, 0, conv_bytes<MODE>(a, sizeof(T)));
+  const dim3 grid(static_cast<unsigned>(wgs)), block(KG * 64);
+  const double bytes = conv_bytes<MODE>(a, sizeof(T));
+  if constexpr (parts_tile<T, MODE, BM, BN, KG>())
+    if (product_in_parts<MODE, BM, BN>(a, wgs * KG))
+      return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF, FS, true>, grid, block, a, parts_name.c_str(), flops, 0, bytes);
+  return launch(ctx, igemm4_kernel<T, MODE, TM, TN, KG, NBUF, FS>, grid, block, a, name.c_str(), flops, 0, bytes);
 }
 
 // The 3x3 patch kernel: stride 1, pad 1, input channels in blocks of 64, rows short enough for the patch
@@ -3200,7 +3225,7 @@ const TileCost kSumsCost[] = {
     {kPatch64, 64, 64, 6.22f, 1.16f, 0.293f, 0.131f, 0.88f}, {kPatch64Deep, 64, 64, 5.70f, 2.80f, 0.066f, 0.155f, 0.80f},
     {kPatch128x64Deep, 128, 64, 5.98f, 3.45f, 0.170f, 0.194f, 1.03f}};
 // fp32 where the output has fewer than one and a half 128 x 128 tiles per compute unit: the reduction is split inside the
-// workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 takes at least six times the multiplies of bf16, so it
+// workgroup (igemm4_kernel), with smaller tiles as the grid shrinks.  fp32 takes at least eight times the multiplies of bf16, so it
 // gains from spreading them over every SIMD (784 x 256 over 2304: 77.6 -> 14.8 us, with fp32 multiplies).  -1: none of them.
 // The lines, with mean times over the layers of the three models in each class (244 launches, fp32 multiplies), the choice = 1:
 //   up to one 32 x 32 tile per CU, K >= 1024 (53): eight wavefronts; four 1.11.  K < 1024 (25): four; eight 1.01
@@ -3510,8 +3535,8 @@ int64_t conv2d_wgrad_workspace_bytes(const ConvShape& s, int dtype, int splits) 
 }
 
 // tile of a weight gradient without a tiling from the caller: 128 x 128 where it leaves at least 128 workgroups, in fp32 1024
-// (TCH_WGRAD_BIG_TILE_WGS: another count).  An fp32 gradient takes its operands apart for six multiplies: 144 workgroups of 128 x 128 use
-// those of 144 compute units, and their 52 KB of LDS (64 x 64: 28) keep main-lane workgroups away.  In the step (fp32 multiplies), from 128 /
+// (TCH_WGRAD_BIG_TILE_WGS: another count).  An fp32 gradient is bound by the matrix pipes: 144 workgroups of 128 x 128 use
+// those of 144 compute units, and their 40 KB of LDS (64 x 64: 24; in parts 52 and 28) keep main-lane workgroups away.  In the step (fp32 multiplies), from 128 /
 // 256 / 512 / 1024 / 2000 on / never: GPT-2 2 x 256 6.48 / 6.39 / 6.22 / 6.22 / 6.19 / 6.25 ms, 1 x 512 7.34 / 6.98 / 6.88 / 6.88 /
 // 6.86 / 6.89, 8 x 512 31.48 / 31.50 / 31.56 / 31.50 / 31.94 / 31.88.
 bool wgrad_big_tile(int dtype, int gemm_m, int gemm_n, int64_t splits) {

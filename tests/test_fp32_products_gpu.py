@@ -5,6 +5,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 TILINGS = [-1, 0, 1, 2, 15, 16, 17, 18, 19, 20]
+# The second is multiplied in parts by every kernel that can (the first by none): ragged for every tile, more than 256 tiles of
+# 128 x 128, eight reduction steps and a remainder for each of eight wavefronts.
+SIZES = [(68, 72, 272), (2100, 2084, 1040)]
+sizes = pytest.mark.parametrize("rows,cols,depth", SIZES)
 
 
 def product(op, rows, cols, depth, tile_cfg, a, b):
@@ -25,9 +29,15 @@ def product(op, rows, cols, depth, tile_cfg, a, b):
     return y.view(rows, cols)
 
 
+def against_64_bits(op, rows, cols, depth, tile_cfg, a, b):
+    """the product, what it is in 64 bits, and the sum of the sizes of its terms"""
+    a64, b64 = a.double(), b.double()
+    return product(op, rows, cols, depth, tile_cfg, a, b).double(), a64 @ b64.t(), a64.abs() @ b64.abs().t()
+
+
 # depths on both sides of the line, with and without a remainder for the steps, the wavefronts and the LDS tiles
 CASES = [(op, rows, cols, depth) for op in ("fwd", "dgrad", "wgrad")
-         for rows, cols, depth in ((36, 40, 128), (36, 40, 144), (132, 200, 272), (64, 64, 1024), (260, 132, 656))]
+         for rows, cols, depth in ((36, 40, 128), (36, 40, 144), (132, 200, 272), (64, 64, 1024), (260, 132, 656), (2100, 2084, 272), (2100, 2084, 1040))]
 
 
 @pytest.mark.parametrize("tile_cfg", TILINGS)
@@ -38,8 +48,7 @@ def test_error_is_that_of_fp32(op, rows, cols, depth, tile_cfg):
     g = torch.Generator().manual_seed(depth + rows)
     a = torch.randn(rows, depth, generator=g).mul_(torch.exp(2 * torch.randn(rows, depth, generator=g)))
     b = torch.randn(cols, depth, generator=g)
-    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).double().cpu()
-    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    got, want, size = against_64_bits(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda())
     assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
     # and over the whole result what sums of independent roundings have, not what the bound above allows
     assert (got - want).norm() <= 4 * 2.0 ** -24 * max(1, depth / 64) ** 0.5 * want.norm()
@@ -73,84 +82,83 @@ PAIRS = [("normal", "normal"), ("relu", "normal"), ("uniform", "uniform"), ("wid
          ("tiny", "large")]
 
 
-@pytest.mark.parametrize("depth", [144, 656])
+@sizes
 @pytest.mark.parametrize("first,second", PAIRS)
-def test_error_is_no_larger_than_with_fp32_multiplies(first, second, depth):
+def test_error_is_no_larger_than_with_fp32_multiplies(first, second, rows, cols, depth):
     """Against 64 bits, over a whole result, next to fp32 multiplies in the same order; every value counts by the sum of |a b|.  What is
     left out of a product and what the small products' sum rounds is 2^-5 of a unit in the last place where one product is all of a
     sum (test_single_products_are_rounded_once), against a rounding of 0.29 units: 0.6 % more; elsewhere parts round less often.
-    The allowance of 3 % is that and what two sets of 34 320 roundings differ by (1 %)."""
+    The allowance of 3 % is that and what two sets of 4896 roundings differ by (2 %)."""
     g = torch.Generator("cuda").manual_seed(depth)
-    a, b = DISTRIBUTIONS[first]((260, depth), g), DISTRIBUTIONS[second]((132, depth), g)
+    a, b = DISTRIBUTIONS[first]((rows, depth), g), DISTRIBUTIONS[second]((cols, depth), g)
     want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     error = lambda y: ((y.double() - want) / size).norm().item()
     off = {groups: error(fp32_multiplies(a, b, groups)) for groups in (1, 4, 8)}
     for op in ("fwd", "dgrad", "wgrad"):
         for tile_cfg in (0, 2) if op == "wgrad" else GROUPS:
             groups = 1 if op == "wgrad" else GROUPS[tile_cfg]
-            ratio = error(product(op, 260, 132, depth, tile_cfg, a, b)) / off[groups]
+            ratio = error(product(op, rows, cols, depth, tile_cfg, a, b)) / off[groups]
             print(f"{first} x {second} over {depth}, {op} tiling {tile_cfg}: {ratio:.3f}")
             assert ratio <= 1.03, (op, tile_cfg, ratio)
             if tile_cfg == 2 and op != "wgrad":   # fp32 multiplies: the reference is what they give
                 assert ratio >= 0.97, (op, ratio)
 
 
+@sizes
 @pytest.mark.parametrize("tile_cfg", TILINGS)
 @pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
-def test_single_products_are_rounded_once(op, tile_cfg):
+def test_single_products_are_rounded_once(op, tile_cfg, rows, cols, depth):
     """Sums of one product and zeros: half a unit in the last place, as a product in fp32, and 2^-5 of a unit.  With both values in
     [1, 2) the second parts are below 2^-7 and the third below 2^-15: x2 y2, which is left out, is below 2^-30; the small products' sum
     is below 2^-5, so that each of the three additions that can round there does by 2^-30 at most.  A unit is at least 2^-23."""
     g = torch.Generator("cuda").manual_seed(4)
-    rows, cols, depth = 260, 132, 144
     a, b = torch.zeros(rows, depth, device="cuda"), torch.randn(cols, depth, device="cuda", generator=g)
     a[torch.arange(rows), torch.arange(rows) % depth] = torch.randn(rows, device="cuda", generator=g)
-    got, want = product(op, rows, cols, depth, tile_cfg, a, b).double(), a.double() @ b.double().t()
+    got, want, _ = against_64_bits(op, rows, cols, depth, tile_cfg, a, b)
     unit = torch.exp2(torch.floor(torch.log2(want.abs())) - 23)
     assert ((got - want).abs() <= (0.5 + 2.0 ** -5) * unit).all()
 
 
+@sizes
 @pytest.mark.parametrize("tile_cfg", TILINGS)
 @pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
 @pytest.mark.parametrize("first,second", [(-112, 0), (0, -112), (-126, 100), (-70, -40), (-60, -60), (104, 0), (50, 50)])
-def test_values_of_any_size_keep_their_bits(first, second, op, tile_cfg):
-    """Operands and results down to the smallest normal values and beyond what the parts hold: the bound of test_error_is_that_of_fp32, and for results the
-    grid of the denormals, 2^-149, that the additions of a denormal sum round to."""
-    rows, cols, depth = 68, 72, 272
+def test_values_of_any_size_keep_their_bits(first, second, op, tile_cfg, rows, cols, depth):
+    """Operands and results down to the smallest normal values and beyond what the parts hold: the bound of
+    test_error_is_that_of_fp32, and for results the grid of the denormals, 2^-149, that the additions of a denormal sum round to."""
     g = torch.Generator().manual_seed(-first)
     a = (1 + torch.rand(rows, depth, generator=g)) * 2.0 ** first
     b = (1 + torch.rand(cols, depth, generator=g)) * 2.0 ** second * (1 - 2 * torch.randint(0, 2, (cols, depth), generator=g))
-    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).double().cpu()
-    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    got, want, size = against_64_bits(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda())
     assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size + depth * 2.0 ** -150).all()
 
 
+@sizes
 @pytest.mark.parametrize("tile_cfg", TILINGS)
 @pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
-def test_infinities_nan_and_the_largest_values(op, tile_cfg):
-    rows, cols, depth = 68, 72, 272
+def test_infinities_nan_and_the_largest_values(op, tile_cfg, rows, cols, depth):
     g = torch.Generator().manual_seed(1)
     a, b = torch.randn(rows, depth, generator=g), torch.randn(cols, depth, generator=g)
     inf, largest = float("inf"), torch.finfo(torch.float32).max
     a[3, 17], a[9, 200], a[33, 5], a[40, 271] = inf, float("nan"), largest, -largest
     a[50, 3], a[50, 100] = inf, -inf
     b[20, 17], b[21, 5], b[:, 271] = 0.0, 0.5, b[:, 271].clamp(-0.9, 0.9)
-    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).cpu()
-    want = a.double() @ b.double().t()
+    a, b = a.cuda(), b.cuda()
+    got, want, _ = against_64_bits(op, rows, cols, depth, tile_cfg, a, b)
     want = torch.where(want.abs() > largest, torch.sign(want) * inf, want)
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
-    assert torch.equal(got[got.isinf()].double(), want[want.isinf()])
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
     ok = want.isfinite()
     size = (torch.where(a.isfinite(), a, 0).double().abs() @ b.double().abs().t())[ok]
-    assert ((got.double() - want)[ok].abs() <= (depth + 2) * 2.0 ** -24 * size).all()
+    assert ((got - want)[ok].abs() <= (depth + 2) * 2.0 ** -24 * size).all()
 
 
+@sizes
 @pytest.mark.parametrize("tile_cfg", TILINGS)
 @pytest.mark.parametrize("op", ["fwd", "dgrad", "wgrad"])
-def test_results_next_to_the_largest_value_are_finite(op, tile_cfg):
+def test_results_next_to_the_largest_value_are_finite(op, tile_cfg, rows, cols, depth):
     """The first part of a value may be larger than the value.  Products of first parts, and sums of such products, overflow then
     where the result does not: 1.999 * 2^127, and 253 times 1.0040^2 * 2^120 (0.996 * 2^128; 1.0078^2 in first parts)."""
-    rows, cols, depth = 68, 72, 272
     g = torch.Generator().manual_seed(2)
     a, b = torch.randn(rows, depth, generator=g), torch.randn(cols, depth, generator=g)
     for row, col, sign in ((5, 7, 1.0), (40, 50, -1.0)):
@@ -159,8 +167,7 @@ def test_results_next_to_the_largest_value_are_finite(op, tile_cfg):
         a[row, :253], b[col, :253] = sign * 1.0040 * 2.0 ** 62, 1.0040 * 2.0 ** 58
         a[row, 17] = b[col, 17] = 0.0     # leaves the others' large values alone
         a[row, 253], b[col, 253] = a[row, 0], b[col, 0]
-    got = product(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda()).double().cpu()
-    want, size = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    got, want, size = against_64_bits(op, rows, cols, depth, tile_cfg, a.cuda(), b.cuda())
     assert want.abs().max() < torch.finfo(torch.float32).max and (want.abs() > 2.0 ** 127).sum() >= 4
     assert ((got - want).abs() <= (depth + 2) * 2.0 ** -24 * size).all()
 
@@ -169,7 +176,7 @@ def test_results_next_to_the_largest_value_are_finite(op, tile_cfg):
 def test_in_order_rows_are_the_same_bits_at_every_number_of_rows(op):
     """tile_cfg = IN_ORDER: 64 x 64 tiles, which multiply in fp32 anyway, up to 384 tiles of 128 x 64; those; and 128 x 128."""
     from sirius_amd import ops
-    cols, depth = 128, 144
+    cols, depth = 128, 272
     g = torch.Generator("cuda").manual_seed(3)
     a, b = (torch.randn(n, depth, device="cuda", generator=g) for n in (49280, cols))
     first, *others = [product(op, rows, cols, depth, ops.IN_ORDER, a[:rows], b)[:66] for rows in (66, 24700, 49280)]

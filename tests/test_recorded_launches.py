@@ -227,6 +227,38 @@ def test_fp32_choice_on_both_sides_of_its_lines(rec, rows, cols, depth, want):
     assert product(rec, F32, rows, cols, depth, -2).startswith("igemm_kernel<f32,fwd,")
 
 
+# rows, output columns, reduction, tiling and whether a forward product and a data gradient multiply in bf16 parts: both sides of
+# every line of that choice
+F32_PARTS = [
+    (257, 1024, 512, "32x32,4way", False, False), (132, 1024, 1024, "32x32,8way", True, False), (128, 1024, 1024, "32x32,8way", False, False),
+    (513, 1024, 768, "64x64,8way", True, True), (1025, 1024, 16368, "64x32,4way", True, False), (1025, 1024, 16384, "64x32,4way", False, False),
+    (257, 1024, 1536, "64x32,8way", True, False), (1025, 1024, 256, "64x64,4way", True, True), (784, 1024, 256, "64x64,4way", False, False),
+    (6017, 1024, 256, "128x128", True, True), (6017, 1024, 240, "128x128", False, False),
+]
+
+
+@pytest.mark.parametrize("rows,cols,depth,tiling,parts,dgrad_parts", F32_PARTS)
+def test_fp32_products_in_parts(rec, rows, cols, depth, tiling, parts, dgrad_parts):
+    name = product(rec, F32, rows, cols, depth, -1)
+    assert tiling in name and name.endswith(",parts>") == parts, name
+    assert "parts" not in product(rec, F32, rows, cols, depth, -2)
+    rec.begin()
+    check(lib().tch_conv2d_dgrad(rec.ctx, F32, address(0), address(1), address(2), None, None, rows, 1, 1, cols, depth, 1, 1, 1, 0, -1, 0, 1))
+    check(lib().tch_conv2d_dgrad(rec.ctx, F32, address(0), address(1), address(2), None, None, rows, 1, 1, cols, depth, 1, 1, 1, 0, -2, 0, 1))
+    check(lib().tch_conv2d_fwd_bnstats(rec.ctx, F32, address(0), address(1), address(2), rows, 1, 1, depth, cols, 1, 1, 1, 0, -1, 0, address(3)))
+    names = [r[0] for r in rec.end()]
+    assert [n.endswith(",parts>") for n in names] == [dgrad_parts, False, False], names
+
+
+@pytest.mark.parametrize("pixels,cols,tiling,parts", [(65, 1040, 2, True), (64, 1040, 2, False), (65, 1024, 2, False), (65, 2112, 0, True)])
+def test_fp32_weight_gradients_in_parts(rec, pixels, cols, tiling, parts):
+    rows = 2048 if tiling == 0 else 1024
+    rec.begin()
+    check(lib().tch_conv2d_wgrad(rec.ctx, F32, address(0), address(1), address(2), None, 1, 0, pixels, 1, 1, cols, rows, 1, 1, 1, 0, tiling, 0))
+    (name, _, _), = rec.end()
+    assert name.endswith(",parts>") == parts, name
+
+
 def test_bf16_choice_for_large_products_and_in_order(rec):
     """From 384 tiles of 128 x 128 on a plain product takes no smaller one; with one order of additions asked for neither a
     split tiling nor the 3x3 patch kernel runs."""
