@@ -3195,9 +3195,12 @@ int pick_tile(int dtype, int gemm_m, int gemm_n, int gemm_k) {
 // 556 different convolutions where they stand in a step or request, one launch at a time (operands as cold or warm as their
 // producers leave them; 3 us of event among it), each with every tiling: ResNet-152 at 1-64 images, GPT-2 at 512-8192
 // tokens, Swin-B at 3-32 images; the second table for ResNet's data gradients with the BatchNorm sums, whose epilogue
-// reads two more tensors.  (kSplit16: two points of requests of one image, 208 and 832 workgroups, see igemm4_kernel.  The patch tilings, 5 and 28-31, were fitted in the same way to ResNet-152's 3x3 convolutions alone:
-// one round of workgroups is fastest with nine filter tiles, several with three, of which two workgroups fit on a CU.)  (Fits to launches repeated on warm operands prefer large tiles: a request of 24 images took
-// 2437 us with them, 2098 with these.)  Against the fastest of all tilings per launch, summed over a step or request: 1-2 %, one image 3.
+// reads two more tensors.  (The patch tilings, 5 and 28-31, were fitted in the same way to ResNet-152's 3x3 convolutions alone: one
+// round of workgroups is fastest with nine filter tiles, several with three, of which two workgroups fit on a CU.  kSplit16: two points
+// of requests of one image, 208 and 832 workgroups.  The 302 products of 7-512 rows for which it is the choice from these prices, kernel
+// times on filters that four launches in turn have read, as shares of the fastest of kSplit32, kSplit32Deep and kSplit64x32, forward / data
+// gradient: over 1024 and more 0.85 / 0.86, 768 0.92 / 0.94, 512 0.94 / 0.98, 256 0.97 / 1.01, 128 0.99 / 1.05: from 256 on.)  (Fits to
+// launches repeated on warm operands prefer large tiles: a request of 24 images took 2437 us with them, 2098 with these.)  Against the fastest of all tilings per launch, summed over a step or request: 1-2 %, one image 3.
 // Tilings without an entry (3, 6, 7, 11, kSplit64, kSplit64Pair, kSplit64x32Deep: for callers that ask, and for tuners) are
 // the fastest on some launches, by 1 % on average and 9 % at most.
 struct TileCost {
@@ -3321,7 +3324,7 @@ int heuristic_tile(int asked, const TileQuery& q) {
     if (t.cfg >= 12 && t.cfg <= 14 && !short_steps()) continue;
     if (patch_tile(t.cfg) && (!q.patch || asked == kAutoInOrder)) continue;
     if (t.bm * t.bn <= 64 * 32 && asked == kAutoInOrder) continue;   // igemm4_kernel's
-    if (t.bm < 32 && q.counted) continue;
+    if (t.bm < 32 && (q.counted || q.gemm_k < 256)) continue;   // less than a reduction step for each of eight wavefronts
     take(t);
   }
   // Data gradients run beside weight gradients, whose LDS has no room on a compute unit that igemm5_kernel holds; from about 2560

@@ -259,6 +259,12 @@ def test_fp32_weight_gradients_in_parts(rec, pixels, cols, tiling, parts):
     assert name.endswith(",parts>") == parts, name
 
 
+def test_bf16_choice_of_16x16_tiles(rec):
+    """Up to a workgroup on every compute unit, and from a reduction step for each of the eight wavefronts on."""
+    assert "16x16,8way" in product(rec, BF16, 98, 256, 256, -1) and "16x16" not in product(rec, BF16, 98, 256, 192, -1)
+    assert "16x16,8way" in product(rec, BF16, 256, 256, 512, -1) and "16x16" not in product(rec, BF16, 272, 256, 512, -1)
+
+
 def test_bf16_choice_for_large_products_and_in_order(rec):
     """From 384 tiles of 128 x 128 on a plain product takes no smaller one; with one order of additions asked for neither a
     split tiling nor the 3x3 patch kernel runs."""
