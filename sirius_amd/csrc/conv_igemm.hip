@@ -3026,8 +3026,12 @@ int launch_mode(Context* ctx, IgemmArgs& a, int tile_cfg, double flops) {
   static_assert(MODE == kFwd || MODE == kDgrad, "weight gradients go through launch_wgrad");
   switch (tile_cfg) {
     case kSplit16:
-      if constexpr (sizeof(T) == 2) return launch_cfg4<T, MODE, 1, 1, 8, 4, 16>(ctx, a, flops);
-      return launch_cfg4<T, MODE, 1, 1, 8, 2>(ctx, a, flops);   // not reached: effective_tile
+      if constexpr (sizeof(T) == 2) {
+        return launch_cfg4<T, MODE, 1, 1, 8, 4, 16>(ctx, a, flops);
+      } else {   // effective_tile() gives fp32 kSplit32Deep, whose row tiles are others
+        set_error("igemm: 16 x 16 tiles are for bf16");
+        return -22;
+      }
     case kSplit32:
       return launch_cfg4<T, MODE, 1, 1, 4, 4>(ctx, a, flops);
     case kSplit32Deep:
