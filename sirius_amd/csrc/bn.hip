@@ -645,7 +645,7 @@ __global__ __launch_bounds__(256) void bn_acc_apply_kernel(AccApplyArgs p) {
     const int c = c0 + tid;
     double s, q;
     acc_totals(p.acc, p.C, p.acc_copies, c, &s, &q);
-      const bool writer = blockIdx.y == 0;
+    const bool writer = blockIdx.y == 0;
     if (!BWD) {
       const double mean = s / static_cast<double>(p.rows.n);
       double var = q / static_cast<double>(p.rows.n) - mean * mean;

@@ -552,8 +552,10 @@ __device__ inline void finish_walk(const IgemmArgs& p, EpilogueOperands<T, MODE,
 
 // The form for accumulators spread over the wavefronts of a tile, one 32-row band at a time.  EARLY: the operands are
 // requested when the kernel starts and wait in registers until the accumulators are done (the kernels that can spare the
-// registers), instead of costing a trip to memory behind the last multiply.  They leave behind the first operand tiles: the counted waits
-// of the loop then wait for no operand of the epilogue, which may come from further away.
+// registers), instead of costing a trip to memory behind the last multiply.  They leave behind the requests of the first operand tiles, which
+// then wait for nothing of the epilogue's.  The loop's counted waits do not know of them: requests land in order, so a wait for a
+// tile requested behind them waits for them as well, and the first wait, which leaves a fixed number outstanding, for
+// as many more operand loads as there are such requests.
 template <typename T, int MODE, int WM, int WN, int TM, int TN, bool EARLY>
 struct TileEpilogue {
   static constexpr int BN = WN * TN * 32, NT = WM * WN * 64, CH = BN / Elem<T>::kPerChunk;
