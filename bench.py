@@ -32,10 +32,10 @@ HANDOVER_PAGE_MB = 128
 # do not depend on the choice of tilings; another kernel at the top of the step has no figure.
 PROFILE_FILE = "profiles/resnet152_bf16_bs64_step_kernel_stats_and_traffic.txt"
 MEASURED_TRAFFIC_MIB = {
-    "wgrad_kernel<bf16,64x64>": 64.44 + 5.60,
-    "wgrad_kernel<bf16,128x128>": 34.38 + 17.23,
+    "wgrad_kernel<bf16,64x64>": 63.91 + 5.42,
+    "wgrad_kernel<bf16,128x128>": 35.27 + 16.06,
     "bn_fin_apply_kernel<bf16,bwd>": 24.37 + 11.91,
-    "bn_fin_apply_kernel<bf16,fwd>": 20.39 + 12.03,
+    "bn_fin_apply_kernel<bf16,fwd>": 20.38 + 12.03,
 }
 
 

@@ -155,8 +155,9 @@ int tch_context_get_cu_limit(tch_context* ctx);
  * out_f32 != 0 stores y as fp32 whatever dtype is.  tile_cfg: -1 auto: the choice, and with it the order a reduction is
  * added up in, follows the number of rows, so a sample's result may differ in rounding with the samples batched beside it
  * (bf16 ResNet-152 logits by about 2e-3).  -2 auto among the tilings that add up a reduction front to back (a row's result
- * does not depend on the number of rows).  -3 and -4: the same two for the linear layers of a transformer, which leave the
- * choice the persistent kernel as well (25 - 27; front to back).  0 = 128x128, 1 = 128x64, 2 = 64x64,
+ * does not depend on the number of rows; fp32 is multiplied in fp32, which otherwise may go through the bf16 matrix pipes in parts
+ * that hold every bit: no less exact, but rounded elsewhere).  -3 and -4: the same two for the linear layers of a transformer, which
+ * leave the choice the persistent kernel as well (25 - 27; front to back).  0 = 128x128, 1 = 128x64, 2 = 64x64,
  * 3 = 64x64 on the register-staged kernel even where the direct-to-LDS kernel applies, 5 = 128x64 with the
  * activation side of all nine taps of a channel block held in LDS as one patch (bf16, 3x3, stride 1, pad 1,
  * channels a multiple of 64, rows of at most 63 pixels; any other convolution runs tiling 1 for it).  The patch
