@@ -181,3 +181,42 @@ def test_in_order_rows_are_the_same_bits_at_every_number_of_rows(op):
     a, b = (torch.randn(n, depth, device="cuda", generator=g) for n in (49280, cols))
     first, *others = [product(op, rows, cols, depth, ops.IN_ORDER, a[:rows], b)[:66] for rows in (66, 24700, 49280)]
     assert all(torch.equal(first, o) for o in others)
+
+
+@pytest.mark.parametrize("stride", [1, 2])
+def test_convolutions_in_parts(stride):
+    """3x3 layers with ragged edges on more than 256 tiles, where taps leave the image, the weight gradient with its reduction split,
+    added to what is there and with the bias gradient.  Per value as in test_error_is_that_of_fp32."""
+    from sirius_amd import ops
+    ctx = ops.Context()
+    g = torch.Generator("cuda").manual_seed(stride)
+    n, side, c, k = 17 * stride * stride, 45, 80, 112
+    out = ops.conv_out_hw(side, side, 3, 3, stride, 1)[0]
+    x, w, dy = (torch.randn(*shape, device="cuda", generator=g) for shape in ((n, side, side, c), (k, 3, 3, c), (n, out, out, k)))
+
+    def in_64_bits(x, w, dy):
+        x = x.double().permute(0, 3, 1, 2).requires_grad_(True)
+        w = w.double().permute(0, 3, 1, 2).requires_grad_(True)
+        y = torch.nn.functional.unfold(x, 3, padding=1, stride=stride).transpose(1, 2).reshape(-1, 9 * c) @ w.reshape(k, -1).t()
+        dx, dw = torch.autograd.grad(y, (x, w), dy.double().reshape(-1, k))
+        return y.detach().view(dy.shape), dx.permute(0, 2, 3, 1), dw.permute(0, 2, 3, 1)
+
+    want, size = in_64_bits(x, w, dy), in_64_bits(x.abs(), w.abs(), dy.abs())
+    near = lambda got, i, depth: bool(((got.double() - want[i]).abs() <= (depth + 2) * 2.0 ** -24 * size[i]).all())
+    y, dx = torch.empty_like(dy), torch.empty_like(x)
+    for tile_cfg in (0, 1, 16, 17, 18, 19, 20):
+        y.fill_(float("nan"))
+        ops.conv2d_fwd(ctx, x, w, y, stride, 1, tile_cfg=tile_cfg)
+        assert near(y, 0, 9 * c), tile_cfg
+    for tile_cfg in (0, 1, 18, 19):
+        dx.fill_(float("nan"))
+        ops.conv2d_dgrad(ctx, dy, w.permute(3, 1, 2, 0).contiguous(), dx, stride, 1, tile_cfg=tile_cfg)
+        assert near(dx, 1, 9 * k), tile_cfg
+    pixels, splits = n * out * out, 60
+    workspace = torch.empty(ops.conv2d_wgrad_workspace_bytes(0, k, 3, 3, c, splits) // 4, device="cuda")
+    for tile_cfg in (0, 1, 2):
+        dw, dbias = torch.ones_like(w), torch.ones(k, device="cuda")
+        ops.conv2d_wgrad(ctx, x, dy, dw, stride, 1, workspace=workspace, splits=splits, accumulate=True, tile_cfg=tile_cfg, dbias=dbias)
+        assert near(dw.double() - 1, 2, pixels), tile_cfg
+        sums, sizes = dy.double().sum((0, 1, 2)), dy.double().abs().sum((0, 1, 2))
+        assert ((dbias.double() - 1 - sums).abs() <= pixels * 2.0 ** -24 * sizes).all()
